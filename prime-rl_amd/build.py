@@ -11,7 +11,8 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libmoe_i8.so"
-SOURCES = ["align.hip", "quant.hip", "sum.hip", "router.hip", "gemm_stream.hip", "gemm_tile.hip", "gemm_narrow.hip", "api.hip"]
+SOURCES = ["align.hip", "quant.hip", "sum.hip", "router.hip", "gemm_stream.hip", "gemm_tile.hip", "gemm_narrow.hip", "gemm_dense.hip",
+           "api.hip"]
 PROBE_LIB_PATH = PKG_DIR / "libmoe_i8_probe.so"  # the benchmark's MFMA rate probe, a library of its own
 
 # packed-fp32 VALU ops are switched off for all device code (hipcc's host pass warns that it does

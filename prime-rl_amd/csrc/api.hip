@@ -728,7 +728,8 @@ int moe_i8_fused_experts_static(const void* hidden, const int8_t* w1, const int8
                               stream);
 }
 
-// Workspace of the dense entry points (every region 256-byte aligned):
+// Workspace of the dense entry points (every region 256-byte aligned; int8 rows are padded to a multiple
+// of 128 bytes):
 //   x_q i8[M*K] | a1 f32[M] | sorted i32[cap] | expert_ids i32[cap/64] | npp i32[1] |
 //   (mlp only) act bf16[M*I] | act_q i8[M*I] | a2 f32[M]
 namespace {
@@ -746,30 +747,60 @@ DenseCarve dense_carve(int64_t m, int k, int inter) {
     off = align_up(off + bytes, 256);
     return at;
   };
-  c.x_q = take(m * k);
+  c.x_q = take(m * moe_i8::dense_row_stride(k));
   c.a1 = take(m * 4);
   c.sorted = take(c.cap * 4);
   c.eids = take((c.cap + kDenseBlock - 1) / kDenseBlock * 4);
   c.npp = take(4);
   if (inter > 0) {
     c.act = take(m * inter * 2);
-    c.act_q = take(m * inter);
+    c.act_q = take(m * moe_i8::dense_row_stride(inter));
     c.a2 = take(m * 4);
   }
   c.total = off;
   return c;
 }
 
-int dense_prologue(const void* x, int64_t m, int k, void* workspace, int64_t workspace_bytes,
-                   const DenseCarve& c, void* stream) {
-  if (m > INT32_MAX - kDenseBlock) return fail(MOE_I8_EINVAL, "too many rows");
-  if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(MOE_I8_EINVAL, "workspace must be 256-byte aligned");
-  if (workspace_bytes < c.total)
-    return fail(MOE_I8_EWORKSPACE, "workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)c.total);
-  char* ws = static_cast<char*>(workspace);
-  // one launch: the ties-to-even row quantiser, whose threads also write the identity routing
-  if (k < 8 || k % 8) return fail(MOE_I8_EINVAL, "k (%d) must be a positive multiple of 8", k);
-  if (!aligned16(x)) return fail(MOE_I8_EINVAL, "x must be 16-byte aligned");
+// A dense problem as the grouped families see it: one expert that every row visits.
+moe_i8::GemmArgs dense_group(int mode, const DenseCarve& c, char* ws, const int8_t* a_q, const float* a_scale,
+                             const int8_t* w, const float* w_scale, void* out, int64_t m, int n, int k) {
+  const int32_t* sorted = reinterpret_cast<int32_t*>(ws + c.sorted);
+  const int32_t* eids = reinterpret_cast<int32_t*>(ws + c.eids);
+  const int32_t* npp = reinterpret_cast<int32_t*>(ws + c.npp);
+  moe_i8::GemmArgs g = mode == moe_i8::kGateUpSilu
+                           ? gate_up_args(a_q, a_scale, w, w_scale, sorted, eids, npp, m, 1, 1, k, n / 2, kDenseBlock, c.cap, out)
+                           : down_args(a_q, a_scale, w, w_scale, nullptr, sorted, eids, npp, m, 1, n, k, kDenseBlock, c.cap, out);
+  g.expert_ids_ascend = true;  // one expert
+  return g;
+}
+
+// Whether one GEMM of a dense entry point runs on the dense kernel (which needs no routing arrays): unless
+// a family is demanded or the 256-row tiles of the LDS-tiled family are expected to be faster.
+bool takes_dense_kernel(moe_i8::GemmArgs g, int variant) {
+  if (variant != MOE_I8_GEMM_AUTO) return false;
+  g.tile_geometry = moe_i8::kTileWide;
+  return moe_i8::gemm_dense_takes(g.num_pairs, g.n, g.k, moe_i8::gemm_tile_supports(g));
+}
+
+int run_dense(const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
+  if (int rc = check_gemm_common(g.a_q, g.w, g.sorted_token_ids, g.expert_ids, g.num_tokens_post_padded, g.out, g.num_pairs,
+                                 1, g.n, g.k, g.block_size, g.sorted_cap, variant))
+    return rc;
+  if (!aligned16(g.w_scale)) return fail(MOE_I8_EINVAL, "weight scales must be 16-byte aligned");
+  if (takes_dense_kernel(g, variant)) {
+    const moe_i8::DenseArgs d{g.mode, g.a_q, g.a_scale, g.w, g.w_scale, g.out, g.num_pairs, g.n, g.k};
+    return check_launch(moe_i8::launch_gemm_dense(d, stream), "gemm_dense");
+  }
+  moe_i8::GemmArgs wide = g;
+  wide.tile_geometry = moe_i8::kTileWide;
+  if (variant == MOE_I8_GEMM_AUTO && moe_i8::gemm_tile_supports(wide)) variant = MOE_I8_GEMM_TILE_WIDE;
+  return run_gemm(g, variant, stream);
+}
+
+// The ties-to-even row quantiser of the dense path; `padded`: rows for the dense kernel; `route`: its
+// threads also write the identity routing the grouped families read (one launch less).
+int dense_quant(const void* x, int64_t m, int k, int8_t* q, float* scale, bool padded, bool route, const DenseCarve& c,
+                char* ws, hipStream_t stream) {
   moe_i8::QuantArgs a;
   a.x = static_cast<const uint16_t*>(x);
   a.src_rows = m;
@@ -778,15 +809,28 @@ int dense_prologue(const void* x, int64_t m, int k, void* workspace, int64_t wor
   a.gather = nullptr;
   a.gather_div = 1;
   a.rows = m;
-  a.q = reinterpret_cast<int8_t*>(ws + c.x_q);
-  a.scale = reinterpret_cast<float*>(ws + c.a1);
+  a.q = q;
+  a.scale = scale;
   a.round_even = 1;
-  a.route_sorted = reinterpret_cast<int32_t*>(ws + c.sorted);
-  a.route_expert_ids = reinterpret_cast<int32_t*>(ws + c.eids);
-  a.route_npp = reinterpret_cast<int32_t*>(ws + c.npp);
-  a.route_block = kDenseBlock;
-  a.route_cap = c.cap;
-  return check_launch(moe_i8::launch_quant_rows(a, static_cast<hipStream_t>(stream)), "quant_rows");
+  if (padded) a.q_stride = moe_i8::dense_row_stride(k);
+  if (route) {
+    a.route_sorted = reinterpret_cast<int32_t*>(ws + c.sorted);
+    a.route_expert_ids = reinterpret_cast<int32_t*>(ws + c.eids);
+    a.route_npp = reinterpret_cast<int32_t*>(ws + c.npp);
+    a.route_block = kDenseBlock;
+    a.route_cap = c.cap;
+  }
+  return check_launch(moe_i8::launch_quant_rows(a, stream), "quant_rows");
+}
+
+int check_dense(const void* x, int64_t m, int k, void* workspace, int64_t workspace_bytes, const DenseCarve& c) {
+  if (m > INT32_MAX - kDenseBlock) return fail(MOE_I8_EINVAL, "too many rows");
+  if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(MOE_I8_EINVAL, "workspace must be 256-byte aligned");
+  if (workspace_bytes < c.total)
+    return fail(MOE_I8_EWORKSPACE, "workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)c.total);
+  if (k < 8 || k % 8) return fail(MOE_I8_EINVAL, "k (%d) must be a positive multiple of 8", k);
+  if (!aligned16(x)) return fail(MOE_I8_EINVAL, "x must be 16-byte aligned");
+  return MOE_I8_OK;
 }
 }  // namespace
 
@@ -801,12 +845,15 @@ int moe_i8_w8a8_linear(const void* x, const int8_t* w, const float* w_scale, voi
   if (m == 0) return MOE_I8_OK;
   if (!x || !w || !w_scale || !out || !workspace) return fail(MOE_I8_EINVAL, "null pointer");
   const DenseCarve c = dense_carve(m, k, 0);
-  if (int rc = dense_prologue(x, m, k, workspace, workspace_bytes, c, stream)) return rc;
+  if (int rc = check_dense(x, m, k, workspace, workspace_bytes, c)) return rc;
   char* ws = static_cast<char*>(workspace);
-  return moe_i8_gemm_down(reinterpret_cast<int8_t*>(ws + c.x_q), reinterpret_cast<float*>(ws + c.a1), w, w_scale,
-                          nullptr, reinterpret_cast<int32_t*>(ws + c.sorted), reinterpret_cast<int32_t*>(ws + c.eids),
-                          reinterpret_cast<int32_t*>(ws + c.npp), m, 1, n, k, kDenseBlock, c.cap, out, variant,
-                          stream);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  int8_t* x_q = reinterpret_cast<int8_t*>(ws + c.x_q);
+  float* a1 = reinterpret_cast<float*>(ws + c.a1);
+  const moe_i8::GemmArgs g = dense_group(moe_i8::kDown, c, ws, x_q, a1, w, w_scale, out, m, n, k);
+  const bool dense = takes_dense_kernel(g, variant);
+  if (int rc = dense_quant(x, m, k, x_q, a1, dense, !dense, c, ws, s)) return rc;
+  return run_dense(g, variant, s);
 }
 
 int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, const int8_t* w2,
@@ -817,39 +864,33 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   if (!x || !w13 || !w13_scale || !w2 || !w2_scale || !out || !workspace) return fail(MOE_I8_EINVAL, "null pointer");
   if (inter < 64 || inter % 64) return fail(MOE_I8_EINVAL, "inter (%d) must be a positive multiple of 64", inter);
   const DenseCarve c = dense_carve(m, hidden, inter);
-  if (int rc = dense_prologue(x, m, hidden, workspace, workspace_bytes, c, stream)) return rc;
+  if (int rc = check_dense(x, m, hidden, workspace, workspace_bytes, c)) return rc;
   char* ws = static_cast<char*>(workspace);
+  hipStream_t s = static_cast<hipStream_t>(stream);
   int8_t* x_q = reinterpret_cast<int8_t*>(ws + c.x_q);
   float* a1 = reinterpret_cast<float*>(ws + c.a1);
-  int32_t* sorted = reinterpret_cast<int32_t*>(ws + c.sorted);
-  int32_t* eids = reinterpret_cast<int32_t*>(ws + c.eids);
-  int32_t* npp = reinterpret_cast<int32_t*>(ws + c.npp);
   int8_t* act_q = reinterpret_cast<int8_t*>(ws + c.act_q);
   float* a2 = reinterpret_cast<float*>(ws + c.a2);
-  if (int rc = moe_i8_gemm_gate_up_silu(x_q, a1, w13, w13_scale, sorted, eids, npp, m, 1, 1, hidden, inter,
-                                        kDenseBlock, c.cap, ws + c.act, variant, stream))
-    return rc;
-  // A few rows (decode): the streaming down GEMM quantises them itself (ties to even here), one
+  const moe_i8::GemmArgs gu = dense_group(moe_i8::kGateUpSilu, c, ws, x_q, a1, w13, w13_scale, ws + c.act, m, 2 * inter, hidden);
+  moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, ws, act_q, a2, w2, w2_scale, out, m, hidden, inter);
+  const bool dense_gu = takes_dense_kernel(gu, variant), dense_dg = takes_dense_kernel(dg, variant);
+  if (int rc = dense_quant(x, m, hidden, x_q, a1, dense_gu, !dense_gu || !dense_dg, c, ws, s)) return rc;
+  if (int rc = run_dense(gu, variant, s)) return rc;
+  // Few rows on the streaming family: its down GEMM quantises them itself (ties to even here), one
   // launch less.
-  moe_i8::GemmArgs dg = down_args(act_q, a2, w2, w2_scale, nullptr, sorted, eids, npp, m, 1, hidden, inter,
-                                  kDenseBlock, c.cap, out);
-  dg.expert_ids_ascend = true;
-  const int family = picks_family(dg, variant);
-  if (family < 0) return MOE_I8_EUNSUPPORTED;
-  if (family == MOE_I8_GEMM_STREAM && m <= kDenseSelfQuantRows && moe_i8::gemm_stream_fuses_quant(inter)) {
-    if (int rc = check_gemm_common(ws + c.act, w2, sorted, eids, npp, out, m, 1, hidden, inter, kDenseBlock, c.cap,
-                                   MOE_I8_GEMM_STREAM))
+  if (variant == MOE_I8_GEMM_STREAM && m <= kDenseSelfQuantRows && moe_i8::gemm_stream_fuses_quant(inter)) {
+    if (int rc = check_gemm_common(ws + c.act, w2, dg.sorted_token_ids, dg.expert_ids, dg.num_tokens_post_padded, out, m, 1,
+                                   hidden, inter, kDenseBlock, c.cap, MOE_I8_GEMM_STREAM))
       return rc;
     if (!aligned16(w2_scale)) return fail(MOE_I8_EINVAL, "w2_scale must be 16-byte aligned");
     dg.a_q = nullptr;
     dg.a_scale = nullptr;
     dg.a_bf16 = reinterpret_cast<const uint16_t*>(ws + c.act);
     dg.a_round_even = true;
-    return check_launch(moe_i8::launch_gemm_stream(dg, static_cast<hipStream_t>(stream)), "gemm_stream");
+    return check_launch(moe_i8::launch_gemm_stream(dg, s), "gemm_stream");
   }
-  if (int rc = moe_i8_scaled_int8_quant(ws + c.act, MOE_I8_DTYPE_BF16, m, inter, inter, act_q, a2, stream)) return rc;
-  return moe_i8_gemm_down(act_q, a2, w2, w2_scale, nullptr, sorted, eids, npp, m, 1, hidden, inter, kDenseBlock,
-                          c.cap, out, variant, stream);
+  if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, false, c, ws, s)) return rc;
+  return run_dense(dg, variant, s);
 }
 
 }  // extern "C"

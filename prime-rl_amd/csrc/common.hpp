@@ -157,6 +157,7 @@ struct QuantArgs {
   int64_t out_rows_per_group = 0;
   int64_t out_row_offset = 0;
   int round_even = 0;  // activations: ties to even instead of away from zero
+  int q_stride = 0;    // row quantiser only: bytes from one row of q to the next, zero-filled behind cols; 0 = cols
   // Row quantiser only: also write the routing of a dense layer seen as one expert that every row
   // visits (rows in order, padded to whole blocks with the sentinel, used blocks owned by expert
   // 0, the rest of both arrays marked unused) — one launch less in front of a dense GEMM.
@@ -237,6 +238,24 @@ bool gemm_tile_prefers_deep(const GemmArgs& a);
 int gemm_tile_geometry(const GemmArgs& a);  // kTileWide or kTileDeep (kTileRing on demand): what a launch of the family would use
 hipError_t launch_gemm_narrow(const GemmArgs& a, hipStream_t stream);
 bool gemm_narrow_supports(const GemmArgs& a);
+
+// One weight matrix that every row visits: out = epilogue(a_q[m, k] x w[n, k]^T).
+struct DenseArgs {
+  int mode;  // kGateUpSilu or kDown
+  const int8_t* a_q;  // rows of dense_row_stride(k) bytes, zero from k on
+  const float* a_scale;
+  const int8_t* w;
+  const float* w_scale;
+  void* out;
+  int64_t m;
+  int n;
+  int k;
+};
+int dense_row_stride(int k);
+// Whether the dense kernel is the one for this problem; `wide_allowed`: the 256-row tiles of the LDS-tiled
+// family can run it too and are preferred where they are expected to be faster.
+bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed);
+hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream);
 
 hipError_t launch_moe_sum(const uint16_t* in, uint16_t* out, int64_t m, int top_k, int hidden,
                           hipStream_t stream);

@@ -1,0 +1,396 @@
+// Dense int8 GEMM for gfx950: one weight matrix that every row visits (linear layers, shared experts).
+//
+// The grouped families cut such a problem into tiles of 128 or 256 channels, sized for a layer whose
+// experts fill the chip.  One matrix does not: 5 rows x 2816 channels were 22-44 workgroups on 256
+// compute units, each alone with the latency of its reduction.  Here the tile is chosen so that about
+// one workgroup per compute unit results, down to 16 rows x 16 channels, and inside a workgroup the
+// REDUCTION is split: its wavefronts form KS groups, group g multiplies the 128-byte pieces g, g + KS, ...
+// of every row through LDS stages of its own, and the int32 partial sums (exact in any order) meet in
+// LDS at the end.  With one wavefront per group no barrier is needed before that.  What bounds a
+// workgroup is the rate at which its operands arrive (about 50 bytes per clock and compute unit), so up
+// to 150 KB of loads stay in flight (S stages) and 128 bytes of every row are fetched at a time.
+//
+// Measured against the grouped families' choice on the same operands (us, rows x channels x reduction):
+// 5x2816x4096 23.9 -> 4.1, 64x4096x4096 30.2 -> 5.9, 333x4096x2048 30.5 -> 8.0, 1115x1792x1536 26.5 -> 7.4,
+// 8170x2384x3200 89.8 -> 74; from a few thousand rows and channels on the 256 x 256 tiles win again
+// (8192x8192x2048 154 against 139): see kConfigs.
+//
+// Loads go global -> LDS (16 bytes per lane, 8 rows x 128 bytes each) with the 16-byte chunk index
+// XOR-swizzled with the row, as in the grouped families.  They are issued a few at a time between the
+// multiplications of a step: all of them at its start hold up the wavefront until the address unit has
+// taken them (333x4096x2048 8.8 -> 8.0 us).  Activation rows are padded with zeros to a multiple of 128
+// bytes (the quantiser writes them), which lets a reduction of any multiple of 64 run on the same path.
+#include "common.hpp"
+
+namespace moe_i8 {
+namespace {
+
+constexpr int kStepBytes = 128;  // reduction bytes of a row per wave-group and step
+constexpr int kXcds = 8;
+
+struct DenseParams {
+  const int8_t* a_q;     // [M, lda], zero between K and lda
+  const float* a_scale;  // [M]
+  const int8_t* w;       // [N, K]
+  const float* w_scale;  // [N]
+  uint16_t* out;         // [M, N] (down) or [M, N / 2] (gate_up)
+  int M;
+  int N;
+  int K;
+  int lda;
+  int mtiles;
+  int ntiles;
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+}
+
+__device__ __forceinline__ uint64_t uniform_address(const void* base) {
+  const uint64_t b = reinterpret_cast<uint64_t>(base);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+  return (uint64_t)lo | ((uint64_t)hi << 32);
+}
+__device__ __forceinline__ void load_to_lds_16(const void* base, uint32_t offset, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(uniform_address(base))
+               : "memory", "m0");
+}
+// 4 bytes per lane from any address of the lane's own
+__device__ __forceinline__ void load_to_lds_4(const void* addr, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               :
+               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(reinterpret_cast<uint64_t>(addr))
+               : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)p);
+}
+__device__ __forceinline__ int swizzle_of_row(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+// Waits until at most n * kPer of this wavefront's vector-memory operations are pending, n <= kMost.
+template <int kPer, int kMost>
+__device__ __forceinline__ void wait_groups(int n) {
+  if constexpr (kMost == 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (n >= kMost)
+      wait_vmcnt<kPer * kMost>();
+    else
+      wait_groups<kPer, kMost - 1>(n);
+  }
+}
+
+template <int MF>
+struct Mfma;
+template <>
+struct Mfma<32> {
+  typedef v16i Acc;
+  static constexpr int kRegs = 16;
+  static constexpr int kSub = 4;  // MFMAs per 128 reduction bytes
+  static __device__ __forceinline__ Acc mul(v4i a, v4i b, Acc c) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Mfma<16> {
+  typedef v4i Acc;
+  static constexpr int kRegs = 4;
+  static constexpr int kSub = 2;
+  static __device__ __forceinline__ Acc mul(v4i a, v4i b, Acc c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
+};
+
+template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int WPE>
+__global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(DenseParams p) {
+  constexpr int G = WM * WN;                   // wavefronts of a group: they share the group's stages
+  constexpr int kThreads = 64 * KS * G;
+  constexpr int L = (TM + TN) / 8 / G;         // 1 KB loads per wavefront and step
+  static_assert((TM + TN) % (8 * G) == 0, "a group's loads divide evenly");
+  static_assert((S - 2) * L <= 63 && S >= 2, "counted waits");
+  constexpr int kGroupBytes = (TM + TN) * kStepBytes;
+  constexpr int kStage = KS * kGroupBytes;
+  constexpr int MT = TM / WM, NT = TN / WN;
+  constexpr int MF = MT % 32 == 0 && NT % 32 == 0 ? 32 : 16;
+  constexpr int MI = MT / MF, NI = NT / MF;
+  using F = Mfma<MF>;
+  constexpr int kPartRow = TN * 4 + 16;        // bytes of a token's row of partial sums
+  constexpr int kPart = TM * kPartRow;
+  constexpr int kLds = S * kStage > KS * kPart ? S * kStage : KS * kPart;
+  static_assert(kLds + 4 * (TM + TN) <= 160 * 1024, "LDS");
+  __shared__ __align__(16) char lds[kLds];
+  __shared__ __align__(16) float scales[(TM + TN + 63) / 64 * 64];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = wave / G, wg = wave % G;
+  const int wm = wg / WN, wn = wg % WN;
+
+  // tile of this workgroup: the workgroups of one XCD (id % 8) take neighbouring tiles, token tiles fastest
+  const int total = p.mtiles * p.ntiles;
+  const int per_xcd = (total + kXcds - 1) / kXcds;
+  const int tile = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+  if (tile >= total || (int)(blockIdx.x / kXcds) >= per_xcd) return;
+  constexpr int kBand = 8;  // token tiles that run together over all channel tiles
+  const int band = tile / (kBand * p.ntiles);
+  const int in_band = tile - band * kBand * p.ntiles;
+  const int band_m = p.mtiles - band * kBand < kBand ? p.mtiles - band * kBand : kBand;
+  const int m0 = (band * kBand + in_band % band_m) * TM;
+  const int nt = in_band / band_m;
+  const int inter = p.N / 2;
+
+  auto weight_row = [&](int r) {  // LDS weight row r of the tile -> row of w
+    if constexpr (MODE == kGateUpSilu) {
+      const int half = TN / 2;
+      const int ch = nt * half + (r < half ? r : r - half);
+      return (ch < inter ? ch : inter - 1) + (r < half ? 0 : inter);
+    } else {
+      const int n = nt * TN + r;
+      return n < p.N ? n : p.N - 1;
+    }
+  };
+
+  const uint32_t lds0 = lds_address(lds);
+  // scales of the tile's channels and rows, the first things in flight
+  for (int j0 = wave * 64; j0 < TM + TN; j0 += kThreads) {
+    const int j = j0 + lane < TM + TN ? j0 + lane : TM + TN - 1;
+    const int m = m0 + j - TN;
+    load_to_lds_4(j < TN ? p.w_scale + weight_row(j) : p.a_scale + (m < p.M ? m : p.M - 1), lds_address(scales + j0));
+  }
+
+  // ---- loads: 1 KB load i of this wavefront fills rows 8 * (wg * L + i) .. + 8 of its group's stage ----
+  uint32_t off[L];
+  bool hi[L];  // weight chunk in the upper 64 bytes of the step
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int rb = wg * L + i;
+    const int r = rb * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ swizzle_of_row(r);
+    if (rb * 8 < TN) {
+      off[i] = (uint32_t)weight_row(r) * (uint32_t)p.K + chunk * 16;
+      hi[i] = chunk >= 4;
+    } else {
+      const int m = m0 + r - TN;
+      off[i] = (uint32_t)(m < p.M ? m : p.M - 1) * (uint32_t)p.lda + chunk * 16;
+      hi[i] = false;
+    }
+  }
+  const int nk = (p.K + kStepBytes - 1) / kStepBytes;  // 128-byte pieces of the reduction; piece s * KS + g is this group's step s
+  const int steps = (nk + KS - 1) / KS;
+  const int mine = (nk - g + KS - 1) / KS;
+  const bool ragged = p.K % kStepBytes != 0;
+  auto issue = [&](int s, int slot, int from, int to) {
+    const int piece = s * KS + g;
+    const int koff = piece * kStepBytes;
+    const uint32_t base = lds0 + slot * kStage + g * kGroupBytes;
+    // Last 64 bytes of a ragged reduction: the activation rows are zero there, so the weights may be anything
+    // readable: the lower half again (the next row would lie past the end of the matrix for the last one).
+    const uint32_t back = ragged && piece == nk - 1 ? 64u : 0u;
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      if (i < from || i >= to) continue;
+      const int rb = wg * L + i;
+      const bool is_w = rb * 8 < TN;
+      load_to_lds_16((is_w ? p.w : p.a_q) + koff, off[i] - (hi[i] ? back : 0u), base + rb * 1024);
+    }
+  };
+
+  int w_ld[NI], x_ld[MI], chunk[F::kSub];
+  const int lrow = lane % MF;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) w_ld[i] = (wn * NT + i * MF + lrow) * kStepBytes;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) x_ld[i] = (TN + wm * MT + i * MF + lrow) * kStepBytes;
+#pragma unroll
+  for (int kk = 0; kk < F::kSub; ++kk) chunk[kk] = ((kk * (64 / MF) + lane / MF) ^ swizzle_of_row(lrow)) * 16;
+
+  typename F::Acc acc[NI][MI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+#pragma unroll
+      for (int r = 0; r < F::kRegs; ++r) acc[i][j][r] = 0;
+
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < mine) issue(s, s, 0, L);
+
+  int slot = 0;
+  for (int s = 0; s < steps; ++s) {
+    // this wavefront's loads of step s are in (those of the next S - 2 steps, as far as there are any, stay in flight)
+    const int later = mine - 1 - s;
+    wait_groups<L, S - 2>(later < 0 ? 0 : later);
+    if constexpr (G > 1)
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int fill = slot == 0 ? S - 1 : slot - 1;  // the slot of step s - 1: everybody is done reading it
+    const bool more = s + S - 1 < mine;
+    if (s < mine) {
+      const char* st = lds + slot * kStage + g * kGroupBytes;
+      v4i a[2][NI], b[2][MI];
+      auto read = [&](int kk) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) a[kk & 1][i] = *reinterpret_cast<const v4i*>(st + w_ld[i] + chunk[kk]);
+#pragma unroll
+        for (int j = 0; j < MI; ++j) b[kk & 1][j] = *reinterpret_cast<const v4i*>(st + x_ld[j] + chunk[kk]);
+      };
+      read(0);
+#pragma unroll
+      for (int kk = 0; kk < F::kSub; ++kk) {
+        if (kk + 1 < F::kSub) read(kk + 1);
+        // the loads of the step S - 1 ahead go out a few at a time between the multiplications
+        // (with two stages they have only this step to arrive in: all of them first)
+        if (more && (S > 2 || kk == 0)) issue(s + S - 1, fill, S > 2 ? kk * L / F::kSub : 0, S > 2 ? (kk + 1) * L / F::kSub : L);
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < MI; ++j) acc[i][j] = F::mul(a[kk & 1][i], b[kk & 1][j], acc[i][j]);
+      }
+    }
+    slot = slot + 1 == S ? 0 : slot + 1;
+  }
+  wait_vmcnt<0>();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // ---- partial sums of the KS groups meet in LDS, [group][token][channel] ----
+  char* part = lds + g * kPart;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+#pragma unroll
+      for (int q = 0; q < F::kRegs / 4; ++q) {
+        const int tok = wm * MT + j * MF + lrow;
+        const int ch = wn * NT + i * MF + (MF == 32 ? 8 * q : 0) + 4 * (lane / MF);
+        *reinterpret_cast<v4i*>(part + tok * kPartRow + ch * 4) =
+            v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+      }
+  __syncthreads();
+
+  constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;  // output channels of the tile
+  constexpr int kPieces = kOut / 8;                        // 16-byte pieces of an output row
+  const int width = MODE == kGateUpSilu ? inter : p.N;
+  auto total4 = [&](int tok, int ch, int (&v)[4]) {
+    v4i s = *reinterpret_cast<const v4i*>(lds + tok * kPartRow + ch * 4);
+#pragma unroll
+    for (int k = 1; k < KS; ++k) s += *reinterpret_cast<const v4i*>(lds + k * kPart + tok * kPartRow + ch * 4);
+    v[0] = s[0], v[1] = s[1], v[2] = s[2], v[3] = s[3];
+  };
+  for (int u = threadIdx.x; u < TM * kPieces; u += kThreads) {
+    const int tok = u / kPieces, c = u % kPieces * 8;
+    const int m = m0 + tok, n = nt * kOut + c;
+    if (m >= p.M || n >= width) continue;
+    const float as = scales[TN + tok];
+    uint2 o[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int ch = c + 4 * h;
+      int v[4];
+      total4(tok, ch, v);
+      const float4 ws = *reinterpret_cast<const float4*>(scales + ch);
+      if constexpr (MODE == kGateUpSilu) {
+        int up[4];
+        total4(tok, ch + kOut, up);
+        o[h] = silu_mul_epilogue4(v, up, as, ws, *reinterpret_cast<const float4*>(scales + ch + kOut));
+      } else {
+        o[h] = down_epilogue4(v, as, ws, 1.0f);
+      }
+    }
+    *reinterpret_cast<uint4*>(p.out + (int64_t)m * width + n) = make_uint4(o[0].x, o[0].y, o[1].x, o[1].y);
+  }
+}
+
+template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int WPE>
+hipError_t launch_config(const DenseParams& p0, hipStream_t stream) {
+  DenseParams p = p0;
+  constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;
+  const int width = MODE == kGateUpSilu ? p.N / 2 : p.N;
+  p.mtiles = (p.M + TM - 1) / TM;
+  p.ntiles = (width + kOut - 1) / kOut;
+  const int per_xcd = (p.mtiles * p.ntiles + kXcds - 1) / kXcds;
+  hipLaunchKernelGGL((gemm_dense_kernel<MODE, TM, TN, KS, WM, WN, S, WPE>), dim3((unsigned)(per_xcd * kXcds)),
+                     dim3(64 * KS * WM * WN), 0, stream, p);
+  return hipGetLastError();
+}
+
+// One way to cut the problem up and what it costs.  A launch takes about
+//   start + rounds * per_round + max(rounds * per_k * K / 1024, padded operations / rate)
+// where a round is as many workgroups as the device holds at a time: small tiles are bound by a round's
+// latency and by how fast a compute unit takes in its two operands, large ones by the matrix pipes at the
+// clock the power limit allows.
+struct Config {
+  int tm, tn;       // tile
+  int per_cu;       // workgroups a compute unit holds at a time
+  float start;      // us
+  float per_round;  // us
+  float per_k;      // us per 1024 reduction bytes
+  float rate;       // 1e15 operations per second
+  hipError_t (*gate_up)(const DenseParams&, hipStream_t);
+  hipError_t (*down)(const DenseParams&, hipStream_t);
+};
+#define MOE_I8_DENSE(TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, RATE)                 \
+  {TM, TN, PER_CU, START, ROUND, PER_K, RATE, launch_config<kGateUpSilu, TM, TN, KS, WM, WN, S, WPE>, \
+   launch_config<kDown, TM, TN, KS, WM, WN, S, WPE>}
+// The constants are least-squares fits to 150 problems drawn over 1..8192 rows, 512..16384 channels and
+// 512..8192 reduction bytes (rms error of a fit 6-14 %).  The configuration the estimates pick takes on
+// average 0.8 % longer than the fastest one of the table.
+const Config kConfigs[] = {
+    MOE_I8_DENSE(16, 16, 8, 1, 1, 2, 4, 1, 2.45f, 0.53f, 0.38f, 1e9f),
+    MOE_I8_DENSE(16, 32, 8, 1, 1, 3, 2, 1, 1.49f, 1.46f, 0.58f, 1e9f),
+    MOE_I8_DENSE(32, 32, 8, 1, 1, 2, 2, 1, 1.35f, 1.64f, 0.70f, 1e9f),
+    MOE_I8_DENSE(32, 64, 4, 1, 2, 3, 2, 1, 1.27f, 2.03f, 1.06f, 0.98f),
+    MOE_I8_DENSE(64, 64, 2, 2, 2, 4, 2, 1, 1.56f, 2.08f, 1.38f, 1.12f),
+    MOE_I8_DENSE(64, 128, 2, 2, 2, 3, 2, 1, 0.55f, 3.15f, 2.15f, 1.58f),
+    MOE_I8_DENSE(128, 128, 1, 2, 4, 4, 2, 1, 1.75f, 3.18f, 3.49f, 1.59f),
+    MOE_I8_DENSE(128, 128, 1, 2, 2, 2, 2, 2, 0.71f, 3.66f, 5.59f, 1.72f),
+};
+// The 256-row tiles of the grouped family (one persistent workgroup per compute unit).
+const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, nullptr, nullptr};
+
+float estimate(const Config& c, int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = ((m + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn);
+  const int64_t room = (int64_t)device_cu_count() * c.per_cu;
+  const float rounds = (float)((tiles + room - 1) / room);
+  const float latency = rounds * c.per_k * (float)k / 1024.0f;
+  const float ops = (float)(tiles * c.tm * c.tn) * (float)k * 2.0f / (c.rate * 1e9f);
+  return c.start + rounds * c.per_round + (latency > ops ? latency : ops);
+}
+
+const Config* pick(int64_t m, int64_t n, int64_t k, bool wide_allowed) {
+  const Config* best = wide_allowed ? &kWide : nullptr;
+  float least = wide_allowed ? estimate(kWide, m, n, k) : 0.0f;
+  for (const Config& c : kConfigs) {
+    const float t = estimate(c, m, n, k);
+    if (!best || t < least) least = t, best = &c;
+  }
+  return best;
+}
+
+}  // namespace
+
+int dense_row_stride(int k) { return (k + kStepBytes - 1) / kStepBytes * kStepBytes; }
+
+bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed) {
+  // per-lane source offsets are 32-bit: the weights and the activation matrix must each span less than 4 GiB
+  if (m < 1 || (int64_t)n * k >= (1ll << 32) || m * dense_row_stride(k) >= (1ll << 32)) return false;
+  return pick(m, n, k, wide_allowed) != &kWide;
+}
+
+hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream) {
+  DenseParams p{};
+  p.a_q = a.a_q;
+  p.a_scale = a.a_scale;
+  p.w = a.w;
+  p.w_scale = a.w_scale;
+  p.out = static_cast<uint16_t*>(a.out);
+  p.M = (int)a.m;
+  p.N = a.n;
+  p.K = a.k;
+  p.lda = dense_row_stride(a.k);
+  const Config* c = pick(a.m, a.n, a.k, false);
+  return a.mode == kGateUpSilu ? c->gate_up(p, stream) : c->down(p, stream);
+}
+
+}  // namespace moe_i8

@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kThreads) void quant_rows_kernel(QuantArgs a) {
 
 template <int kMode>
 void launch_quant_rows_mode(const QuantArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
-  switch (quant_vectors_per_lane(a.cols)) {
+  switch (quant_vectors_per_lane(a.q_stride > a.cols ? a.q_stride : a.cols)) {
     case 1: hipLaunchKernelGGL((quant_rows_kernel<1, kMode>), grid, block, 0, stream, a); break;
     case 2: hipLaunchKernelGGL((quant_rows_kernel<2, kMode>), grid, block, 0, stream, a); break;
     case 4: hipLaunchKernelGGL((quant_rows_kernel<4, kMode>), grid, block, 0, stream, a); break;

@@ -114,8 +114,10 @@ __device__ __forceinline__ void quant_one_row(const QuantArgs& a, int64_t row) {
   const int64_t orow = a.rows_per_group > 0
                            ? (row / a.rows_per_group) * a.out_rows_per_group + a.out_row_offset + row % a.rows_per_group
                            : row;
-  uint2* out = reinterpret_cast<uint2*>(a.q + orow * (int64_t)a.cols);
+  const int stride = kMode == kQuantWeights || a.q_stride == 0 ? a.cols : a.q_stride;
+  uint2* out = reinterpret_cast<uint2*>(a.q + orow * (int64_t)stride);
   const int nvec = a.cols / kQuantVec;
+  const int ovec = stride / kQuantVec;  // vectors of the output row: zeros behind the input's
 
   if constexpr (VPL > 0) {
     uint4 v[VPL];
@@ -142,7 +144,7 @@ __device__ __forceinline__ void quant_one_row(const QuantArgs& a, int64_t row) {
 #pragma unroll
       for (int i = 0; i < VPL; ++i) {
         const int c = lane + i * kWave;
-        if (c < nvec) out[c] = quant8<kMode == kQuantEven>(v[i], inv);
+        if (c < ovec) out[c] = quant8<kMode == kQuantEven>(v[i], inv);
       }
     }
   } else {
@@ -163,7 +165,7 @@ __device__ __forceinline__ void quant_one_row(const QuantArgs& a, int64_t row) {
       }
     }
     auto second_pass = [&](auto quantise) {
-      for (int c0 = lane; c0 < nvec; c0 += kUnroll * kWave) {
+      for (int c0 = lane; c0 < ovec; c0 += kUnroll * kWave) {
         uint4 t[kUnroll];
 #pragma unroll
         for (int i = 0; i < kUnroll; ++i) {
@@ -173,7 +175,7 @@ __device__ __forceinline__ void quant_one_row(const QuantArgs& a, int64_t row) {
 #pragma unroll
         for (int i = 0; i < kUnroll; ++i) {
           const int c = c0 + i * kWave;
-          if (c < nvec) out[c] = have ? quantise(t[i]) : make_uint2(0u, 0u);
+          if (c < ovec) out[c] = have ? quantise(t[i]) : make_uint2(0u, 0u);
         }
       }
     };

@@ -1,0 +1,31 @@
+"""GPU parity of the dense GEMM kernel at the sizes where its tiles and its split reduction can go wrong:
+one row, tile edges and remainders of every tile the library picks by itself, channels that fill no tile,
+reductions shorter than a workgroup's split and odd multiples of 64."""
+
+import pytest
+import torch
+
+DEV = "cuda:0"
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 16, 64), (1, 2144, 1536), (3, 528, 6080), (16, 4096, 704), (17, 2528, 5056), (31, 48, 192), (33, 4096, 1088),
+    (64, 8192, 1984), (65, 1904, 3968), (129, 4112, 2112), (333, 4096, 2048), (500, 10240, 1472), (1000, 6144, 832),
+    (2049, 4096, 576), (5000, 528, 1024),
+])
+def test_linear_and_mlp(pra, oracle, M, N, K):
+    g = torch.Generator().manual_seed(M * 7 + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    s = torch.rand(N, generator=g) * 0.008 + 0.002
+    out = pra.apply_int8_linear(x.to(DEV), w.to(DEV), s.to(DEV))
+    assert torch.equal(out.cpu(), oracle.w8a8_linear(x, w, s))
+    # the gated MLP: gate_up over N rows of weights, down back to K channels, against the streaming family
+    inter = N // 2 // 64 * 64
+    if inter:
+        w13, s13 = w[: 2 * inter].to(DEV), (s[: 2 * inter] * 0.1).to(DEV)
+        w2 = torch.randint(-127, 128, (K, inter), generator=g, dtype=torch.int8).to(DEV)
+        s2 = (torch.rand(K, generator=g) * 1e-3 + 1e-3).to(DEV)
+        got = pra.w8a8_mlp(x.to(DEV), w13, s13, w2, s2)
+        assert torch.equal(got, pra.w8a8_mlp(x.to(DEV), w13, s13, w2, s2, gemm_variant="stream"))
