@@ -7,6 +7,7 @@ built, or exports fewer symbols than the header declares, importing callers get 
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from pathlib import Path
 
@@ -71,6 +72,7 @@ SIGNATURES = {
 STATIC_SCRATCH_BYTES = 32 << 20
 
 _lib = None
+_host = None
 
 
 class MoeI8Error(RuntimeError):
@@ -98,6 +100,22 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+def host():
+    """The native call path of the Python entry points (``csrc/host.cpp``), loaded on first use; raises if it
+    has not been built."""
+    global _host
+    if _host is None:
+        load()
+        path = PKG_DIR / "_host.so"
+        if not path.exists():
+            raise ImportError(f"{path} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
+        spec = importlib.util.spec_from_file_location("_host", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def check(code: int) -> None:

@@ -522,6 +522,12 @@ def route_topk(
     uint8 / uint16 ``[M, layers, topk]`` tensor, the compact routed-experts record of
     ``src/prime_rl/inference/vllm/routed_experts.py:11-33``.
     """
+    if score_func in _SCORE_FUNCS:
+        record, layer = routed_experts_out or (None, 0)
+        r = _abi.host().route(gating_output, topk, _SCORE_FUNCS[score_func], 1 if renormalize else 0, float(route_scale),
+                              selection_bias, num_expert_group, topk_group, 1 if group_score_top2 else 0, record, layer)
+        if r is not None:
+            return _result(r)
     _require_gpu("gating_output", gating_output)
     if gating_output.dtype != torch.float32:
         raise NotImplementedError(f"router logits must be float32, got {gating_output.dtype}")
@@ -692,6 +698,9 @@ def apply_int8_linear(
         raise NotImplementedError("static or asymmetric activation quantisation is not supported")
     if bias is not None:
         raise NotImplementedError("bias is not supported")
+    r = _abi.host().linear(input, weight, weight_scale, _variant(gemm_variant), workspace)
+    if r is not None:
+        return _result(r)
     _require_gpu("input", input)
     if input.dtype != torch.bfloat16:
         raise NotImplementedError(f"only bfloat16 activations are supported, got {input.dtype}")
@@ -723,6 +732,9 @@ def w8a8_mlp(
     routed output, ``src/prime_rl/trainer/models/layers/moe.py:453-462``; ``FeedForward.forward``,
     ``src/prime_rl/trainer/models/layers/mlp.py:29-32``): ``w13`` int8 ``[2I, H]`` gate rows first, ``w2``
     int8 ``[H, I]``, per-channel scales; both activations quantised per token with ties to even."""
+    r = _abi.host().mlp(x, w13, w13_scale, w2, w2_scale, _variant(gemm_variant), workspace)
+    if r is not None:
+        return _result(r)
     _require_gpu("x", x)
     if x.dtype != torch.bfloat16:
         raise NotImplementedError(f"only bfloat16 activations are supported, got {x.dtype}")
@@ -872,17 +884,19 @@ def _capturing(device: torch.device) -> bool:
     return bool(torch.cuda.is_available() and torch.cuda.is_current_stream_capturing())
 
 
-def _workspace(device: torch.device, stream: int, nbytes: int, pin: bool = False) -> torch.Tensor:
+def _workspace(device: torch.device, stream: int, nbytes: int, pin: bool = False, spare: int = 0) -> torch.Tensor:
     """Default workspace of a (device, stream).  A buffer that ``reserve_workspace`` allocated, or that a
     call made under graph capture used, is *pinned*: a captured graph may hold its address, so it is never
     replaced in place or evicted; when a later eager call needs more, the pinned buffer moves to a keep-alive
     list (it stays allocated for the life of the process) and a larger one takes its place in the cache.
-    Only buffers that no capture has seen are freed, when the cache is over its size or they are outgrown."""
+    Only buffers that no capture has seen are freed, when the cache is over its size or they are outgrown.
+    ``spare`` bytes more are asked for where that costs nothing that matters (outside a capture).  The native
+    call path is told of every change."""
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     with _workspaces_lock:
         ws = _workspaces.get(key)
         capturing = _capturing(device)
-        if ws is not None and ws.numel() >= nbytes:
+        if ws is not None and ws.numel() >= nbytes + (0 if capturing else spare):
             _workspaces.move_to_end(key)
             if pin or capturing:
                 _pinned_workspaces.add(key)
@@ -896,8 +910,12 @@ def _workspace(device: torch.device, stream: int, nbytes: int, pin: bool = False
         if ws is not None and key in _pinned_workspaces:
             _retired_workspaces.append(ws)  # a graph may replay on it: keep it allocated
             _pinned_workspaces.discard(key)
-        ws = torch.empty((max(nbytes, 256),), dtype=torch.uint8, device=device)
+        if ws is not None and ws.is_cuda:
+            _abi.host().forget(*key)  # before the old buffer can go
+        ws = torch.empty((max(nbytes + spare, 256),), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
+        if ws.is_cuda:
+            _abi.host().remember(*key, ws.data_ptr(), ws.numel())
         _workspaces.move_to_end(key)
         if pin:
             _pinned_workspaces.add(key)
@@ -905,7 +923,8 @@ def _workspace(device: torch.device, stream: int, nbytes: int, pin: bool = False
             for old_key in [k for k in _workspaces if k not in _pinned_workspaces and k != key]:
                 if len(_workspaces) <= _MAX_CACHED_WORKSPACES:
                     break
-                del _workspaces[old_key]
+                if _workspaces.pop(old_key).is_cuda:
+                    _abi.host().forget(*old_key)
         return ws
 
 
@@ -918,7 +937,19 @@ def reserve_workspace(max_tokens: int, top_k: int, num_experts: int, hidden: int
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     stream = torch.cuda.current_stream(device).cuda_stream
     return _workspace(device, stream, workspace_bytes(max_tokens, top_k, num_experts, hidden, inter, block_size_m),
-                      pin=True)
+                      pin=True, spare=_routing_bytes(max_tokens, top_k))
+
+
+def _routing_bytes(m: int, top_k: int) -> int:
+    """What ``fused_moe`` keeps behind the layer's workspace: fp32 weights and int32 ids of every pair."""
+    return 8 * m * top_k
+
+
+def _result(r):
+    """What the native call path returned: the result, or the C-ABI's error code."""
+    if type(r) is int:
+        _abi.check(r)
+    return r
 
 
 def fused_experts(
@@ -960,6 +991,12 @@ def fused_experts(
     token must be distinct, as every router produces them: the kernels size their work on an expert
     holding at most one row per token.
     """
+    if (use_int8_w8a8 is True and per_channel_quant is True and activation == "silu" and expert_map is None
+            and block_shape is None and not apply_router_weight_on_input and global_num_experts == -1):
+        r = _abi.host().experts(hidden_states, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, block_size_m,
+                                _variant(gemm_variant), inplace, out, workspace)
+        if r is not None:
+            return _result(r)
     if not use_int8_w8a8:
         raise NotImplementedError("this library implements only the use_int8_w8a8=True path")
     if not per_channel_quant:
@@ -1016,7 +1053,7 @@ def fused_experts(
     need = workspace_bytes(M, k, E, H, I, block_size_m)
     stream = _stream(hidden_states)
     if workspace is None:
-        workspace = _workspace(hidden_states.device, stream, need)
+        workspace = _workspace(hidden_states.device, stream, need, spare=_routing_bytes(M, k))
     else:
         _require_gpu("workspace", workspace)
         if workspace.numel() * workspace.element_size() < need:
@@ -1068,6 +1105,25 @@ def fused_moe(
     ``src/prime_rl/trainer/models/layers/moe.py:262-269``)."""
     if custom_routing_function is not None:
         raise NotImplementedError("custom_routing_function is not supported")
+    if (use_int8_w8a8 is True and per_channel_quant is True and activation == "silu" and expert_map is None
+            and block_shape is None and global_num_experts == -1 and scoring_func in ("softmax", "sigmoid")
+            and (not use_grouped_topk or (num_expert_group and topk_group))):
+        groups, kept = (num_expert_group, topk_group) if use_grouped_topk else (1, 1)
+        record, layer = routed_experts_out or (None, 0)
+        args = (
+            hidden_states, w1, w2, w1_scale, w2_scale, block_size_m, _variant(gemm_variant), inplace, workspace,
+            gating_output, topk, _SCORE_FUNCS[scoring_func], 1 if renormalize else 0, float(routed_scaling_factor),
+            e_score_correction_bias, groups, kept,
+            1 if use_grouped_topk and e_score_correction_bias is not None else 0, record, layer,
+        )
+        r = _abi.host().moe(*args)
+        if r is False:
+            M, H = hidden_states.shape
+            _workspace(hidden_states.device, _stream(hidden_states),
+                       workspace_bytes(M, topk, w1.shape[0], H, w1.shape[1] // 2, block_size_m), spare=_routing_bytes(M, topk))
+            r = _abi.host().moe(*args)
+        if r is not None and r is not False:
+            return _result(r)
     if gating_output.dtype != torch.float32:
         gating_output = gating_output.float()
     if use_grouped_topk:

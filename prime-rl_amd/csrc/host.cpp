@@ -1,0 +1,347 @@
+// The Python entry points' everyday call, in one native step: argument checks, output allocation, workspace
+// lookup and the C-ABI call.  A decode-sized layer takes 10-35 us on the GPU; the same steps in Python took
+// 17-39 us of host time per call, i.e. more than the kernels they launch.
+//
+// Every function returns the result tensor(s); None when anything about the call is out of the ordinary (a
+// type, shape, device or layout it does not expect, no workspace large enough, a capture in progress), in
+// which case the caller runs the Python path, which handles or names it; or a negative int, the C-ABI's error
+// code.  Nothing is launched before all checks are done, so None always means nothing has happened yet.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/moe_i8.h"
+
+namespace {
+
+// Default workspaces the Python side has made, by (device, stream); it owns them and withdraws an entry before
+// it lets go of the tensor.  Guarded by the interpreter lock.
+struct Workspace {
+  int device;
+  hipStream_t stream;
+  char* data;
+  int64_t bytes;
+};
+constexpr int kMaxWorkspaces = 64;
+Workspace g_workspaces[kMaxWorkspaces];
+int g_num_workspaces = 0;
+
+Workspace* find_workspace(int device, hipStream_t stream) {
+  for (int i = 0; i < g_num_workspaces; ++i)
+    if (g_workspaces[i].device == device && g_workspaces[i].stream == stream) return &g_workspaces[i];
+  return nullptr;
+}
+
+// The device and stream a call runs on; false: leave it to the Python path.
+struct Where {
+  int device;
+  hipStream_t stream;
+  bool init(const at::Tensor& t) {
+    device = t.get_device();
+    if (device != c10::hip::current_device()) return false;
+    stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return status == hipStreamCaptureStatusNone;
+  }
+};
+
+// A tensor argument: contiguous, of the type, on the GPU (of `where`, once that is known).
+bool plain(PyObject* o, at::ScalarType type, const at::Tensor** out) {
+  if (!THPVariable_Check(o)) return false;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  if (!t.is_cuda() || t.scalar_type() != type || !t.is_contiguous()) return false;
+  *out = &t;
+  return true;
+}
+
+at::Tensor make(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor& like) {
+  return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
+}
+
+char* bytes_of(const at::Tensor& t) { return static_cast<char*>(t.data_ptr()); }
+
+// A caller's workspace, or the default one of the stream.
+bool workspace(PyObject* o, const Where& at, int64_t need, char** data, int64_t* size) {
+  if (o == Py_None) {
+    const Workspace* w = find_workspace(at.device, at.stream);
+    if (!w || w->bytes < need) return false;
+    *data = w->data;
+    *size = w->bytes;
+    return true;
+  }
+  if (!THPVariable_Check(o)) return false;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  if (!t.is_cuda() || t.get_device() != at.device || !t.is_contiguous() || (int64_t)t.nbytes() < need) return false;
+  *data = bytes_of(t);
+  *size = (int64_t)t.nbytes();
+  return true;
+}
+
+bool as_int(PyObject* o, int64_t* v) {
+  if (!PyLong_CheckExact(o)) return false;
+  *v = PyLong_AsLongLong(o);
+  if (*v == -1 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+// [N, K] int8 weights, contiguous or as the transposed [K, N] view of such a tensor, with N scales.
+bool dense_weight(PyObject* wo, PyObject* so, const at::Tensor** w, const at::Tensor** s, int64_t* n, int64_t* k) {
+  if (!THPVariable_Check(wo)) return false;
+  const at::Tensor& t = THPVariable_Unpack(wo);
+  if (!t.is_cuda() || t.scalar_type() != at::kChar || t.dim() != 2) return false;
+  if (t.is_contiguous()) {
+    *n = t.size(0), *k = t.size(1);
+  } else if (t.stride(0) == 1 && t.stride(1) == t.size(0)) {
+    *n = t.size(1), *k = t.size(0);
+  } else {
+    return false;
+  }
+  *w = &t;
+  return plain(so, at::kFloat, s) && (*s)->numel() == *n;
+}
+
+#define MOE_I8_ARGS(count) \
+  if (nargs != count) { PyErr_SetString(PyExc_TypeError, "wrong number of arguments"); return nullptr; }
+
+PyObject* wrap_guarded(PyObject* (*fn)(PyObject* const*, Py_ssize_t), PyObject* const* args, Py_ssize_t nargs) {
+  try {
+    return fn(args, nargs);
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+template <PyObject* (*fn)(PyObject* const*, Py_ssize_t)>
+PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return wrap_guarded(fn, args, nargs);
+}
+
+// remember(device, stream, data, bytes): the default workspace of (device, stream) is now this one.
+PyObject* remember(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(4);
+  const long long d = PyLong_AsLongLong(args[0]), b = PyLong_AsLongLong(args[3]);
+  void* s = PyLong_AsVoidPtr(args[1]);
+  void* p = PyLong_AsVoidPtr(args[2]);
+  if (PyErr_Occurred()) return nullptr;
+  Workspace* w = find_workspace((int)d, (hipStream_t)s);
+  if (!w && g_num_workspaces < kMaxWorkspaces) w = &g_workspaces[g_num_workspaces++];
+  if (w) *w = {(int)d, (hipStream_t)s, (char*)p, (int64_t)b};
+  Py_RETURN_NONE;
+}
+
+// forget(device, stream)
+PyObject* forget(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(2);
+  const long long d = PyLong_AsLongLong(args[0]);
+  void* s = PyLong_AsVoidPtr(args[1]);
+  if (PyErr_Occurred()) return nullptr;
+  if (Workspace* w = find_workspace((int)d, (hipStream_t)s)) *w = g_workspaces[--g_num_workspaces];
+  Py_RETURN_NONE;
+}
+
+// linear(input, weight, weight_scale, variant, workspace)
+PyObject* linear(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(5);
+  const at::Tensor *x, *w, *s;
+  int64_t n, k, variant, size;
+  char* ws;
+  Where at;
+  if (!plain(args[0], at::kBFloat16, &x) || !dense_weight(args[1], args[2], &w, &s, &n, &k) || !as_int(args[3], &variant) ||
+      x->dim() < 1 || x->size(-1) != k || k == 0 || n > INT32_MAX || k > INT32_MAX || !at.init(*x) ||
+      w->get_device() != at.device || s->get_device() != at.device)
+    Py_RETURN_NONE;
+  const int64_t m = x->numel() / k;
+  if (m == 0 || !workspace(args[4], at, moe_i8_dense_workspace_bytes(m, (int)k, 0), &ws, &size)) Py_RETURN_NONE;
+  c10::SmallVector<int64_t, 4> shape(x->sizes().begin(), x->sizes().end());
+  shape.back() = n;
+  at::Tensor out = make(shape, at::kBFloat16, *x);
+  if (int rc = moe_i8_w8a8_linear(x->data_ptr(), (const int8_t*)w->data_ptr(), (const float*)s->data_ptr(), out.data_ptr(), m,
+                                  (int)n, (int)k, ws, size, (int)variant, at.stream))
+    return PyLong_FromLong(rc);
+  return THPVariable_Wrap(std::move(out));
+}
+
+// mlp(x, w13, w13_scale, w2, w2_scale, variant, workspace)
+PyObject* mlp(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(7);
+  const at::Tensor *x, *w13, *s13, *w2, *s2;
+  int64_t two_i, h, h2, i, variant, size;
+  char* ws;
+  Where at;
+  if (!plain(args[0], at::kBFloat16, &x) || !dense_weight(args[1], args[2], &w13, &s13, &two_i, &h) ||
+      !dense_weight(args[3], args[4], &w2, &s2, &h2, &i) || !as_int(args[5], &variant) || x->dim() < 1 || two_i != 2 * i ||
+      h2 != h || h == 0 || x->size(-1) != h || h > INT32_MAX || two_i > INT32_MAX || !at.init(*x) ||
+      w13->get_device() != at.device || s13->get_device() != at.device || w2->get_device() != at.device ||
+      s2->get_device() != at.device)
+    Py_RETURN_NONE;
+  const int64_t m = x->numel() / h;
+  if (m == 0 || !workspace(args[6], at, moe_i8_dense_workspace_bytes(m, (int)h, (int)i), &ws, &size)) Py_RETURN_NONE;
+  at::Tensor out = make(x->sizes(), at::kBFloat16, *x);
+  if (int rc = moe_i8_w8a8_mlp(x->data_ptr(), (const int8_t*)w13->data_ptr(), (const float*)s13->data_ptr(),
+                               (const int8_t*)w2->data_ptr(), (const float*)s2->data_ptr(), out.data_ptr(), m, (int)h, (int)i, ws,
+                               size, (int)variant, at.stream))
+    return PyLong_FromLong(rc);
+  return THPVariable_Wrap(std::move(out));
+}
+
+// The layer's tensors, checked against each other.
+struct Layer {
+  const at::Tensor *x, *w1, *w2, *s1, *s2;
+  int64_t m, e, h, i;
+  Where at;
+  bool init(PyObject* xo, PyObject* w1o, PyObject* w2o, PyObject* s1o, PyObject* s2o) {
+    if (!plain(xo, at::kBFloat16, &x) || !plain(w1o, at::kChar, &w1) || !plain(w2o, at::kChar, &w2) ||
+        !plain(s1o, at::kFloat, &s1) || !plain(s2o, at::kFloat, &s2) || x->dim() != 2 || w1->dim() != 3 || w2->dim() != 3)
+      return false;
+    m = x->size(0), h = x->size(1), e = w1->size(0), i = w1->size(1) / 2;
+    if (m == 0 || w1->size(1) % 2 || w1->size(2) != h || w2->size(0) != e || w2->size(1) != h || w2->size(2) != i ||
+        s1->numel() != e * 2 * i || s2->numel() != e * h || e < 1 || e > MOE_I8_MAX_EXPERTS || h % 64 || i % 64 || h > INT32_MAX ||
+        i > INT32_MAX / 2 || !at.init(*x))
+      return false;
+    for (const at::Tensor* t : {w1, w2, s1, s2})
+      if (t->get_device() != at.device) return false;
+    return true;
+  }
+  // `out`: None (a new tensor; the input itself if `inplace`) or the tensor to write
+  bool output(PyObject* o, bool inplace, at::Tensor* out) const {
+    if (o == Py_None) {
+      *out = inplace ? *x : make(x->sizes(), at::kBFloat16, *x);
+      return true;
+    }
+    const at::Tensor* t;
+    if (!plain(o, at::kBFloat16, &t) || t->sizes() != x->sizes() || t->get_device() != at.device) return false;
+    *out = *t;
+    return true;
+  }
+  int run(const float* weights, const int32_t* ids, int k, int block, int variant, at::Tensor& out, char* ws, int64_t size) const {
+    return moe_i8_fused_experts(x->data_ptr(), (const int8_t*)w1->data_ptr(), (const int8_t*)w2->data_ptr(), weights, ids,
+                                (const float*)s1->data_ptr(), (const float*)s2->data_ptr(), out.data_ptr(), m, k, (int)e, (int)h,
+                                (int)i, block, ws, size, variant, at.stream);
+  }
+};
+
+// experts(hidden, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, block, variant, inplace, out, workspace)
+PyObject* experts(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(12);
+  Layer l;
+  const at::Tensor *tw, *ids;
+  int64_t block, variant, size;
+  char* ws;
+  at::Tensor out;
+  if (!l.init(args[0], args[1], args[2], args[5], args[6]) || !plain(args[3], at::kFloat, &tw) || !plain(args[4], at::kInt, &ids) ||
+      !as_int(args[7], &block) || !as_int(args[8], &variant) || ids->dim() != 2 || ids->size(0) != l.m || tw->sizes() != ids->sizes() ||
+      tw->get_device() != l.at.device || ids->get_device() != l.at.device || ids->size(1) < 1 || ids->size(1) > l.e)
+    Py_RETURN_NONE;
+  const int k = (int)ids->size(1);
+  const int64_t need = moe_i8_workspace_bytes(l.m, k, (int)l.e, (int)l.h, (int)l.i, (int)block);
+  if (need < 0 || !workspace(args[11], l.at, need, &ws, &size) || !l.output(args[10], args[9] == Py_True, &out)) Py_RETURN_NONE;
+  if (int rc = l.run((const float*)tw->data_ptr(), (const int32_t*)ids->data_ptr(), k, (int)block, (int)variant, out, ws, size))
+    return PyLong_FromLong(rc);
+  return THPVariable_Wrap(std::move(out));
+}
+
+// The router's arguments: (logits, top_k, score_func, renormalize, scale, bias, groups, topk_groups, top2,
+// record, layer), in this order from `a` on.
+struct Router {
+  const at::Tensor* logits;
+  const at::Tensor* bias = nullptr;
+  const at::Tensor* record = nullptr;
+  int64_t m, e, k, score, renormalize, groups, topk_groups, top2, layer = 0;
+  double scale;
+  bool init(PyObject* const* a) {
+    if (!plain(a[0], at::kFloat, &logits) || logits->dim() != 2 || !as_int(a[1], &k) || !as_int(a[2], &score) ||
+        !as_int(a[3], &renormalize) || !PyFloat_CheckExact(a[4]) || !as_int(a[6], &groups) || !as_int(a[7], &topk_groups) ||
+        !as_int(a[8], &top2) || k < 1 || k > 64)
+      return false;
+    scale = PyFloat_AS_DOUBLE(a[4]);
+    m = logits->size(0), e = logits->size(1);
+    if (m == 0 || e < 1 || e > MOE_I8_MAX_EXPERTS || k > e || groups > e || topk_groups > e) return false;
+    if (a[5] != Py_None && (!plain(a[5], at::kFloat, &bias) || bias->numel() != e || bias->get_device() != logits->get_device()))
+      return false;
+    if (a[9] != Py_None) {
+      if (!THPVariable_Check(a[9]) || !as_int(a[10], &layer)) return false;
+      record = &THPVariable_Unpack(a[9]);
+      if (!record->is_cuda() || !record->is_contiguous() || record->get_device() != logits->get_device() ||
+          (record->scalar_type() != at::kByte && record->scalar_type() != at::kUInt16) || record->dim() != 3 ||
+          record->size(0) != m || record->size(2) != k || layer < 0 || layer >= record->size(1))
+        return false;
+    }
+    return true;
+  }
+  int run(float* weights, int32_t* ids, hipStream_t stream) const {
+    return moe_i8_route_topk((const float*)logits->data_ptr(), m, (int)e, (int)k, (int)score,
+                             bias ? (const float*)bias->data_ptr() : nullptr, (int)groups, (int)topk_groups, (int)top2,
+                             (int)renormalize, (float)scale, weights, ids, record ? record->data_ptr() : nullptr,
+                             record ? (record->scalar_type() == at::kByte ? 1 : 2) : 0, record ? record->size(1) * k : 0,
+                             record ? layer * k : 0, stream);
+  }
+};
+
+// route(<router>) -> (weights, ids)
+PyObject* route(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(11);
+  Router r;
+  Where at;
+  if (!r.init(args) || !at.init(*r.logits)) Py_RETURN_NONE;
+  at::Tensor weights = make({r.m, r.k}, at::kFloat, *r.logits), ids = make({r.m, r.k}, at::kInt, *r.logits);
+  if (int rc = r.run((float*)weights.data_ptr(), (int32_t*)ids.data_ptr(), at.stream)) return PyLong_FromLong(rc);
+  PyObject* w = THPVariable_Wrap(std::move(weights));
+  PyObject* i = THPVariable_Wrap(std::move(ids));
+  PyObject* both = w && i ? PyTuple_Pack(2, w, i) : nullptr;
+  Py_XDECREF(w);
+  Py_XDECREF(i);
+  return both;
+}
+
+// moe(hidden, w1, w2, w1_scale, w2_scale, block, variant, inplace, workspace, <router>): router, then experts.
+// The routing stays in the workspace, behind what the layer needs.  False: only a default workspace of that
+// size is missing.
+PyObject* moe(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(20);
+  Layer l;
+  Router r;
+  int64_t block, variant, size;
+  char* ws;
+  at::Tensor out;
+  if (!l.init(args[0], args[1], args[2], args[3], args[4]) || !as_int(args[5], &block) || !as_int(args[6], &variant) ||
+      !r.init(args + 9) || r.m != l.m || r.e != l.e || r.logits->get_device() != l.at.device)
+    Py_RETURN_NONE;
+  const int64_t need = moe_i8_workspace_bytes(l.m, (int)r.k, (int)l.e, (int)l.h, (int)l.i, (int)block);
+  if (need < 0) Py_RETURN_NONE;
+  if (!workspace(args[8], l.at, need + 8 * l.m * r.k, &ws, &size)) {
+    if (args[8] == Py_None) Py_RETURN_FALSE;
+    Py_RETURN_NONE;
+  }
+  if (!l.output(Py_None, args[7] == Py_True, &out)) Py_RETURN_NONE;
+  float* weights = reinterpret_cast<float*>(ws + need);
+  int32_t* ids = reinterpret_cast<int32_t*>(weights + l.m * r.k);
+  if (int rc = r.run(weights, ids, l.at.stream)) return PyLong_FromLong(rc);
+  if (int rc = l.run(weights, ids, (int)r.k, (int)block, (int)variant, out, ws, size)) return PyLong_FromLong(rc);
+  return THPVariable_Wrap(std::move(out));
+}
+
+PyMethodDef kMethods[] = {
+    {"remember", (PyCFunction)(void*)guarded<remember>, METH_FASTCALL, nullptr},
+    {"forget", (PyCFunction)(void*)guarded<forget>, METH_FASTCALL, nullptr},
+    {"linear", (PyCFunction)(void*)guarded<linear>, METH_FASTCALL, nullptr},
+    {"mlp", (PyCFunction)(void*)guarded<mlp>, METH_FASTCALL, nullptr},
+    {"experts", (PyCFunction)(void*)guarded<experts>, METH_FASTCALL, nullptr},
+    {"route", (PyCFunction)(void*)guarded<route>, METH_FASTCALL, nullptr},
+    {"moe", (PyCFunction)(void*)guarded<moe>, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&kModule); }
