@@ -127,6 +127,15 @@ int moe_i8_quant_weights(const void* w, int dtype, int64_t rows, int64_t cols, i
                          void* stream);
 
 /*
+ * The three projections of one expert layer, each as moe_i8_quant_weights does it, in one launch: gate and
+ * up bf16 [E, I, H] into the halves of w13 int8 [E, 2I, H] (gate rows first), down bf16 [E, H, I] into w2
+ * int8 [E, H, I]; scales fp32 [E, 2I] and [E, H].
+ */
+int moe_i8_quant_expert_weights(const void* gate, const void* up, const void* down, int dtype, int64_t num_experts,
+                                int64_t inter, int64_t hidden, int8_t* w13, float* w13_scale, int8_t* w2,
+                                float* w2_scale, void* stream);
+
+/*
  * Replaces vLLM `fused_moe_kernel` (gate_up GEMM, use_int8_w8a8, per-channel) +
  * `silu_and_mul` (csrc/activation_kernels.cu).  In-tree semantics: grouped GEMM
  * contract tests/unit/train/models/test_moe.py:60-66; gate-then-up stacking

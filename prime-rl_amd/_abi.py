@@ -45,6 +45,7 @@ SIGNATURES = {
          c_int64, _P],
     ),
     "moe_i8_quant_weights": (c_int, [_P, c_int, c_int64, c_int64, c_int64, c_int64, c_int64, _P, _P, _P]),
+    "moe_i8_quant_expert_weights": (c_int, [_P, _P, _P, c_int, c_int64, c_int64, c_int64, _P, _P, _P, _P, _P]),
     "moe_i8_gemm_gate_up_silu": (
         c_int,
         [_P, _P, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64, _P, c_int, _P],

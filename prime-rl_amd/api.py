@@ -245,7 +245,7 @@ def quantize_expert_weights(
     down_proj: torch.Tensor,
     out: tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    """Trainer expert weights → the int8 kernel layout ``fused_experts`` reads, in three launches and
+    """Trainer expert weights → the int8 kernel layout ``fused_experts`` reads, in one launch and
     with no concatenated bf16 intermediate.
 
     ``gate_proj, up_proj`` bf16 ``[E, I, H]`` and ``down_proj`` bf16 ``[E, H, I]`` (``w1, w3, w2`` of
@@ -254,6 +254,9 @@ def quantize_expert_weights(
     [E, 2I]``, ``w2 int8 [E, H, I]``, ``w2_scale fp32 [E, H]``.  ``out=(w13, w13_scale, w2,
     w2_scale)`` overwrites the parameters of a running engine in place.
     """
+    if out is not None and len(out) == 4:
+        if _result(_abi.host().requantise(gate_proj, up_proj, down_proj, *out)) is not None:
+            return tuple(out)
     _check_bf16_weight("gate_proj", gate_proj, 3)
     _check_bf16_weight("up_proj", up_proj, 3)
     _check_bf16_weight("down_proj", down_proj, 3)
@@ -281,9 +284,12 @@ def quantize_expert_weights(
                 raise ValueError(f"out tensor {name} must be {dtype} with {numel} elements")
         if w13.shape != (E, 2 * I, H) or w2.shape != (E, H, I):
             raise ValueError("out weights must be w13 [E, 2I, H] and w2 [E, H, I]")
-    _quant_weights_into(gate_proj, w13, s13, I, 2 * I, 0)
-    _quant_weights_into(up_proj, w13, s13, I, 2 * I, I)
-    _quant_weights_into(down_proj, w2, s2)
+    _abi.check(
+        _abi.load().moe_i8_quant_expert_weights(
+            _ptr(gate_proj), _ptr(up_proj), _ptr(down_proj), _abi.DTYPE_BF16, E, I, H, _ptr(w13), _ptr(s13), _ptr(w2),
+            _ptr(s2), _stream(gate_proj),
+        )
+    )
     return w13, s13, w2, s2
 
 

@@ -335,9 +335,9 @@ int moe_i8_route_topk(const float* logits, int64_t m, int num_experts, int top_k
   return check_launch(moe_i8::launch_route_topk(a, static_cast<hipStream_t>(stream)), "route_topk");
 }
 
-int moe_i8_quant_weights(const void* w, int dtype, int64_t rows, int64_t cols, int64_t rows_per_group,
-                         int64_t out_rows_per_group, int64_t out_row_offset, int8_t* q, float* scale,
-                         void* stream) {
+static int weight_quant_args(const void* w, int dtype, int64_t rows, int64_t cols, int64_t rows_per_group,
+                             int64_t out_rows_per_group, int64_t out_row_offset, int8_t* q, float* scale,
+                             moe_i8::QuantArgs* out) {
   if (dtype != MOE_I8_DTYPE_BF16) return fail(MOE_I8_EUNSUPPORTED, "only bf16 weights are supported");
   if (rows < 0) return fail(MOE_I8_EINVAL, "negative row count");
   if (rows == 0) return MOE_I8_OK;
@@ -362,7 +362,31 @@ int moe_i8_quant_weights(const void* w, int dtype, int64_t rows, int64_t cols, i
   a.rows_per_group = rows_per_group;
   a.out_rows_per_group = out_rows_per_group;
   a.out_row_offset = out_row_offset;
-  return check_launch(moe_i8::launch_quant_weights(a, static_cast<hipStream_t>(stream)), "quant_weights");
+  *out = a;
+  return MOE_I8_OK;
+}
+
+int moe_i8_quant_weights(const void* w, int dtype, int64_t rows, int64_t cols, int64_t rows_per_group,
+                         int64_t out_rows_per_group, int64_t out_row_offset, int8_t* q, float* scale,
+                         void* stream) {
+  moe_i8::QuantArgs a;
+  if (int rc = weight_quant_args(w, dtype, rows, cols, rows_per_group, out_rows_per_group, out_row_offset, q, scale, &a))
+    return rc;
+  if (rows == 0) return MOE_I8_OK;
+  return check_launch(moe_i8::launch_quant_weights(&a, 1, static_cast<hipStream_t>(stream)), "quant_weights");
+}
+
+int moe_i8_quant_expert_weights(const void* gate, const void* up, const void* down, int dtype, int64_t num_experts,
+                                int64_t inter, int64_t hidden, int8_t* w13, float* w13_scale, int8_t* w2,
+                                float* w2_scale, void* stream) {
+  if (num_experts < 0 || inter < 1 || hidden < 1) return fail(MOE_I8_EINVAL, "bad layer shape");
+  if (num_experts == 0) return MOE_I8_OK;
+  moe_i8::QuantArgs a[3];
+  if (int rc = weight_quant_args(gate, dtype, num_experts * inter, hidden, inter, 2 * inter, 0, w13, w13_scale, &a[0])) return rc;
+  if (int rc = weight_quant_args(up, dtype, num_experts * inter, hidden, inter, 2 * inter, inter, w13, w13_scale, &a[1]))
+    return rc;
+  if (int rc = weight_quant_args(down, dtype, num_experts * hidden, inter, 0, 0, 0, w2, w2_scale, &a[2])) return rc;
+  return check_launch(moe_i8::launch_quant_weights(a, 3, static_cast<hipStream_t>(stream)), "quant_weights");
 }
 
 // The gate_up GEMM behind the entry point; `from_align`: the routing arrays are moe_align's own

@@ -192,8 +192,9 @@ struct RouteArgs {
 int route_experts_per_lane(int num_experts);
 hipError_t launch_route_topk(const RouteArgs& a, hipStream_t stream);
 
-// Per-output-channel weight quantisation (round to nearest even of w / scale, scale = absmax / 127).
-hipError_t launch_quant_weights(const QuantArgs& a, hipStream_t stream);
+// Per-output-channel weight quantisation (round to nearest even of w / scale, scale = absmax / 127) of 1 to
+// 3 matrices; the first two of three have the same row length.
+hipError_t launch_quant_weights(const QuantArgs* a, int count, hipStream_t stream);
 // moe_align and the quantisation of `q` in one launch; only when align_quant_fusable() says so.
 bool align_quant_fusable(const AlignArgs& a, const QuantArgs& q);
 hipError_t launch_align_quant(const AlignArgs& a, const QuantArgs& q, hipStream_t stream);

@@ -330,6 +330,29 @@ PyObject* moe(PyObject* const* args, Py_ssize_t nargs) {
   return THPVariable_Wrap(std::move(out));
 }
 
+// requantise(gate, up, down, w13, w13_scale, w2, w2_scale) -> True
+PyObject* requantise(PyObject* const* args, Py_ssize_t nargs) {
+  MOE_I8_ARGS(7);
+  const at::Tensor *g, *u, *d, *w13, *s13, *w2, *s2;
+  Where at;
+  if (!plain(args[0], at::kBFloat16, &g) || !plain(args[1], at::kBFloat16, &u) || !plain(args[2], at::kBFloat16, &d) ||
+      !plain(args[3], at::kChar, &w13) || !plain(args[4], at::kFloat, &s13) || !plain(args[5], at::kChar, &w2) ||
+      !plain(args[6], at::kFloat, &s2) || g->dim() != 3 || d->dim() != 3 || w13->dim() != 3 || u->sizes() != g->sizes())
+    Py_RETURN_NONE;
+  const int64_t e = g->size(0), i = g->size(1), h = g->size(2);
+  if (e == 0 || i == 0 || h == 0 || h % 8 || i % 8 || d->size(0) != e || d->size(1) != h || d->size(2) != i || w13->size(0) != e ||
+      w13->size(1) != 2 * i || w13->size(2) != h || w2->sizes() != d->sizes() || s13->numel() != e * 2 * i || s2->numel() != e * h ||
+      !at.init(*g))
+    Py_RETURN_NONE;
+  for (const at::Tensor* t : {u, d, w13, s13, w2, s2})
+    if (t->get_device() != at.device) Py_RETURN_NONE;
+  if (int rc = moe_i8_quant_expert_weights(g->data_ptr(), u->data_ptr(), d->data_ptr(), MOE_I8_DTYPE_BF16, e, i, h,
+                                           (int8_t*)w13->data_ptr(), (float*)s13->data_ptr(), (int8_t*)w2->data_ptr(),
+                                           (float*)s2->data_ptr(), at.stream))
+    return PyLong_FromLong(rc);
+  Py_RETURN_TRUE;
+}
+
 PyMethodDef kMethods[] = {
     {"remember", (PyCFunction)(void*)guarded<remember>, METH_FASTCALL, nullptr},
     {"forget", (PyCFunction)(void*)guarded<forget>, METH_FASTCALL, nullptr},
@@ -338,6 +361,7 @@ PyMethodDef kMethods[] = {
     {"experts", (PyCFunction)(void*)guarded<experts>, METH_FASTCALL, nullptr},
     {"route", (PyCFunction)(void*)guarded<route>, METH_FASTCALL, nullptr},
     {"moe", (PyCFunction)(void*)guarded<moe>, METH_FASTCALL, nullptr},
+    {"requantise", (PyCFunction)(void*)guarded<requantise>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -257,3 +257,15 @@ def test_model_level_weight_update_from_a_name_tensor_stream(pra, oracle):
     want = oracle.quantize_expert_weights(*newer)
     assert torch.equal(params["model.layers.1.mlp.experts.w13_weight"].cpu(), want[0])   # the valid layer was written
     assert {k: v.data_ptr() for k, v in params.items()} == ptrs
+
+
+@pytest.mark.parametrize("E,I,H", [(1, 8, 8), (2, 24, 520), (3, 640, 1344), (1, 1032, 2056), (2, 16, 8200), (5, 4104, 64)])
+def test_one_launch_for_a_layer_equals_the_oracle(pra, oracle, E, I, H):
+    """The layer's three projections in one launch, at row lengths of every register variant (and beyond, where
+    they run separately), pairs of them, and more or fewer rows than the launch has wavefronts for."""
+    gate, up, down = _weights(E, I, H, seed=E + I)
+    got = pra.quantize_expert_weights(gate.to(DEV), up.to(DEV), down.to(DEV))
+    for g, w in zip(got, oracle.quantize_expert_weights(gate, up, down)):
+        assert torch.equal(g.cpu(), w)
+    again = pra.quantize_expert_weights(gate.to(DEV), up.to(DEV), down.to(DEV), out=tuple(torch.zeros_like(g) for g in got))
+    assert all(torch.equal(a, g) for a, g in zip(again, got))
