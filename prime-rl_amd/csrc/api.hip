@@ -57,6 +57,7 @@ int check_gemm_common(const void* a_q, const void* w, const int32_t* sorted, con
 // or where there is at most one routed row per expert on average.
 constexpr int kStreamMaxRows = 16;
 constexpr int kStreamRowsPerExpert = 1;
+constexpr int kSelfQuantMaxInter = 1024;  // longest reduction moe_i8_gemm_down_bf16 takes for any routing
 
 int tile_geometry_of(int variant) {
   return variant == MOE_I8_GEMM_TILE_WIDE ? moe_i8::kTileWide
@@ -454,23 +455,33 @@ int moe_i8_gemm_down(const int8_t* h_q, const float* a_scale, const int8_t* w2,
                         variant, 0, false, stream);
 }
 
-int moe_i8_gemm_down_bf16(const void* act, const int8_t* w2, const float* w2_scale, const float* topk_weights,
-                          const int32_t* sorted_token_ids, const int32_t* expert_ids,
-                          const int32_t* num_tokens_post_padded, int64_t num_pairs, int num_experts, int hidden,
-                          int inter, int block_size, int64_t sorted_cap, void* out, void* stream) {
+// The self-quantising down GEMM behind the entry point; `max_rows` as in gemm_down_impl.
+static int gemm_down_bf16_impl(const void* act, const int8_t* w2, const float* w2_scale, const float* topk_weights,
+                               const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                               const int32_t* num_tokens_post_padded, int64_t num_pairs, int num_experts, int hidden,
+                               int inter, int block_size, int64_t sorted_cap, void* out, int64_t max_rows, void* stream) {
   if (num_pairs == 0) return MOE_I8_OK;
   if (int rc = check_gemm_common(act, w2, sorted_token_ids, expert_ids, num_tokens_post_padded, out, num_pairs,
                                  num_experts, hidden, inter, block_size, sorted_cap, MOE_I8_GEMM_STREAM))
     return rc;
   if (!w2_scale) return fail(MOE_I8_EINVAL, "null scale pointer");
   if (!aligned16(w2_scale)) return fail(MOE_I8_EINVAL, "w2_scale must be 16-byte aligned");
-  if (!moe_i8::gemm_stream_fuses_quant(inter))
-    return fail(MOE_I8_EUNSUPPORTED, "inter (%d) is too long for the GEMM that quantises its own activations", inter);
   moe_i8::GemmArgs g = down_args(nullptr, nullptr, w2, w2_scale, topk_weights, sorted_token_ids, expert_ids,
                                  num_tokens_post_padded, num_pairs, num_experts, hidden, inter, block_size,
                                  sorted_cap, out);
   g.a_bf16 = static_cast<const uint16_t*>(act);
+  g.max_rows_per_expert = max_rows;
   return check_launch(moe_i8::launch_gemm_stream(g, static_cast<hipStream_t>(stream)), "gemm_stream");
+}
+
+int moe_i8_gemm_down_bf16(const void* act, const int8_t* w2, const float* w2_scale, const float* topk_weights,
+                          const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                          const int32_t* num_tokens_post_padded, int64_t num_pairs, int num_experts, int hidden,
+                          int inter, int block_size, int64_t sorted_cap, void* out, void* stream) {
+  if (num_pairs > 0 && inter > kSelfQuantMaxInter)
+    return fail(MOE_I8_EUNSUPPORTED, "inter (%d) is too long for the GEMM that quantises its own activations", inter);
+  return gemm_down_bf16_impl(act, w2, w2_scale, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_padded, num_pairs,
+                             num_experts, hidden, inter, block_size, sorted_cap, out, 0, stream);
 }
 
 int moe_i8_gemm_acc_i32(const int8_t* a_q, const int8_t* w, const int32_t* sorted_token_ids,
@@ -573,7 +584,7 @@ LayerPlan plan_layer(int64_t m, int top_k, int num_experts, int hidden, int inte
   // Very few rows per expert (decode): the streaming down GEMM quantises its activations itself, one
   // launch less.  Every workgroup of a block repeats that quantisation, so from about four rows
   // per expert on (measured) the separate launch is the cheaper one again.
-  plan.down_quantises = plan.down_kernel == MOE_I8_GEMM_STREAM && moe_i8::gemm_stream_fuses_quant(inter) &&
+  plan.down_quantises = plan.down_kernel == MOE_I8_GEMM_STREAM && moe_i8::gemm_stream_fuses_quant(dg) &&
                         p <= (int64_t)3 * num_experts;
   moe_i8::AlignArgs aa{};
   aa.num_pairs = p;
@@ -671,8 +682,8 @@ int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
                                  block_size, c.cap, act, variant, true, stream))
     return rc;
   if (plan.down_quantises) {
-    if (int rc = moe_i8_gemm_down_bf16(act, w2, w2_scale, topk_weights, sorted, eids, npp, p, num_experts,
-                                       hidden_size, inter, block_size, c.cap, down, stream))
+    if (int rc = gemm_down_bf16_impl(act, w2, w2_scale, topk_weights, sorted, eids, npp, p, num_experts,
+                                     hidden_size, inter, block_size, c.cap, down, m, stream))
       return rc;
   } else {
     if (int rc = moe_i8_quant_rows(act, MOE_I8_DTYPE_BF16, p, inter, inter, nullptr, 1, p, act_q, a2, stream))
@@ -902,7 +913,7 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   if (int rc = run_dense(gu, variant, s)) return rc;
   // Few rows on the streaming family: its down GEMM quantises them itself (ties to even here), one
   // launch less.
-  if (variant == MOE_I8_GEMM_STREAM && m <= kDenseSelfQuantRows && moe_i8::gemm_stream_fuses_quant(inter)) {
+  if (variant == MOE_I8_GEMM_STREAM && m <= kDenseSelfQuantRows && inter <= kSelfQuantMaxInter) {
     if (int rc = check_gemm_common(ws + c.act, w2, dg.sorted_token_ids, dg.expert_ids, dg.num_tokens_post_padded, out, m, 1,
                                    hidden, inter, kDenseBlock, c.cap, MOE_I8_GEMM_STREAM))
       return rc;

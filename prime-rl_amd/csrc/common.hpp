@@ -232,7 +232,11 @@ hipError_t launch_gemm_stream(const GemmArgs& a, hipStream_t stream);
 int64_t mfma_probe_sink_bytes(int workgroups);
 double mfma_probe_ops(int workgroups, int iters);
 hipError_t launch_mfma_probe(bool random_operands, int workgroups, int iters, int32_t* sink, hipStream_t stream);
-bool gemm_stream_fuses_quant(int k);  // the down GEMM can quantise bf16 activations of this length itself
+bool gemm_stream_fuses_quant(const GemmArgs& a);  // the down GEMM of this family can quantise bf16 activations itself
+// The streaming family's kernel for a handful of tokens (launch_gemm_stream uses it where it takes the problem).
+bool gemm_split_takes(const GemmArgs& a);
+bool gemm_split_fuses_quant(int k);
+hipError_t launch_gemm_split(const GemmArgs& a, hipStream_t stream);
 hipError_t launch_gemm_tile(const GemmArgs& a, hipStream_t stream);
 bool gemm_tile_supports(const GemmArgs& a);
 bool gemm_tile_prefers_deep(const GemmArgs& a);

@@ -20,12 +20,11 @@
 // multiplications of a step: all of them at its start hold up the wavefront until the address unit has
 // taken them (333x4096x2048 8.8 -> 8.0 us).  Activation rows are padded with zeros to a multiple of 128
 // bytes (the quantiser writes them), which lets a reduction of any multiple of 64 run on the same path.
-#include "common.hpp"
+#include "lds_loads.hpp"
 
 namespace moe_i8 {
 namespace {
 
-constexpr int kStepBytes = 128;  // reduction bytes of a row per wave-group and step
 constexpr int kXcds = 8;
 
 struct DenseParams {
@@ -40,65 +39,6 @@ struct DenseParams {
   int lda;
   int mtiles;
   int ntiles;
-};
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
-}
-
-__device__ __forceinline__ uint64_t uniform_address(const void* base) {
-  const uint64_t b = reinterpret_cast<uint64_t>(base);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  return (uint64_t)lo | ((uint64_t)hi << 32);
-}
-__device__ __forceinline__ void load_to_lds_16(const void* base, uint32_t offset, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(uniform_address(base))
-               : "memory", "m0");
-}
-// 4 bytes per lane from any address of the lane's own
-__device__ __forceinline__ void load_to_lds_4(const void* addr, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-               :
-               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(reinterpret_cast<uint64_t>(addr))
-               : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-  return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)p);
-}
-__device__ __forceinline__ int swizzle_of_row(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-// Waits until at most n * kPer of this wavefront's vector-memory operations are pending, n <= kMost.
-template <int kPer, int kMost>
-__device__ __forceinline__ void wait_groups(int n) {
-  if constexpr (kMost == 0) {
-    wait_vmcnt<0>();
-  } else {
-    if (n >= kMost)
-      wait_vmcnt<kPer * kMost>();
-    else
-      wait_groups<kPer, kMost - 1>(n);
-  }
-}
-
-template <int MF>
-struct Mfma;
-template <>
-struct Mfma<32> {
-  typedef v16i Acc;
-  static constexpr int kRegs = 16;
-  static constexpr int kSub = 4;  // MFMAs per 128 reduction bytes
-  static __device__ __forceinline__ Acc mul(v4i a, v4i b, Acc c) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0); }
-};
-template <>
-struct Mfma<16> {
-  typedef v4i Acc;
-  static constexpr int kRegs = 4;
-  static constexpr int kSub = 2;
-  static __device__ __forceinline__ Acc mul(v4i a, v4i b, Acc c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
 };
 
 template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int WPE>

@@ -448,17 +448,16 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-bool gemm_stream_fuses_quant(int k) { return k <= kFusedMaxK; }
+bool gemm_stream_fuses_quant(const GemmArgs& a) {
+  return a.k <= kFusedMaxK || (gemm_split_takes(a) && gemm_split_fuses_quant(a.k));
+}
 
 hipError_t launch_gemm_stream(const GemmArgs& a, hipStream_t stream) {
+  if (a.a_bf16 && (!gemm_stream_fuses_quant(a) || a.row_div != 1)) return hipErrorInvalidValue;
+  if (gemm_split_takes(a) && (!a.a_bf16 || gemm_split_fuses_quant(a.k))) return launch_gemm_split(a, stream);
   switch (a.mode) {
     case kGateUpSilu: return launch_mode<kGateUpSilu>(a, stream);
-    case kDown:
-      if (a.a_bf16) {
-        if (a.k > kFusedMaxK || a.row_div != 1) return hipErrorInvalidValue;
-        return launch_mode<kDown, true>(a, stream);
-      }
-      return launch_mode<kDown>(a, stream);
+    case kDown: return a.a_bf16 ? launch_mode<kDown, true>(a, stream) : launch_mode<kDown>(a, stream);
     case kAccI32: return launch_mode<kAccI32>(a, stream);
     default: return hipErrorInvalidValue;
   }

@@ -1,0 +1,46 @@
+"""GPU parity of the streaming family's split-reduction kernel (a handful of tokens): one block and many, row
+counts up to its limit, ragged channels and reductions, self-quantising or not, on both sides of the hand-over to
+the streaming kernel; and of the top-k combine at every k that has its own variant."""
+
+import pytest
+import torch
+
+from _util import inputs_mod
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("E,k,H,I,M,B", [
+    (1, 1, 64, 64, 1, 16), (8, 2, 192, 128, 2, 64), (16, 8, 2048, 768, 1, 64), (16, 8, 2048, 768, 5, 64),
+    (4, 4, 4096, 1408, 3, 32), (3, 3, 7168, 2048, 2, 64), (2, 1, 8192, 64, 16, 128), (1, 1, 1088, 960, 16, 64),
+    (9, 9, 4096, 1408, 1, 64), (40, 6, 512, 2112, 9, 16),
+])
+def test_few_tokens_equal_the_tiled_families_stages(pra, oracle, E, k, H, I, M, B):
+    im = inputs_mod()
+    inp = im.make_inputs(im.LayerShape("f", E=E, k=k, H=H, I=I), M, seed=E + M + H)
+    st = oracle.fused_experts_staged(inp.hidden_states, inp.w1, inp.w2, inp.topk_weights, inp.topk_ids, inp.w1_scale,
+                                     inp.w2_scale, B)
+    d = inp.to(DEV)
+    s, e, npp = pra.moe_align_block_size(d.topk_ids, B, E)
+    act = pra.gemm_gate_up_silu(st["x_q"].to(DEV), st["a1_scale"].to(DEV), d.w1, d.w1_scale, s, e, npp, k, B, M * k, "stream")
+    # the epilogue's exponential is the one thing the oracle does not share bit for bit
+    diff = (act.float().cpu() - st["cache2"].float()).abs() > 0.02 * st["cache2"].float().abs() + 1e-6
+    assert not bool(diff.any())
+    down = pra.gemm_down(st["h_q"].to(DEV), st["a2_scale"].to(DEV), d.w2, d.w2_scale, d.topk_weights, s, e, npp, B, "stream")
+    assert torch.equal(down.cpu(), st["cache3"].reshape(M * k, H))
+    # the layer, which may quantise inside the down GEMM, against its own stages
+    hq, a2 = pra.per_token_quant_int8(act)
+    want = torch.empty(M, H, dtype=torch.bfloat16, device=DEV)
+    pra.moe_sum(pra.gemm_down(hq, a2, d.w2, d.w2_scale, d.topk_weights, s, e, npp, B, "stream").view(M, k, H), want)
+    got = pra.fused_experts(*d.fused_experts_args(), **d.fused_experts_kwargs(), block_size_m=B, gemm_variant="stream")
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 16])
+@pytest.mark.parametrize("M,H", [(1, 8), (3, 2048), (33, 7168)])
+def test_combine_at_every_k(pra, oracle, k, M, H):
+    x = torch.randn(M, k, H, generator=torch.Generator().manual_seed(k)).to(torch.bfloat16)
+    out = torch.empty(M, H, dtype=torch.bfloat16, device=DEV)
+    pra.moe_sum(x.to(DEV), out)
+    assert torch.equal(out.cpu(), oracle.moe_sum(x))
