@@ -3,54 +3,64 @@
 //
 // In this regime every expert is active, a block of 64 rows is all the reuse a weight byte gets,
 // and the layer is bound by streaming the weights from HBM once.  What matters is that the stream
-// never stops: a workgroup keeps two reduction steps of loads in flight at all times, also across
-// the end of a tile and through its epilogue.
+// never stops, and that the compute units end together: one workgroup of eight wavefronts per
+// compute unit walks its tiles with a ring of six or seven LDS stages, so that five or six reduction
+// steps of loads (80-96 KB of weights) are in flight at all times, also across the end of a tile and
+// through its epilogue.
 //
-// A workgroup is 4 wavefronts and two of them share a compute unit.  A tile is 64 token rows (one
-// 64-row sub-block of a moe_align block) x 128 weight rows; the reduction runs in steps of 128
-// bytes through a ring of three 24 KB LDS stages that both operands reach by global -> LDS loads
-// (global_load_lds_dwordx4, no staging registers).  Wavefront w multiplies weight rows
-// [32w, 32w + 32) of the tile with all 64 token rows as two v_mfma_i32_32x32x32_i8 tiles, used
-// "transposed" (A operand = weight rows), so a lane ends up with runs of 4 consecutive channels of
-// one token and stores its results straight from registers, 8 bytes at a time.  For the gate_up
-// GEMM the 32 weight rows of a wavefront are 16 gate rows and the 16 matching up rows, which puts a
-// gate value and its up value into the same lane.
+// A tile's loads and a step's work are kept off the stream's critical path: tasks are looked up 64 at a time,
+// token ids travel two tiles ahead, and a step reads its operands before it issues the loads of a later step
+// between its multiplications.  Against two workgroups of four wavefronts with three stages each (64 KB in
+// flight, a look-up of two dependent scalar reads per tile, loads first): same tiles, but half as long per tile
+// and twice as many per workgroup, which evens out the last round; 0.57 us per step = 7.3 TB/s of weights.
+// Layer us before -> after: 128 experts of 2048 x 768 at 17 / 100 / 203 / 512 tokens 85.0 / 118.1 / 122.0 / 138.3
+// -> 81.6 / 112.5 / 116.9 / 132.6, 4096 x 1408 with skewed routing at 17 / 64 / 200 tokens 113.8 / 155.0 / 250.4 ->
+// 105.7 / 151.0 / 242.4, 256 experts of 7168 x 2048 at 17 / 128 / 256 tokens 557 / 1109 / 1268 -> 537 / 1026 / 1199.
+//
+// A tile is TOK token rows (32 or 64: part of a moe_align block) x 128 weight rows; the reduction runs
+// in steps of 128 bytes and both operands reach LDS by global -> LDS loads (global_load_lds_dwordx4, no
+// staging registers).  Wavefront w multiplies weight rows [32 * (w % 4), + 32) of the tile with token half
+// w / 4, used "transposed" (A operand = weight rows), so a lane ends up with runs of 4 consecutive
+// channels of one token and stores its results straight from registers, 8 bytes at a time.  For the
+// gate_up GEMM the 32 weight rows of a wavefront are 16 gate rows and the 16 matching up rows, which
+// puts a gate value and its up value into the same lane.
 //
 // Nothing in the steady state is a compiler-visible vector load: token ids, activation scales,
-// routed weights and channel scales of the NEXT tile also travel global -> LDS (4 bytes per lane)
-// while the current tile is reduced, into a small double-buffered area.  The only waits on vector
-// memory are therefore the explicit ones of the ring, which leave the most recent group of loads
-// in flight.  (The vector-memory counter retires loads and stores in order, so the ring waits
-// before it issues a tile's stores and never has to count them.)
+// routed weights and channel scales of later tiles also travel global -> LDS (4 bytes per lane) while
+// the current tile is reduced, into a small triple-buffered area.  The only waits on vector memory are
+// therefore the explicit ones of the ring.  They count a wavefront's stage loads only: the few other
+// operations (those 4-byte loads, an epilogue's stores) make a wait slightly stricter than needed,
+// never weaker.
 //
 // LDS rows are 128 bytes; the 16-byte chunk index is XOR-swizzled with row bits so that the MFMA
-// operand reads (32 consecutive rows, same chunk) spread over all banks; because a load fills LDS
-// linearly the swizzle is applied to the global source address of each lane.
-#include "common.hpp"
+// operand reads spread over all banks; because a load fills LDS linearly the swizzle is applied to the
+// global source address of each lane.
+#include "lds_loads.hpp"
 
 namespace moe_i8 {
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / kWave;
-constexpr int kTok = 64;    // token rows per tile
 constexpr int kCh = 128;    // weight rows per tile
-constexpr int kBK = 128;    // reduction bytes per step
-constexpr int kStages = 3;
-constexpr int kTokOffset = kCh * kBK;
-constexpr int kStageBytes = (kCh + kTok) * kBK;  // 24 KB
-constexpr int kStageLoads = 6;                   // 1 KB loads per wavefront and step: 4 weight + 2 token
 constexpr int kXcds = 8;
-constexpr int kFirstGroup = 2;                   // the last loads of the start-up: token rows of step 1
-constexpr int kMinSteps = 4;  // the look-ahead of the next tile's inputs needs this many steps per tile
+constexpr int kMinSteps = 4;
+
+template <int TOK>
+struct Shape {
+  static constexpr int kStages = TOK == 64 ? 6 : 7;
+  static constexpr int kStageBytes = (kCh + TOK) * kStepBytes;  // 24 | 20 KB
+  static constexpr int kTokWaves = TOK / 8;                     // wavefronts that load token rows (8 rows each)
+  static constexpr int MF = TOK / 2;                            // MFMA edge: 32 or 16
+};
 
 // Inputs of one tile's epilogue (and of the loads of its token rows), filled by 4-byte global -> LDS
-// loads while the previous tile is reduced.
+// loads while earlier tiles are reduced.  Every wavefront fetches what it reads itself.
 struct TileAux {
-  int32_t ids[kTok];    // sorted_token_ids of the tile's rows
-  float a_scale[kTok];  // activation scale of each row (0 index for padding rows)
-  float row_w[kTok];    // routed weight of each row (down GEMM)
-  float w_scale[kCh];   // down: scales of the tile's 128 channels; gate_up: 64 gate scales, 64 up scales
+  int32_t ids[64];    // sorted_token_ids of the tile's rows
+  float a_scale[64];  // activation scale of each row (0 index for padding rows)
+  float row_w[64];    // routed weight of each row (down GEMM)
+  float w_scale[kCh]; // down: scales of the tile's 128 channels; gate_up: 64 gate scales, 64 up scales
 };
 
 struct NarrowParams {
@@ -72,163 +82,117 @@ struct NarrowParams {
   void* out;
 };
 
-// s_waitcnt with only the vector-memory counter constrained (gfx9 encoding: vmcnt = bits 3:0 and
-// 15:14; expcnt 6:4 and lgkmcnt 11:8 left at their maximum).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
-}
-
-__device__ __forceinline__ uint64_t uniform_address(const void* base) {
-  const uint64_t b = reinterpret_cast<uint64_t>(base);
-  // readfirstlane yields a signed int: go through uint32_t so that the low half is not sign-extended
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  return (uint64_t)lo | ((uint64_t)hi << 32);
-}
-
-// 16 (or 4) bytes per lane from global memory straight into LDS: lane i lands at lds_addr + 16 * i
-// (+ 4 * i).  lds_addr is wave-uniform and goes through M0; the source is a wave-uniform base plus
-// an unsigned 32-bit byte offset per lane.  Inline assembly, so that the compiler neither counts
-// these loads nor waits for them: the ring's explicit waits do.
-__device__ __forceinline__ void load_to_lds_16(const void* base, uint32_t offset, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(uniform_address(base))
-               : "memory", "m0");
-}
-// The same with the non-temporal hint: for weight rows that no other tile of this launch reads (the
-// expert's rows fit in one tile).  Streamed that way they do not displace the token rows and the
-// other tiles' shared weights from L2: measured 8-13 % on launches bound by the weight stream, and
-// a loss wherever a second tile of the expert would have found the rows in L2, hence per task.
-__device__ __forceinline__ void load_to_lds_16_stream(const void* base, uint32_t offset, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-               :
-               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(uniform_address(base))
-               : "memory", "m0");
-}
-__device__ __forceinline__ void load_to_lds_4(const void* base, uint32_t offset, uint32_t lds_addr) {
+__device__ __forceinline__ void load_to_lds_dword(const void* base, uint32_t offset, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :
                : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(uniform_address(base))
                : "memory", "m0");
 }
 
-// Two ints from wave-uniform addresses through the scalar (read-only) path, one wait for both.
-// After the inline assembly above the compiler no longer proves that global memory is unchanged and
-// would fetch such values with vector loads, whose wait would drain the ring; this only waits for
-// itself.  Only for data written before the launch (the scalar cache does not see this kernel's
-// stores).
-__device__ __forceinline__ void scalar_load2(const int32_t* pa, const int32_t* pb, int32_t& a, int32_t& b) {
-  asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)"
-               : "=&s"(a), "=&s"(b)
-               : "s"(uniform_address(pa)), "s"(uniform_address(pb))
-               : "memory");
-}
-
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-  return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)p);
-}
-
-__device__ __forceinline__ int swizzle_of_row(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
 struct Task {
   int e;          // expert; -1 = no more work
   int ct;         // channel tile
   int64_t slot0;  // first slot of the tile in sorted_ids
-  bool single;    // the expert's rows fit in this one tile: nothing else reads its weight rows
+  bool single;    // nothing else reads the expert's weight rows
 };
 
 struct TaskLoads {
   const int8_t* wbase;  // weights of the task's expert (wave-uniform)
   bool stream;          // fetch the weight rows with the non-temporal hint
-  uint32_t woff[4];     // per lane: byte offset of its chunk of weight row i from wbase
-  uint32_t xoff[2];     // per lane: byte offset of its chunk of token row i from a_q
+  uint32_t woff[2];     // per lane: byte offset of its chunk of weight row i from wbase
+  uint32_t xoff;        // per lane: byte offset of its chunk of its token row from a_q
 };
 
-// Extra 4-byte loads per wavefront in the step that fetches the next tile's scales.
-template <int MODE>
-constexpr int aux_loads() {
-  return MODE == kDown ? 4 : MODE == kGateUpSilu ? 3 : 0;
-}
-
-// Waits until at most the `n` most recent vector-memory operations of this wavefront are pending;
-// n is the size of the group issued last, one of four values.
-template <int MODE>
-__device__ __forceinline__ void wait_all_but(int n) {
-  if (n == kStageLoads)
-    wait_vmcnt<kStageLoads>();
-  else if (n == kFirstGroup)
-    wait_vmcnt<kFirstGroup>();
-  else if (n == kStageLoads + 1)
-    wait_vmcnt<kStageLoads + 1>();
-  else
-    wait_vmcnt<kStageLoads + aux_loads<MODE>()>();
-}
-
-template <int MODE>
+template <int MODE, int TOK>
 __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p) {
+  using S = Shape<TOK>;
+  using F = Mfma<S::MF>;
+  constexpr int kStages = S::kStages;
+  constexpr int kStageBytes = S::kStageBytes;
+  constexpr int kTokOffset = kCh * kStepBytes;
+  constexpr int NI = 32 / S::MF;  // MFMA tiles of a wavefront's 32 weight rows
   __shared__ __align__(16) char stages[kStages * kStageBytes];
-  __shared__ __align__(16) TileAux aux[2];
+  __shared__ __align__(16) TileAux aux[3];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lrow = lane & 31;
-  const int lhalf = lane >> 5;
+  const int cg = wave & 3;   // channel quarter
+  const int th = wave >> 2;  // token half
+  const int lrow = lane % S::MF;
+  const int lgrp = lane / S::MF;
   const int K = p.K;
-  const int nk = K / kBK;
+  const int nk = K / kStepBytes;
   const int inter = p.N / 2;
+  const bool loads_tokens = wave < S::kTokWaves;
+  // Steps the loads run ahead of the multiplication: the ring's depth, less for very short reductions (the
+  // rows of the next tile are set up in the first step of the current one).
+  const int ahead = nk - 1 < kStages - 1 ? nk - 1 : kStages - 1;
 
-  // ---- this workgroup's tasks: (tile, channel tile), channel tile fastest, split into 8 contiguous
+  // ---- this workgroup's tasks: (block, channel tile), channel tile fastest, split into 8 contiguous
   // ranges, one per XCD (workgroup id % 8), so that workgroups that run side by side share token
-  // rows and expert weights in that XCD's L2 ----
+  // rows and expert weights in that XCD's L2.  A block of more than TOK rows is walked in as many
+  // phases: the first TOK rows of all blocks, then the next (most of those are padding and skipped).
   const int npp = *p.npp;
-  const int sub_per_block = p.B / kTok;
-  const int total = (npp / kTok) * p.ntiles;
+  const int nblocks = npp / p.B;
+  const int sub_per_block = p.B / TOK;
+  const int total = nblocks * p.ntiles;
   const int per_xcd = (total + kXcds - 1) / kXcds;
   const int xcd = blockIdx.x % kXcds;
   const int stride = gridDim.x / kXcds;
-  const int range_end = (xcd + 1) * per_xcd < total ? (xcd + 1) * per_xcd : total;
+  const int in_range = total - xcd * per_xcd < per_xcd ? total - xcd * per_xcd : per_xcd;
+  const int phase_len = (per_xcd + stride - 1) / stride * stride;
 
-  // The first task at or after candidate `it` (in steps of `stride`) whose expert id is valid and
-  // whose rows are not all padding (valid rows are a prefix of a block).
-  auto find_task = [&](int& it) {
+  // Candidate tasks of this workgroup: `first_slot + i * stride` of its XCD's range, phase by phase.  Lane i
+  // looks up candidate 64 * chunk + i, so that taking the next task is a bit scan and a few lane reads: looked
+  // up one by one (two dependent scalar reads, about 1 us) they held up every tile, whose steps are 0.6 us.
+  // A task needs a valid expert id and rows that are not all padding (valid rows are a prefix of a block).
+  const int candidates = phase_len / stride * sub_per_block;
+  uint64_t open = 0;  // candidates of the current chunk not handed out yet
+  int chunk_base = 0, lane_e = 0, lane_blk = 0, lane_ct = 0, lane_flags = 0;
+  auto look_up = [&]() {
+    const int i = chunk_base + lane;
+    const int sub = i / (phase_len / stride);
+    const int at = (int)(blockIdx.x / kXcds) + (i - sub * (phase_len / stride)) * stride;
+    bool ok = i < candidates && at < in_range;
+    const int task = xcd * per_xcd + (ok ? at : 0);
+    const int blk = ok ? task / p.ntiles : 0;
+    const int64_t slot0 = (int64_t)blk * p.B + (int64_t)(ok ? sub : 0) * TOK;
+    const int e = p.expert_ids[blk];
+    const int32_t first = p.sorted_ids[slot0];
+    // Does the expert hold other tiles?  Its neighbours in the block list, and the next tile of the same block
+    // (the next tile's first slot says whether it is in use; any tile but the first has the one in front of it).
+    const int before = p.expert_ids[blk > 0 ? blk - 1 : blk];
+    const int after = p.expert_ids[blk + 1 < nblocks ? blk + 1 : blk];
+    const int32_t other = p.sorted_ids[slot0 + (sub + 1 < sub_per_block && ok ? TOK : 0)];
+    // all of them used here, so that the compiler waits for these loads here and not inside the ring's loop
+    asm volatile("" ::"v"(e), "v"(first), "v"(before), "v"(after), "v"(other));
+    ok = ok && e >= 0 && e < p.E && first >= 0 && first < p.P;
+    const bool single = sub == 0 && (blk == 0 || before != e) && (blk + 1 >= nblocks || after != e) &&
+                        (sub_per_block == 1 || !(other >= 0 && other < p.P));
+    lane_e = e;
+    lane_blk = blk;
+    lane_ct = task - blk * p.ntiles;
+    lane_flags = sub * 2 + (single ? 1 : 0);
+    open = __ballot(ok);
+  };
+  auto next_task = [&]() {
     Task tk;
     tk.e = -1;
     tk.ct = 0;
     tk.slot0 = 0;
     tk.single = false;
-    for (; xcd * per_xcd + it < range_end; it += stride) {
-      const int task = xcd * per_xcd + it;
-      const int tile = task / p.ntiles;
-      const int blk = tile / sub_per_block;
-      const int64_t slot0 = (int64_t)blk * p.B + (int64_t)(tile % sub_per_block) * kTok;
-      int32_t e, first;
-      scalar_load2(p.expert_ids + blk, p.sorted_ids + slot0, e, first);
-      if (e >= 0 && e < p.E && first >= 0 && first < p.P) {
-        tk.e = e;
-        tk.ct = task - tile * p.ntiles;
-        tk.slot0 = slot0;
-        // Does the expert hold other tiles?  Its neighbours in the block list, and the other
-        // 64-row half of a 128-row block (valid rows are a prefix: a second half means the first is
-        // full, and the second half's first slot says whether it is in use).
-        const int nblocks = npp / p.B;
-        int32_t before, after;
-        scalar_load2(p.expert_ids + (blk > 0 ? blk - 1 : blk), p.expert_ids + (blk + 1 < nblocks ? blk + 1 : blk), before,
-                     after);
-        bool single = (blk == 0 || before != e) && (blk + 1 >= nblocks || after != e);
-        if (single && sub_per_block > 1) {
-          if (tile % sub_per_block != 0) {
-            single = false;
-          } else {
-            int32_t other, unused;
-            scalar_load2(p.sorted_ids + slot0 + kTok, p.sorted_ids + slot0, other, unused);
-            single = !(other >= 0 && other < p.P);
-          }
-        }
-        tk.single = single;
-        break;
-      }
+    while (open == 0 && chunk_base + kWave < candidates) {
+      chunk_base += kWave;
+      look_up();
+    }
+    if (open != 0) {
+      const int i = __ffsll((unsigned long long)open) - 1;
+      open &= open - 1;
+      const int flags = __builtin_amdgcn_readlane(lane_flags, i);
+      tk.e = __builtin_amdgcn_readlane(lane_e, i);
+      tk.ct = __builtin_amdgcn_readlane(lane_ct, i);
+      tk.slot0 = (int64_t)__builtin_amdgcn_readlane(lane_blk, i) * p.B + (flags >> 1) * TOK;
+      tk.single = flags & 1;
     }
     return tk;
   };
@@ -237,12 +201,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
 
   // ---- global -> LDS loads ----
   // Lane fills LDS slot (lane & 7) of row base + 8 * i + (lane >> 3): it fetches the logical chunk
-  // (lane & 7) ^ swizzle(row) of that row, and swizzle(row) = (lane >> 3) ^ (i & 1).
+  // (lane & 7) ^ swizzle(row) of that row.
   auto setup_weight_loads = [&](const Task& tk, TaskLoads& ld) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 32 * wave + 8 * i + (lane >> 3);  // LDS weight row; wavefront row / 32 multiplies it
-      const int chunk = ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;
+    for (int i = 0; i < 2; ++i) {
+      const int row = 16 * wave + 8 * i + (lane >> 3);  // LDS weight row; wavefront row / 32 (mod 4) multiplies it
+      const int chunk = ((lane & 7) ^ swizzle_of_row(row)) * 16;
       int n;
       if constexpr (MODE == kGateUpSilu) {
         const int j = row & 31;
@@ -258,211 +222,231 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
     ld.stream = tk.single;
   };
   auto setup_token_loads = [&](const TileAux& ax, TaskLoads& ld) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = 16 * wave + 8 * i + (lane >> 3);
-      const int chunk = ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;
-      const int32_t tok = ax.ids[row];
-      const uint32_t arow = (tok >= 0 && tok < p.P) ? (uint32_t)(tok / p.row_div) : 0u;
-      ld.xoff[i] = arow * (uint32_t)K + chunk;
-    }
+    const int row = (8 * wave + (lane >> 3)) & (TOK - 1);
+    const int chunk = ((lane & 7) ^ swizzle_of_row(row)) * 16;
+    const int32_t tok = ax.ids[row];
+    const uint32_t arow = (tok >= 0 && tok < p.P) ? (uint32_t)(tok / p.row_div) : 0u;
+    ld.xoff = arow * (uint32_t)K + chunk;
   };
   auto issue_weights = [&](const TaskLoads& ld, int stage, int koff) {
-    const uint32_t base = stage0 + stage * kStageBytes;
+    const uint32_t base = stage0 + stage * kStageBytes + wave * 2048;
     if (ld.stream) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) load_to_lds_16_stream(ld.wbase + koff, ld.woff[i], base + (wave * 4 + i) * 1024);
+      for (int i = 0; i < 2; ++i) load_to_lds_16_stream(ld.wbase + koff, ld.woff[i], base + i * 1024);
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) load_to_lds_16(ld.wbase + koff, ld.woff[i], base + (wave * 4 + i) * 1024);
+      for (int i = 0; i < 2; ++i) load_to_lds_16(ld.wbase + koff, ld.woff[i], base + i * 1024);
     }
   };
   auto issue_tokens = [&](const TaskLoads& ld, int stage, int koff) {
-    const uint32_t base = stage0 + stage * kStageBytes + kTokOffset;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) load_to_lds_16(p.a_q + koff, ld.xoff[i], base + (wave * 2 + i) * 1024);
+    if (loads_tokens) load_to_lds_16(p.a_q + koff, ld.xoff, stage0 + stage * kStageBytes + kTokOffset + wave * 1024);
   };
-  auto issue_stage = [&](const TaskLoads& ld, int stage, int koff) {
-    issue_weights(ld, stage, koff);
-    issue_tokens(ld, stage, koff);
-  };
-  // Every wavefront fetches the whole (tiny) set: identical values to identical places, and each
-  // wavefront's own wait covers what it reads.
   auto issue_ids = [&](const Task& tk, TileAux& ax) {
-    load_to_lds_4(p.sorted_ids + tk.slot0, (uint32_t)lane * 4u, lds_address(ax.ids));
+    load_to_lds_dword(p.sorted_ids + tk.slot0, (uint32_t)(lane & (TOK - 1)) * 4u, lds_address(ax.ids));
   };
   auto issue_scales = [&](const Task& tk, TileAux& ax) {
     if constexpr (MODE == kAccI32) return;
-    const int32_t tok = ax.ids[lane];
+    const int32_t tok = ax.ids[lane & (TOK - 1)];
     const uint32_t t = (tok >= 0 && tok < p.P) ? (uint32_t)tok : 0u;
-    load_to_lds_4(p.a_scale, (t / (uint32_t)p.row_div) * 4u, lds_address(ax.a_scale));
+    load_to_lds_dword(p.a_scale, (t / (uint32_t)p.row_div) * 4u, lds_address(ax.a_scale));
     const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
     if constexpr (MODE == kDown) {
       // without routed weights the slot is filled with something readable and never used
       if (p.row_weight)
-        load_to_lds_4(p.row_weight, t * 4u, lds_address(ax.row_w));
+        load_to_lds_dword(p.row_weight, t * 4u, lds_address(ax.row_w));
       else
-        load_to_lds_4(p.a_scale, 0u, lds_address(ax.row_w));
+        load_to_lds_dword(p.a_scale, 0u, lds_address(ax.row_w));
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int n = tk.ct * kCh + 64 * j + lane;
-        load_to_lds_4(wsc, (uint32_t)(n < p.N ? n : p.N - 1) * 4u, lds_address(ax.w_scale + 64 * j));
+        load_to_lds_dword(wsc, (uint32_t)(n < p.N ? n : p.N - 1) * 4u, lds_address(ax.w_scale + 64 * j));
       }
     } else {
       const int ch = tk.ct * 64 + lane;
       const uint32_t c = (uint32_t)(ch < inter ? ch : inter - 1);
-      load_to_lds_4(wsc, c * 4u, lds_address(ax.w_scale));
-      load_to_lds_4(wsc, (c + (uint32_t)inter) * 4u, lds_address(ax.w_scale + 64));
+      load_to_lds_dword(wsc, c * 4u, lds_address(ax.w_scale));
+      load_to_lds_dword(wsc, (c + (uint32_t)inter) * 4u, lds_address(ax.w_scale + 64));
     }
   };
+  // this wavefront's loads of all but the `steps` most recent steps are in
+  auto wait_all_but = [&](int steps) {
+    if (loads_tokens)
+      wait_groups<3, kStages - 2>(steps);
+    else
+      wait_groups<2, kStages - 2>(steps);
+  };
 
-  // ---- MFMA operand reads: lane feeds row (lane & 31), 16-byte chunk 2 * kk + (lane >> 5) ----
-  const int w_ld = (32 * wave + lrow) * kBK;
-  int x_ld[2], chunk[4];
+  // ---- MFMA operand reads ----
+  int w_ld[NI], chunk[F::kSub];
 #pragma unroll
-  for (int tj = 0; tj < 2; ++tj) x_ld[tj] = kTokOffset + (tj * 32 + lrow) * kBK;
+  for (int i = 0; i < NI; ++i) w_ld[i] = (32 * cg + S::MF * i + lrow) * kStepBytes;
+  const int x_ld = kTokOffset + (th * S::MF + lrow) * kStepBytes;
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) chunk[kk] = ((2 * kk + lhalf) ^ swizzle_of_row(lrow)) * 16;
+  for (int kk = 0; kk < F::kSub; ++kk) chunk[kk] = ((kk * (64 / S::MF) + lgrp) ^ swizzle_of_row(lrow)) * 16;
 
-  // acc[tj][4q + r] is weight row 8q + 4 * (lane >> 5) + r of this wavefront's 32, token row
-  // tj * 32 + (lane & 31) of the tile.
-  auto epilogue = [&](const Task& tk, const TileAux& ax, v16i (&acc)[2]) {
+  // Token row th * MF + lrow of the tile; acc[i][4q + r] is weight row MF * i + 8q + 4 * lgrp + r (q = 0 for
+  // the 16-row tiles) of this wavefront's 32.
+  auto epilogue = [&](const Task& tk, const TileAux& ax, typename F::Acc (&acc)[NI]) {
+    const int row = th * S::MF + lrow;
+    const int32_t tok = ax.ids[row];
+    if (tok < 0 || tok >= p.P) return;
+    auto piece = [&](int j, int (&v)[4]) {  // weight rows 8 * j + 4 * lgrp + r (j = 0..3); 16-row tiles: 16 * j + 4 * lgrp + r
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const int row = tj * 32 + lrow;
-      const int32_t tok = ax.ids[row];
-      if (tok < 0 || tok >= p.P) continue;
-      if constexpr (MODE == kAccI32) {
-        int32_t* out = static_cast<int32_t*>(p.out) + (int64_t)tok * p.N;
+      for (int r = 0; r < 4; ++r) v[r] = S::MF == 32 ? acc[0][(4 * j + r) % F::kRegs] : acc[j % NI][r];
+    };
+    constexpr int kPieces = S::MF == 32 ? 4 : 2;
+    constexpr int kPieceRows = S::MF == 32 ? 8 : 16;
+    if constexpr (MODE == kGateUpSilu) {
+      // weight rows 0..15 of the wavefront are gate channels, 16..31 the matching up channels
+      uint16_t* out = static_cast<uint16_t*>(p.out) + (int64_t)tok * inter;
+      const float as = ax.a_scale[row];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = tk.ct * kCh + 32 * wave + 8 * q + 4 * lhalf;
-          if (n < p.N)
-            *reinterpret_cast<v4i*>(out + n) =
-                v4i{acc[tj][4 * q], acc[tj][4 * q + 1], acc[tj][4 * q + 2], acc[tj][4 * q + 3]};
-        }
-      } else if constexpr (MODE == kDown) {
-        uint16_t* out = static_cast<uint16_t*>(p.out) + (int64_t)tok * p.N;
-        const float as = ax.a_scale[row];
-        const float rw = p.row_weight ? ax.row_w[row] : 1.0f;
+      for (int j = 0; j < kPieces / 2; ++j) {
+        const int c = 16 * cg + kPieceRows * j + 4 * lgrp;
+        const int n = tk.ct * 64 + c;
+        const float4 wg = *reinterpret_cast<const float4*>(ax.w_scale + c);
+        const float4 wu = *reinterpret_cast<const float4*>(ax.w_scale + 64 + c);
+        int g[4], u[4];
+        piece(j, g);
+        piece(j + kPieces / 2, u);
+        if (n < inter) *reinterpret_cast<uint2*>(out + n) = silu_mul_epilogue4(g, u, as, wg, wu);
+      }
+    } else {
+      const float as = MODE == kDown ? ax.a_scale[row] : 0.0f;
+      const float rw = MODE == kDown && p.row_weight ? ax.row_w[row] : 1.0f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int c = 32 * wave + 8 * q + 4 * lhalf;
-          const int n = tk.ct * kCh + c;
+      for (int j = 0; j < kPieces; ++j) {
+        const int c = 32 * cg + kPieceRows * j + 4 * lgrp;
+        const int n = tk.ct * kCh + c;
+        if (n >= p.N) continue;
+        int v[4];
+        piece(j, v);
+        if constexpr (MODE == kAccI32) {
+          *reinterpret_cast<v4i*>(static_cast<int32_t*>(p.out) + (int64_t)tok * p.N + n) = v4i{v[0], v[1], v[2], v[3]};
+        } else {
           const float4 ws = *reinterpret_cast<const float4*>(ax.w_scale + c);
-          const int v[4] = {acc[tj][4 * q], acc[tj][4 * q + 1], acc[tj][4 * q + 2], acc[tj][4 * q + 3]};
-          if (n < p.N) *reinterpret_cast<uint2*>(out + n) = down_epilogue4(v, as, ws, rw);
-        }
-      } else {
-        // weight rows 0..15 of the wavefront are gate channels, 16..31 the matching up channels
-        uint16_t* out = static_cast<uint16_t*>(p.out) + (int64_t)tok * inter;
-        const float as = ax.a_scale[row];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int c = 16 * wave + 8 * q + 4 * lhalf;
-          const int n = tk.ct * 64 + c;
-          const float4 wg = *reinterpret_cast<const float4*>(ax.w_scale + c);
-          const float4 wu = *reinterpret_cast<const float4*>(ax.w_scale + 64 + c);
-          const int g[4] = {acc[tj][4 * q], acc[tj][4 * q + 1], acc[tj][4 * q + 2], acc[tj][4 * q + 3]};
-          const int u[4] = {acc[tj][4 * q + 8], acc[tj][4 * q + 9], acc[tj][4 * q + 10], acc[tj][4 * q + 11]};
-          if (n < inter) *reinterpret_cast<uint2*>(out + n) = silu_mul_epilogue4(g, u, as, wg, wu);
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)tok * p.N + n) = down_epilogue4(v, as, ws, rw);
         }
       }
     }
   };
 
-  // ---- start-up: the first task's token ids, its weights (which need no ids) behind them, then
-  // what depends on the ids: token rows and scales ----
-  int it = blockIdx.x / kXcds;
-  Task tk = find_task(it);
+  // ---- start-up: the first task's weights need nothing but its expert; then what depends on its row ids.
+  // Then the rows of the second task (its loads start `ahead` steps before the first one's last).
+  if (total == 0) return;
+  look_up();
+  Task tk = next_task();
   if (tk.e < 0) return;
-  int par = 0;
-  TaskLoads ld;
+  TaskLoads ld, nld;
+  constexpr int kEarly = 2;  // steps whose weights are requested before the row ids are in
   issue_ids(tk, aux[0]);
   setup_weight_loads(tk, ld);
-  issue_weights(ld, 0, 0);
-  issue_weights(ld, 1, kBK);
-  wait_vmcnt<8>();  // the ids are in; every wavefront fetched its own copy, so no barrier is needed
+#pragma unroll
+  for (int s = 0; s < kEarly; ++s) issue_weights(ld, s, s * kStepBytes);
+  Task nx = next_task();
+  issue_ids(nx.e >= 0 ? nx : tk, aux[1]);
+  Task n2 = next_task();
+  // the ids of the first task are the oldest load; every wavefront fetched its own copy, so no barrier is needed
+  wait_vmcnt<2 * kEarly>();
   setup_token_loads(aux[0], ld);
+#pragma unroll
+  for (int s = 0; s < kEarly; ++s) issue_tokens(ld, s, s * kStepBytes);
   issue_scales(tk, aux[0]);
-  issue_tokens(ld, 0, 0);
-  issue_tokens(ld, 1, kBK);
-  int last_group = kFirstGroup;  // size of the most recent group of loads: the token rows of step 1
-  int nit = it + stride;
-  Task nx = find_task(nit);
-  int nnit = nit;
-  Task nnx = nx;
-  TaskLoads nld = ld;
+  for (int s = kEarly; s < ahead; ++s) {
+    issue_weights(ld, s, s * kStepBytes);
+    issue_tokens(ld, s, s * kStepBytes);
+  }
+  nld = ld;
+  wait_all_but(ahead - kEarly);  // steps 0 and 1 (their loads are not in the order of the steps)
 
-  bool landed = false;  // the loads of the coming step are known to have landed (waited for before the stores)
-  int stage = 0;        // ring position of the step being multiplied
+  int par = 0;    // aux of the current task; the next ones follow
+  int stage = 0;  // ring position of the step being multiplied
+  bool fresh = true;
   while (true) {
-    v16i acc[2];
+    typename F::Acc acc[NI];
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[tj][r] = 0;
+      for (int r = 0; r < F::kRegs; ++r) acc[i][r] = 0;
+    // a wavefront whose half of the tile is padding (valid rows are a prefix) only loads
+    const int32_t half_first = __builtin_amdgcn_readfirstlane(aux[par].ids[th * S::MF]);
+    const bool active = half_first >= 0 && half_first < p.P;
+    TileAux& ax_next = aux[par + 1 < 3 ? par + 1 : par - 2];
+    TileAux& ax_n2 = aux[par + 2 < 3 ? par + 2 : par - 1];
 
     for (int s = 0; s < nk; ++s) {
-      // this wavefront's loads of step s have landed (only the group issued last is still in flight) ...
-      if (!landed) wait_all_but<MODE>(last_group);
-      landed = false;
+      // this wavefront's loads of step s have landed ...
+      if (!fresh) wait_all_but(ahead - 1);
+      fresh = false;
       // ... and so have everybody's; everybody is also done reading the stage that is filled next
-      __builtin_amdgcn_s_barrier();
-      const int fill = stage >= 1 ? stage - 1 : kStages - 1;  // (stage + 2) % 3
-      last_group = kStageLoads;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      int fill = stage + ahead;
+      if (fill >= kStages) fill -= kStages;
       if (s == 0) {
-        // ids of the next tile (of this one again if it is the last: harmless)
-        issue_ids(nx.e >= 0 ? nx : tk, aux[par ^ 1]);
-        last_group = kStageLoads + 1;
-      } else if (s == 2) {
-        // they are in (issued two steps ago): the next tile's row addresses and scales
-        const Task& t2 = nx.e >= 0 ? nx : tk;
-        setup_weight_loads(t2, nld);
-        setup_token_loads(aux[par ^ 1], nld);
-        issue_scales(t2, aux[par ^ 1]);
-        last_group = kStageLoads + aux_loads<MODE>();
+        // the next task's rows (their ids were fetched a task ago) and, for the one after it, the ids
+        const Task& t1 = nx.e >= 0 ? nx : tk;
+        setup_weight_loads(t1, nld);
+        setup_token_loads(nx.e >= 0 ? ax_next : aux[par], nld);
+        if (n2.e >= 0) issue_ids(n2, ax_n2);
       }
-      if (s + 2 < nk)
-        issue_stage(ld, fill, (s + 2) * kBK);
-      else if (nx.e >= 0)
-        issue_stage(nld, fill, (s + 2 - nk) * kBK);
-      else
-        issue_stage(ld, fill, (nk - 1) * kBK);  // nothing left to fetch: keeps the group sizes uniform
-      if (s == 3 && nx.e >= 0) {
-        // The task after the next is looked up here, where the wait for the two scalar loads hides
-        // behind the loads just issued, and not between two tiles.
-        nnit = nit + stride;
-        nnx = find_task(nnit);
-      }
+      // Operands first, then the loads of the step `ahead` of this one a piece at a time between the
+      // multiplications: the address unit takes 16 clocks per load and the whole workgroup's 20-24 of them in front
+      // of the operand reads made a step 0.45 us even where every load hit L2.
       const char* st = stages + stage * kStageBytes;
+      v4i a[F::kSub][NI], b[F::kSub];
+      if (active) {
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const v4i a = *reinterpret_cast<const v4i*>(st + w_ld + chunk[kk]);
-        const v4i b0 = *reinterpret_cast<const v4i*>(st + x_ld[0] + chunk[kk]);
-        const v4i b1 = *reinterpret_cast<const v4i*>(st + x_ld[1] + chunk[kk]);
-        acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b0, acc[0], 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b1, acc[1], 0, 0, 0);
+        for (int kk = 0; kk < F::kSub; ++kk) {
+          b[kk] = *reinterpret_cast<const v4i*>(st + x_ld + chunk[kk]);
+#pragma unroll
+          for (int i = 0; i < NI; ++i) a[kk][i] = *reinterpret_cast<const v4i*>(st + w_ld[i] + chunk[kk]);
+        }
       }
+      // the step fetched: of this task, of the next one, or (nothing left) the last one again, which keeps the
+      // counts uniform
+      const bool in_task = s + ahead < nk || nx.e < 0;
+      const int fs = s + ahead < nk ? s + ahead : nx.e < 0 ? nk - 1 : s + ahead - nk;
+      const int8_t* wsrc = (in_task ? ld.wbase : nld.wbase) + fs * kStepBytes;
+      const bool nt = in_task ? ld.stream : nld.stream;
+      const uint32_t wdst = stage0 + fill * kStageBytes + wave * 2048;
+      const uint32_t w0 = in_task ? ld.woff[0] : nld.woff[0], w1 = in_task ? ld.woff[1] : nld.woff[1];
+      const uint32_t x0 = in_task ? ld.xoff : nld.xoff;
+      auto mul = [&](int kk) {
+        if (active)
+#pragma unroll
+          for (int i = 0; i < NI; ++i) acc[i] = F::mul(a[kk][i], b[kk], acc[i]);
+      };
+      auto one_weight = [&](uint32_t off, uint32_t dst) {
+        if (nt)
+          load_to_lds_16_stream(wsrc, off, dst);
+        else
+          load_to_lds_16(wsrc, off, dst);
+      };
+      mul(0);
+      one_weight(w0, wdst);
+      if constexpr (F::kSub == 4) mul(1);
+      one_weight(w1, wdst + 1024);
+      mul(F::kSub == 4 ? 2 : 1);
+      if (loads_tokens) load_to_lds_16(p.a_q + fs * kStepBytes, x0, stage0 + fill * kStageBytes + kTokOffset + wave * 1024);
+      if constexpr (F::kSub == 4) mul(3);
+      if (s == 1 && nx.e >= 0) issue_scales(nx, ax_next);
       stage = stage + 1 < kStages ? stage + 1 : 0;
     }
-    // Before the stores, everything but the group issued in the last step is complete: the coming
-    // step's loads have landed, and the stores need not be counted by the next wait.
-    wait_all_but<MODE>(last_group);
-    landed = true;
-    epilogue(tk, aux[par], acc);
+    // Before the stores the coming step's loads have landed, and the next wait need not get past them.
+    wait_all_but(ahead - 1);
+    fresh = true;
+    if (active) epilogue(tk, aux[par], acc);
     if (nx.e < 0) break;
     tk = nx;
     ld = nld;
-    par ^= 1;
-    it = nit;
-    nit = nnit;
-    nx = nnx;
+    nx = n2;
+    n2 = next_task();
+    par = par + 1 < 3 ? par + 1 : 0;
   }
   wait_vmcnt<0>();
 }
 
-template <int MODE>
+template <int MODE, int TOK>
 hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   NarrowParams p;
   p.a_q = a.a_q;
@@ -481,9 +465,18 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.B = a.block_size;
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 63) / 64 : (a.n + kCh - 1) / kCh;
   p.out = a.out;
-  const int grid = 2 * (device_cu_count() / kXcds * kXcds);  // two workgroups per compute unit
-  hipLaunchKernelGGL(gemm_narrow_kernel<MODE>, dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
+  const int grid = device_cu_count() / kXcds * kXcds;
+  hipLaunchKernelGGL((gemm_narrow_kernel<MODE, TOK>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
   return hipGetLastError();
+}
+
+// Tiles of 32 token rows where no expert can hold more (a block's second half would be all padding): the
+// smaller stage leaves room for a seventh one and a third of the token loads goes away (17 tokens 84.6 -> 81.6 us,
+// 40 tokens 109.5 -> 107.0).  Beyond that one expert with more rows would make its weights travel twice (skewed
+// routing, 45 tokens: 139.6 -> 151.5).
+bool small_tiles(const GemmArgs& a) {
+  const int64_t most_rows = a.max_rows_per_expert > 0 && a.max_rows_per_expert < a.num_pairs ? a.max_rows_per_expert : a.num_pairs;
+  return most_rows <= 32;
 }
 
 }  // namespace
@@ -492,16 +485,17 @@ bool gemm_narrow_supports(const GemmArgs& a) {
   // per-lane source offsets are 32-bit: one expert's weights, the activation matrix and the per-pair
   // arrays must each span less than 4 GiB
   const int64_t act_rows = (a.num_pairs + a.row_div - 1) / a.row_div;
-  return (a.block_size == 64 || a.block_size == 128) && a.k % kBK == 0 && a.k >= kMinSteps * kBK && a.n % 16 == 0 &&
+  return (a.block_size == 64 || a.block_size == 128) && a.k % kStepBytes == 0 && a.k >= kMinSteps * kStepBytes && a.n % 16 == 0 &&
          (int64_t)a.n * a.k < (1ll << 32) && act_rows * a.k < (1ll << 32) && a.num_pairs < (1ll << 30) &&
-         a.sorted_cap / kTok * ((a.n + 63) / 64) < (1ll << 31);
+         a.sorted_cap / 32 * ((a.n + 63) / 64) < (1ll << 31);
 }
 
 hipError_t launch_gemm_narrow(const GemmArgs& a, hipStream_t stream) {
+  const bool small = small_tiles(a);
   switch (a.mode) {
-    case kGateUpSilu: return launch_mode<kGateUpSilu>(a, stream);
-    case kDown: return launch_mode<kDown>(a, stream);
-    case kAccI32: return launch_mode<kAccI32>(a, stream);
+    case kGateUpSilu: return small ? launch_mode<kGateUpSilu, 32>(a, stream) : launch_mode<kGateUpSilu, 64>(a, stream);
+    case kDown: return small ? launch_mode<kDown, 32>(a, stream) : launch_mode<kDown, 64>(a, stream);
+    case kAccI32: return small ? launch_mode<kAccI32, 32>(a, stream) : launch_mode<kAccI32, 64>(a, stream);
     default: return hipErrorInvalidValue;
   }
 }

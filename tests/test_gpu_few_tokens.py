@@ -44,3 +44,22 @@ def test_combine_at_every_k(pra, oracle, k, M, H):
     out = torch.empty(M, H, dtype=torch.bfloat16, device=DEV)
     pra.moe_sum(x.to(DEV), out)
     assert torch.equal(out.cpu(), oracle.moe_sum(x))
+
+
+@pytest.mark.parametrize("E,k,H,I,M,B", [
+    (3, 1, 512, 512, 17, 64), (40, 8, 640, 768, 20, 64), (5, 5, 1408, 896, 32, 128), (128, 2, 512, 1024, 33, 64),
+    (300, 4, 2048, 512, 90, 128), (2, 2, 4096, 1408, 65, 64), (700, 6, 512, 640, 31, 64),
+])
+def test_narrow_tiles_at_short_reductions_and_many_tasks(pra, oracle, E, k, H, I, M, B):
+    """The narrow family at its shortest reductions (where its loads run fewer steps ahead), with 32- and 64-row
+    tiles, one task per workgroup and more than 64 candidates per workgroup."""
+    im = inputs_mod()
+    d = im.make_inputs(im.LayerShape("n", E=E, k=k, H=H, I=I, routing="zipf"), M, seed=E + M).to(DEV)
+    s, e, npp = pra.moe_align_block_size(d.topk_ids, B, E)
+    xq, a1 = pra.per_token_quant_int8(d.hidden_states)
+    for w, row_div, a in ((d.w1, k, xq), (d.w2, 1, torch.randint(-127, 128, (M * k, I), dtype=torch.int8, device=DEV))):
+        got = pra.gemm_acc_i32(a, w, s, e, npp, row_div, B, M * k, "narrow")
+        assert torch.equal(got, pra.gemm_acc_i32(a, w, s, e, npp, row_div, B, M * k, "stream"))
+    kw = d.fused_experts_kwargs()
+    out = pra.fused_experts(*d.fused_experts_args(), **kw, block_size_m=B, gemm_variant="narrow")
+    assert torch.equal(out, pra.fused_experts(*d.fused_experts_args(), **kw, block_size_m=B, gemm_variant="stream"))
