@@ -226,7 +226,8 @@ struct GemmArgs {
   int tile_geometry = 0;            // LDS-tiled family: kTileAuto, kTileWide (256-row tiles), kTileDeep (128-row tiles) or kTileRing (256-row tiles, four-stage ring; on demand only)
 };
 constexpr int kTileAuto = 0, kTileWide = 1, kTileDeep = 2, kTileRing = 3;
-constexpr int kTileDeepRowsPerExpert = 96;  // the LDS-tiled family picks its deep geometry up to this many routed rows per expert
+// The LDS-tiled family picks its deep geometry up to this many routed rows per expert (launches with 2 GB of weights and more: fewer).
+constexpr int kTileDeepRowsPerExpert = 96, kTileDeepRowsLongStream = 64;
 hipError_t launch_gemm_stream(const GemmArgs& a, hipStream_t stream);
 // register-only int8 MFMA loop (measurement aid): sink holds mfma_probe_sink_bytes(workgroups)
 int64_t mfma_probe_sink_bytes(int workgroups);
@@ -241,6 +242,8 @@ hipError_t launch_gemm_tile(const GemmArgs& a, hipStream_t stream);
 bool gemm_tile_supports(const GemmArgs& a);
 bool gemm_tile_prefers_deep(const GemmArgs& a);
 int gemm_tile_geometry(const GemmArgs& a);  // kTileWide or kTileDeep (kTileRing on demand): what a launch of the family would use
+bool gemm_wide_supports(const GemmArgs& a);
+hipError_t launch_gemm_wide(const GemmArgs& a, hipStream_t stream);
 hipError_t launch_gemm_narrow(const GemmArgs& a, hipStream_t stream);
 bool gemm_narrow_supports(const GemmArgs& a);
 

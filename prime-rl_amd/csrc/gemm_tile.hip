@@ -1,4 +1,5 @@
-// Grouped int8 GEMM for gfx950, LDS-tiled family (prefill: from a few dozen routed rows per expert up).
+// Grouped int8 GEMM for gfx950, LDS-tiled family: its deep tiles (around a hundred routed rows per expert), the
+// ring pipeline and the choice of the family's kernel; the wide tiles are in gemm_wide.hip.
 //
 // Persistent workgroups (one per CU, 512 threads = 8 wavefronts) walk a list of tiles.  A tile is
 // a run of 64-row moe_align sub-blocks of ONE expert (aligned to the start of the expert's segment)
@@ -6,15 +7,11 @@
 // (v_mfma_i32_32x32x32_i8) is used "transposed" (A operand = weight rows, B operand = token rows),
 // so a lane ends up with runs of 4 consecutive channels of one token.
 //
-// Two geometries (template parameter DEEP):
-//  * wide: up to 256 token rows per tile, two 64 KB LDS stages, loads one step ahead.  Wavefront w
-//    owns token sub-block w / 2 x channel half w % 2 as 4 x 2 MFMA tiles (128 accumulator VGPRs).
-//    Bound by the matrix pipe; a weight tile is reused by up to four sub-blocks.
-//  * deep: up to 128 token rows per tile, a ring of three 48 KB stages, loads two steps ahead.  With
-//    few rows per expert a step holds little arithmetic and the kernel is bound by the weight stream
-//    from HBM, i.e. by the bytes a compute unit keeps in flight.  All eight wavefronts multiply in
-//    every task: with two active sub-blocks wavefront w owns sub-block w / 4 and a quarter of the
-//    channels, with one an eighth of the channels.
+// Deep tiles hold up to 128 token rows, with a ring of three 48 KB stages and loads two steps ahead.  With
+// few rows per expert a step holds little arithmetic and the kernel is bound by the weight stream
+// from HBM, i.e. by the bytes a compute unit keeps in flight.  All eight wavefronts multiply in
+// every task: with two active sub-blocks wavefront w owns sub-block w / 4 and a quarter of the
+// channels, with one an eighth of the channels.
 //
 // Both operands go global -> LDS directly (global_load_lds_dwordx4: no staging registers, no
 // ds_write), with one s_barrier per step and explicit vmcnt waits.  Every wavefront-level load
@@ -41,18 +38,11 @@ constexpr int kBN = 256;       // weight rows per tile
 constexpr int kBK = 128;       // reduction bytes per step
 constexpr int kTokOffset = kBN * kBK;
 
-// Two geometries.  Wide: tiles of up to 256 token rows, two 64 KB stages (loads one step ahead).
-// Deep: tiles of up to 128 token rows, a ring of three 48 KB stages (loads two steps ahead): with
-// few rows per expert a step holds little arithmetic, and what bounds the kernel is how many bytes
-// of the weight stream a compute unit keeps in flight.
-template <bool DEEP>
-struct Geometry {
-  static constexpr int kTileTok = DEEP ? 128 : 256;               // token rows per tile
-  static constexpr int kSlots = DEEP ? 3 : 2;                     // LDS stages
-  static constexpr int kStageBytes = (kBN + kTileTok) * kBK;      // 48 KB | 64 KB
-  static constexpr int kMaxTiles = DEEP ? 2048 : 6144;            // capacity of the in-LDS tile list
-  static constexpr int kTokLoads = kTileTok / 64;                 // wave-level loads of 8 token rows per wavefront and step
-};
+constexpr int kTileTok = 128;                          // token rows per tile
+constexpr int kSlots = 3;                              // LDS stages
+constexpr int kStageBytes = (kBN + kTileTok) * kBK;    // 48 KB
+constexpr int kMaxTiles = 2048;                        // capacity of the in-LDS tile list
+constexpr int kTokLoads = kTileTok / 64;               // wave-level loads of 8 token rows per wavefront and step
 constexpr int kXcds = 8;
 constexpr int kGroupTiles = 8;  // token tiles of one expert whose tasks are interleaved per channel tile
 
@@ -279,9 +269,8 @@ struct TaskLoads {
 // Weights: lane fills LDS slot (lane & 7) of row 32 * wave + 8 * i + (lane >> 3): it fetches the logical
 // chunk (lane & 7) ^ swizzle(row) of that row, and swizzle(row) = (lane >> 3) ^ (i & 1).  Token rows
 // likewise, of row (8 * kTokLoads) * wave + 8 * i + (lane >> 3).
-template <int MODE, bool DEEP>
+template <int MODE>
 __device__ __forceinline__ void setup_loads(const TileParams& p, const Task& tk, int wave, int lane, TaskLoads& ld) {
-  constexpr int kTokLoads = Geometry<DEEP>::kTokLoads;
   const int K = p.K;
   const int inter = p.N / 2;
 #pragma unroll
@@ -310,13 +299,11 @@ __device__ __forceinline__ void setup_loads(const TileParams& p, const Task& tk,
   ld.wbase = p.w + (int64_t)tk.e * p.N * K;
 }
 
-// `tokens`: this wavefront's token rows belong to an active sub-block.  The deep geometry issues the
-// token loads regardless (rows of inactive sub-blocks fetch row 0), so that every wavefront has the
-// same number of loads in flight per step and the counted waits of the ring hold for all of them.
-template <bool DEEP, bool NT>
+// The token loads are issued regardless of the active sub-blocks (rows of inactive ones fetch row 0), so that
+// every wavefront has the same number of loads in flight per step and the counted waits of the ring hold for all.
+template <bool NT>
 __device__ __forceinline__ void issue_stage_loads(const TaskLoads& ld, const int8_t* a_q, uint32_t stage_addr,
-                                                  int wave, int koff, bool tokens) {
-  constexpr int kTokLoads = Geometry<DEEP>::kTokLoads;
+                                                  int wave, int koff) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if constexpr (NT)
@@ -324,11 +311,9 @@ __device__ __forceinline__ void issue_stage_loads(const TaskLoads& ld, const int
     else
       load_to_lds_16(ld.wbase + koff, ld.woff[i], stage_addr + (wave * 4 + i) * 1024);
   }
-  if (DEEP || tokens) {
 #pragma unroll
-    for (int i = 0; i < kTokLoads; ++i)
-      load_to_lds_16(a_q + koff, ld.xoff[i], stage_addr + kTokOffset + (wave * kTokLoads + i) * 1024);
-  }
+  for (int i = 0; i < kTokLoads; ++i)
+    load_to_lds_16(a_q + koff, ld.xoff[i], stage_addr + kTokOffset + (wave * kTokLoads + i) * 1024);
 }
 
 struct TileReads {
@@ -337,12 +322,10 @@ struct TileReads {
   int chunk[4];  // swizzled byte offset of logical chunk 2 * kk + (lane >> 5)
 };
 
-// How the eight wavefronts share a task.  A task with NCI = 4 has three or four active 64-row
-// sub-blocks: wavefront w owns sub-block w / 2 and half of the channels (4 MFMA tiles of 32 weight
-// rows, twice 32 token rows).  With two active sub-blocks (NCI = 2) it owns sub-block w / 4 and a
-// quarter of the channels, with one (NCI = 1) an eighth of the channels: every wavefront multiplies
-// in every task, so a tile with few rows costs its loads and not the serial MFMA chain of the one
-// or two wavefronts its rows would otherwise belong to.
+// How the eight wavefronts share a task.  With two active sub-blocks (NCI = 2) wavefront w owns sub-block w / 4
+// and a quarter of the channels (two MFMA tiles of 32 weight rows, twice 32 token rows), with one (NCI = 1) an
+// eighth of the channels: every wavefront multiplies in every task, so a tile with few rows costs its loads
+// and not the serial MFMA chain of the one or two wavefronts its rows would otherwise belong to.
 template <int MODE, int NCI>
 __device__ __forceinline__ void make_reads(int wave, int lane, TileReads& rd) {
   constexpr int kParts = 8 / NCI;
@@ -354,9 +337,7 @@ __device__ __forceinline__ void make_reads(int wave, int lane, TileReads& rd) {
     int row;
     if constexpr (MODE == kGateUpSilu) {
       // LDS rows 0..127 hold gate channels, 128..255 the matching up channels
-      if constexpr (NCI == 4)
-        row = (ci < 2 ? 0 : 128) + cpart * 64 + (ci & 1) * 32 + lrow;
-      else if constexpr (NCI == 2)
+      if constexpr (NCI == 2)
         row = ci * 128 + cpart * 32 + lrow;
       else
         row = (lrow < 16 ? 0 : 128 - 16) + cpart * 16 + lrow;  // 16 gate rows, then their 16 up rows
@@ -388,26 +369,6 @@ __device__ __forceinline__ void multiply_stage(const TileReads& rd, const char* 
 #pragma unroll
       for (int tj = 0; tj < 2; ++tj)
         acc[ci][tj] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[kk][ci], b[kk][tj], acc[ci][tj], 0, 0, 0);
-  if constexpr (NCI == 4) {
-    // Fine interleave, one group ahead: the first MFMA issues as soon as three operands are in and
-    // every later read is issued at least one MFMA group before its first use, so it is hidden
-    // behind MFMAs already queued (8 wavefronts share the LDS: a long burst of reads in front of the
-    // first MFMA would leave the matrix pipe idle at the start of every step).
-    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);  // b0 a0 b1 of sub-step 0
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a0 b0
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a1
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a0 b1
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a2
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // a1
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a3
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // a2
-      if (kk < 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // next b0 a0
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // a3
-      if (kk < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // next b1
-    }
-  }
 }
 
 // acc[ci][tj][4q + r] is weight row 32 * ci + 8q + 4 * (lane >> 5) + r of the wavefront's MFMA tiles
@@ -549,12 +510,10 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
   }
 }
 
-template <int MODE, bool DEEP>
+template <int MODE>
 __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
-  using G = Geometry<DEEP>;
-  constexpr int kStageBytes = G::kStageBytes;
-  __shared__ __align__(16) char stages[G::kSlots * kStageBytes];
-  __shared__ uint32_t tile_desc[G::kMaxTiles];
+  __shared__ __align__(16) char stages[kSlots * kStageBytes];
+  __shared__ uint32_t tile_desc[kMaxTiles];
   __shared__ int wave_part[kWaves];
   __shared__ __align__(16) float channel_scales[kWaves * 128];
   __shared__ int total_tiles;
@@ -562,19 +521,18 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int load_sub = wave * G::kTokLoads / 8;  // token sub-block whose rows this wavefront loads
   const int nk = p.K / kBK;
 
   const int npp = *p.npp;
   const int nblocks = npp / p.B;
   const int sub_per_block = p.B / 64;
-  const int per_tile = G::kTileTok / p.B;  // 1, 2 or 4 blocks
+  const int per_tile = kTileTok / p.B;  // 1 or 2 blocks
   const int ntile =
-      p.ascend ? build_tile_list_ascending(p.expert_ids, nblocks, p.E, per_tile == 4 ? 2 : per_tile == 2 ? 1 : 0,
+      p.ascend ? build_tile_list_ascending(p.expert_ids, nblocks, p.E, per_tile == 2 ? 1 : 0,
                                            reinterpret_cast<int*>(stages), wave_part, tile_desc, &total_tiles,
-                                           G::kMaxTiles)
+                                           kMaxTiles)
                : build_tile_list(p.expert_ids, nblocks, per_tile, reinterpret_cast<int*>(stages), wave_part, tile_desc,
-                                 &total_tiles, G::kMaxTiles);
+                                 &total_tiles, kMaxTiles);
   const int total = ntile * p.ntiles;
   const int per_xcd = (total + kXcds - 1) / kXcds;
   const int xcd = blockIdx.x % kXcds;
@@ -630,14 +588,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
   while (tk.e == -2) tk = decode(it += stride);
   if (tk.e < 0) return;
   TaskLoads ld;
-  setup_loads<MODE, DEEP>(p, tk, wave, lane, ld);
-  bool my_tokens = load_sub < tk.nsub;
+  setup_loads<MODE>(p, tk, wave, lane, ld);
   int slot = 0;  // stage of the step being multiplied
   // The scratch of the tile list lived in the stage memory; everybody is past it (the builder ends
-  // with a barrier), so the first stage(s) can be filled now.
-  issue_stage_loads<DEEP, NT>(ld, p.a_q, stage0, wave, 0, my_tokens);
-  if constexpr (DEEP) issue_stage_loads<DEEP, NT>(ld, p.a_q, stage0 + kStageBytes, wave, kBK, my_tokens);
-  constexpr int kLoadsPerStep = 4 + G::kTokLoads;  // per wavefront (deep geometry: always that many)
+  // with a barrier), so the first stages can be filled now.
+  issue_stage_loads<NT>(ld, p.a_q, stage0, wave, 0);
+  issue_stage_loads<NT>(ld, p.a_q, stage0 + kStageBytes, wave, kBK);
+  constexpr int kLoadsPerStep = 4 + kTokLoads;  // per wavefront
 
   bool stores_pending = false;
   while (true) {
@@ -646,11 +603,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
     Task nx = decode(nit);
     while (nx.e == -2) nx = decode(nit += stride);
     TaskLoads nld = ld;
-    if (nx.e >= 0) setup_loads<MODE, DEEP>(p, nx, wave, lane, nld);
-    const bool nx_tokens = load_sub < nx.nsub;
+    if (nx.e >= 0) setup_loads<MODE>(p, nx, wave, lane, nld);
 
-    // NCI = MFMA tiles of 32 weight rows per wavefront; `active`: the wavefront multiplies in this task
-    auto run_task = [&](auto nci_tag, bool active) {
+    // NCI = MFMA tiles of 32 weight rows per wavefront
+    auto run_task = [&](auto nci_tag) {
       constexpr int NCI = decltype(nci_tag)::value;
       v16i acc[NCI][2];
 #pragma unroll
@@ -664,52 +620,42 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
         // This wavefront's loads of step s have landed ...  A wavefront that has just run an
         // epilogue waited for all its loads there and only has the epilogue's stores pending: it
         // lets them drain behind the first step instead of stalling on them.
-        if constexpr (DEEP) {
-          // in flight behind step s: the loads of step s + 1 (issued one step ago), if there is one
-          if (s > 0 || !stores_pending) {
-            if (s + 1 < nk || nx.e >= 0)
-              wait_vmcnt<kLoadsPerStep>();
-            else
-              wait_vmcnt<0>();
-          }
-        } else {
-          if (s > 0 || !stores_pending) wait_vmcnt<0>();
+        // in flight behind step s: the loads of step s + 1 (issued one step ago), if there is one
+        if (s > 0 || !stores_pending) {
+          if (s + 1 < nk || nx.e >= 0)
+            wait_vmcnt<kLoadsPerStep>();
+          else
+            wait_vmcnt<0>();
         }
         // ... and so have everybody's; everybody is also done reading the stage of the step before,
         // which is the one to fill next
         __builtin_amdgcn_s_barrier();
-        constexpr int kAhead = G::kSlots - 1;
+        constexpr int kAhead = kSlots - 1;
         int fill = slot + kAhead;
-        if (fill >= G::kSlots) fill -= G::kSlots;
+        if (fill >= kSlots) fill -= kSlots;
         const uint32_t fill_addr = stage0 + fill * kStageBytes;
         if (s + kAhead < nk)
-          issue_stage_loads<DEEP, NT>(ld, p.a_q, fill_addr, wave, (s + kAhead) * kBK, my_tokens);
+          issue_stage_loads<NT>(ld, p.a_q, fill_addr, wave, (s + kAhead) * kBK);
         else if (nx.e >= 0)
-          issue_stage_loads<DEEP, NT>(nld, p.a_q, fill_addr, wave, (s + kAhead - nk) * kBK, nx_tokens);
-        if (active) multiply_stage<NCI>(rd, stages + slot * kStageBytes, acc);
-        slot = slot + 1 == G::kSlots ? 0 : slot + 1;
+          issue_stage_loads<NT>(nld, p.a_q, fill_addr, wave, (s + kAhead - nk) * kBK);
+        multiply_stage<NCI>(rd, stages + slot * kStageBytes, acc);
+        slot = slot + 1 == kSlots ? 0 : slot + 1;
       }
       // everybody is done reading the stage of the last step: it becomes the epilogue's staging area
       // (the next task's first loads went to the other stages)
       __builtin_amdgcn_s_barrier();
-      const int last = slot == 0 ? G::kSlots - 1 : slot - 1;
-      if (active)
-        epilogue<MODE, NCI>(p, tk, wave, lane, acc, stages + last * kStageBytes + wave * 8192 / (4 / NCI),
+      const int last = slot == 0 ? kSlots - 1 : slot - 1;
+      epilogue<MODE, NCI>(p, tk, wave, lane, acc, stages + last * kStageBytes + wave * 8192 / (4 / NCI),
                             channel_scales + wave * 128);
-      stores_pending = active && MODE != kAccI32;
+      stores_pending = MODE != kAccI32;
     };
-    if constexpr (DEEP) {
-      if (tk.nsub >= 2)
-        run_task(std::integral_constant<int, 2>{}, true);
-      else
-        run_task(std::integral_constant<int, 1>{}, true);
-    } else {
-      run_task(std::integral_constant<int, 4>{}, load_sub < tk.nsub);
-    }
+    if (tk.nsub >= 2)
+      run_task(std::integral_constant<int, 2>{});
+    else
+      run_task(std::integral_constant<int, 1>{});
     if (nx.e < 0) break;
     tk = nx;
     ld = nld;
-    my_tokens = nx_tokens;
     it = nit;
   }
   wait_vmcnt<0>();
@@ -1110,7 +1056,7 @@ bool ring_supports(const GemmArgs& a) {
   return tiles <= 6144 && blocks <= (int64_t)(kRingSlots * kRingStage / sizeof(int)) && blocks <= 65535;
 }
 
-template <int MODE, bool DEEP, bool RING = false>
+template <int MODE, bool RING>
 hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   TileParams p;
   p.a_q = a.a_q;
@@ -1134,45 +1080,45 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   if constexpr (RING)
     hipLaunchKernelGGL((gemm_ring_kernel<MODE>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
   else
-    hipLaunchKernelGGL((gemm_tile_kernel<MODE, DEEP>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((gemm_tile_kernel<MODE>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
   return hipGetLastError();
 }
 
-template <bool DEEP>
-bool geometry_supports(const GemmArgs& a) {
-  using G = Geometry<DEEP>;
+bool deep_supports(const GemmArgs& a) {
   // per-lane source offsets are 32-bit: one expert's weights and the activation matrix must each
   // span less than 4 GiB
   const int64_t act_rows = (a.num_pairs + a.row_div - 1) / a.row_div;
-  if (!((a.block_size == 64 || a.block_size == 128) && a.k % kBK == 0 && a.k >= G::kSlots * kBK && a.n % 16 == 0 &&
+  if (!((a.block_size == 64 || a.block_size == 128) && a.k % kBK == 0 && a.k >= kSlots * kBK && a.n % 16 == 0 &&
         (int64_t)a.n * a.k < (1ll << 32) && act_rows * a.k < (1ll << 32)))
     return false;
   // The tile list lives in LDS.  A run of equal expert ids of L blocks makes ceil(L / blocks per
   // tile) tiles; moe_align's ids ascend, so there is one run per expert.  Ids of unknown order could
   // make every block a tile of its own.  While the list is built the block ids sit in the stages.
   const int64_t blocks = (a.sorted_cap + a.block_size - 1) / a.block_size;
-  const int per_tile = G::kTileTok / a.block_size;
+  const int per_tile = kTileTok / a.block_size;
   const int64_t tiles = a.expert_ids_ascend ? (blocks + per_tile - 1) / per_tile + a.num_experts : blocks;
-  return tiles <= G::kMaxTiles && blocks <= (int64_t)(G::kSlots * G::kStageBytes / sizeof(int)) && blocks <= 65535;
+  return tiles <= kMaxTiles && blocks <= (int64_t)(kSlots * kStageBytes / sizeof(int)) && blocks <= 65535;
 }
 
 }  // namespace
 
 bool gemm_tile_supports(const GemmArgs& a) {
   switch (a.tile_geometry) {
-    case kTileWide: return geometry_supports<false>(a);
-    case kTileDeep: return geometry_supports<true>(a);
+    case kTileWide: return gemm_wide_supports(a);
+    case kTileDeep: return deep_supports(a);
     case kTileRing: return ring_supports(a);
-    default: return geometry_supports<false>(a) || geometry_supports<true>(a);
+    default: return gemm_wide_supports(a) || deep_supports(a);
   }
 }
 
-// Measured on three layer shapes (Qwen3-30B-A3B, GLM-4.5-Air, DeepSeek-V3): the deep geometry wins up
-// to about a hundred routed rows per expert, where a 256-row tile would be mostly padding and the
-// kernel is bound by the weight stream; beyond that the wide tile's reuse of a weight tile by up to
-// four sub-blocks wins.
+// Measured on three layer shapes (Qwen3-30B-A3B, GLM-4.5-Air, DeepSeek-V3): the deep tiles win where a 256-row
+// tile would be mostly padding and the kernel is bound by the weight stream.  Layer us at 64 / 80 / 96 / 107 routed
+// rows per expert, deep against wide: 155 / 165 / 171 / - against 162 / 170 / 177 / - with 0.2-0.4 GB of weights per
+// launch, 471 / - / - / 570 against 485 / - / - / 541 with 0.7-1.5 GB; with 3.8-7.5 GB 2040 / - / 2339 against 2015 / - /
+// 2234.
 bool gemm_tile_prefers_deep(const GemmArgs& a) {
-  return a.num_pairs <= (int64_t)kTileDeepRowsPerExpert * a.num_experts;
+  const bool long_stream = (int64_t)a.num_experts * a.n * a.k >= (2048ll << 20);
+  return a.num_pairs <= (int64_t)(long_stream ? kTileDeepRowsLongStream : kTileDeepRowsPerExpert) * a.num_experts;
 }
 
 // The geometry a launch of this family uses for `a` (kTileWide or kTileDeep; kTileRing only on demand).
@@ -1180,20 +1126,12 @@ int gemm_tile_geometry(const GemmArgs& a) {
   if (a.tile_geometry == kTileWide) return kTileWide;
   if (a.tile_geometry == kTileDeep) return kTileDeep;
   if (a.tile_geometry == kTileRing) return kTileRing;
-  return geometry_supports<true>(a) && (gemm_tile_prefers_deep(a) || !geometry_supports<false>(a)) ? kTileDeep : kTileWide;
+  return deep_supports(a) && (gemm_tile_prefers_deep(a) || !gemm_wide_supports(a)) ? kTileDeep : kTileWide;
 }
 
 hipError_t launch_gemm_tile(const GemmArgs& a, hipStream_t stream) {
   const int geometry = gemm_tile_geometry(a);
   if (geometry == kTileRing) {
-    switch (a.mode) {
-      case kGateUpSilu: return launch_mode<kGateUpSilu, false, true>(a, stream);
-      case kDown: return launch_mode<kDown, false, true>(a, stream);
-      case kAccI32: return launch_mode<kAccI32, false, true>(a, stream);
-      default: return hipErrorInvalidValue;
-    }
-  }
-  if (geometry == kTileDeep) {
     switch (a.mode) {
       case kGateUpSilu: return launch_mode<kGateUpSilu, true>(a, stream);
       case kDown: return launch_mode<kDown, true>(a, stream);
@@ -1201,12 +1139,15 @@ hipError_t launch_gemm_tile(const GemmArgs& a, hipStream_t stream) {
       default: return hipErrorInvalidValue;
     }
   }
-  switch (a.mode) {
-    case kGateUpSilu: return launch_mode<kGateUpSilu, false>(a, stream);
-    case kDown: return launch_mode<kDown, false>(a, stream);
-    case kAccI32: return launch_mode<kAccI32, false>(a, stream);
-    default: return hipErrorInvalidValue;
+  if (geometry == kTileDeep) {
+    switch (a.mode) {
+      case kGateUpSilu: return launch_mode<kGateUpSilu, false>(a, stream);
+      case kDown: return launch_mode<kDown, false>(a, stream);
+      case kAccI32: return launch_mode<kAccI32, false>(a, stream);
+      default: return hipErrorInvalidValue;
+    }
   }
+  return launch_gemm_wide(a, stream);
 }
 
 }  // namespace moe_i8
