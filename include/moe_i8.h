@@ -223,7 +223,9 @@ int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
 /*
  * What moe_i8_fused_experts would launch for a layer shape, decided on the host from the sizes alone (no GPU
  * call): the GEMM kernel of each projection (MOE_I8_GEMM_STREAM, _NARROW, _TILE_WIDE or _TILE_DEEP) and the
- * number of kernel launches of one call.  A diagnostic with no counterpart in the reference (upstream picks its
+ * number of kernel launches of one call through its chain of stages (alignment, quantisation, GEMMs, combine).
+ * Calls of a few tokens with MOE_I8_GEMM_AUTO replace that chain by two launches of their own; for them the answer
+ * is the chain that a demanded family would run.  A diagnostic with no counterpart in the reference (upstream picks its
  * kernel configuration from tuned tables per shape): it lets a test pin which measured kernel each benchmark
  * point runs on, so that a retune of the hand-over points cannot silently move one.  Any output pointer may be
  * null.  Returns MOE_I8_EUNSUPPORTED when `variant` demands a family that does not handle the shape.

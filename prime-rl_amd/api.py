@@ -122,7 +122,8 @@ def layer_plan(m: int, top_k: int, num_experts: int, hidden: int, inter: int,
                block_size: int = 64, gemm_variant: str | int = "auto") -> dict:
     """Which GEMM kernel ``fused_experts`` runs for each projection of a layer of this shape and how many
     kernel launches one call makes: ``{"gate_up": name, "down": name, "launches": n}``.  Decided on the host
-    from the sizes alone (no GPU needed), by the same code the driver uses."""
+    from the sizes alone (no GPU needed), by the same code the driver uses.  Of a few tokens that ``"auto"`` runs
+    in two launches of their own it names the chain of stages they replace."""
     import ctypes
 
     gu, dn, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()

@@ -640,6 +640,27 @@ int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
   void* down = ws + c.down;
   const int64_t p = m * top_k;
 
+  // A few tokens: no rows to gather per expert, the whole layer in two launches.
+  if (variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, hidden_size, inter) && aligned16(hidden) && aligned16(w1) &&
+      aligned16(w2) && num_experts <= MOE_I8_MAX_EXPERTS) {
+    moe_i8::FewTokensArgs f;
+    f.x = static_cast<const uint16_t*>(hidden);
+    f.w1 = w1;
+    f.w1_scale = w1_scale;
+    f.w2 = w2;
+    f.w2_scale = w2_scale;
+    f.topk_weights = topk_weights;
+    f.topk_ids = topk_ids;
+    f.act = static_cast<uint16_t*>(act);
+    f.out = static_cast<uint16_t*>(out);
+    f.tokens = (int)m;
+    f.top_k = top_k;
+    f.num_experts = num_experts;
+    f.hidden = hidden_size;
+    f.inter = inter;
+    return check_launch(moe_i8::launch_few_tokens(f, static_cast<hipStream_t>(stream)), "few_tokens");
+  }
+
   const LayerPlan plan = plan_layer(m, top_k, num_experts, hidden_size, inter, block_size, variant);
   if (plan.gate_up_kernel < 0 || plan.down_kernel < 0) return MOE_I8_EUNSUPPORTED;
 

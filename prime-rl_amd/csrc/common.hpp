@@ -265,6 +265,27 @@ int dense_row_stride(int k);
 bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed);
 hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream);
 
+// The whole layer of a few tokens in two launches: act holds tokens * top_k rows of inter bf16.
+struct FewTokensArgs {
+  const uint16_t* x;  // [tokens, hidden]
+  const int8_t* w1;   // [num_experts, 2 * inter, hidden]
+  const float* w1_scale;
+  const int8_t* w2;   // [num_experts, hidden, inter]
+  const float* w2_scale;
+  const float* topk_weights;
+  const int32_t* topk_ids;
+  uint16_t* act;
+  uint16_t* out;
+  int tokens;
+  int top_k;
+  int num_experts;
+  int hidden;
+  int inter;
+};
+constexpr int kFewTokensMaxPairs = 64;  // one lane per pair
+bool few_tokens_takes(int64_t tokens, int top_k, int hidden, int inter);
+hipError_t launch_few_tokens(const FewTokensArgs& a, hipStream_t stream);
+
 hipError_t launch_moe_sum(const uint16_t* in, uint16_t* out, int64_t m, int top_k, int hidden,
                           hipStream_t stream);
 
