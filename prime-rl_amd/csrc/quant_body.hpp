@@ -21,20 +21,26 @@ __device__ __forceinline__ float absmax8(const uint4& v) {
   return m;
 }
 
-// kEven: ties to even (rintf) instead of away from zero (roundf).
+// The low bytes of y[0..3] in one dword (selector: 0-3 = bytes of the 2nd operand, 4-7 = of the 1st).
+__device__ __forceinline__ uint32_t pack_low_bytes(const uint32_t* y) {
+  return __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0400u) | __builtin_amdgcn_perm(y[3], y[2], 0x04000c0cu);
+}
+
+// round(x * inv) as int8, ties to even (kEven) or away from zero; |x * inv| < 128.  The product is rounded to fp32 and
+// then to an integer, each in one operation: adding 1.5 * 2^23 leaves the nearest integer, ties to even, as a two's
+// complement byte in the low mantissa bits; truncation after adding 0.49999997 towards the sign (the largest float
+// below one half) rounds ties away from zero.  Both equal rintf / roundf for every float below 128 in magnitude
+// (checked one by one), at 4 and 6 operations per element instead of 8 and 11.
 template <bool kEven = false>
 __device__ __forceinline__ uint2 quant8(const uint4& v, float inv) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  uint32_t out[2] = {0u, 0u};
+  uint32_t y[8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float flo = __uint_as_float(w[i] << 16) * inv, fhi = __uint_as_float(w[i] & 0xffff0000u) * inv;
-    const int lo = (int)(kEven ? rintf(flo) : roundf(flo));
-    const int hi = (int)(kEven ? rintf(fhi) : roundf(fhi));
-    const uint32_t pair = ((uint32_t)lo & 0xffu) | (((uint32_t)hi & 0xffu) << 8);
-    out[i >> 1] |= pair << ((i & 1) * 16);
+  for (int i = 0; i < 8; ++i) {
+    const float p = __uint_as_float(i & 1 ? w[i >> 1] & 0xffff0000u : w[i >> 1] << 16) * inv;
+    y[i] = kEven ? __float_as_uint(p + 12582912.0f) : (uint32_t)(int)(p + copysignf(0.49999997f, p));
   }
-  return make_uint2(out[0], out[1]);
+  return make_uint2(pack_low_bytes(y), pack_low_bytes(y + 4));
 }
 
 // Largest |x| of 8 packed bf16 as a float.  Without the sign bit, bf16 patterns order like unsigned
@@ -88,15 +94,7 @@ __device__ __forceinline__ uint2 quant8_weights(const uint4& v, const WeightRcp&
 #pragma unroll
     for (int i = 0; i < 8; ++i) y[i] = __float_as_uint(rintf(x[i] / s.scale) + kMagic);
   }
-  uint32_t out[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    // low bytes of four results -> one dword (selector: 0-3 = bytes of the 2nd operand, 4-7 = of the 1st)
-    const uint32_t p01 = __builtin_amdgcn_perm(y[4 * h + 1], y[4 * h], 0x0c0c0400u);
-    const uint32_t p23 = __builtin_amdgcn_perm(y[4 * h + 3], y[4 * h + 2], 0x04000c0cu);
-    out[h] = p01 | p23;
-  }
-  return make_uint2(out[0], out[1]);
+  return make_uint2(pack_low_bytes(y), pack_low_bytes(y + 4));
 }
 
 // VPL = 16-byte vectors per lane held in registers (covers cols <= VPL * 512).
