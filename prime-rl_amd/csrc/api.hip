@@ -838,11 +838,15 @@ bool takes_dense_kernel(moe_i8::GemmArgs g, int variant) {
   return moe_i8::gemm_dense_takes(g.num_pairs, g.n, g.k, moe_i8::gemm_tile_supports(g));
 }
 
-int run_dense(const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
+int check_dense_gemm(const moe_i8::GemmArgs& g, int variant) {
   if (int rc = check_gemm_common(g.a_q, g.w, g.sorted_token_ids, g.expert_ids, g.num_tokens_post_padded, g.out, g.num_pairs,
                                  1, g.n, g.k, g.block_size, g.sorted_cap, variant))
     return rc;
-  if (!aligned16(g.w_scale)) return fail(MOE_I8_EINVAL, "weight scales must be 16-byte aligned");
+  return aligned16(g.w_scale) ? MOE_I8_OK : fail(MOE_I8_EINVAL, "weight scales must be 16-byte aligned");
+}
+
+int run_dense(const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
+  if (int rc = check_dense_gemm(g, variant)) return rc;
   if (takes_dense_kernel(g, variant)) {
     const moe_i8::DenseArgs d{g.mode, g.a_q, g.a_scale, g.w, g.w_scale, g.out, g.num_pairs, g.n, g.k};
     return check_launch(moe_i8::launch_gemm_dense(d, stream), "gemm_dense");
@@ -851,6 +855,15 @@ int run_dense(const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
   wide.tile_geometry = moe_i8::kTileWide;
   if (variant == MOE_I8_GEMM_AUTO && moe_i8::gemm_tile_supports(wide)) variant = MOE_I8_GEMM_TILE_WIDE;
   return run_gemm(g, variant, stream);
+}
+
+// A few rows: the launch quantises them itself.  Whether it runs, unless a family is demanded.
+bool takes_dense_few(const void* x, const moe_i8::GemmArgs& g, int variant) {
+  return variant == MOE_I8_GEMM_AUTO && moe_i8::dense_few_takes(g.num_pairs, g.n, g.k) && aligned16(x) && aligned16(g.w);
+}
+int run_dense_few(const void* x, const moe_i8::GemmArgs& g, hipStream_t stream) {
+  const moe_i8::DenseFewArgs d{g.mode, static_cast<const uint16_t*>(x), g.w, g.w_scale, static_cast<uint16_t*>(g.out), (int)g.num_pairs, g.n, g.k};
+  return check_launch(moe_i8::launch_dense_few(d, stream), "dense_few");
 }
 
 // The ties-to-even row quantiser of the dense path; `padded`: rows for the dense kernel; `route`: its
@@ -907,6 +920,10 @@ int moe_i8_w8a8_linear(const void* x, const int8_t* w, const float* w_scale, voi
   int8_t* x_q = reinterpret_cast<int8_t*>(ws + c.x_q);
   float* a1 = reinterpret_cast<float*>(ws + c.a1);
   const moe_i8::GemmArgs g = dense_group(moe_i8::kDown, c, ws, x_q, a1, w, w_scale, out, m, n, k);
+  if (takes_dense_few(x, g, variant)) {
+    if (int rc = check_dense_gemm(g, variant)) return rc;
+    return run_dense_few(x, g, s);
+  }
   const bool dense = takes_dense_kernel(g, variant);
   if (int rc = dense_quant(x, m, k, x_q, a1, dense, !dense, c, ws, s)) return rc;
   return run_dense(g, variant, s);
@@ -929,6 +946,12 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   float* a2 = reinterpret_cast<float*>(ws + c.a2);
   const moe_i8::GemmArgs gu = dense_group(moe_i8::kGateUpSilu, c, ws, x_q, a1, w13, w13_scale, ws + c.act, m, 2 * inter, hidden);
   moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, ws, act_q, a2, w2, w2_scale, out, m, hidden, inter);
+  if (takes_dense_few(x, gu, variant) && takes_dense_few(ws + c.act, dg, variant)) {
+    if (int rc = check_dense_gemm(gu, variant)) return rc;
+    if (int rc = check_dense_gemm(dg, variant)) return rc;
+    if (int rc = run_dense_few(x, gu, s)) return rc;
+    return run_dense_few(ws + c.act, dg, s);
+  }
   const bool dense_gu = takes_dense_kernel(gu, variant), dense_dg = takes_dense_kernel(dg, variant);
   if (int rc = dense_quant(x, m, hidden, x_q, a1, dense_gu, !dense_gu || !dense_dg, c, ws, s)) return rc;
   if (int rc = run_dense(gu, variant, s)) return rc;

@@ -82,6 +82,16 @@ __device__ __forceinline__ int wave_inclusive_scan_add(int v) {
   return v;
 }
 
+// sum over the wavefront, in every lane
+__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_inclusive_scan_add(v), 63); }
+
+// acc + the products of 16 int8 pairs (v_dot4_i32_i8)
+__device__ __forceinline__ int dot16(const v4i& a, const v4i& b, int acc) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_sdot4(a[i], b[i], acc, false);
+  return acc;
+}
+
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 
@@ -264,6 +274,21 @@ int dense_row_stride(int k);
 // family can run it too and are preferred where they are expected to be faster.
 bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed);
 hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream);
+
+// The same for a few rows, which the launch quantises itself (ties to even).
+struct DenseFewArgs {
+  int mode;           // kGateUpSilu or kDown
+  const uint16_t* x;  // [m, k] bf16
+  const int8_t* w;
+  const float* w_scale;
+  uint16_t* out;
+  int m;
+  int n;
+  int k;
+};
+constexpr int kDenseFewRows = 16;
+bool dense_few_takes(int64_t m, int n, int k);
+hipError_t launch_dense_few(const DenseFewArgs& a, hipStream_t stream);
 
 // The whole layer of a few tokens in two launches: act holds tokens * top_k rows of inter bf16.
 struct FewTokensArgs {

@@ -1,0 +1,158 @@
+// Dense W8A8 layer of a few rows in one launch, for gfx950: quantisation of the rows, product and epilogue.
+//
+// For a handful of rows the quantisation launch in front of a dense GEMM costs as much as the GEMM (3.0 and 5.2 us
+// for 5 rows x 2816 channels x 4096).  Here every workgroup quantises all rows itself, one wavefront per row, into
+// LDS, while its own weights are on their way from memory; a wavefront holds R weight rows in registers (16
+// consecutive reduction bytes per lane) and multiplies them with row after row by v_dot4_i32_i8; the lanes' int32 sums
+// (exact in any order) meet by lane permutes.  What bounds it: one memory latency and the weights' bytes, as long
+// as repeating the quantisation per workgroup stays hidden behind them.
+#include "quant_body.hpp"
+
+namespace moe_i8 {
+namespace {
+
+constexpr int kWaves = 8;
+
+// C: 1 KB pieces of a row (k <= 1024 * C); R: weight rows of a wavefront (gate_up: half gate, half up)
+template <int MODE, int C, int R>
+__global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) {
+  extern __shared__ __align__(16) int8_t xq[];  // [m][C * 1024], zero behind k
+  __shared__ float a_scale[kDenseFewRows];
+  constexpr int kOut = MODE == kGateUpSilu ? R / 2 : R;  // channels of a wavefront
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int K = p.k, width = MODE == kGateUpSilu ? p.n / 2 : p.n;
+
+  // the row first: its loads are waited for first
+  uint4 v[2 * C];
+  auto fetch = [&](int row) {
+    const uint4* x = reinterpret_cast<const uint4*>(p.x + (int64_t)row * K);
+#pragma unroll
+    for (int i = 0; i < 2 * C; ++i) v[i] = row < p.m && i * kWave + lane < K / kQuantVec ? x[i * kWave + lane] : make_uint4(0u, 0u, 0u, 0u);
+  };
+  fetch(wave);
+  v4i w[R][C], next[R][C];
+  float ws, wu = 0.0f, next_ws, next_wu = 0.0f;
+  auto fetch_weights = [&](int ch0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int c0 = ch0 + r % kOut < width ? ch0 + r % kOut : width - 1;
+      const v4i* row = reinterpret_cast<const v4i*>(p.w + (int64_t)(r < kOut ? c0 : width + c0) * K);
+#pragma unroll
+      for (int c = 0; c < C; ++c) next[r][c] = __builtin_nontemporal_load(row + (c * kWave + lane < K / 16 ? c * kWave + lane : 0));
+    }
+    // lane l < kOut: scales of channel ch0 + l
+    const int mine = ch0 + lane < width ? ch0 + lane : width - 1;
+    next_ws = p.w_scale[mine];
+    if constexpr (MODE == kGateUpSilu) next_wu = p.w_scale[width + mine];
+  };
+  int ch0 = (blockIdx.x * kWaves + wave) * kOut;
+  const int stride = gridDim.x * kWaves * kOut;
+  fetch_weights(ch0);
+
+  for (int row = wave; row < p.m; row += kWaves) {
+    if (row != wave) fetch(row);
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2 * C; ++i) m = fmaxf(m, absmax8_packed(v[i]));
+    const float absmax = fmaxf(wave_max(m), 1e-10f);
+    const float inv = 127.0f / absmax;
+    if (lane == 0) a_scale[row] = absmax / 127.0f;
+#pragma unroll
+    for (int i = 0; i < 2 * C; ++i)
+      *reinterpret_cast<uint2*>(xq + row * (C * 1024) + (i * kWave + lane) * kQuantVec) = quant8<true>(v[i], inv);
+  }
+  __syncthreads();
+
+  while (true) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int c = 0; c < C; ++c) w[r][c] = next[r][c];
+    ws = next_ws, wu = next_wu;
+    const bool more = ch0 + stride < width;
+    if (more) fetch_weights(ch0 + stride);
+    for (int row = 0; row < p.m; ++row) {
+      v4i q[C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) q[c] = *reinterpret_cast<const v4i*>(xq + row * (C * 1024) + (c * kWave + lane) * 16);
+      int g = 0, u = 0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        int acc = 0;
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc = dot16(w[r][c], q[c], acc);
+        const int sum = wave_total(acc);
+        if (r < kOut)
+          g = lane == r ? sum : g;
+        else
+          u = lane == r - kOut ? sum : u;
+      }
+      if (lane < kOut && ch0 + lane < width) {
+        const int g4[4] = {g, g, g, g}, u4[4] = {u, u, u, u};
+        const float4 s4 = make_float4(ws, ws, ws, ws);
+        const uint2 o = MODE == kGateUpSilu ? silu_mul_epilogue4(g4, u4, a_scale[row], s4, make_float4(wu, wu, wu, wu))
+                                            : down_epilogue4(g4, a_scale[row], s4, 1.0f);
+        p.out[(int64_t)row * width + ch0 + lane] = (uint16_t)o.x;
+      }
+    }
+    if (!more) break;
+    ch0 += stride;
+  }
+}
+
+template <int MODE, int C, int R>
+hipError_t launch_rows(const DenseFewArgs& a, hipStream_t stream) {
+  constexpr int kOut = kWaves * (MODE == kGateUpSilu ? R / 2 : R);
+  const int width = MODE == kGateUpSilu ? a.n / 2 : a.n;
+  const size_t lds = (size_t)a.m * C * 1024;
+  const int groups = (width + kOut - 1) / kOut, most = device_cu_count();  // a workgroup per compute unit: one quantisation each
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)dense_few_kernel<MODE, C, R>, hipFuncAttributeMaxDynamicSharedMemorySize, kDenseFewRows * C * 1024);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((dense_few_kernel<MODE, C, R>), dim3((unsigned)(groups < most ? groups : most)), dim3(64 * kWaves), lds, stream, a);
+  return hipGetLastError();
+}
+
+template <int MODE, int C>
+hipError_t launch_pieces(const DenseFewArgs& a, hipStream_t stream) {
+  // as many weight rows per wavefront, up to 16 KB, as leave work for every compute unit
+  const int most = a.n / (kWaves * 200);
+  if constexpr (C <= 2)
+    if (most >= 8) return launch_rows<MODE, C, 8>(a, stream);
+  if constexpr (C <= 4)
+    if (most >= 4) return launch_rows<MODE, C, 4>(a, stream);
+  return launch_rows<MODE, C, 2>(a, stream);
+}
+
+template <int MODE>
+hipError_t launch_mode(const DenseFewArgs& a, hipStream_t stream) {
+  switch ((a.k + 1023) / 1024) {
+    case 1: return launch_pieces<MODE, 1>(a, stream);
+    case 2: return launch_pieces<MODE, 2>(a, stream);
+    case 3: return launch_pieces<MODE, 3>(a, stream);
+    case 4: return launch_pieces<MODE, 4>(a, stream);
+    case 5: return launch_pieces<MODE, 5>(a, stream);
+    case 6: return launch_pieces<MODE, 6>(a, stream);
+    case 7: return launch_pieces<MODE, 7>(a, stream);
+    default: return launch_pieces<MODE, 8>(a, stream);
+  }
+}
+
+}  // namespace
+
+// Every row adds its quantisation and its products, on the vector units, to each workgroup; a quantisation launch and
+// the matrix units cost the same for 1 or 16 rows.  us per call here / there at 1, 4, 8 and 16 rows: 512 x 512 channels x
+// reduction 4.6 4.6 4.6 6.4 / 7.6, 4096 x 2048 4.9 4.8 5.1 7.8 / 7.5, 1440 x 5696 5.1 6.0 8.0 12.8 / 8.5, 8192 x 4096 6.9 8.7
+// 10.8 16.7 / 10.3, 8192 x 8192 12.9 14.6 19.3 28.8 / 15.8; gated MLP of 4096 x 1408 7.5 9.5 12.2 19.3 / 14.8.
+bool dense_few_takes(int64_t m, int n, int k) {
+  const int64_t weights = (int64_t)n * k;
+  const int64_t most = weights <= 1 << 20 ? kDenseFewRows : weights <= 12 << 20 ? 8 : weights <= 40 << 20 ? 6 : 4;
+  return m <= most && n % 16 == 0 && k % 16 == 0 && k <= 8 * 1024;
+}
+
+hipError_t launch_dense_few(const DenseFewArgs& a, hipStream_t stream) {
+  return a.mode == kGateUpSilu ? launch_mode<kGateUpSilu>(a, stream) : launch_mode<kDown>(a, stream);
+}
+
+}  // namespace moe_i8

@@ -24,14 +24,6 @@ constexpr int kGateWaves = 4;
 constexpr int down_rows(int c) { return c <= 2 ? 8 : 4; }     // channels of a down workgroup
 constexpr int down_waves(int c) { return c == 1 ? 16 : 8; }  // its wavefronts at most
 
-__device__ __forceinline__ int dot16(const v4i& a, const v4i& b, int acc) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_sdot4(a[i], b[i], acc, false);
-  return acc;
-}
-// sum over the wavefront, in every lane
-__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_inclusive_scan_add(v), 63); }
-
 // C: 1 KB pieces of a row (hidden <= 1024 * C)
 // kOne: one token, so no expert has two pairs
 template <int C, bool kOne>

@@ -29,3 +29,23 @@ def test_linear_and_mlp(pra, oracle, M, N, K):
         s2 = (torch.rand(K, generator=g) * 1e-3 + 1e-3).to(DEV)
         got = pra.w8a8_mlp(x.to(DEV), w13, s13, w2, s2)
         assert torch.equal(got, pra.w8a8_mlp(x.to(DEV), w13, s13, w2, s2, gemm_variant="stream"))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 16, 64), (1, 8192, 8192), (2, 304, 1088), (3, 9344, 2048), (4, 4096, 8128), (5, 2816, 4096), (6, 8192, 4096),
+    (7, 1648, 3008), (8, 2064, 5120), (8, 12288, 960), (9, 400, 1024), (16, 1024, 1024), (13, 176, 5952),
+])
+def test_few_rows_in_one_launch(pra, oracle, M, N, K):
+    """Rows quantised by the workgroups that multiply them: every row count per wavefront, remainders of
+    channels and of the 1 KB pieces of a reduction, more channel groups than workgroups."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    x[0, : K // 2] = torch.arange(K // 2) % 255 - 127  # exact ties and the largest values
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    s = torch.rand(N, generator=g) * 0.008 + 0.002
+    assert torch.equal(pra.apply_int8_linear(x.to(DEV), w.to(DEV), s.to(DEV)).cpu(), oracle.w8a8_linear(x, w, s))
+    inter = N // 2 // 64 * 64
+    if inter:
+        w2 = torch.randint(-127, 128, (K, inter), generator=g, dtype=torch.int8).to(DEV)
+        args = (x.to(DEV), w[: 2 * inter].to(DEV), (s[: 2 * inter] * 0.1).to(DEV), w2, (torch.rand(K, generator=g) * 1e-3).to(DEV))
+        assert torch.equal(pra.w8a8_mlp(*args), pra.w8a8_mlp(*args, gemm_variant="stream"))
