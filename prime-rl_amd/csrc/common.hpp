@@ -82,8 +82,45 @@ __device__ __forceinline__ int wave_inclusive_scan_add(int v) {
   return v;
 }
 
-// sum over the wavefront, in every lane
-__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_inclusive_scan_add(v), 63); }
+// Sums of R values over the wavefront, R = 2, 4 or 8: value l % R's in lane l.  Two values are folded into one by every
+// lane keeping the one it will end with and handing the other to its partner: 28 operations for eight values where
+// eight reductions of their own take 56.
+template <int R>
+__device__ __forceinline__ int wave_totals(const int (&v)[R]) {
+  const int lane = lane_id();
+  // partner at distance 1, 2 (quads), 4 (a shift up or down by half of eight lanes), 8 (rotation of a row of sixteen)
+  auto partner1 = [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0xb1, 0xf, 0xf, false); };
+  auto partner2 = [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x4e, 0xf, 0xf, false); };
+  auto partner4 = [](int x) {
+    const int up = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, false);   // row_shl:4 into lanes 0-3 and 8-11 of a row
+    return __builtin_amdgcn_update_dpp(up, x, 0x114, 0xf, 0xa, false);          // row_shr:4 into the others
+  };
+  auto fold = [&](int a, int b, int bit, auto partner) { return (lane & bit ? b : a) + partner(lane & bit ? a : b); };
+  int x;
+  if constexpr (R == 2) {
+    x = fold(v[0], v[1], 1, partner1);
+    x += partner2(x);
+    x += partner4(x);
+  } else if constexpr (R == 4) {
+    x = fold(fold(v[0], v[1], 1, partner1), fold(v[2], v[3], 1, partner1), 2, partner2);
+    x += partner4(x);
+  } else {
+    static_assert(R == 8, "2, 4 or 8 values");
+    x = fold(fold(fold(v[0], v[1], 1, partner1), fold(v[2], v[3], 1, partner1), 2, partner2),
+             fold(fold(v[4], v[5], 1, partner1), fold(v[6], v[7], 1, partner1), 2, partner2), 4, partner4);
+  }
+  x += __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, false);  // row_ror:8
+  const auto rows = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  x = (int)rows[0] + (int)rows[1];
+  const auto halves = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return (int)halves[0] + (int)halves[1];
+}
+
+// lane l: the value of lane l + kBy of its row of sixteen (0 past its end)
+template <int kBy>
+__device__ __forceinline__ int dpp_shift_down(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0x100 + kBy, 0xf, 0xf, true);
+}
 
 // acc + the products of 16 int8 pairs (v_dot4_i32_i8)
 __device__ __forceinline__ int dot16(const v4i& a, const v4i& b, int acc) {
@@ -124,6 +161,16 @@ __device__ __forceinline__ uint2 silu_mul_epilogue4(const int (&g)[4], const int
     h[r + 1] = __uint_as_float(s2 & 0xffff0000u) * __uint_as_float(u2 & 0xffff0000u);
   }
   return make_uint2(pack_bf16(h[0], h[1]), pack_bf16(h[2], h[3]));
+}
+
+// The same of one pair; the result in the low 16 bits.
+__device__ __forceinline__ uint32_t silu_mul_epilogue1(int g, int u, float a_scale, float wg, float wu) {
+  const uint32_t gu = pack_bf16((float)g * a_scale * wg, (float)u * a_scale * wu);
+  const uint32_t s = pack_bf16(fast_silu(__uint_as_float(gu << 16)), 0.0f);
+  return pack_bf16(__uint_as_float(s << 16) * __uint_as_float(gu & 0xffff0000u), 0.0f);
+}
+__device__ __forceinline__ uint32_t down_epilogue1(int acc, float a_scale, float ws, float rw) {
+  return pack_bf16((float)acc * a_scale * ws * rw, 0.0f);
 }
 
 // Four down-projection accumulators -> four bf16 outputs: acc * a_scale * w_scale * routed weight.

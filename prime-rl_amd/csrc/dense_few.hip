@@ -13,12 +13,22 @@ namespace {
 
 constexpr int kWaves = 8;
 
+// lane l: the value of lane l ^ (R / 2)
+template <int R>
+__device__ __forceinline__ int partner_half(int v) {
+  if constexpr (R == 2) return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, false);
+  if constexpr (R == 4) return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, false);
+  const int up = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xf, 0x5, false);
+  return __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false);
+}
+
 // C: 1 KB pieces of a row (k <= 1024 * C); R: weight rows of a wavefront (gate_up: half gate, half up)
 template <int MODE, int C, int R>
 __global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) {
   extern __shared__ __align__(16) int8_t xq[];  // [m][C * 1024], zero behind k
   __shared__ float a_scale[kDenseFewRows];
   constexpr int kOut = MODE == kGateUpSilu ? R / 2 : R;  // channels of a wavefront
+  constexpr int kRowsAtOnce = kWave / kOut < kDenseFewRows ? kWave / kOut : kDenseFewRows;  // rows that share an epilogue
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int K = p.k, width = MODE == kGateUpSilu ? p.n / 2 : p.n;
@@ -41,8 +51,8 @@ __global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) 
 #pragma unroll
       for (int c = 0; c < C; ++c) next[r][c] = __builtin_nontemporal_load(row + (c * kWave + lane < K / 16 ? c * kWave + lane : 0));
     }
-    // lane l < kOut: scales of channel ch0 + l
-    const int mine = ch0 + lane < width ? ch0 + lane : width - 1;
+    // lane l: scales of channel ch0 + l % kOut
+    const int mine = ch0 + lane % kOut < width ? ch0 + lane % kOut : width - 1;
     next_ws = p.w_scale[mine];
     if constexpr (MODE == kGateUpSilu) next_wu = p.w_scale[width + mine];
   };
@@ -72,28 +82,34 @@ __global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) 
     ws = next_ws, wu = next_wu;
     const bool more = ch0 + stride < width;
     if (more) fetch_weights(ch0 + stride);
+    int g = 0, u = 0;  // lane row * kOut + l: the sums of row `row`, channel ch0 + l
     for (int row = 0; row < p.m; ++row) {
       v4i q[C];
 #pragma unroll
       for (int c = 0; c < C; ++c) q[c] = *reinterpret_cast<const v4i*>(xq + row * (C * 1024) + (c * kWave + lane) * 16);
-      int g = 0, u = 0;
+      int acc[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        int acc = 0;
+        acc[r] = 0;
 #pragma unroll
-        for (int c = 0; c < C; ++c) acc = dot16(w[r][c], q[c], acc);
-        const int sum = wave_total(acc);
-        if (r < kOut)
-          g = lane == r ? sum : g;
-        else
-          u = lane == r - kOut ? sum : u;
+        for (int c = 0; c < C; ++c) acc[r] = dot16(w[r][c], q[c], acc[r]);
       }
-      if (lane < kOut && ch0 + lane < width) {
-        const int g4[4] = {g, g, g, g}, u4[4] = {u, u, u, u};
-        const float4 s4 = make_float4(ws, ws, ws, ws);
-        const uint2 o = MODE == kGateUpSilu ? silu_mul_epilogue4(g4, u4, a_scale[row], s4, make_float4(wu, wu, wu, wu))
-                                            : down_epilogue4(g4, a_scale[row], s4, 1.0f);
-        p.out[(int64_t)row * width + ch0 + lane] = (uint16_t)o.x;
+      const int totals = wave_totals<R>(acc);
+      const bool mine = lane / kOut == row % kRowsAtOnce;
+      if constexpr (MODE == kGateUpSilu) {
+        // R totals repeat through the lanes: gate in the lower half of R lanes, up in the upper
+        const int other = partner_half<R>(totals);
+        const bool upper = lane & kOut;
+        g = mine ? (upper ? other : totals) : g;
+        u = mine ? (upper ? totals : other) : u;
+      } else {
+        g = mine ? totals : g;
+      }
+      if (row % kRowsAtOnce == kRowsAtOnce - 1 || row == p.m - 1) {
+        const int first = row - row % kRowsAtOnce, at = first + lane / kOut, ch = ch0 + lane % kOut;
+        if (at <= row && lane < kRowsAtOnce * kOut && ch < width)
+          p.out[(int64_t)at * width + ch] = (uint16_t)(MODE == kGateUpSilu ? silu_mul_epilogue1(g, u, a_scale[at], ws, wu)
+                                                                           : down_epilogue1(g, a_scale[at], ws, 1.0f));
       }
     }
     if (!more) break;

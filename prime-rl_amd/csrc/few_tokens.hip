@@ -77,7 +77,7 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_up_few_kernel(FewTokensA
   while (true) {
     float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kVec; ++i) m = fmaxf(m, absmax8(v[i]));
+    for (int i = 0; i < kVec; ++i) m = fmaxf(m, absmax8_packed(v[i]));
     m = wave_max(m);
     if (lane == 0) part[wave] = m;
     __syncthreads();
@@ -96,26 +96,19 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_up_few_kernel(FewTokensA
       pair = __builtin_ctzll(same);
       fetch();
     }
-    int g = 0, u = 0;
     v4i q[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) q[c] = *reinterpret_cast<const v4i*>(xq + (c * kWave + lane) * 16);
+    int acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      int acc = 0;
+      acc[r] = 0;
 #pragma unroll
-      for (int c = 0; c < C; ++c) acc = dot16(w[r][c], q[c], acc);
-      const int sum = wave_total(acc);
-      if (r < R / 2)
-        g = lane == r ? sum : g;
-      else
-        u = lane == r - R / 2 ? sum : u;
+      for (int c = 0; c < C; ++c) acc[r] = dot16(w[r][c], q[c], acc[r]);
     }
-    if (lane < R / 2 && ch0 + lane < p.inter) {
-      const int g4[4] = {g, g, g, g}, u4[4] = {u, u, u, u};
-      const uint2 o = silu_mul_epilogue4(g4, u4, a_scale, make_float4(wg, wg, wg, wg), make_float4(wu, wu, wu, wu));
-      p.act[out] = (uint16_t)o.x;
-    }
+    const int g = wave_totals<R>(acc);
+    const int u = dpp_shift_down<R / 2>(g);
+    if (lane < R / 2 && ch0 + lane < p.inter) p.act[out] = (uint16_t)silu_mul_epilogue1(g, u, a_scale, wg, wu);
     if (!same) return;
   }
 }
@@ -177,7 +170,7 @@ __global__ __launch_bounds__(64 * (kOne ? 16 : down_waves(C))) void down_few_ker
       const int at = pair;
       float m = 0.0f;
 #pragma unroll
-      for (int c = 0; c < 2 * C; ++c) m = fmaxf(m, absmax8(v[c]));
+      for (int c = 0; c < 2 * C; ++c) m = fmaxf(m, absmax8_packed(v[c]));
       const float absmax = fmaxf(wave_max(m), 1e-10f);
       const float inv = 127.0f / absmax, a_scale = absmax / 127.0f;
       v4i q[C];
@@ -188,20 +181,16 @@ __global__ __launch_bounds__(64 * (kOne ? 16 : down_waves(C))) void down_few_ker
       }
       const bool more = !kOne && same != 0;
       if (more) fetch();
-      int mine = 0;
+      int acc[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        int acc = 0;
+        acc[r] = 0;
 #pragma unroll
-        for (int c = 0; c < C; ++c) acc = dot16(w[r][c], q[c], acc);
-        const int sum = wave_total(acc);
-        mine = lane == r ? sum : mine;
+        for (int c = 0; c < C; ++c) acc[r] = dot16(w[r][c], q[c], acc[r]);
       }
+      const int mine = wave_totals<R>(acc);
       const float rw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(routed), at));
-      if (lane < R) {
-        const int a4[4] = {mine, mine, mine, mine};
-        rows[at][lane] = bf16_bits_to_f32(down_epilogue4(a4, a_scale, make_float4(ws, ws, ws, ws), rw).x & 0xffffu);
-      }
+      if (lane < R) rows[at][lane] = bf16_bits_to_f32(down_epilogue1(mine, a_scale, ws, rw) & 0xffffu);
       if (!more) break;
     }
   }
