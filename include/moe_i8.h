@@ -221,6 +221,18 @@ int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
                          void* workspace, int64_t workspace_bytes, int variant, void* stream);
 
 /*
+ * moe_i8_route_topk and moe_i8_fused_experts in one call: topk_weights [M, top_k] and topk_ids [M, top_k] are outputs
+ * here (with the routed-experts record, if one is asked for) and the layer runs on them.  Same arguments, checks and
+ * results as the two calls; a single token is routed inside the layer's first launch.
+ */
+int moe_i8_fused_moe(const void* hidden, const float* logits, const int8_t* w1, const int8_t* w2, const float* w1_scale,
+                     const float* w2_scale, void* out, int64_t m, int top_k, int num_experts, int hidden_size, int inter,
+                     int block_size, int score_func, const float* selection_bias, int num_groups, int topk_groups,
+                     int group_score_top2, int renormalize, float route_scale, float* topk_weights, int32_t* topk_ids,
+                     void* capture, int capture_dtype, int64_t capture_token_stride, int64_t capture_offset,
+                     void* workspace, int64_t workspace_bytes, int variant, void* stream);
+
+/*
  * What moe_i8_fused_experts would launch for a layer shape, decided on the host from the sizes alone (no GPU
  * call): the GEMM kernel of each projection (MOE_I8_GEMM_STREAM, _NARROW, _TILE_WIDE or _TILE_DEEP) and the
  * number of kernel launches of one call through its chain of stages (alignment, quantisation, GEMMs, combine).

@@ -283,11 +283,11 @@ int moe_i8_scaled_int8_quant(const void* x, int dtype, int64_t rows, int64_t col
   return quant_rows_impl(x, dtype, rows, cols, row_stride, nullptr, 1, rows, q, scale, 1, stream);
 }
 
-int moe_i8_route_topk(const float* logits, int64_t m, int num_experts, int top_k, int score_func,
+// The router's arguments, checked; nothing is filled in for zero tokens.
+static int route_args(const float* logits, int64_t m, int num_experts, int top_k, int score_func,
                       const float* selection_bias, int num_groups, int topk_groups, int group_score_top2,
                       int renormalize, float route_scale, float* topk_weights, int32_t* topk_ids,
-                      void* capture, int capture_dtype, int64_t capture_token_stride,
-                      int64_t capture_offset, void* stream) {
+                      void* capture, int capture_dtype, int64_t capture_token_stride, int64_t capture_offset, moe_i8::RouteArgs* out) {
   if (m < 0) return fail(MOE_I8_EINVAL, "negative token count");
   if (num_experts < 1 || num_experts > MOE_I8_MAX_EXPERTS)
     return fail(MOE_I8_EINVAL, "num_experts (%d) must be in [1, %d]", num_experts, MOE_I8_MAX_EXPERTS);
@@ -315,7 +315,7 @@ int moe_i8_route_topk(const float* logits, int64_t m, int num_experts, int top_k
     return fail(MOE_I8_EINVAL, "capture needs a buffer and offset + top_k <= token stride");
   if (m == 0) return MOE_I8_OK;
   if (!logits || !topk_weights || !topk_ids) return fail(MOE_I8_EINVAL, "null pointer");
-  moe_i8::RouteArgs a;
+  moe_i8::RouteArgs& a = *out;
   a.logits = logits;
   a.m = m;
   a.num_experts = num_experts;
@@ -333,6 +333,20 @@ int moe_i8_route_topk(const float* logits, int64_t m, int num_experts, int top_k
   a.capture_bytes = capture_dtype;
   a.capture_stride = capture_token_stride;
   a.capture_offset = capture_offset;
+  return MOE_I8_OK;
+}
+
+int moe_i8_route_topk(const float* logits, int64_t m, int num_experts, int top_k, int score_func,
+                      const float* selection_bias, int num_groups, int topk_groups, int group_score_top2,
+                      int renormalize, float route_scale, float* topk_weights, int32_t* topk_ids,
+                      void* capture, int capture_dtype, int64_t capture_token_stride,
+                      int64_t capture_offset, void* stream) {
+  moe_i8::RouteArgs a;
+  if (int rc = route_args(logits, m, num_experts, top_k, score_func, selection_bias, num_groups, topk_groups, group_score_top2,
+                          renormalize, route_scale, topk_weights, topk_ids, capture, capture_dtype, capture_token_stride,
+                          capture_offset, &a))
+    return rc;
+  if (m == 0) return MOE_I8_OK;
   return check_launch(moe_i8::launch_route_topk(a, static_cast<hipStream_t>(stream)), "route_topk");
 }
 
@@ -611,11 +625,13 @@ int64_t moe_i8_workspace_bytes(int64_t m, int top_k, int num_experts, int hidden
   return carve(m, top_k, num_experts, hidden, inter, block_size).total;
 }
 
-int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
+// `route`: the routing is still to be done (topk_weights and topk_ids are written first).
+static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t* w2,
                          const float* topk_weights, const int32_t* topk_ids,
                          const float* w1_scale, const float* w2_scale, void* out, int64_t m,
                          int top_k, int num_experts, int hidden_size, int inter, int block_size,
-                         void* workspace, int64_t workspace_bytes, int variant, void* stream) {
+                         void* workspace, int64_t workspace_bytes, int variant,
+                         const moe_i8::RouteArgs* route, void* stream) {
   if (m < 0) return fail(MOE_I8_EINVAL, "negative m");
   if (m == 0) return MOE_I8_OK;
   if (!hidden || !w1 || !w2 || !topk_weights || !topk_ids || !w1_scale || !w2_scale || !out || !workspace)
@@ -658,11 +674,16 @@ int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
     f.num_experts = num_experts;
     f.hidden = hidden_size;
     f.inter = inter;
-    return check_launch(moe_i8::launch_few_tokens(f, static_cast<hipStream_t>(stream)), "few_tokens");
+    const bool routes = route && moe_i8::few_tokens_routes(*route);
+    if (route && !routes)
+      if (int rc = check_launch(moe_i8::launch_route_topk(*route, static_cast<hipStream_t>(stream)), "route_topk")) return rc;
+    return check_launch(moe_i8::launch_few_tokens(f, routes ? route : nullptr, static_cast<hipStream_t>(stream)), "few_tokens");
   }
 
   const LayerPlan plan = plan_layer(m, top_k, num_experts, hidden_size, inter, block_size, variant);
   if (plan.gate_up_kernel < 0 || plan.down_kernel < 0) return MOE_I8_EUNSUPPORTED;
+  if (route)
+    if (int rc = check_launch(moe_i8::launch_route_topk(*route, static_cast<hipStream_t>(stream)), "route_topk")) return rc;
 
   // Small batches: moe_align (one workgroup) and the quantisation of the input share one launch.
   moe_i8::AlignArgs aa;
@@ -714,6 +735,30 @@ int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
       return rc;
   }
   return moe_i8_sum(down, out, m, top_k, hidden_size, stream);
+}
+
+int moe_i8_fused_experts(const void* hidden, const int8_t* w1, const int8_t* w2,
+                         const float* topk_weights, const int32_t* topk_ids,
+                         const float* w1_scale, const float* w2_scale, void* out, int64_t m,
+                         int top_k, int num_experts, int hidden_size, int inter, int block_size,
+                         void* workspace, int64_t workspace_bytes, int variant, void* stream) {
+  return fused_experts_impl(hidden, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, out, m, top_k, num_experts, hidden_size,
+                            inter, block_size, workspace, workspace_bytes, variant, nullptr, stream);
+}
+
+int moe_i8_fused_moe(const void* hidden, const float* logits, const int8_t* w1, const int8_t* w2, const float* w1_scale,
+                     const float* w2_scale, void* out, int64_t m, int top_k, int num_experts, int hidden_size, int inter,
+                     int block_size, int score_func, const float* selection_bias, int num_groups, int topk_groups,
+                     int group_score_top2, int renormalize, float route_scale, float* topk_weights, int32_t* topk_ids,
+                     void* capture, int capture_dtype, int64_t capture_token_stride, int64_t capture_offset,
+                     void* workspace, int64_t workspace_bytes, int variant, void* stream) {
+  moe_i8::RouteArgs route;
+  if (int rc = route_args(logits, m, num_experts, top_k, score_func, selection_bias, num_groups, topk_groups, group_score_top2,
+                          renormalize, route_scale, topk_weights, topk_ids, capture, capture_dtype, capture_token_stride,
+                          capture_offset, &route))
+    return rc;
+  return fused_experts_impl(hidden, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, out, m, top_k, num_experts, hidden_size,
+                            inter, block_size, workspace, workspace_bytes, variant, &route, stream);
 }
 
 int moe_i8_layer_plan(int64_t m, int top_k, int num_experts, int hidden_size, int inter, int block_size,

@@ -16,6 +16,7 @@
 // is used.  What bounds it: one memory latency and the bytes at one token of a small layer, the bytes alone
 // where experts are large.
 #include "quant_body.hpp"
+#include "router_body.hpp"
 
 namespace moe_i8 {
 namespace {
@@ -25,9 +26,10 @@ constexpr int down_rows(int c) { return c <= 2 ? 8 : 4; }     // channels of a d
 constexpr int down_waves(int c) { return c == 1 ? 16 : 8; }  // its wavefronts at most
 
 // C: 1 KB pieces of a row (hidden <= 1024 * C)
-// kOne: one token, so no expert has two pairs
-template <int C, bool kOne>
-__global__ __launch_bounds__(64 * kGateWaves) void gate_up_few_kernel(FewTokensArgs p) {
+// kOne: one token, so no expert has two pairs.  kRoute > 0: of one token, which every wavefront routes itself (kRoute
+// experts per lane), as far as its pair; the first one writes the routing for the down launch and the caller.
+template <int C, bool kOne, int kRoute = 0>
+__global__ __launch_bounds__(64 * kGateWaves) void gate_up_few_kernel(FewTokensArgs p, RouteArgs route) {
   constexpr int kThreads = 64 * kGateWaves;
   constexpr int R = C <= 2 ? 8 : C <= 4 ? 4 : 2;  // weight rows of a wavefront: half gate, half up
   constexpr int kVec = (C * 1024 / kQuantVec + kThreads - 1) / kThreads;
@@ -38,9 +40,27 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_up_few_kernel(FewTokensA
   const int pairs = p.tokens * p.top_k, K = p.hidden;
   int pair = blockIdx.y;
   // the pairs of this pair's expert: the first one's workgroups take them all
+  // the token's row and logits first: their loads are waited for first
+  uint4 v[kVec];
+  auto fetch = [&] {
+    const uint4* x = reinterpret_cast<const uint4*>(p.x + (int64_t)(pair / p.top_k) * K);
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) v[i] = i * kThreads + tid < K / kQuantVec ? x[i * kThreads + tid] : make_uint4(0u, 0u, 0u, 0u);
+  };
+  fetch();
+  float logits[kRoute > 0 ? kRoute : 1];
+  if constexpr (kRoute > 0) route_logits<kRoute>(route, 0, logits);
+
   int e;
   uint64_t same = 0;
-  if constexpr (kOne) {
+  if constexpr (kRoute > 0) {
+    const bool writes = blockIdx.x == 0 && pair == 0 && wave == 0;
+    int id;
+    float w;
+    route_select<kRoute>(route, logits, writes ? p.top_k : pair + 1, id, w);
+    if (writes) route_write(route, 0, id, w);
+    e = __builtin_amdgcn_readlane(id, pair);
+  } else if constexpr (kOne) {
     e = p.topk_ids[pair];
   } else {
     const int id = lane < pairs ? p.topk_ids[lane] : -1;
@@ -49,15 +69,6 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_up_few_kernel(FewTokensA
     if (__builtin_ctzll(same) != pair) return;
   }
   if (e < 0 || e >= p.num_experts) return;
-
-  // the token's row first: its loads are waited for first
-  uint4 v[kVec];
-  auto fetch = [&] {
-    const uint4* x = reinterpret_cast<const uint4*>(p.x + (int64_t)(pair / p.top_k) * K);
-#pragma unroll
-    for (int i = 0; i < kVec; ++i) v[i] = i * kThreads + tid < K / kQuantVec ? x[i * kThreads + tid] : make_uint4(0u, 0u, 0u, 0u);
-  };
-  fetch();
 
   const int ch0 = (blockIdx.x * kGateWaves + wave) * (R / 2);
   v4i w[R][C];
@@ -210,13 +221,18 @@ __global__ __launch_bounds__(64 * (kOne ? 16 : down_waves(C))) void down_few_ker
 }
 
 template <int C>
-hipError_t launch_gate_up(const FewTokensArgs& a, hipStream_t stream) {
+hipError_t launch_gate_up(const FewTokensArgs& a, const RouteArgs* route, hipStream_t stream) {
   constexpr int kChannels = (C <= 2 ? 8 : C <= 4 ? 4 : 2) / 2 * kGateWaves;
   const dim3 grid((unsigned)((a.inter + kChannels - 1) / kChannels), (unsigned)(a.tokens * a.top_k)), block(64 * kGateWaves);
-  if (a.tokens == 1)
-    hipLaunchKernelGGL((gate_up_few_kernel<C, true>), grid, block, 0, stream, a);
+  const RouteArgs r = route ? *route : RouteArgs{};
+  if (route && route_experts_per_lane(a.num_experts) <= 2)
+    hipLaunchKernelGGL((gate_up_few_kernel<C, true, 2>), grid, block, 0, stream, a, r);
+  else if (route)
+    hipLaunchKernelGGL((gate_up_few_kernel<C, true, 4>), grid, block, 0, stream, a, r);
+  else if (a.tokens == 1)
+    hipLaunchKernelGGL((gate_up_few_kernel<C, true>), grid, block, 0, stream, a, r);
   else
-    hipLaunchKernelGGL((gate_up_few_kernel<C, false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((gate_up_few_kernel<C, false>), grid, block, 0, stream, a, r);
   return hipGetLastError();
 }
 template <int C>
@@ -245,17 +261,22 @@ bool few_tokens_takes(int64_t tokens, int top_k, int hidden, int inter) {
          hidden <= 8 * 1024 && inter <= 4 * 1024;
 }
 
-hipError_t launch_few_tokens(const FewTokensArgs& a, hipStream_t stream) {
+bool few_tokens_routes(const RouteArgs& r) {
+  // an expert group is a run of whole lanes: with other numbers of experts per lane than these two a launch of its own
+  return r.m == 1 && (route_experts_per_lane(r.num_experts) == 2 || route_experts_per_lane(r.num_experts) == 4);
+}
+
+hipError_t launch_few_tokens(const FewTokensArgs& a, const RouteArgs* route, hipStream_t stream) {
   hipError_t err;
   switch ((a.hidden + 1023) / 1024) {
-    case 1: err = launch_gate_up<1>(a, stream); break;
-    case 2: err = launch_gate_up<2>(a, stream); break;
-    case 3: err = launch_gate_up<3>(a, stream); break;
-    case 4: err = launch_gate_up<4>(a, stream); break;
-    case 5: err = launch_gate_up<5>(a, stream); break;
-    case 6: err = launch_gate_up<6>(a, stream); break;
-    case 7: err = launch_gate_up<7>(a, stream); break;
-    default: err = launch_gate_up<8>(a, stream); break;
+    case 1: err = launch_gate_up<1>(a, route, stream); break;
+    case 2: err = launch_gate_up<2>(a, route, stream); break;
+    case 3: err = launch_gate_up<3>(a, route, stream); break;
+    case 4: err = launch_gate_up<4>(a, route, stream); break;
+    case 5: err = launch_gate_up<5>(a, route, stream); break;
+    case 6: err = launch_gate_up<6>(a, route, stream); break;
+    case 7: err = launch_gate_up<7>(a, route, stream); break;
+    default: err = launch_gate_up<8>(a, route, stream); break;
   }
   if (err != hipSuccess) return err;
   switch ((a.inter + 1023) / 1024) {

@@ -282,9 +282,11 @@ struct Router {
     return moe_i8_route_topk((const float*)logits->data_ptr(), m, (int)e, (int)k, (int)score,
                              bias ? (const float*)bias->data_ptr() : nullptr, (int)groups, (int)topk_groups, (int)top2,
                              (int)renormalize, (float)scale, weights, ids, record ? record->data_ptr() : nullptr,
-                             record ? (record->scalar_type() == at::kByte ? 1 : 2) : 0, record ? record->size(1) * k : 0,
-                             record ? layer * k : 0, stream);
+                             record_dtype(), record_stride(), record_offset(), stream);
   }
+  int record_dtype() const { return record ? (record->scalar_type() == at::kByte ? 1 : 2) : 0; }
+  int64_t record_stride() const { return record ? record->size(1) * k : 0; }
+  int64_t record_offset() const { return record ? layer * k : 0; }
 };
 
 // route(<router>) -> (weights, ids)
@@ -325,8 +327,13 @@ PyObject* moe(PyObject* const* args, Py_ssize_t nargs) {
   if (!l.output(Py_None, args[7] == Py_True, &out)) Py_RETURN_NONE;
   float* weights = reinterpret_cast<float*>(ws + need);
   int32_t* ids = reinterpret_cast<int32_t*>(weights + l.m * r.k);
-  if (int rc = r.run(weights, ids, l.at.stream)) return PyLong_FromLong(rc);
-  if (int rc = l.run(weights, ids, (int)r.k, (int)block, (int)variant, out, ws, size)) return PyLong_FromLong(rc);
+  if (int rc = moe_i8_fused_moe(l.x->data_ptr(), (const float*)r.logits->data_ptr(), (const int8_t*)l.w1->data_ptr(),
+                                (const int8_t*)l.w2->data_ptr(), (const float*)l.s1->data_ptr(), (const float*)l.s2->data_ptr(),
+                                out.data_ptr(), l.m, (int)r.k, (int)l.e, (int)l.h, (int)l.i, (int)block, (int)r.score,
+                                r.bias ? (const float*)r.bias->data_ptr() : nullptr, (int)r.groups, (int)r.topk_groups, (int)r.top2,
+                                (int)r.renormalize, (float)r.scale, weights, ids, r.record ? r.record->data_ptr() : nullptr,
+                                r.record_dtype(), r.record_stride(), r.record_offset(), ws, size, (int)variant, l.at.stream))
+    return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(out));
 }
 

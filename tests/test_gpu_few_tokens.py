@@ -81,3 +81,31 @@ def test_layer_of_a_few_tokens_equals_the_chain_of_stages(pra, E, k, H, I, M):
     x = d.hidden_states.clone()
     got = pra.fused_experts(x, *d.fused_experts_args()[1:], **d.fused_experts_kwargs(), inplace=True)
     assert got.data_ptr() == x.data_ptr() and torch.equal(x, want)
+
+
+@pytest.mark.parametrize("E,k,H,I,groups,score,bias,M", [
+    (128, 8, 2048, 768, None, "softmax", False, 1), (256, 8, 7168, 256, (8, 4), "sigmoid", True, 1),
+    (100, 3, 512, 64, None, "sigmoid", True, 1), (192, 16, 1088, 192, None, "softmax", False, 1),
+    (40, 2, 256, 128, None, "softmax", False, 1), (300, 4, 256, 64, None, "softmax", False, 1), (128, 8, 512, 128, None, "softmax", False, 4),
+])
+def test_routed_call_of_a_few_tokens_equals_router_and_layer(pra, E, k, H, I, groups, score, bias, M):
+    """Routing inside the layer's first launch (one token), in front of the two launches, or of the chain."""
+    im = inputs_mod()
+    d = im.make_inputs(im.LayerShape("r", E=E, k=k, H=H, I=I), M, seed=E + k).to(DEV)
+    g = torch.Generator(device=DEV).manual_seed(E)
+    logits = torch.randn(M, E, device=DEV, generator=g)
+    how = dict(scoring_func=score, routed_scaling_factor=2.5 if bias else 1.0,
+               e_score_correction_bias=torch.randn(E, device=DEV, generator=g) * 0.1 if bias else None)
+    if groups:
+        how.update(use_grouped_topk=True, num_expert_group=groups[0], topk_group=groups[1])
+    kw = {n: v for n, v in d.fused_experts_kwargs().items() if n not in ("topk_weights", "topk_ids")}
+    record = torch.zeros(M, 3, k, dtype=torch.uint16, device=DEV)
+    x, w1, w2 = d.fused_experts_args()[:3]
+    got = pra.fused_moe(x, w1, w2, logits, k, True, routed_experts_out=(record, 1), **how, **kw)
+    if groups:
+        w, ids = pra.grouped_topk(x, logits, k, True, *groups, score, 2.5, how["e_score_correction_bias"])
+    else:
+        w, ids = pra.route_topk(logits, k, score_func=score, renormalize=True, route_scale=how["routed_scaling_factor"],
+                                selection_bias=how["e_score_correction_bias"])
+    assert torch.equal(record[:, 1].to(torch.int32), ids) and int(record[:, ::2].to(torch.int32).sum()) == 0
+    assert torch.equal(got, pra.fused_experts(x, w1, w2, w, ids, **kw, gemm_variant="stream"))
