@@ -233,8 +233,52 @@ __global__ __launch_bounds__(kSingleThreads) void align_single_kernel(
   align_single_body(ids, P, E, B, nbits, sorted, sorted_cap, expert_ids, expert_cap, npp_out, smem, use_masks != 0);
 }
 
-// One launch for small batches: workgroup 0 runs moe_align, every other workgroup quantises 16
-// activation rows (one per wavefront).  The two halves are independent.
+// The rows that a workgroup of a fused launch quantises: one per wavefront, or, where a row is longer than a wavefront of a
+// 1024-thread workgroup can hold (8 vectors per lane of its 128 registers), one per four wavefronts, which take a quarter
+// each and share the maximum through LDS.  Bound by memory; with rows read twice, four loads of a lane at a time, the
+// launch took 97 us for 16384 rows of 7168 (3.6 TB/s) and 9.8 us for 64, now 73 us (4.8 TB/s) and 6 us.
+constexpr int kLongRow = 16;        // vectors per lane that a single wavefront would need
+constexpr int kLongRowWaves = 4;
+template <int VPL>
+constexpr int rows_per_workgroup() { return VPL == kLongRow ? kSingleWaves / kLongRowWaves : kSingleWaves; }
+
+template <int VPL>
+__device__ __forceinline__ void quant_workgroup_rows(const QuantArgs& q, int64_t group) {
+  const int wave = threadIdx.x / kWave;
+  if constexpr (VPL == kLongRow) {
+    constexpr int kVec = kLongRow / kLongRowWaves;
+    __shared__ __align__(16) float part[kSingleWaves];
+    const int64_t row = group * rows_per_workgroup<VPL>() + wave / kLongRowWaves;
+    const int c0 = (wave % kLongRowWaves) * (kVec * kWave) + lane_id();
+    const int nvec = q.cols / kQuantVec;
+    const bool have = row < q.rows;
+    const uint4* in = reinterpret_cast<const uint4*>(q.x + (have ? row : 0) * q.row_stride);
+    uint4 v[kVec];
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) v[i] = have && c0 + i * kWave < nvec ? in[c0 + i * kWave] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) m = fmaxf(m, absmax8(v[i]));
+    m = wave_max(m);
+    if (lane_id() == 0) part[wave] = m;
+    __syncthreads();
+    if (!have) return;
+    const float4 all = *reinterpret_cast<const float4*>(part + wave / kLongRowWaves * kLongRowWaves);
+    const float absmax = fmaxf(fmaxf(fmaxf(all.x, all.y), fmaxf(all.z, all.w)), 1e-10f);
+    const float inv = 127.0f / absmax;
+    if (threadIdx.x % (kLongRowWaves * kWave) == 0) q.scale[row] = absmax / 127.0f;
+    uint2* out = reinterpret_cast<uint2*>(q.q + row * (int64_t)q.cols);
+#pragma unroll
+    for (int i = 0; i < kVec; ++i)
+      if (c0 + i * kWave < nvec) out[c0 + i * kWave] = quant8(v[i], inv);
+  } else {
+    const int64_t row = group * kSingleWaves + wave;
+    if (row < q.rows) quant_one_row<VPL>(q, row);
+  }
+}
+
+// One launch for small batches: workgroup 0 runs moe_align, every other workgroup quantises its activation rows.  The
+// two halves are independent.
 template <int VPL>
 __global__ __launch_bounds__(kSingleThreads) void align_quant_kernel(
     const int32_t* __restrict__ ids, int P, int E, int B, int nbits,
@@ -245,8 +289,7 @@ __global__ __launch_bounds__(kSingleThreads) void align_quant_kernel(
     align_single_body(ids, P, E, B, nbits, sorted, sorted_cap, expert_ids, expert_cap, npp_out, smem, use_masks != 0);
     return;
   }
-  const int64_t row = (int64_t)(blockIdx.x - 1) * kSingleWaves + threadIdx.x / kWave;
-  if (row < q.rows) quant_one_row<VPL>(q, row);
+  quant_workgroup_rows<VPL>(q, (int64_t)blockIdx.x - 1);
 }
 
 // ---- multi-launch path -------------------------------------------------------------------
@@ -335,8 +378,7 @@ __global__ __launch_bounds__(kSingleThreads) void align_scan_quant_kernel(
     align_scan_body(E, B, units, unit_hist, unit_base, seg_out, expert_ids, expert_cap, npp_out);
     return;
   }
-  const int64_t row = (int64_t)(blockIdx.x - 1) * kSingleWaves + threadIdx.x / kWave;
-  if (row < q.rows) quant_one_row<VPL>(q, row);
+  quant_workgroup_rows<VPL>(q, (int64_t)blockIdx.x - 1);
 }
 
 __global__ __launch_bounds__(kMultiThreads) void align_scatter_kernel(
@@ -459,8 +501,7 @@ __global__ __launch_bounds__(kSingleThreads) void align_count_quant_kernel(
     align_count_body(ids, P, E, B, chunk_base, seg_out, expert_ids, expert_cap, npp_out, smem);
     return;
   }
-  const int64_t row = (int64_t)(blockIdx.x - 1) * kSingleWaves + threadIdx.x / kWave;
-  if (row < q.rows) quant_one_row<VPL>(q, row);
+  quant_workgroup_rows<VPL>(q, (int64_t)blockIdx.x - 1);
   fill_sentinel(sorted, sorted_cap, P, (int)blockIdx.x - 1, (int)gridDim.x - 1);
 }
 
@@ -544,6 +585,7 @@ hipError_t set_chunked_lds_limits() {
   MOE_I8_LIMIT(2);
   MOE_I8_LIMIT(4);
   MOE_I8_LIMIT(8);
+  MOE_I8_LIMIT(kLongRow);
 #undef MOE_I8_LIMIT
   return hipFuncSetAttribute((const void*)align_scatter_chunk_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                              kSingleLdsMax);
@@ -559,13 +601,13 @@ hipError_t launch_scatter_chunks(const AlignArgs& a, const int32_t* chunk_base, 
 }
 }  // namespace
 
-// The fused kernels are 1024-thread workgroups (the aligning one needs them), which caps a thread at
-// 128 registers: a row held in 16 vectors per lane would spill (measured: 33 us instead of 6 us for 64
-// rows of 7168), so rows that long take the variant that reads the row twice, the second time from
-// the cache (the `default` of the switches below).
+// Rows of up to 4096 elements are held by one wavefront, of up to 8192 by four (see above; 16 vectors per lane would spill,
+// 33 us instead of 6 us for 64 rows of 7168); longer ones are read twice, the second time from the cache.
 hipError_t launch_align_quant(const AlignArgs& a, const QuantArgs& q, hipStream_t stream) {
   const int E = a.num_experts;
-  const dim3 grid(1 + (unsigned)((q.rows + kSingleWaves - 1) / kSingleWaves));
+  const int vpl = quant_vectors_per_lane(q.cols);
+  const int64_t per_group = vpl == kLongRow ? rows_per_workgroup<kLongRow>() : kSingleWaves;
+  const dim3 grid(1 + (unsigned)((q.rows + per_group - 1) / per_group));
   if (a.num_pairs > kSingleMaxPairs && a.num_pairs <= kChunkedMaxPairs) {
     // two launches as launch_align, the first one (a single counting workgroup) also quantises
     static const hipError_t attr = set_chunked_lds_limits();
@@ -576,11 +618,12 @@ hipError_t launch_align_quant(const AlignArgs& a, const QuantArgs& q, hipStream_
   hipLaunchKernelGGL(align_count_quant_kernel<V>, grid, dim3(kSingleThreads), single_lds_bytes(E), stream,  \
                      a.topk_ids, a.num_pairs, E, a.block_size, chunk_base, seg, a.sorted_token_ids,         \
                      a.sorted_cap, a.expert_ids, a.expert_cap, a.num_tokens_post_padded, q)
-    switch (quant_vectors_per_lane(q.cols)) {
+    switch (vpl) {
       case 1: MOE_I8_COUNT_QUANT(1); break;
       case 2: MOE_I8_COUNT_QUANT(2); break;
       case 4: MOE_I8_COUNT_QUANT(4); break;
       case 8: MOE_I8_COUNT_QUANT(8); break;
+      case kLongRow: MOE_I8_COUNT_QUANT(kLongRow); break;
       default: MOE_I8_COUNT_QUANT(0); break;
     }
 #undef MOE_I8_COUNT_QUANT
@@ -603,11 +646,12 @@ hipError_t launch_align_quant(const AlignArgs& a, const QuantArgs& q, hipStream_
 #define MOE_I8_SCAN_QUANT(V)                                                                           \
   hipLaunchKernelGGL(align_scan_quant_kernel<V>, grid, dim3(kSingleThreads), 0, stream, E, a.block_size, \
                      units, unit_hist, unit_base, seg, a.expert_ids, a.expert_cap, a.num_tokens_post_padded, q)
-    switch (quant_vectors_per_lane(q.cols)) {
+    switch (vpl) {
       case 1: MOE_I8_SCAN_QUANT(1); break;
       case 2: MOE_I8_SCAN_QUANT(2); break;
       case 4: MOE_I8_SCAN_QUANT(4); break;
       case 8: MOE_I8_SCAN_QUANT(8); break;
+      case kLongRow: MOE_I8_SCAN_QUANT(kLongRow); break;
       default: MOE_I8_SCAN_QUANT(0); break;
     }
 #undef MOE_I8_SCAN_QUANT
@@ -631,11 +675,12 @@ hipError_t launch_align_quant(const AlignArgs& a, const QuantArgs& q, hipStream_
                        a.sorted_token_ids, a.sorted_cap, a.expert_ids, a.expert_cap,                \
                        a.num_tokens_post_padded, use_masks ? 1 : 0, q);                             \
   } while (0)
-  switch (quant_vectors_per_lane(q.cols)) {
+  switch (vpl) {
     case 1: MOE_I8_FUSED_LAUNCH(1); break;
     case 2: MOE_I8_FUSED_LAUNCH(2); break;
     case 4: MOE_I8_FUSED_LAUNCH(4); break;
     case 8: MOE_I8_FUSED_LAUNCH(8); break;
+    case kLongRow: MOE_I8_FUSED_LAUNCH(kLongRow); break;
     default: MOE_I8_FUSED_LAUNCH(0); break;
   }
 #undef MOE_I8_FUSED_LAUNCH

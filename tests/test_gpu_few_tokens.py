@@ -109,3 +109,20 @@ def test_routed_call_of_a_few_tokens_equals_router_and_layer(pra, E, k, H, I, gr
                                 selection_bias=how["e_score_correction_bias"])
     assert torch.equal(record[:, 1].to(torch.int32), ids) and int(record[:, ::2].to(torch.int32).sum()) == 0
     assert torch.equal(got, pra.fused_experts(x, w1, w2, w, ids, **kw, gemm_variant="stream"))
+
+
+@pytest.mark.parametrize("H", [4096, 4160, 7168, 8192, 8256])
+@pytest.mark.parametrize("M", [9, 1101, 4101])  # alignment in one, two and three launches
+def test_layer_quantises_long_rows_as_the_row_quantiser_does(pra, H, M):
+    """Rows held by one wavefront, by four, and read twice, in each launch that quantises the layer's input."""
+    E, k, I, B = 8, 8, 64, 64
+    im = inputs_mod()
+    d = im.make_inputs(im.LayerShape("q", E=E, k=k, H=H, I=I), M, seed=H + M).to(DEV)
+    s, e, npp = pra.moe_align_block_size(d.topk_ids, B, E)
+    x_q, a1 = pra.per_token_quant_int8(d.hidden_states)
+    act = pra.gemm_gate_up_silu(x_q, a1, d.w1, d.w1_scale, s, e, npp, k, B, M * k, "stream")
+    h_q, a2 = pra.per_token_quant_int8(act)
+    want = torch.empty(M, H, dtype=torch.bfloat16, device=DEV)
+    pra.moe_sum(pra.gemm_down(h_q, a2, d.w2, d.w2_scale, d.topk_weights, s, e, npp, B, "stream").view(M, k, H), want)
+    got = pra.fused_experts(*d.fused_experts_args(), **d.fused_experts_kwargs(), block_size_m=B, gemm_variant="stream")
+    assert torch.equal(got, want)
