@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) 
     if (row != wave) fetch(row);
     float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 2 * C; ++i) m = fmaxf(m, absmax8_packed(v[i]));
+    for (int i = 0; i < 2 * C; ++i) m = fmaxf(m, absmax8(v[i]));
     const float absmax = fmaxf(wave_max(m), 1e-10f);
     const float inv = 127.0f / absmax;
     if (lane == 0) a_scale[row] = absmax / 127.0f;

@@ -88,7 +88,7 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_up_few_kernel(FewTokensA
   while (true) {
     float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kVec; ++i) m = fmaxf(m, absmax8_packed(v[i]));
+    for (int i = 0; i < kVec; ++i) m = fmaxf(m, absmax8(v[i]));
     m = wave_max(m);
     if (lane == 0) part[wave] = m;
     __syncthreads();
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(64 * (kOne ? 16 : down_waves(C))) void down_few_ker
       const int at = pair;
       float m = 0.0f;
 #pragma unroll
-      for (int c = 0; c < 2 * C; ++c) m = fmaxf(m, absmax8_packed(v[c]));
+      for (int c = 0; c < 2 * C; ++c) m = fmaxf(m, absmax8(v[c]));
       const float absmax = fmaxf(wave_max(m), 1e-10f);
       const float inv = 127.0f / absmax, a_scale = absmax / 127.0f;
       v4i q[C];

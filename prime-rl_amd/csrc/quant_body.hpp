@@ -10,6 +10,8 @@ constexpr int kQuantVec = 8;  // bf16 elements per 16-byte load
 
 __device__ __forceinline__ float wave_max(float v) { return wave_reduce_max(v); }
 
+// Largest |x| of 8 packed bf16.  A NaN is skipped: a row that holds one keeps the scale of its other elements (and
+// the NaN becomes 0, in quant8).
 __device__ __forceinline__ float absmax8(const uint4& v) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
   float m = 0.0f;
@@ -26,11 +28,12 @@ __device__ __forceinline__ uint32_t pack_low_bytes(const uint32_t* y) {
   return __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0400u) | __builtin_amdgcn_perm(y[3], y[2], 0x04000c0cu);
 }
 
-// round(x * inv) as int8, ties to even (kEven) or away from zero; |x * inv| < 128.  The product is rounded to fp32 and
-// then to an integer, each in one operation: adding 1.5 * 2^23 leaves the nearest integer, ties to even, as a two's
-// complement byte in the low mantissa bits; truncation after adding 0.49999997 towards the sign (the largest float
-// below one half) rounds ties away from zero.  Both equal rintf / roundf for every float below 128 in magnitude
-// (checked one by one), at 4 and 6 operations per element instead of 8 and 11.
+// round(x * inv) as int8, ties to even (kEven) or away from zero; NaN gives 0.  |x * inv| < 128 for every other x, as
+// long as inv comes from a maximum that no element exceeds: absmax8's, which a NaN does not hide.  The product is
+// rounded to fp32 and then to an integer, each in one operation: adding 1.5 * 2^23 leaves the nearest integer, ties to
+// even, as a two's complement byte in the low mantissa bits; truncation after adding 0.49999997 towards the sign (the
+// largest float below one half) rounds ties away from zero.  Both equal rintf / roundf for every float below 128 in
+// magnitude (checked one by one), at 4 and 6 operations per element instead of 8 and 11.
 template <bool kEven = false>
 __device__ __forceinline__ uint2 quant8(const uint4& v, float inv) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -43,8 +46,9 @@ __device__ __forceinline__ uint2 quant8(const uint4& v, float inv) {
   return make_uint2(pack_low_bytes(y), pack_low_bytes(y + 4));
 }
 
-// Largest |x| of 8 packed bf16 as a float.  Without the sign bit, bf16 patterns order like unsigned
-// integers, so the maximum is taken on packed 16-bit lanes (two elements per operation).
+// The same for finite values only (weights): without the sign bit, bf16 patterns order like unsigned integers, so the
+// maximum is taken on packed 16-bit lanes (two elements per operation).  A NaN would be the largest of its 8 elements
+// and hide them from the float maximum of the row.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float absmax8_packed(const uint4& v) {
   const uint32_t w[4] = {v.x & 0x7fff7fffu, v.y & 0x7fff7fffu, v.z & 0x7fff7fffu, v.w & 0x7fff7fffu};
