@@ -94,6 +94,12 @@ bool as_int(PyObject* o, int64_t* v) {
   return true;
 }
 
+// A switch that is True or False; any other value's truth is for the Python path to ask.
+bool as_bool(PyObject* o, bool* v) {
+  *v = o == Py_True;
+  return PyBool_Check(o);
+}
+
 // [N, K] int8 weights, contiguous or as the transposed [K, N] view of such a tensor, with N scales.
 bool dense_weight(PyObject* wo, PyObject* so, const at::Tensor** w, const at::Tensor** s, int64_t* n, int64_t* k) {
   if (!THPVariable_Check(wo)) return false;
@@ -236,15 +242,16 @@ PyObject* experts(PyObject* const* args, Py_ssize_t nargs) {
   Layer l;
   const at::Tensor *tw, *ids;
   int64_t block, variant, size;
+  bool inplace;
   char* ws;
   at::Tensor out;
   if (!l.init(args[0], args[1], args[2], args[5], args[6]) || !plain(args[3], at::kFloat, &tw) || !plain(args[4], at::kInt, &ids) ||
-      !as_int(args[7], &block) || !as_int(args[8], &variant) || ids->dim() != 2 || ids->size(0) != l.m || tw->sizes() != ids->sizes() ||
+      !as_int(args[7], &block) || !as_int(args[8], &variant) || !as_bool(args[9], &inplace) || ids->dim() != 2 || ids->size(0) != l.m || tw->sizes() != ids->sizes() ||
       tw->get_device() != l.at.device || ids->get_device() != l.at.device || ids->size(1) < 1 || ids->size(1) > l.e)
     Py_RETURN_NONE;
   const int k = (int)ids->size(1);
   const int64_t need = moe_i8_workspace_bytes(l.m, k, (int)l.e, (int)l.h, (int)l.i, (int)block);
-  if (need < 0 || !workspace(args[11], l.at, need, &ws, &size) || !l.output(args[10], args[9] == Py_True, &out)) Py_RETURN_NONE;
+  if (need < 0 || !workspace(args[11], l.at, need, &ws, &size) || !l.output(args[10], inplace, &out)) Py_RETURN_NONE;
   if (int rc = l.run((const float*)tw->data_ptr(), (const int32_t*)ids->data_ptr(), k, (int)block, (int)variant, out, ws, size))
     return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(out));
@@ -313,9 +320,11 @@ PyObject* moe(PyObject* const* args, Py_ssize_t nargs) {
   Layer l;
   Router r;
   int64_t block, variant, size;
+  bool inplace;
   char* ws;
   at::Tensor out;
   if (!l.init(args[0], args[1], args[2], args[3], args[4]) || !as_int(args[5], &block) || !as_int(args[6], &variant) ||
+      !as_bool(args[7], &inplace) ||
       !r.init(args + 9) || r.m != l.m || r.e != l.e || r.logits->get_device() != l.at.device)
     Py_RETURN_NONE;
   const int64_t need = moe_i8_workspace_bytes(l.m, (int)r.k, (int)l.e, (int)l.h, (int)l.i, (int)block);
@@ -324,7 +333,7 @@ PyObject* moe(PyObject* const* args, Py_ssize_t nargs) {
     if (args[8] == Py_None) Py_RETURN_FALSE;
     Py_RETURN_NONE;
   }
-  if (!l.output(Py_None, args[7] == Py_True, &out)) Py_RETURN_NONE;
+  if (!l.output(Py_None, inplace, &out)) Py_RETURN_NONE;
   float* weights = reinterpret_cast<float*>(ws + need);
   int32_t* ids = reinterpret_cast<int32_t*>(weights + l.m * r.k);
   if (int rc = moe_i8_fused_moe(l.x->data_ptr(), (const float*)r.logits->data_ptr(), (const int8_t*)l.w1->data_ptr(),
