@@ -5,7 +5,8 @@
  * (passed as void*).  The library never allocates or frees device memory,
  * never synchronises and never touches any stream but the one it is given, so
  * every call can be recorded into a HIP graph.  The caller owns all buffers,
- * including the workspace.
+ * including the workspace.  Threads may share a workspace on one stream: a call
+ * issues all its launches before another one on the same workspace issues any.
  *
  * Return value: 0 on success, a negative MOE_I8_E* code otherwise; the text of
  * the last error of the calling thread is available from moe_i8_last_error().

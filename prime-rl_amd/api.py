@@ -918,11 +918,11 @@ def _workspace(device: torch.device, stream: int, nbytes: int, pin: bool = False
             _retired_workspaces.append(ws)  # a graph may replay on it: keep it allocated
             _pinned_workspaces.discard(key)
         if ws is not None and ws.is_cuda:
-            _abi.host().forget(*key)  # before the old buffer can go
+            _abi.host().forget(*key)
         ws = torch.empty((max(nbytes + spare, 256),), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
         if ws.is_cuda:
-            _abi.host().remember(*key, ws.data_ptr(), ws.numel())
+            _abi.host().remember(*key, ws)
         _workspaces.move_to_end(key)
         if pin:
             _pinned_workspaces.add(key)

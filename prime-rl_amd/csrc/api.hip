@@ -3,7 +3,10 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
+#include <condition_variable>
 #include <mutex>
+#include <vector>
 
 #include "../../include/moe_i8.h"
 #include "common.hpp"
@@ -24,6 +27,40 @@ int check_launch(hipError_t err, const char* what) {
   if (err == hipSuccess) return MOE_I8_OK;
   return fail(MOE_I8_ELAUNCH, "%s: %s", what, hipGetErrorString(err));
 }
+
+// A call's turn on its workspace, while it issues its launches.  Calls of several threads on one stream may share a
+// workspace, since the stream runs them one after the other, but only if their launches do not interleave.  A thread
+// that waits here waits for calls on the same workspace and for nothing else.
+class WorkspaceTurn {
+ public:
+  explicit WorkspaceTurn(const void* workspace) : workspace_(workspace) {
+    std::unique_lock<std::mutex> lock(state().mutex);
+    while (std::find(state().busy.begin(), state().busy.end(), workspace_) != state().busy.end()) state().ended.wait(lock);
+    state().busy.push_back(workspace_);
+  }
+  ~WorkspaceTurn() {
+    {
+      std::lock_guard<std::mutex> lock(state().mutex);
+      std::vector<const void*>& busy = state().busy;
+      *std::find(busy.begin(), busy.end(), workspace_) = busy.back();
+      busy.pop_back();
+    }
+    state().ended.notify_all();
+  }
+  WorkspaceTurn(const WorkspaceTurn&) = delete;
+
+ private:
+  struct State {
+    std::mutex mutex;
+    std::condition_variable ended;
+    std::vector<const void*> busy;  // one entry per thread inside a call
+  };
+  static State& state() {
+    static State* s = new State;  // never destroyed: threads may outlive static objects
+    return *s;
+  }
+  const void* workspace_;
+};
 
 bool valid_block_size(int b) { return b == 16 || b == 32 || b == 64 || b == 128; }
 
@@ -655,6 +692,7 @@ static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t
   float* a2 = reinterpret_cast<float*>(ws + c.a2);
   void* down = ws + c.down;
   const int64_t p = m * top_k;
+  const WorkspaceTurn turn(workspace);
 
   // A few tokens: no rows to gather per expert, the whole layer in two launches.
   if (variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, hidden_size, inter) && aligned16(hidden) && aligned16(w1) &&
@@ -965,6 +1003,7 @@ int moe_i8_w8a8_linear(const void* x, const int8_t* w, const float* w_scale, voi
   int8_t* x_q = reinterpret_cast<int8_t*>(ws + c.x_q);
   float* a1 = reinterpret_cast<float*>(ws + c.a1);
   const moe_i8::GemmArgs g = dense_group(moe_i8::kDown, c, ws, x_q, a1, w, w_scale, out, m, n, k);
+  const WorkspaceTurn turn(workspace);
   if (takes_dense_few(x, g, variant)) {
     if (int rc = check_dense_gemm(g, variant)) return rc;
     return run_dense_few(x, g, s);
@@ -991,6 +1030,7 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   float* a2 = reinterpret_cast<float*>(ws + c.a2);
   const moe_i8::GemmArgs gu = dense_group(moe_i8::kGateUpSilu, c, ws, x_q, a1, w13, w13_scale, ws + c.act, m, 2 * inter, hidden);
   moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, ws, act_q, a2, w2, w2_scale, out, m, hidden, inter);
+  const WorkspaceTurn turn(workspace);
   if (takes_dense_few(x, gu, variant) && takes_dense_few(ws + c.act, dg, variant)) {
     if (int rc = check_dense_gemm(gu, variant)) return rc;
     if (int rc = check_dense_gemm(dg, variant)) return rc;

@@ -6,6 +6,10 @@
 // type, shape, device or layout it does not expect, no workspace large enough, a capture in progress), in
 // which case the caller runs the Python path, which handles or names it; or a negative int, the C-ABI's error
 // code.  Nothing is launched before all checks are done, so None always means nothing has happened yet.
+//
+// The interpreter lock is held while arguments are read and given up around every call that may block (the output's
+// allocation, the launches, the capture query): a launch waits where the queue is full, and what it waits for may be
+// a host callback that needs the lock.  Whatever the launches use is therefore read, or kept alive, beforehand.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <ATen/ATen.h>
@@ -13,25 +17,36 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <utility>
+#include <vector>
+
 #include "../../include/moe_i8.h"
 
 namespace {
 
-// Default workspaces the Python side has made, by (device, stream); it owns them and withdraws an entry before
-// it lets go of the tensor.  Guarded by the interpreter lock.
+// The interpreter lock given up for a scope.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// Default workspaces the Python side has made, by (device, stream); it withdraws an entry when it lets go of the
+// tensor.  A call holds a reference of its own until its launches are in the stream: another thread may replace the
+// entry meanwhile.  Guarded by the interpreter lock.
 struct Workspace {
   int device;
   hipStream_t stream;
-  char* data;
-  int64_t bytes;
+  at::Tensor tensor;
 };
-constexpr int kMaxWorkspaces = 64;
-Workspace g_workspaces[kMaxWorkspaces];
-int g_num_workspaces = 0;
+constexpr size_t kMaxWorkspaces = 64;
+std::vector<Workspace>& workspaces() {
+  static auto* all = new std::vector<Workspace>();  // never destroyed: the allocator may be gone by then
+  return *all;
+}
 
 Workspace* find_workspace(int device, hipStream_t stream) {
-  for (int i = 0; i < g_num_workspaces; ++i)
-    if (g_workspaces[i].device == device && g_workspaces[i].stream == stream) return &g_workspaces[i];
+  for (Workspace& w : workspaces())
+    if (w.device == device && w.stream == stream) return &w;
   return nullptr;
 }
 
@@ -44,6 +59,7 @@ struct Where {
     if (device != c10::hip::current_device()) return false;
     stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const Unlocked unlocked;
     if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
       (void)hipGetLastError();
       return false;
@@ -61,27 +77,35 @@ bool plain(PyObject* o, at::ScalarType type, const at::Tensor** out) {
   return true;
 }
 
-at::Tensor make(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor& like) {
-  return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
+at::Tensor make(at::IntArrayRef sizes, at::ScalarType type, const Where& at) {
+  return at::empty(sizes, at::TensorOptions().dtype(type).device(at::Device(at::kCUDA, (c10::DeviceIndex)at.device)));
 }
 
-char* bytes_of(const at::Tensor& t) { return static_cast<char*>(t.data_ptr()); }
-
 // A caller's workspace, or the default one of the stream.
-bool workspace(PyObject* o, const Where& at, int64_t need, char** data, int64_t* size) {
-  if (o == Py_None) {
-    const Workspace* w = find_workspace(at.device, at.stream);
-    if (!w || w->bytes < need) return false;
-    *data = w->data;
-    *size = w->bytes;
+struct Scratch {
+  at::Tensor keep;
+  char* data;
+  int64_t bytes;
+  bool init(PyObject* o, const Where& at, int64_t need) {
+    if (o == Py_None) {
+      const Workspace* w = find_workspace(at.device, at.stream);
+      if (!w) return false;
+      keep = w->tensor;
+    } else {
+      if (!THPVariable_Check(o)) return false;
+      keep = THPVariable_Unpack(o);
+      if (!keep.is_cuda() || keep.get_device() != at.device || !keep.is_contiguous()) return false;
+    }
+    bytes = (int64_t)keep.nbytes();
+    if (bytes < need) return false;
+    data = static_cast<char*>(keep.data_ptr());
     return true;
   }
-  if (!THPVariable_Check(o)) return false;
-  const at::Tensor& t = THPVariable_Unpack(o);
-  if (!t.is_cuda() || t.get_device() != at.device || !t.is_contiguous() || (int64_t)t.nbytes() < need) return false;
-  *data = bytes_of(t);
-  *size = (int64_t)t.nbytes();
-  return true;
+};
+
+template <class T>
+T* data(const at::Tensor* t) {
+  return t ? static_cast<T*>(t->data_ptr()) : nullptr;
 }
 
 bool as_int(PyObject* o, int64_t* v) {
@@ -132,16 +156,22 @@ PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return wrap_guarded(fn, args, nargs);
 }
 
-// remember(device, stream, data, bytes): the default workspace of (device, stream) is now this one.
+// remember(device, stream, tensor): the default workspace of (device, stream) is now this one.
 PyObject* remember(PyObject* const* args, Py_ssize_t nargs) {
-  MOE_I8_ARGS(4);
-  const long long d = PyLong_AsLongLong(args[0]), b = PyLong_AsLongLong(args[3]);
+  MOE_I8_ARGS(3);
+  const long long d = PyLong_AsLongLong(args[0]);
   void* s = PyLong_AsVoidPtr(args[1]);
-  void* p = PyLong_AsVoidPtr(args[2]);
   if (PyErr_Occurred()) return nullptr;
-  Workspace* w = find_workspace((int)d, (hipStream_t)s);
-  if (!w && g_num_workspaces < kMaxWorkspaces) w = &g_workspaces[g_num_workspaces++];
-  if (w) *w = {(int)d, (hipStream_t)s, (char*)p, (int64_t)b};
+  if (!THPVariable_Check(args[2])) {
+    PyErr_SetString(PyExc_TypeError, "a workspace is a tensor");
+    return nullptr;
+  }
+  const at::Tensor& t = THPVariable_Unpack(args[2]);
+  if (Workspace* w = find_workspace((int)d, (hipStream_t)s)) {
+    w->tensor = t;
+  } else if (workspaces().size() < kMaxWorkspaces) {
+    workspaces().push_back({(int)d, (hipStream_t)s, t});
+  }
   Py_RETURN_NONE;
 }
 
@@ -151,7 +181,11 @@ PyObject* forget(PyObject* const* args, Py_ssize_t nargs) {
   const long long d = PyLong_AsLongLong(args[0]);
   void* s = PyLong_AsVoidPtr(args[1]);
   if (PyErr_Occurred()) return nullptr;
-  if (Workspace* w = find_workspace((int)d, (hipStream_t)s)) *w = g_workspaces[--g_num_workspaces];
+  if (Workspace* w = find_workspace((int)d, (hipStream_t)s)) {
+    std::swap(*w, workspaces().back());
+    const at::Tensor last = std::move(workspaces().back().tensor);  // let go of once the table is in order again
+    workspaces().pop_back();
+  }
   Py_RETURN_NONE;
 }
 
@@ -159,31 +193,37 @@ PyObject* forget(PyObject* const* args, Py_ssize_t nargs) {
 PyObject* linear(PyObject* const* args, Py_ssize_t nargs) {
   MOE_I8_ARGS(5);
   const at::Tensor *x, *w, *s;
-  int64_t n, k, variant, size;
-  char* ws;
+  int64_t n, k, variant;
   Where at;
+  Scratch ws;
   if (!plain(args[0], at::kBFloat16, &x) || !dense_weight(args[1], args[2], &w, &s, &n, &k) || !as_int(args[3], &variant) ||
       x->dim() < 1 || x->size(-1) != k || k == 0 || n > INT32_MAX || k > INT32_MAX || !at.init(*x) ||
       w->get_device() != at.device || s->get_device() != at.device)
     Py_RETURN_NONE;
   const int64_t m = x->numel() / k;
-  if (m == 0 || !workspace(args[4], at, moe_i8_dense_workspace_bytes(m, (int)k, 0), &ws, &size)) Py_RETURN_NONE;
+  if (m == 0 || !ws.init(args[4], at, moe_i8_dense_workspace_bytes(m, (int)k, 0))) Py_RETURN_NONE;
   c10::SmallVector<int64_t, 4> shape(x->sizes().begin(), x->sizes().end());
   shape.back() = n;
-  at::Tensor out = make(shape, at::kBFloat16, *x);
-  if (int rc = moe_i8_w8a8_linear(x->data_ptr(), (const int8_t*)w->data_ptr(), (const float*)s->data_ptr(), out.data_ptr(), m,
-                                  (int)n, (int)k, ws, size, (int)variant, at.stream))
-    return PyLong_FromLong(rc);
-  return THPVariable_Wrap(std::move(out));
+  const void* xp = data<void>(x);
+  const int8_t* wp = data<int8_t>(w);
+  const float* sp = data<float>(s);
+  at::Tensor out;
+  int rc;
+  {
+    const Unlocked unlocked;
+    out = make(shape, at::kBFloat16, at);
+    rc = moe_i8_w8a8_linear(xp, wp, sp, out.data_ptr(), m, (int)n, (int)k, ws.data, ws.bytes, (int)variant, at.stream);
+  }
+  return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
 }
 
 // mlp(x, w13, w13_scale, w2, w2_scale, variant, workspace)
 PyObject* mlp(PyObject* const* args, Py_ssize_t nargs) {
   MOE_I8_ARGS(7);
   const at::Tensor *x, *w13, *s13, *w2, *s2;
-  int64_t two_i, h, h2, i, variant, size;
-  char* ws;
+  int64_t two_i, h, h2, i, variant;
   Where at;
+  Scratch ws;
   if (!plain(args[0], at::kBFloat16, &x) || !dense_weight(args[1], args[2], &w13, &s13, &two_i, &h) ||
       !dense_weight(args[3], args[4], &w2, &s2, &h2, &i) || !as_int(args[5], &variant) || x->dim() < 1 || two_i != 2 * i ||
       h2 != h || h == 0 || x->size(-1) != h || h > INT32_MAX || two_i > INT32_MAX || !at.init(*x) ||
@@ -191,13 +231,19 @@ PyObject* mlp(PyObject* const* args, Py_ssize_t nargs) {
       s2->get_device() != at.device)
     Py_RETURN_NONE;
   const int64_t m = x->numel() / h;
-  if (m == 0 || !workspace(args[6], at, moe_i8_dense_workspace_bytes(m, (int)h, (int)i), &ws, &size)) Py_RETURN_NONE;
-  at::Tensor out = make(x->sizes(), at::kBFloat16, *x);
-  if (int rc = moe_i8_w8a8_mlp(x->data_ptr(), (const int8_t*)w13->data_ptr(), (const float*)s13->data_ptr(),
-                               (const int8_t*)w2->data_ptr(), (const float*)s2->data_ptr(), out.data_ptr(), m, (int)h, (int)i, ws,
-                               size, (int)variant, at.stream))
-    return PyLong_FromLong(rc);
-  return THPVariable_Wrap(std::move(out));
+  if (m == 0 || !ws.init(args[6], at, moe_i8_dense_workspace_bytes(m, (int)h, (int)i))) Py_RETURN_NONE;
+  const c10::SmallVector<int64_t, 4> shape(x->sizes().begin(), x->sizes().end());
+  const void* xp = data<void>(x);
+  const int8_t *w13p = data<int8_t>(w13), *w2p = data<int8_t>(w2);
+  const float *s13p = data<float>(s13), *s2p = data<float>(s2);
+  at::Tensor out;
+  int rc;
+  {
+    const Unlocked unlocked;
+    out = make(shape, at::kBFloat16, at);
+    rc = moe_i8_w8a8_mlp(xp, w13p, s13p, w2p, s2p, out.data_ptr(), m, (int)h, (int)i, ws.data, ws.bytes, (int)variant, at.stream);
+  }
+  return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
 }
 
 // The layer's tensors, checked against each other.
@@ -218,21 +264,16 @@ struct Layer {
       if (t->get_device() != at.device) return false;
     return true;
   }
-  // `out`: None (a new tensor; the input itself if `inplace`) or the tensor to write
+  // `out`: None (a new tensor, made with the launches; the input itself if `inplace`) or the tensor to write
   bool output(PyObject* o, bool inplace, at::Tensor* out) const {
     if (o == Py_None) {
-      *out = inplace ? *x : make(x->sizes(), at::kBFloat16, *x);
+      if (inplace) *out = *x;
       return true;
     }
     const at::Tensor* t;
     if (!plain(o, at::kBFloat16, &t) || t->sizes() != x->sizes() || t->get_device() != at.device) return false;
     *out = *t;
     return true;
-  }
-  int run(const float* weights, const int32_t* ids, int k, int block, int variant, at::Tensor& out, char* ws, int64_t size) const {
-    return moe_i8_fused_experts(x->data_ptr(), (const int8_t*)w1->data_ptr(), (const int8_t*)w2->data_ptr(), weights, ids,
-                                (const float*)s1->data_ptr(), (const float*)s2->data_ptr(), out.data_ptr(), m, k, (int)e, (int)h,
-                                (int)i, block, ws, size, variant, at.stream);
   }
 };
 
@@ -241,20 +282,30 @@ PyObject* experts(PyObject* const* args, Py_ssize_t nargs) {
   MOE_I8_ARGS(12);
   Layer l;
   const at::Tensor *tw, *ids;
-  int64_t block, variant, size;
+  int64_t block, variant;
   bool inplace;
-  char* ws;
+  Scratch ws;
   at::Tensor out;
   if (!l.init(args[0], args[1], args[2], args[5], args[6]) || !plain(args[3], at::kFloat, &tw) || !plain(args[4], at::kInt, &ids) ||
-      !as_int(args[7], &block) || !as_int(args[8], &variant) || !as_bool(args[9], &inplace) || ids->dim() != 2 || ids->size(0) != l.m || tw->sizes() != ids->sizes() ||
-      tw->get_device() != l.at.device || ids->get_device() != l.at.device || ids->size(1) < 1 || ids->size(1) > l.e)
+      !as_int(args[7], &block) || !as_int(args[8], &variant) || !as_bool(args[9], &inplace) || ids->dim() != 2 ||
+      ids->size(0) != l.m || tw->sizes() != ids->sizes() || tw->get_device() != l.at.device || ids->get_device() != l.at.device ||
+      ids->size(1) < 1 || ids->size(1) > l.e)
     Py_RETURN_NONE;
   const int k = (int)ids->size(1);
   const int64_t need = moe_i8_workspace_bytes(l.m, k, (int)l.e, (int)l.h, (int)l.i, (int)block);
-  if (need < 0 || !workspace(args[11], l.at, need, &ws, &size) || !l.output(args[10], inplace, &out)) Py_RETURN_NONE;
-  if (int rc = l.run((const float*)tw->data_ptr(), (const int32_t*)ids->data_ptr(), k, (int)block, (int)variant, out, ws, size))
-    return PyLong_FromLong(rc);
-  return THPVariable_Wrap(std::move(out));
+  if (need < 0 || !ws.init(args[11], l.at, need) || !l.output(args[10], inplace, &out)) Py_RETURN_NONE;
+  const void* xp = data<void>(l.x);
+  const int8_t *w1 = data<int8_t>(l.w1), *w2 = data<int8_t>(l.w2);
+  const float *twp = data<float>(tw), *s1 = data<float>(l.s1), *s2 = data<float>(l.s2);
+  const int32_t* idp = data<int32_t>(ids);
+  int rc;
+  {
+    const Unlocked unlocked;
+    if (!out.defined()) out = make({l.m, l.h}, at::kBFloat16, l.at);
+    rc = moe_i8_fused_experts(xp, w1, w2, twp, idp, s1, s2, out.data_ptr(), l.m, k, (int)l.e, (int)l.h, (int)l.i, (int)block,
+                              ws.data, ws.bytes, (int)variant, l.at.stream);
+  }
+  return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
 }
 
 // The router's arguments: (logits, top_k, score_func, renormalize, scale, bias, groups, topk_groups, top2,
@@ -285,12 +336,6 @@ struct Router {
     }
     return true;
   }
-  int run(float* weights, int32_t* ids, hipStream_t stream) const {
-    return moe_i8_route_topk((const float*)logits->data_ptr(), m, (int)e, (int)k, (int)score,
-                             bias ? (const float*)bias->data_ptr() : nullptr, (int)groups, (int)topk_groups, (int)top2,
-                             (int)renormalize, (float)scale, weights, ids, record ? record->data_ptr() : nullptr,
-                             record_dtype(), record_stride(), record_offset(), stream);
-  }
   int record_dtype() const { return record ? (record->scalar_type() == at::kByte ? 1 : 2) : 0; }
   int64_t record_stride() const { return record ? record->size(1) * k : 0; }
   int64_t record_offset() const { return record ? layer * k : 0; }
@@ -302,8 +347,21 @@ PyObject* route(PyObject* const* args, Py_ssize_t nargs) {
   Router r;
   Where at;
   if (!r.init(args) || !at.init(*r.logits)) Py_RETURN_NONE;
-  at::Tensor weights = make({r.m, r.k}, at::kFloat, *r.logits), ids = make({r.m, r.k}, at::kInt, *r.logits);
-  if (int rc = r.run((float*)weights.data_ptr(), (int32_t*)ids.data_ptr(), at.stream)) return PyLong_FromLong(rc);
+  const float *logits = data<float>(r.logits), *bias = data<float>(r.bias);
+  void* record = data<void>(r.record);
+  const int record_dtype = r.record_dtype();
+  const int64_t stride = r.record_stride(), offset = r.record_offset();
+  at::Tensor weights, ids;
+  int rc;
+  {
+    const Unlocked unlocked;
+    weights = make({r.m, r.k}, at::kFloat, at);
+    ids = make({r.m, r.k}, at::kInt, at);
+    rc = moe_i8_route_topk(logits, r.m, (int)r.e, (int)r.k, (int)r.score, bias, (int)r.groups, (int)r.topk_groups, (int)r.top2,
+                           (int)r.renormalize, (float)r.scale, static_cast<float*>(weights.data_ptr()),
+                           static_cast<int32_t*>(ids.data_ptr()), record, record_dtype, stride, offset, at.stream);
+  }
+  if (rc) return PyLong_FromLong(rc);
   PyObject* w = THPVariable_Wrap(std::move(weights));
   PyObject* i = THPVariable_Wrap(std::move(ids));
   PyObject* both = w && i ? PyTuple_Pack(2, w, i) : nullptr;
@@ -319,9 +377,9 @@ PyObject* moe(PyObject* const* args, Py_ssize_t nargs) {
   MOE_I8_ARGS(20);
   Layer l;
   Router r;
-  int64_t block, variant, size;
+  int64_t block, variant;
   bool inplace;
-  char* ws;
+  Scratch ws;
   at::Tensor out;
   if (!l.init(args[0], args[1], args[2], args[3], args[4]) || !as_int(args[5], &block) || !as_int(args[6], &variant) ||
       !as_bool(args[7], &inplace) ||
@@ -329,21 +387,28 @@ PyObject* moe(PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   const int64_t need = moe_i8_workspace_bytes(l.m, (int)r.k, (int)l.e, (int)l.h, (int)l.i, (int)block);
   if (need < 0) Py_RETURN_NONE;
-  if (!workspace(args[8], l.at, need + 8 * l.m * r.k, &ws, &size)) {
+  if (!ws.init(args[8], l.at, need + 8 * l.m * r.k)) {
     if (args[8] == Py_None) Py_RETURN_FALSE;
     Py_RETURN_NONE;
   }
   if (!l.output(Py_None, inplace, &out)) Py_RETURN_NONE;
-  float* weights = reinterpret_cast<float*>(ws + need);
+  float* weights = reinterpret_cast<float*>(ws.data + need);
   int32_t* ids = reinterpret_cast<int32_t*>(weights + l.m * r.k);
-  if (int rc = moe_i8_fused_moe(l.x->data_ptr(), (const float*)r.logits->data_ptr(), (const int8_t*)l.w1->data_ptr(),
-                                (const int8_t*)l.w2->data_ptr(), (const float*)l.s1->data_ptr(), (const float*)l.s2->data_ptr(),
-                                out.data_ptr(), l.m, (int)r.k, (int)l.e, (int)l.h, (int)l.i, (int)block, (int)r.score,
-                                r.bias ? (const float*)r.bias->data_ptr() : nullptr, (int)r.groups, (int)r.topk_groups, (int)r.top2,
-                                (int)r.renormalize, (float)r.scale, weights, ids, r.record ? r.record->data_ptr() : nullptr,
-                                r.record_dtype(), r.record_stride(), r.record_offset(), ws, size, (int)variant, l.at.stream))
-    return PyLong_FromLong(rc);
-  return THPVariable_Wrap(std::move(out));
+  const void* xp = data<void>(l.x);
+  const int8_t *w1 = data<int8_t>(l.w1), *w2 = data<int8_t>(l.w2);
+  const float *s1 = data<float>(l.s1), *s2 = data<float>(l.s2), *logits = data<float>(r.logits), *bias = data<float>(r.bias);
+  void* record = data<void>(r.record);
+  const int record_dtype = r.record_dtype();
+  const int64_t stride = r.record_stride(), offset = r.record_offset();
+  int rc;
+  {
+    const Unlocked unlocked;
+    if (!out.defined()) out = make({l.m, l.h}, at::kBFloat16, l.at);
+    rc = moe_i8_fused_moe(xp, logits, w1, w2, s1, s2, out.data_ptr(), l.m, (int)r.k, (int)l.e, (int)l.h, (int)l.i, (int)block,
+                          (int)r.score, bias, (int)r.groups, (int)r.topk_groups, (int)r.top2, (int)r.renormalize, (float)r.scale,
+                          weights, ids, record, record_dtype, stride, offset, ws.data, ws.bytes, (int)variant, l.at.stream);
+  }
+  return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
 }
 
 // requantise(gate, up, down, w13, w13_scale, w2, w2_scale) -> True
@@ -362,10 +427,15 @@ PyObject* requantise(PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   for (const at::Tensor* t : {u, d, w13, s13, w2, s2})
     if (t->get_device() != at.device) Py_RETURN_NONE;
-  if (int rc = moe_i8_quant_expert_weights(g->data_ptr(), u->data_ptr(), d->data_ptr(), MOE_I8_DTYPE_BF16, e, i, h,
-                                           (int8_t*)w13->data_ptr(), (float*)s13->data_ptr(), (int8_t*)w2->data_ptr(),
-                                           (float*)s2->data_ptr(), at.stream))
-    return PyLong_FromLong(rc);
+  const void *gp = data<void>(g), *up = data<void>(u), *dp = data<void>(d);
+  int8_t *w13p = data<int8_t>(w13), *w2p = data<int8_t>(w2);
+  float *s13p = data<float>(s13), *s2p = data<float>(s2);
+  int rc;
+  {
+    const Unlocked unlocked;
+    rc = moe_i8_quant_expert_weights(gp, up, dp, MOE_I8_DTYPE_BF16, e, i, h, w13p, s13p, w2p, s2p, at.stream);
+  }
+  if (rc) return PyLong_FromLong(rc);
   Py_RETURN_TRUE;
 }
 

@@ -1,6 +1,9 @@
 """What the entry points accept and refuse, and how they write their results, is the same whether the native call path
 takes a call or leaves it to the Python path."""
 
+import sys
+import threading
+
 import pytest
 import torch
 
@@ -30,3 +33,63 @@ def test_inplace_goes_by_truth(pra, M, inplace):
         assert torch.equal(got, result)
         assert (got.data_ptr() == x.data_ptr()) == bool(inplace)
         assert torch.equal(x, result if inplace else d.hidden_states)
+
+
+def _calls(pra, M):
+    """One call of every entry point the native path takes: (call, its result)."""
+    d, args, kw = _layer(M)
+    logits = torch.randn(M, 16, device=DEV)
+    mlp = (d.w1[0], d.w1_scale[0].reshape(-1), d.w2[0], d.w2_scale[0].reshape(-1))
+    gate, up, down = (torch.randn(s, device=DEV).to(torch.bfloat16) for s in ((2, 64, 128), (2, 64, 128), (2, 128, 64)))
+    out = pra.quantize_expert_weights(gate, up, down)
+    calls = (lambda: pra.fused_experts(*args, **kw), lambda: pra.fused_moe(d.hidden_states, d.w1, d.w2, logits, 4, True, **kw),
+             lambda: pra.w8a8_mlp(d.hidden_states, *mlp), lambda: pra.apply_int8_linear(d.hidden_states, *mlp[:2]),
+             lambda: pra.route_topk(logits, 4)[0], lambda: pra.quantize_expert_weights(gate, up, down, out=out)[0])
+    return [(call, call().clone()) for call in calls]
+
+
+def test_other_python_threads_run_during_the_launches(pra):
+    """The interpreter lock is given up inside every call.  With a switch interval longer than the test nothing else
+    makes this thread give it up, so another one gets it only there."""
+    interval = sys.getswitchinterval()
+    for call, _ in _calls(pra, 3):
+        go, ran = threading.Event(), []
+
+        def other():
+            go.wait()
+            ran.append(True)
+
+        thread = threading.Thread(target=other)
+        thread.start()
+        sys.setswitchinterval(60.0)
+        try:
+            go.set()
+            for _ in range(3000):
+                if ran:
+                    break
+                call()
+            seen = bool(ran)
+        finally:
+            sys.setswitchinterval(interval)
+        thread.join()
+        torch.cuda.synchronize()
+        assert seen, call
+
+
+@pytest.mark.parametrize("M", [2, 37, 200])
+def test_threads_share_a_stream_and_its_workspace(pra, M):
+    """Calls of several threads on one stream use one default workspace: their launches must not interleave."""
+    calls, wrong = _calls(pra, M)[:4], []
+    torch.cuda.synchronize()
+
+    def work(call, want):
+        for _ in range(60):
+            if not torch.equal(call(), want):
+                wrong.append(call)
+
+    threads = [threading.Thread(target=work, args=c) for c in calls + calls]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
