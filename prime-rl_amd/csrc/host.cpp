@@ -15,6 +15,7 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <utility>
@@ -146,8 +147,8 @@ bool dense_weight(PyObject* wo, PyObject* so, const at::Tensor** w, const at::Te
 PyObject* wrap_guarded(PyObject* (*fn)(PyObject* const*, Py_ssize_t), PyObject* const* args, Py_ssize_t nargs) {
   try {
     return fn(args, nargs);
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (const std::exception&) {  // as torch's own bindings raise it: an allocation that fails is an OutOfMemoryError
+    torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }

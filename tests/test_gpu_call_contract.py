@@ -93,3 +93,20 @@ def test_threads_share_a_stream_and_its_workspace(pra, M):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_a_result_that_cannot_be_allocated_is_an_out_of_memory_error(pra):
+    n, k = 16384, 64
+    w, s = torch.zeros(n, k, dtype=torch.int8, device=DEV), torch.ones(n, device=DEV)
+    x = torch.zeros(4096, k, dtype=torch.bfloat16, device=DEV)  # a result of 128 MB
+    pra.apply_int8_linear(x, w[:16].contiguous(), s[:16])  # (the default workspace)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (16 << 20)) / total)
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            pra.apply_int8_linear(x, w, s)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert pra.apply_int8_linear(x, w, s).shape == (4096, n)
