@@ -677,6 +677,11 @@ static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t
   if (!valid_block_size(block_size)) return fail(MOE_I8_EINVAL, "block_size must be 16, 32, 64 or 128");
   if (hidden_size < 64 || hidden_size % 64 || inter < 64 || inter % 64)
     return fail(MOE_I8_EINVAL, "hidden (%d) and inter (%d) must be positive multiples of 64", hidden_size, inter);
+  if (num_experts < 1 || num_experts > MOE_I8_MAX_EXPERTS)
+    return fail(MOE_I8_EINVAL, "num_experts must be in [1, %d]", MOE_I8_MAX_EXPERTS);
+  if (!aligned16(hidden) || !aligned16(w1) || !aligned16(w2) || !aligned16(out))
+    return fail(MOE_I8_EINVAL, "activation, weight and output pointers must be 16-byte aligned");
+  if (!aligned16(w1_scale) || !aligned16(w2_scale)) return fail(MOE_I8_EINVAL, "weight scales must be 16-byte aligned");
   if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(MOE_I8_EINVAL, "workspace must be 256-byte aligned");
   const Carve c = carve(m, top_k, num_experts, hidden_size, inter, block_size);
   if (workspace_bytes < c.total)
@@ -695,8 +700,7 @@ static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t
   const WorkspaceTurn turn(workspace);
 
   // A few tokens: no rows to gather per expert, the whole layer in two launches.
-  if (variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, hidden_size, inter) && aligned16(hidden) && aligned16(w1) &&
-      aligned16(w2) && num_experts <= MOE_I8_MAX_EXPERTS) {
+  if (variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, hidden_size, inter)) {
     moe_i8::FewTokensArgs f;
     f.x = static_cast<const uint16_t*>(hidden);
     f.w1 = w1;
@@ -745,8 +749,7 @@ static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t
   qa.rows = m;
   qa.q = x_q;
   qa.scale = a1;
-  if (num_experts >= 1 && num_experts <= MOE_I8_MAX_EXPERTS && aligned16(hidden) &&
-      moe_i8::align_quant_fusable(aa, qa)) {
+  if (moe_i8::align_quant_fusable(aa, qa)) {
     if (int rc = check_launch(moe_i8::launch_align_quant(aa, qa, static_cast<hipStream_t>(stream)),
                               "align_quant"))
       return rc;

@@ -266,3 +266,21 @@ def test_layer_plan_follows_a_demanded_family_and_rejects_what_it_cannot_run(pra
         pra.layer_plan(16, 8, 128, 2048, 700)
     # output pointers are optional
     assert abi.load().moe_i8_layer_plan(16, 8, 128, 2048, 768, 64, abi.GEMM_AUTO, None, None, None) == abi.OK
+
+
+@pytest.mark.parametrize("m", [1, 4, 100])  # a few tokens take launches of their own
+def test_fused_experts_refuses_misaligned_pointers_at_every_size(pra, m):
+    abi = pra._abi
+    lib = abi.load()
+    buf = ctypes.create_string_buffer(1 << 13)
+    base = (ctypes.addressof(buf) + 255) // 256 * 256
+    good = [base] * 8
+
+    def call(pointers, experts=4):
+        return lib.moe_i8_fused_experts(*pointers, m, 2, experts, 128, 64, 64, base, 1 << 30, abi.GEMM_AUTO, None)
+
+    for i in (0, 1, 2, 5, 6, 7):  # hidden, w1, w2, w1_scale, w2_scale, out
+        assert call(good[:i] + [base + 8] + good[i + 1:]) == abi.EINVAL
+        assert "16-byte aligned" in lib.moe_i8_last_error().decode()
+    for experts in (0, 1025):
+        assert call(good, experts) == abi.EINVAL and "num_experts" in lib.moe_i8_last_error().decode()
