@@ -530,7 +530,7 @@ def route_topk(
     ``src/prime_rl/inference/vllm/routed_experts.py:11-33``.
     """
     if score_func in _SCORE_FUNCS:
-        record, layer = routed_experts_out or (None, 0)
+        record, layer = (None, 0) if routed_experts_out is None else routed_experts_out
         r = _abi.host().route(gating_output, topk, _SCORE_FUNCS[score_func], 1 if renormalize else 0, float(route_scale),
                               selection_bias, num_expert_group, topk_group, 1 if group_score_top2 else 0, record, layer)
         if r is not None:
@@ -1116,7 +1116,7 @@ def fused_moe(
             and block_shape is None and global_num_experts == -1 and scoring_func in ("softmax", "sigmoid")
             and (not use_grouped_topk or (num_expert_group and topk_group))):
         groups, kept = (num_expert_group, topk_group) if use_grouped_topk else (1, 1)
-        record, layer = routed_experts_out or (None, 0)
+        record, layer = (None, 0) if routed_experts_out is None else routed_experts_out
         args = (
             hidden_states, w1, w2, w1_scale, w2_scale, block_size_m, _variant(gemm_variant), inplace, workspace,
             gating_output, topk, _SCORE_FUNCS[scoring_func], 1 if renormalize else 0, float(routed_scaling_factor),

@@ -109,14 +109,12 @@ T* data(const at::Tensor* t) {
   return t ? static_cast<T*>(t->data_ptr()) : nullptr;
 }
 
+// An int that the C-ABI's 32 bits hold.
 bool as_int(PyObject* o, int64_t* v) {
   if (!PyLong_CheckExact(o)) return false;
-  *v = PyLong_AsLongLong(o);
-  if (*v == -1 && PyErr_Occurred()) {
-    PyErr_Clear();
-    return false;
-  }
-  return true;
+  int overflow = 0;
+  *v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return !overflow && *v >= INT32_MIN && *v <= INT32_MAX;
 }
 
 // A switch that is True or False; any other value's truth is for the Python path to ask.

@@ -110,3 +110,19 @@ def test_a_result_that_cannot_be_allocated_is_an_out_of_memory_error(pra):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert pra.apply_int8_linear(x, w, s).shape == (4096, n)
+
+
+def test_what_the_python_path_refuses_is_refused(pra):
+    d, args, kw = _layer(3)
+    x, w1, w2 = args[:3]
+    logits = torch.randn(3, 16, device=DEV)
+    for block in (48, 2**32 + 64, 2**70):
+        with pytest.raises(ValueError, match="block_size"):
+            pra.fused_experts(*args, **kw, block_size_m=block)
+        with pytest.raises(ValueError, match="block_size"):
+            pra.fused_moe(x, w1, w2, logits, 4, True, **kw, block_size_m=block)
+    for record in ((), [], False):
+        with pytest.raises((ValueError, TypeError)):
+            pra.route_topk(logits, 4, routed_experts_out=record)
+        with pytest.raises((ValueError, TypeError)):
+            pra.fused_moe(x, w1, w2, logits, 4, True, **kw, routed_experts_out=record)
