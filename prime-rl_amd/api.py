@@ -255,9 +255,10 @@ def quantize_expert_weights(
     [E, 2I]``, ``w2 int8 [E, H, I]``, ``w2_scale fp32 [E, H]``.  ``out=(w13, w13_scale, w2,
     w2_scale)`` overwrites the parameters of a running engine in place.
     """
-    if out is not None and len(out) == 4:
-        if _result(_abi.host().requantise(gate_proj, up_proj, down_proj, *out)) is not None:
-            return tuple(out)
+    if out is not None:
+        out = tuple(out)  # any iterable of the four
+        if len(out) == 4 and _result(_abi.host().requantise(gate_proj, up_proj, down_proj, *out)) is not None:
+            return out
     _check_bf16_weight("gate_proj", gate_proj, 3)
     _check_bf16_weight("up_proj", up_proj, 3)
     _check_bf16_weight("down_proj", down_proj, 3)
@@ -1115,7 +1116,7 @@ def fused_moe(
     if (use_int8_w8a8 is True and per_channel_quant is True and activation == "silu" and expert_map is None
             and block_shape is None and global_num_experts == -1 and scoring_func in ("softmax", "sigmoid")
             and (not use_grouped_topk or (num_expert_group and topk_group))):
-        groups, kept = (num_expert_group, topk_group) if use_grouped_topk else (1, 1)
+        groups, kept = (max(num_expert_group, 1), max(topk_group, 1)) if use_grouped_topk else (1, 1)
         record, layer = (None, 0) if routed_experts_out is None else routed_experts_out
         args = (
             hidden_states, w1, w2, w1_scale, w2_scale, block_size_m, _variant(gemm_variant), inplace, workspace,

@@ -126,3 +126,22 @@ def test_what_the_python_path_refuses_is_refused(pra):
             pra.route_topk(logits, 4, routed_experts_out=record)
         with pytest.raises((ValueError, TypeError)):
             pra.fused_moe(x, w1, w2, logits, 4, True, **kw, routed_experts_out=record)
+
+
+def test_what_the_python_path_accepts_is_accepted(pra):
+    d, args, kw = _layer(3)
+    x, w1, w2 = args[:3]
+    logits = torch.randn(3, 16, device=DEV)
+    # group counts below one mean one group, as in grouped_topk
+    w, ids = pra.grouped_topk(x, logits, 4, True, -1, -1)
+    got = pra.fused_moe(x, w1, w2, logits, 4, True, **kw, use_grouped_topk=True, num_expert_group=-1, topk_group=-1)
+    assert torch.equal(got, pra.fused_experts(x, w1, w2, w, ids, **kw))
+    # the parameters to overwrite come as any iterable
+    gate, up, down = (torch.randn(s, device=DEV).to(torch.bfloat16) for s in ((2, 64, 128), (2, 64, 128), (2, 128, 64)))
+    want = pra.quantize_expert_weights(gate, up, down)
+    for kind in (tuple, list, iter, lambda ts: (t for t in ts)):
+        out = [torch.zeros_like(t) for t in want]
+        got = pra.quantize_expert_weights(gate, up, down, out=kind(out))
+        assert all(g is o and torch.equal(o, w) for g, o, w in zip(got, out, want))
+    with pytest.raises(ValueError):
+        pra.quantize_expert_weights(gate, up, down, out=want[:3])
