@@ -279,6 +279,8 @@ int moe_i8_fused_experts_static(const void* hidden, const int8_t* w1, const int8
  * (FeedForward.forward, src/prime_rl/trainer/models/layers/mlp.py:29-32; added to the routed output at
  * src/prime_rl/trainer/models/layers/moe.py:453-462): w13 int8 [2*inter, hidden] gate rows first,
  * w2 int8 [hidden, inter]; x bf16 [m, hidden] -> out bf16 [m, hidden].
+ *
+ * out may overlap x in both.
  */
 int moe_i8_scaled_int8_quant(const void* x, int dtype, int64_t rows, int64_t cols, int64_t row_stride,
                              int8_t* q, float* scale, void* stream);

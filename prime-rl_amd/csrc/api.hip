@@ -943,9 +943,18 @@ int run_dense(const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
   return run_gemm(g, variant, stream);
 }
 
-// A few rows: the launch quantises them itself.  Whether it runs, unless a family is demanded.
+bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+  const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+  return a0 < b0 + (uintptr_t)b_bytes && b0 < a0 + (uintptr_t)a_bytes;
+}
+
+// A few rows: the launch quantises them itself.  Whether it runs, unless a family is demanded or the output overlaps
+// the rows: every workgroup reads them all, while others already write.  (The other kernels read a copy of the rows
+// that a launch of its own has quantised.)
 bool takes_dense_few(const void* x, const moe_i8::GemmArgs& g, int variant) {
-  return variant == MOE_I8_GEMM_AUTO && moe_i8::dense_few_takes(g.num_pairs, g.n, g.k) && aligned16(x) && aligned16(g.w);
+  const int64_t width = g.mode == moe_i8::kGateUpSilu ? g.n / 2 : g.n;
+  return variant == MOE_I8_GEMM_AUTO && moe_i8::dense_few_takes(g.num_pairs, g.n, g.k) && aligned16(x) && aligned16(g.w) &&
+         !overlap(x, 2 * g.num_pairs * g.k, g.out, 2 * g.num_pairs * width);
 }
 int run_dense_few(const void* x, const moe_i8::GemmArgs& g, hipStream_t stream) {
   const moe_i8::DenseFewArgs d{g.mode, static_cast<const uint16_t*>(x), g.w, g.w_scale, static_cast<uint16_t*>(g.out), (int)g.num_pairs, g.n, g.k};

@@ -145,3 +145,29 @@ def test_what_the_python_path_accepts_is_accepted(pra):
         assert all(g is o and torch.equal(o, w) for g, o, w in zip(got, out, want))
     with pytest.raises(ValueError):
         pra.quantize_expert_weights(gate, up, down, out=want[:3])
+
+
+@pytest.mark.parametrize("M", [1, 4, 16, 50])
+@pytest.mark.parametrize("shift", [0, 16, -64])
+def test_dense_output_may_overlap_its_input(pra, M, shift):
+    """Through the C-ABI: the output on the input's memory, exactly or shifted by some elements."""
+    K = 1024
+    lib, abi = pra._abi.load(), pra._abi
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+    w = torch.randint(-127, 128, (K, K), dtype=torch.int8, device=DEV, generator=g)
+    w13 = torch.randint(-127, 128, (2 * K, K), dtype=torch.int8, device=DEV, generator=g)
+    s = torch.rand(2 * K, device=DEV, generator=g) * 1e-3
+    ws = torch.empty(lib.moe_i8_dense_workspace_bytes(M, K, K), dtype=torch.uint8, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    for want, call in (
+        (pra.apply_int8_linear(x, w, s[:K]), lambda i, o: lib.moe_i8_w8a8_linear(
+            i, w.data_ptr(), s.data_ptr(), o, M, K, K, ws.data_ptr(), ws.numel(), abi.GEMM_AUTO, stream)),
+        (pra.w8a8_mlp(x, w13, s, w, s[:K]), lambda i, o: lib.moe_i8_w8a8_mlp(
+            i, w13.data_ptr(), s.data_ptr(), w.data_ptr(), s.data_ptr(), o, M, K, K, ws.data_ptr(), ws.numel(), abi.GEMM_AUTO, stream)),
+    ):
+        memory = torch.zeros(M * K + 128, dtype=torch.bfloat16, device=DEV)
+        memory[64:64 + M * K] = x.view(-1)
+        at = memory.data_ptr() + 2 * 64
+        abi.check(call(at, at + 2 * shift))
+        assert torch.equal(memory[64 + shift:64 + shift + M * K].view(M, K), want)
