@@ -284,3 +284,39 @@ def test_fused_experts_refuses_misaligned_pointers_at_every_size(pra, m):
         assert "16-byte aligned" in lib.moe_i8_last_error().decode()
     for experts in (0, 1025):
         assert call(good, experts) == abi.EINVAL and "num_experts" in lib.moe_i8_last_error().decode()
+
+
+def test_the_library_builds_with_the_hip_compiler_alone(pra, monkeypatch, tmp_path):
+    import sys
+
+    build, commands = pra.build, []
+
+    def run(cmd):
+        commands.append(cmd)
+        Path(cmd[cmd.index("-o") + 1]).touch()
+
+    monkeypatch.setattr(build, "_run", run)
+    monkeypatch.setattr(build, "PKG_DIR", tmp_path)
+    for name in ("LIB_PATH", "PROBE_LIB_PATH"):
+        monkeypatch.setattr(build, name, tmp_path / getattr(build, name).name)
+    monkeypatch.setitem(sys.modules, "torch", None)  # not installed
+    assert build.build_library().exists()
+    assert len(commands) == len(build.SOURCES) + 3 and all("hipcc" in cmd[0] for cmd in commands)
+
+
+def test_without_a_fitting_extension_calls_take_the_python_path(pra, monkeypatch, tmp_path):
+    abi = pra._abi
+    x = torch.zeros((4, 128), dtype=torch.bfloat16)
+    with monkeypatch.context() as m:  # not built
+        m.setattr(abi, "_host", None)
+        m.setattr(abi, "HOST_PATH", tmp_path / "_host.so")
+        with pytest.warns(RuntimeWarning, match="not built: calls take the slower Python path"):
+            assert abi.host().linear(x, x, x, 0, None) is None
+        with pytest.raises(ValueError, match="GPU tensor"):  # the Python path names what is wrong
+            pra.apply_int8_linear(x, torch.zeros((8, 128), dtype=torch.int8), torch.ones(8))
+    with monkeypatch.context() as m:  # built for another torch
+        m.setattr(abi, "_host", None)
+        m.setattr(torch, "__version__", "0.0.0")
+        with pytest.warns(RuntimeWarning, match="is built for torch"):
+            assert isinstance(abi.host(), abi.PythonPathOnly)
+    assert not isinstance(abi.host(), abi.PythonPathOnly)

@@ -171,3 +171,11 @@ def test_dense_output_may_overlap_its_input(pra, M, shift):
         at = memory.data_ptr() + 2 * 64
         abi.check(call(at, at + 2 * shift))
         assert torch.equal(memory[64 + shift:64 + shift + M * K].view(M, K), want)
+
+
+@pytest.mark.parametrize("M", [1, 5, 200])
+def test_the_python_path_alone_gives_the_same_results(pra, monkeypatch, M):
+    calls = _calls(pra, M)
+    monkeypatch.setattr(pra._abi, "_host", pra._abi.PythonPathOnly())
+    for call, want in calls:
+        assert torch.equal(call(), want)
