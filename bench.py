@@ -23,6 +23,7 @@ import json
 import os
 import sys
 import time
+from collections import Counter
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent
@@ -346,7 +347,7 @@ def time_decode_mix(pkg, torch, shape_name: str, layers: int, steps: int) -> dic
     torch.cuda.synchronize()
     replay = time.perf_counter() - t0
     tokens = sum(sizes)
-    small = sum(1 for M in sizes if M * k <= 3 * E)
+    launches = Counter(pkg.layer_launches(M, k, E, H, I) for M in sizes)
     del stack, graphs
     torch.cuda.empty_cache()
     return {"shape": shape_name, "layers": layers, "steps": steps, "tokens": tokens,
@@ -356,7 +357,7 @@ def time_decode_mix(pkg, torch, shape_name: str, layers: int, steps: int) -> dic
                           "us_per_layer_call": replay / (steps * layers) * 1e6, "buckets": list(DECODE_BUCKETS),
                           "note": "one captured graph of the whole stack per bucket; batch padded up to the bucket; "
                                   "includes the device copies that refresh inputs and routing"},
-            "launches_per_layer": {"4 (down GEMM quantises its own input)": small, "5": steps - small}}
+            "launches_per_layer": {str(n): calls for n, calls in sorted(launches.items())}}  # of the steps' batches
 
 
 def time_mfma_ceiling(pkg, torch) -> dict:

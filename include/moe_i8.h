@@ -234,17 +234,23 @@ int moe_i8_fused_moe(const void* hidden, const float* logits, const int8_t* w1, 
                      void* workspace, int64_t workspace_bytes, int variant, void* stream);
 
 /*
- * What moe_i8_fused_experts would launch for a layer shape, decided on the host from the sizes alone (no GPU
- * call): the GEMM kernel of each projection (MOE_I8_GEMM_STREAM, _NARROW, _TILE_WIDE or _TILE_DEEP) and the
- * number of kernel launches of one call through its chain of stages (alignment, quantisation, GEMMs, combine).
- * Calls of a few tokens with MOE_I8_GEMM_AUTO replace that chain by two launches of their own; for them the answer
- * is the chain that a demanded family would run.  A diagnostic with no counterpart in the reference (upstream picks its
+ * The chain of stages (alignment, quantisation, GEMMs, combine) of a layer shape, decided on the host from the sizes
+ * alone (no GPU call): the GEMM kernel of each projection (MOE_I8_GEMM_STREAM, _NARROW, _TILE_WIDE or _TILE_DEEP) and
+ * the number of the chain's kernel launches.  Calls of a few tokens with MOE_I8_GEMM_AUTO replace the chain by two
+ * launches of their own: moe_i8_layer_launches says whether and how many launches a call makes.  A diagnostic with no counterpart in the reference (upstream picks its
  * kernel configuration from tuned tables per shape): it lets a test pin which measured kernel each benchmark
  * point runs on, so that a retune of the hand-over points cannot silently move one.  Any output pointer may be
  * null.  Returns MOE_I8_EUNSUPPORTED when `variant` demands a family that does not handle the shape.
  */
 int moe_i8_layer_plan(int64_t m, int top_k, int num_experts, int hidden_size, int inter, int block_size,
                       int variant, int* gate_up_kernel, int* down_kernel, int* launches);
+
+/*
+ * The kernel launches one moe_i8_fused_experts call makes, or one moe_i8_fused_moe call if `routed`; same arguments and
+ * errors as moe_i8_layer_plan.
+ */
+int moe_i8_layer_launches(int64_t m, int top_k, int num_experts, int hidden_size, int inter, int block_size, int variant,
+                          int routed, int* launches);
 
 /*
  * moe_i8_fused_experts for callers that cannot allocate device memory (code under HIP graph capture,

@@ -11,6 +11,7 @@ from .api import (  # noqa: F401
     fused_experts,
     fused_moe,
     fused_topk,
+    layer_launches,
     layer_plan,
     grouped_topk,
     route_topk,
@@ -37,6 +38,7 @@ from . import api, build, vllm_plugin  # noqa: F401
 __all__ = [
     "fused_experts",
     "fused_moe",
+    "layer_launches",
     "layer_plan",
     "moe_align_block_size",
     "per_token_quant_int8",

@@ -120,16 +120,28 @@ _KERNEL_NAMES = {_abi.GEMM_STREAM: "stream", _abi.GEMM_NARROW: "narrow", _abi.GE
 
 def layer_plan(m: int, top_k: int, num_experts: int, hidden: int, inter: int,
                block_size: int = 64, gemm_variant: str | int = "auto") -> dict:
-    """Which GEMM kernel ``fused_experts`` runs for each projection of a layer of this shape and how many
-    kernel launches one call makes: ``{"gate_up": name, "down": name, "launches": n}``.  Decided on the host
-    from the sizes alone (no GPU needed), by the same code the driver uses.  Of a few tokens that ``"auto"`` runs
-    in two launches of their own it names the chain of stages they replace."""
+    """The chain of stages of a layer of this shape: the GEMM kernel of each projection and the chain's kernel
+    launches, ``{"gate_up": name, "down": name, "launches": n}``.  Decided on the host from the sizes alone (no GPU
+    needed), by the same code the driver uses.  ``"auto"`` runs a few tokens in two launches of their own instead:
+    ``layer_launches`` counts what a call makes."""
     import ctypes
 
     gu, dn, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     _abi.check(_abi.load().moe_i8_layer_plan(m, top_k, num_experts, hidden, inter, block_size, _variant(gemm_variant),
                                              ctypes.byref(gu), ctypes.byref(dn), ctypes.byref(n)))
     return {"gate_up": _KERNEL_NAMES[gu.value], "down": _KERNEL_NAMES[dn.value], "launches": n.value}
+
+
+def layer_launches(m: int, top_k: int, num_experts: int, hidden: int, inter: int, block_size: int = 64,
+                   gemm_variant: str | int = "auto", routed: bool = False) -> int:
+    """Kernel launches of one ``fused_experts`` call (``routed``: one ``fused_moe`` call) of a layer of this shape,
+    decided on the host as the call itself decides."""
+    import ctypes
+
+    n = ctypes.c_int()
+    _abi.check(_abi.load().moe_i8_layer_launches(m, top_k, num_experts, hidden, inter, block_size, _variant(gemm_variant),
+                                                 1 if routed else 0, ctypes.byref(n)))
+    return n.value
 
 
 # --------------------------------------------------------------------------------------------- #

@@ -653,6 +653,11 @@ LayerPlan plan_layer(int64_t m, int top_k, int num_experts, int hidden, int inte
   plan.launches = moe_i8::align_launches(aa) + (plan.fuse_align_quant ? 0 : 1) + 1 + (plan.down_quantises ? 1 : 2) + 1;
   return plan;
 }
+
+// A few tokens: no rows to gather per expert, the whole layer in two launches instead of that chain.
+bool runs_few_tokens(int64_t m, int top_k, int hidden, int inter, int variant) {
+  return variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, hidden, inter);
+}
 }  // namespace
 
 int64_t moe_i8_workspace_bytes(int64_t m, int top_k, int num_experts, int hidden, int inter,
@@ -699,8 +704,7 @@ static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t
   const int64_t p = m * top_k;
   const WorkspaceTurn turn(workspace);
 
-  // A few tokens: no rows to gather per expert, the whole layer in two launches.
-  if (variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, hidden_size, inter)) {
+  if (runs_few_tokens(m, top_k, hidden_size, inter, variant)) {
     moe_i8::FewTokensArgs f;
     f.x = static_cast<const uint16_t*>(hidden);
     f.w1 = w1;
@@ -716,7 +720,7 @@ static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t
     f.num_experts = num_experts;
     f.hidden = hidden_size;
     f.inter = inter;
-    const bool routes = route && moe_i8::few_tokens_routes(*route);
+    const bool routes = route && moe_i8::few_tokens_routes(m, num_experts);
     if (route && !routes)
       if (int rc = check_launch(moe_i8::launch_route_topk(*route, static_cast<hipStream_t>(stream)), "route_topk")) return rc;
     return check_launch(moe_i8::launch_few_tokens(f, routes ? route : nullptr, static_cast<hipStream_t>(stream)), "few_tokens");
@@ -802,8 +806,7 @@ int moe_i8_fused_moe(const void* hidden, const float* logits, const int8_t* w1, 
                             inter, block_size, workspace, workspace_bytes, variant, &route, stream);
 }
 
-int moe_i8_layer_plan(int64_t m, int top_k, int num_experts, int hidden_size, int inter, int block_size,
-                      int variant, int* gate_up_kernel, int* down_kernel, int* launches) {
+static int layer_shape_args(int64_t m, int top_k, int num_experts, int hidden_size, int inter, int block_size, int variant) {
   if (m < 1 || top_k < 1 || m * top_k > INT32_MAX - 1) return fail(MOE_I8_EINVAL, "m / top_k out of range");
   if (num_experts < 1 || num_experts > MOE_I8_MAX_EXPERTS)
     return fail(MOE_I8_EINVAL, "num_experts must be in [1, %d]", MOE_I8_MAX_EXPERTS);
@@ -812,11 +815,31 @@ int moe_i8_layer_plan(int64_t m, int top_k, int num_experts, int hidden_size, in
     return fail(MOE_I8_EINVAL, "hidden (%d) and inter (%d) must be positive multiples of 64", hidden_size, inter);
   if (variant < MOE_I8_GEMM_AUTO || variant > MOE_I8_GEMM_TILE_RING)
     return fail(MOE_I8_EINVAL, "unknown GEMM variant %d", variant);
+  return MOE_I8_OK;
+}
+
+int moe_i8_layer_plan(int64_t m, int top_k, int num_experts, int hidden_size, int inter, int block_size,
+                      int variant, int* gate_up_kernel, int* down_kernel, int* launches) {
+  if (int rc = layer_shape_args(m, top_k, num_experts, hidden_size, inter, block_size, variant)) return rc;
   const LayerPlan plan = plan_layer(m, top_k, num_experts, hidden_size, inter, block_size, variant);
   if (plan.gate_up_kernel < 0 || plan.down_kernel < 0) return MOE_I8_EUNSUPPORTED;
   if (gate_up_kernel) *gate_up_kernel = plan.gate_up_kernel;
   if (down_kernel) *down_kernel = plan.down_kernel;
   if (launches) *launches = plan.launches;
+  return MOE_I8_OK;
+}
+
+int moe_i8_layer_launches(int64_t m, int top_k, int num_experts, int hidden_size, int inter, int block_size, int variant,
+                          int routed, int* launches) {
+  if (int rc = layer_shape_args(m, top_k, num_experts, hidden_size, inter, block_size, variant)) return rc;
+  if (!launches) return fail(MOE_I8_EINVAL, "null pointer");
+  if (runs_few_tokens(m, top_k, hidden_size, inter, variant)) {
+    *launches = routed && !moe_i8::few_tokens_routes(m, num_experts) ? 3 : 2;
+    return MOE_I8_OK;
+  }
+  const LayerPlan plan = plan_layer(m, top_k, num_experts, hidden_size, inter, block_size, variant);
+  if (plan.gate_up_kernel < 0 || plan.down_kernel < 0) return MOE_I8_EUNSUPPORTED;
+  *launches = plan.launches + (routed ? 1 : 0);
   return MOE_I8_OK;
 }
 

@@ -357,7 +357,7 @@ struct FewTokensArgs {
 constexpr int kFewTokensMaxPairs = 64;  // one lane per pair
 bool few_tokens_takes(int64_t tokens, int top_k, int hidden, int inter);
 // `route`: the first launch routes the token too and writes topk_weights and topk_ids; only when few_tokens_routes() says so.
-bool few_tokens_routes(const RouteArgs& r);
+bool few_tokens_routes(int64_t tokens, int num_experts);
 hipError_t launch_few_tokens(const FewTokensArgs& a, const RouteArgs* route, hipStream_t stream);
 
 hipError_t launch_moe_sum(const uint16_t* in, uint16_t* out, int64_t m, int top_k, int hidden,

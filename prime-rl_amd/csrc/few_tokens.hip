@@ -261,9 +261,9 @@ bool few_tokens_takes(int64_t tokens, int top_k, int hidden, int inter) {
          hidden <= 8 * 1024 && inter <= 4 * 1024;
 }
 
-bool few_tokens_routes(const RouteArgs& r) {
+bool few_tokens_routes(int64_t tokens, int num_experts) {
   // an expert group is a run of whole lanes: with other numbers of experts per lane than these two a launch of its own
-  return r.m == 1 && (route_experts_per_lane(r.num_experts) == 2 || route_experts_per_lane(r.num_experts) == 4);
+  return tokens == 1 && (route_experts_per_lane(num_experts) == 2 || route_experts_per_lane(num_experts) == 4);
 }
 
 hipError_t launch_few_tokens(const FewTokensArgs& a, const RouteArgs* route, hipStream_t stream) {

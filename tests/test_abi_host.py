@@ -214,8 +214,8 @@ def test_header_is_plain_c_and_a_c_client_links(pra, tmp_path):
     assert run.returncode == 0 and run.stdout.strip() == "ok", run.stdout + run.stderr
 
 
-# Which kernel the library picks by itself at every benchmark point (shape, tokens) and how many launches a
-# layer call makes there.  These are the kernels the committed measurements were taken on: a retune of the
+# Which kernels the library picks by itself for the chain of stages at every benchmark point (shape, tokens) and how
+# many launches the chain makes there (calls of a few tokens run without it: test_launches_of_a_call).  These are the kernels the committed measurements were taken on: a retune of the
 # hand-over points between the GEMM families must change this table knowingly.
 _PLAN = [
     ("toy", 256, "tile_deep", "tile_deep", 5),
@@ -320,3 +320,18 @@ def test_without_a_fitting_extension_calls_take_the_python_path(pra, monkeypatch
         with pytest.warns(RuntimeWarning, match="is built for torch"):
             assert isinstance(abi.host(), abi.PythonPathOnly)
     assert not isinstance(abi.host(), abi.PythonPathOnly)
+
+
+@pytest.mark.parametrize("shape_name,M,launches,routed", [
+    ("qwen3-30b-a3b", 1, 2, 2), ("qwen3-30b-a3b", 2, 2, 3), ("qwen3-30b-a3b", 8, 2, 3), ("qwen3-30b-a3b", 9, 4, 5),
+    ("qwen3-30b-a3b", 128, 5, 6), ("qwen3-30b-a3b", 8192, 7, 8), ("glm-4.5-air", 4, 2, 3), ("glm-4.5-air", 5, 5, 6),
+    ("deepseek-v3", 1, 2, 2), ("deepseek-v3", 8, 5, 6), ("deepseek-v3", 2048, 6, 7),
+])
+def test_launches_of_a_call(pra, shape_name, M, launches, routed):
+    shape = pra.inputs.SHAPES[shape_name]
+    args = (M, shape.k + (1 if shape.shared_expert else 0), shape.E_total, shape.H, shape.I)
+    assert pra.layer_launches(*args) == launches and pra.layer_launches(*args, routed=True) == routed
+    # a demanded family runs the chain of stages
+    assert pra.layer_launches(*args, gemm_variant="stream") == pra.layer_plan(*args, gemm_variant="stream")["launches"]
+    with pytest.raises(pra._abi.MoeI8Error):
+        pra.layer_launches(0, *args[1:])

@@ -1,6 +1,7 @@
 """What the entry points accept and refuse, and how they write their results, is the same whether the native call path
 takes a call or leaves it to the Python path."""
 
+import ctypes
 import sys
 import threading
 
@@ -179,3 +180,31 @@ def test_the_python_path_alone_gives_the_same_results(pra, monkeypatch, M):
     monkeypatch.setattr(pra._abi, "_host", pra._abi.PythonPathOnly())
     for call, want in calls:
         assert torch.equal(call(), want)
+
+
+@pytest.mark.parametrize("M", [1, 2, 8, 9, 37, 200, 1500, 9000])
+@pytest.mark.parametrize("E", [16, 128])
+def test_layer_launches_are_what_a_captured_call_records(pra, M, E):
+    k, H, I = 4, 512, 256
+    d, args, kw = _layer(M, E=E, k=k, H=H, I=I)
+    lib = pra._abi.load()  # (its handle finds the HIP runtime it is linked with)
+    logits = torch.randn(M, E, device=DEV)
+    w, ids = torch.empty(M, k, device=DEV), torch.empty(M, k, dtype=torch.int32, device=DEV)
+    out = torch.empty_like(d.hidden_states)
+    ws = torch.empty(pra.workspace_bytes(M, k, E, H, I, 64), dtype=torch.uint8, device=DEV)
+
+    def routed():
+        pra._abi.check(lib.moe_i8_fused_moe(
+            d.hidden_states.data_ptr(), logits.data_ptr(), d.w1.data_ptr(), d.w2.data_ptr(), d.w1_scale.data_ptr(),
+            d.w2_scale.data_ptr(), out.data_ptr(), M, k, E, H, I, 64, 0, None, 1, 1, 0, 1, 1.0, w.data_ptr(), ids.data_ptr(),
+            None, 0, 0, 0, ws.data_ptr(), ws.numel(), 0, torch.cuda.current_stream().cuda_stream))
+
+    for call, is_routed in ((lambda: pra.fused_experts(*args, **kw, workspace=ws, out=out), False), (routed, True)):
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            call()
+        nodes = ctypes.c_size_t()
+        assert lib.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+        assert nodes.value == pra.layer_launches(M, k, E, H, I, routed=is_routed)
