@@ -12,6 +12,11 @@
 // us per launch, streaming kernel -> this one (8 experts per token, gate_up / self-quantising down):
 // 1 token 11.4 -> 7.2 / 8.0 -> 5.9, 2 tokens 12.7 -> 11.3 / 9.2 -> 7.9, 3 tokens 18.1 -> 14.7 / 10.9 -> 9.5; even
 // at 4 to 5 tokens, slower from 6 on (15.3 -> 16.2).
+//
+// Where it runs: calls of a few tokens that the two-launch layer does not take (a reduction of the down GEMM
+// beyond 4096, 5 to 16 tokens on a handful of experts), and the streaming family when it is demanded.  Layer us,
+// streaming kernel -> this one: 8 experts (2 per token) of 2048 x 5632 at 1 / 4 / 10 tokens 54.7 -> 29.5, 63.1 -> 47.8,
+// 73.6 -> 62.1; of 4096 x 1408 at 5 / 9 tokens 41.1 -> 34.9, 42.5 -> 37.0; 4 experts of 8192 x 1024 at 14 tokens 52.8 -> 37.7.
 #include "lds_loads.hpp"
 #include "quant_body.hpp"
 
@@ -249,13 +254,14 @@ hipError_t launch_config(const SplitParams& p0, int64_t blocks, hipStream_t stre
 
 int64_t blocks_of(const GemmArgs& a) { return (a.sorted_cap + a.block_size - 1) / a.block_size; }
 
+// Eight wavefronts on 16 rows while that makes no more than four workgroups per compute unit, then two on 32
+// (fewer, longer workgroups: 11.3 against 11.5-12.0 us at two tokens, 17.7 against 19.6 at four).
+bool eight_wavefronts(int64_t blocks, int n) { return blocks * (n / 16) <= 4 * (int64_t)device_cu_count(); }
+
 template <int MODE, bool kFused>
 hipError_t launch_mode(const SplitParams& p, int64_t blocks, hipStream_t stream) {
-  // eight wavefronts on 16 rows while that makes no more than four workgroups per compute unit, then two on 32
-  // (fewer, longer workgroups: 11.3 against 11.5-12.0 us at two tokens, 17.7 against 19.6 at four)
-  if (blocks * (p.N / 16) <= 4 * (int64_t)device_cu_count())
-    return launch_config<MODE, kFused, 16, 8, 2>(p, blocks, stream);
-  return launch_config<MODE, kFused, 32, 2, 2>(p, blocks, stream);
+  return eight_wavefronts(blocks, p.N) ? launch_config<MODE, kFused, 16, 8, 2>(p, blocks, stream)
+                                       : launch_config<MODE, kFused, 32, 2, 2>(p, blocks, stream);
 }
 
 }  // namespace
@@ -263,12 +269,21 @@ hipError_t launch_mode(const SplitParams& p, int64_t blocks, hipStream_t stream)
 // Measured crossover with the streaming kernel, in the wavefronts that one would have (one per 32 weight rows
 // and block) on a device that holds 3072 of them: gate_up 18.1 -> 14.7 us at 1152, 19.0 -> 17.6 at 1536, even
 // at 2048 and 2304; down 10.9 -> 9.5 at 1536, 12.1 -> 11.1 at 2048, even at 2560, slower at 3072.
+//
+// The token rows lie whole in LDS, so they decide how many workgroups of two wavefronts a compute unit holds, and a second
+// round of workgroups costs more than the split saves.  us per gate_up, streaming kernel / this one: 8 experts of 4096 x
+// 1408 (704 workgroups) 21.7 / 21.3 at 9 rows, three to a unit, and 21.8 / 30.2 at 10, two to a unit; 16 experts of 2048
+// x 1024 (1024 workgroups) 12.4 / 17.3 at 12 rows, three to a unit.
 bool gemm_split_takes(const GemmArgs& a) {
   const int64_t most_rows = a.max_rows_per_expert > 0 && a.max_rows_per_expert < a.num_pairs ? a.max_rows_per_expert : a.num_pairs;
-  const int cus = device_cu_count();
-  return a.mode != kAccI32 && most_rows <= kRows && a.k <= kMaxK && (int64_t)a.n * a.k < (1ll << 32) &&
-         blocks_of(a) * (a.n / 32) <= (a.mode == kGateUpSilu ? 8 : 10) * cus &&
-         ring_bytes(16, 8, 2) + most_rows * (a.k + kRowPad) <= kMaxLds - 1024;
+  const int64_t cus = device_cu_count(), blocks = blocks_of(a);
+  if (a.mode == kAccI32 || most_rows > kRows || a.k > kMaxK || (int64_t)a.n * a.k >= (1ll << 32) ||
+      blocks * (a.n / 32) > (a.mode == kGateUpSilu ? 8 : 10) * cus)
+    return false;
+  const int64_t rows_lds = most_rows * (a.k + kRowPad);
+  if (eight_wavefronts(blocks, a.n)) return ring_bytes(16, 8, 2) + rows_lds <= kMaxLds - 1024;
+  const int64_t used = blocks < a.num_experts ? blocks : a.num_experts;  // (an expert's rows fit one block)
+  return used * ((a.n + 31) / 32) <= cus * (kMaxLds / (ring_bytes(32, 2, 2) + rows_lds));
 }
 bool gemm_split_fuses_quant(int k) { return k <= kMaxFusedK; }
 

@@ -37,6 +37,18 @@ def test_few_tokens_equal_the_tiled_families_stages(pra, oracle, E, k, H, I, M, 
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("E,k,H,I", [(8, 2, 4096, 1408), (16, 2, 2048, 1024), (8, 2, 2048, 5632)])
+@pytest.mark.parametrize("M", [5, 9, 10, 11, 12, 16])
+def test_either_side_of_the_line_between_the_streaming_kernels(pra, E, k, H, I, M):
+    """Token rows in LDS: whether all workgroups of the split-reduction kernel are resident at once decides which
+    kernel runs (9 and 10 rows of 4096, 11 and 12 of 2048)."""
+    im = inputs_mod()
+    d = im.make_inputs(im.LayerShape("s", E=E, k=k, H=H, I=I), M, seed=E + M).to(DEV)
+    kw = d.fused_experts_kwargs()
+    got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream")
+    assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="narrow"))
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 16])
 @pytest.mark.parametrize("M,H", [(1, 8), (3, 2048), (33, 7168)])
 def test_combine_at_every_k(pra, oracle, k, M, H):
