@@ -655,8 +655,8 @@ LayerPlan plan_layer(int64_t m, int top_k, int num_experts, int hidden, int inte
 }
 
 // A few tokens: no rows to gather per expert, the whole layer in two launches instead of that chain.
-bool runs_few_tokens(int64_t m, int top_k, int hidden, int inter, int variant) {
-  return variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, hidden, inter);
+bool runs_few_tokens(int64_t m, int top_k, int num_experts, int hidden, int inter, int variant) {
+  return variant == MOE_I8_GEMM_AUTO && moe_i8::few_tokens_takes(m, top_k, num_experts, hidden, inter);
 }
 }  // namespace
 
@@ -704,7 +704,7 @@ static int fused_experts_impl(const void* hidden, const int8_t* w1, const int8_t
   const int64_t p = m * top_k;
   const WorkspaceTurn turn(workspace);
 
-  if (runs_few_tokens(m, top_k, hidden_size, inter, variant)) {
+  if (runs_few_tokens(m, top_k, num_experts, hidden_size, inter, variant)) {
     moe_i8::FewTokensArgs f;
     f.x = static_cast<const uint16_t*>(hidden);
     f.w1 = w1;
@@ -833,7 +833,7 @@ int moe_i8_layer_launches(int64_t m, int top_k, int num_experts, int hidden_size
                           int routed, int* launches) {
   if (int rc = layer_shape_args(m, top_k, num_experts, hidden_size, inter, block_size, variant)) return rc;
   if (!launches) return fail(MOE_I8_EINVAL, "null pointer");
-  if (runs_few_tokens(m, top_k, hidden_size, inter, variant)) {
+  if (runs_few_tokens(m, top_k, num_experts, hidden_size, inter, variant)) {
     *launches = routed && !moe_i8::few_tokens_routes(m, num_experts) ? 3 : 2;
     return MOE_I8_OK;
   }

@@ -355,7 +355,7 @@ struct FewTokensArgs {
   int inter;
 };
 constexpr int kFewTokensMaxPairs = 64;  // one lane per pair
-bool few_tokens_takes(int64_t tokens, int top_k, int hidden, int inter);
+bool few_tokens_takes(int64_t tokens, int top_k, int num_experts, int hidden, int inter);
 // `route`: the first launch routes the token too and writes topk_weights and topk_ids; only when few_tokens_routes() says so.
 bool few_tokens_routes(int64_t tokens, int num_experts);
 hipError_t launch_few_tokens(const FewTokensArgs& a, const RouteArgs* route, hipStream_t stream);

@@ -252,13 +252,19 @@ hipError_t launch_down(const FewTokensArgs& a, hipStream_t stream) {
 
 // Layer us, blocks of rows per expert -> this, at 1 / 2 / 3 / 4 / 8 tokens: 20.4 / 25.9 / 30.7 / 35.3 / 55.3 -> 10.9 / 16.7 /
 // 22.4 / 27.4 / 47.6 (128 experts of 2048 x 768, 8 per token), 67.3 / 127.3 / 157.3 / 197.5 / 305 -> 55.4 / 107.4 / 141.4 /
-// 179.6 / 308 (256 experts of 7168 x 2048).  An expert that every token visits is taken row after row here: with one
-// (4096 x 1408, skewed routing) 38.5 / 46.2 / 60.5 / 65.5 / - -> 27.5 / 40.7 / 54.0 / 64.8 / - and slower from 6 tokens on;
-// small experts are past it soon.
-bool few_tokens_takes(int64_t tokens, int top_k, int hidden, int inter) {
+// 179.6 / 308 (256 experts of 7168 x 2048).
+//
+// An expert is taken row after row here, so what decides is how many tokens share one.  An expert that every token
+// visits (one of 129 of 4096 x 1408, skewed routing; 17 MB of weights) is the longest chain of the launch: 60.5 / 45.7,
+// 63.7 / 54.1, 72.8 / 68.2, 72.9 / 72.6, 78.4 / 85.6 there / here at 2 to 6 tokens.  With small experts that chain is short
+// against the launches saved.  The line at 8 MB is on the safe side: evenly routed, 8 tokens on 128 experts of 2880 x
+// 960 (7.9 MB) take 98.3 / 74.2, but on ones of 4096 x 1024 (12 MB), which go there, 126.3 / 101.5.
+// Where more than seven tokens share every expert the chain of launches is shorter at any size: 8 tokens on one expert of
+// 2048 x 1024 17.1 / 18.0, on eight of 2048 x 1280 that all visit 31.6 / 34.5 (7 tokens: 16.9 / 16.5, 31.8 / 31.4).
+bool few_tokens_takes(int64_t tokens, int top_k, int num_experts, int hidden, int inter) {
   const bool small_experts = 3ll * hidden * inter <= (8ll << 20);
-  return tokens <= (small_experts ? 8 : 4) && tokens * top_k <= kFewTokensMaxPairs && hidden % 16 == 0 && inter % 16 == 0 &&
-         hidden <= 8 * 1024 && inter <= 4 * 1024;
+  return tokens <= (small_experts ? 8 : 4) && tokens * top_k <= kFewTokensMaxPairs && tokens * top_k <= 7ll * num_experts &&
+         hidden % 16 == 0 && inter % 16 == 0 && hidden <= 8 * 1024 && inter <= 4 * 1024;
 }
 
 bool few_tokens_routes(int64_t tokens, int num_experts) {

@@ -335,3 +335,12 @@ def test_launches_of_a_call(pra, shape_name, M, launches, routed):
     assert pra.layer_launches(*args, gemm_variant="stream") == pra.layer_plan(*args, gemm_variant="stream")["launches"]
     with pytest.raises(pra._abi.MoeI8Error):
         pra.layer_launches(0, *args[1:])
+
+
+@pytest.mark.parametrize("E,k,H,I,M,few", [
+    (1, 1, 2048, 1024, 7, True), (1, 1, 2048, 1024, 8, False), (8, 8, 2048, 1280, 7, True), (8, 8, 2048, 1280, 8, False),
+    (9, 8, 2048, 1280, 8, False), (10, 8, 2048, 1280, 8, True), (128, 8, 2048, 1408, 4, True), (128, 8, 2048, 1408, 5, False),
+    (128, 17, 2048, 768, 3, True), (128, 17, 2048, 768, 4, False), (4, 1, 8256, 64, 1, False), (4, 1, 64, 4160, 1, False),
+])
+def test_line_of_the_two_launch_layer(pra, E, k, H, I, M, few):
+    assert (pra.layer_launches(M, k, E, H, I) == 2) is few

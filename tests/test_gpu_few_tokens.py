@@ -80,7 +80,7 @@ def test_narrow_tiles_at_short_reductions_and_many_tasks(pra, oracle, E, k, H, I
 @pytest.mark.parametrize("E,k,H,I,M", [
     (16, 8, 2048, 768, 1), (4, 4, 64, 64, 1), (40, 20, 1088, 192, 1), (1, 1, 8192, 4096, 1), (9, 9, 4096, 1408, 1),
     (16, 8, 2048, 768, 8), (5, 2, 1024, 1024, 2), (6, 3, 1088, 1088, 3), (4, 4, 7168, 2112, 4), (12, 1, 3072, 3072, 4),
-    (64, 8, 5120, 64, 7), (70, 64, 192, 320, 1), (8, 8, 6144, 128, 8),
+    (64, 8, 5120, 64, 7), (70, 64, 192, 320, 1), (8, 8, 6144, 128, 8), (10, 8, 6144, 128, 8),
 ])
 def test_layer_of_a_few_tokens_equals_the_chain_of_stages(pra, E, k, H, I, M):
     """The two-launch layer against the chain through moe_align, tokens sharing experts or not."""
