@@ -64,7 +64,6 @@ struct WideParams {
   int K;
   int B;
   int per_tile;  // most blocks of a tile
-  int keep;      // store results without the non-temporal hint where weight rows are shared
   int even;      // an expert's blocks are dealt evenly to its tiles, instead of full tiles and a rest
   int ntiles;    // channel tiles
   int ascend;  // expert_ids is known to ascend over the used blocks (it comes from moe_align)
@@ -273,7 +272,9 @@ __device__ __forceinline__ void barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int MODE>
+// KEEP: results are stored without the non-temporal hint where weight rows are shared.  (A template argument: of two
+// stores behind a run-time flag the compiler makes one, without the hint.)
+template <int MODE, bool KEEP>
 __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
   __shared__ __align__(16) char stages[2 * kStage];
   __shared__ __align__(16) char staging[kWaves * kStaging];
@@ -557,7 +558,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
       const float* ws = w_scales[aux];
       auto store = [&](uint16_t* to, const uint4& v) {
         const v4i x = {(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-        if (!NT && p.keep)
+        if constexpr (KEEP && !NT)
           *reinterpret_cast<v4i*>(to) = x;
         else
           __builtin_nontemporal_store(x, reinterpret_cast<v4i*>(to));
@@ -681,13 +682,18 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.even = a.k > 4096;
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kCh - 1) / kCh;
   p.ascend = a.expert_ids_ascend && a.num_experts <= 2 * kThreads ? 1 : 0;
-  // The next launch reads the results back from the last-level cache where they about fit it and the weights do not sweep
-  // it: 128 experts of 2048 x 768 at 4096 / 8192 / 16384 tokens 305.6 / 486 / 864 -> 298 / 480 / 856 us a layer; 256 experts of
-  // 7168 x 2048 2431 -> 2446 at 4096.
-  p.keep = (int64_t)a.num_experts * a.n * a.k < (2048ll << 20) &&
-           a.num_pairs * (MODE == kGateUpSilu ? a.n / 2 : a.n) * 2 < (600ll << 20);
+  // The next launch of a layer reads the results back from the last-level cache where they about fit it and the weights do
+  // not sweep it.  Layer us with / without the hint: 128 experts of 2048 x 768 at 8192 tokens 488 / 480, of 4096 x 1536 at
+  // 4000 881 / 865; the other side of the line: 256 experts of 7168 x 2048 at 8192 tokens 3780 / 3813, a gated MLP of 4096 x
+  // 1408 at 4096 rows, whose weights stay cached, 88.3 / 89.7.
+  const bool keep = MODE != kAccI32 && a.num_experts > 1 && (int64_t)a.num_experts * a.n * a.k < (2048ll << 20) &&
+                    a.num_pairs * (MODE == kGateUpSilu ? a.n / 2 : a.n) * 2 < (600ll << 20);
   p.out = a.out;
-  hipLaunchKernelGGL((gemm_wide_kernel<MODE>), dim3((unsigned)(device_cu_count() / kXcds * kXcds)), dim3(kThreads), 0, stream, p);
+  const dim3 grid((unsigned)(device_cu_count() / kXcds * kXcds));
+  if (keep)
+    hipLaunchKernelGGL((gemm_wide_kernel<MODE, true>), grid, dim3(kThreads), 0, stream, p);
+  else
+    hipLaunchKernelGGL((gemm_wide_kernel<MODE, false>), grid, dim3(kThreads), 0, stream, p);
   return hipGetLastError();
 }
 
