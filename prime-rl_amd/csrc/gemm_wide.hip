@@ -678,8 +678,11 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.B = a.block_size;
   p.per_tile = kTok / a.block_size;
   // Nine blocks as 3 + 3 + 3 instead of 4 + 4 + 1: a step of one block costs far more than a quarter of a full one (its weight
-  // rows are the same).  16384 tokens on 256 experts of 7168 x 2048: 6360 -> 6247 us a layer; even with reductions up to 4096.
-  p.even = a.k > 4096;
+  // rows are the same).  Layer us, full tiles and a rest / even ones: 256 experts of 7168 x 2048 at 8192 / 16384 tokens 4229 / 3790,
+  // 6360 / 6247, 129 of 4096 x 1408, evenly routed, at 4096 1066 / 933 (skewed routing: the same).  Below: no difference
+  // at 2048 x 768 and 2048 x 1408, and even tiles lose at short reductions, where a task is mostly its epilogue: 32
+  // experts of 1024 x 512 at 5000 tokens 101.6 / 103.3, 256 of 2048 x 512 at 4000 297.9 / 303.7.
+  p.even = a.k >= 4096;
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kCh - 1) / kCh;
   p.ascend = a.expert_ids_ascend && a.num_experts <= 2 * kThreads ? 1 : 0;
   // The next launch of a layer reads the results back from the last-level cache where they about fit it and the weights do
