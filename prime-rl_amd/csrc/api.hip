@@ -106,9 +106,10 @@ int tile_geometry_of(int variant) {
 // Routed rows per expert up to which the narrow tiles beat the deep geometry of the LDS-tiled family.
 // The narrow tiles (64 x 128 tasks) start up faster and balance better; the deep tiles stream an
 // expert's weights once for up to 128 rows, which counts the more the longer a launch runs and the
-// more the routing is skewed.  Measured crossovers, with the weight bytes of the launch: 0.2-0.4 GB
-// (Qwen3-30B-A3B, even routing) 40 rows, 0.7-1.5 GB (GLM-4.5-Air, Zipf routing and a shared expert)
-// 24-32, 3.8-7.5 GB (DeepSeek-V3) between 16 (1442 against 1512 us a layer) and 32 (1765 against 1629).
+// more the routing is skewed.  Layer us, narrow / deep, by the weight bytes of the launch and rows per expert: 0.2-0.4 GB
+// (Qwen3-30B-A3B, even routing) 24 rows 125 / 130, 32 135 / 134, 40 142 / 139, 48 159 / 144; 0.7-1.5 GB (GLM-4.5-Air,
+// Zipf routing and a shared expert) 24 289 / 300, 28 317 / 317, 32 338 / 337, 36 366 / 347; 3.8-7.5 GB (DeepSeek-V3)
+// 16 1406 / 1456, 20 1545 / 1577, 24 1627 / 1604, 32 1766 / 1632.
 int narrow_rows_per_expert(const moe_i8::GemmArgs& g) {
   const int64_t weight_bytes = (int64_t)g.num_experts * g.n * g.k;
   return weight_bytes < (512ll << 20) ? 40 : weight_bytes < (2048ll << 20) ? 28 : 16;

@@ -13,9 +13,11 @@
 // between its multiplications.  Against two workgroups of four wavefronts with three stages each (64 KB in
 // flight, a look-up of two dependent scalar reads per tile, loads first): same tiles, but half as long per tile
 // and twice as many per workgroup, which evens out the last round; 0.57 us per step = 7.3 TB/s of weights.
-// Layer us before -> after: 128 experts of 2048 x 768 at 17 / 100 / 203 / 512 tokens 85.0 / 118.1 / 122.0 / 138.3
-// -> 81.6 / 112.5 / 116.9 / 132.6, 4096 x 1408 with skewed routing at 17 / 64 / 200 tokens 113.8 / 155.0 / 250.4 ->
-// 105.7 / 151.0 / 242.4, 256 experts of 7168 x 2048 at 17 / 128 / 256 tokens 557 / 1109 / 1268 -> 537 / 1026 / 1199.
+// Layer us before -> after: 128 experts of 2048 x 768 at 17 / 100 / 203 / 400 / 512 tokens 80.6 / 112.3 / 117.1 / 128.1 /
+// 135.1 -> 78.0 / 109.0 / 113.1 / 126.1 / 135.3, 4096 x 1408 with skewed routing at 17 / 64 tokens 104.7 / 148.6 -> 99.8 /
+// 143.2, but at 200 / 300 tokens, where one expert holds several tiles of rows, 231.0 / 265.1 -> 235.5 / 271.2; 256 experts
+// of 7168 x 2048 at 17 / 64 / 128 / 256 tokens 544 / 909 / 1062 / 1226 -> 535 / 874 / 1033 / 1186.  Launches of
+// several tasks of four steps gain nothing: 256 experts of 2048 x 512 at 90 tokens 134 -> 139.5.
 //
 // A tile is TOK token rows (32 or 64: part of a moe_align block) x 128 weight rows; the reduction runs
 // in steps of 128 bytes and both operands reach LDS by global -> LDS loads (global_load_lds_dwordx4, no
