@@ -41,12 +41,12 @@ extern "C" {
 /* GEMM kernel families; MOE_I8_GEMM_AUTO picks by rows-per-expert. */
 #define MOE_I8_GEMM_AUTO 0
 #define MOE_I8_GEMM_STREAM 1 /* weights streamed global->registers, 16-row MFMA sub-tiles (decode) */
-#define MOE_I8_GEMM_TILE 2   /* LDS-staged tiles, 32x32x32 MFMA (prefill); geometry by rows per expert */
-#define MOE_I8_GEMM_NARROW 3 /* 64-row tiles, three LDS stages kept in flight (tens of rows per expert) */
+#define MOE_I8_GEMM_TILE 2   /* LDS-staged tiles of 128 or 256 rows; geometry by rows per expert */
+#define MOE_I8_GEMM_NARROW 3 /* 32- or 64-row tiles, a ring of seven or six LDS stages (tens of rows per expert) */
 #define MOE_I8_GEMM_TILE_WIDE 4 /* the LDS-tiled family with 256-row tiles and two stages (many rows per expert) */
 #define MOE_I8_GEMM_TILE_DEEP 5 /* the LDS-tiled family with 128-row tiles and three stages (around 100 rows per expert) */
 #define MOE_I8_GEMM_TILE_RING 6 /* 256-row tiles through a ring of four 32 KB stages: a measured alternative to _TILE_WIDE, \
-                                   same results, 7-10 % slower; MOE_I8_GEMM_AUTO never picks it */
+                                   same results, slower; MOE_I8_GEMM_AUTO never picks it */
 
 /* Router score functions (reference TokenChoiceTopKRouter.score_func). */
 #define MOE_I8_SCORE_SOFTMAX 0      /* softmax over all experts */

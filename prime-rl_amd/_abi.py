@@ -136,7 +136,7 @@ def _load_host():
 def host():
     """The native call path of the Python entry points (``csrc/host.cpp``), loaded on first use.  It is an
     extension of one torch build: where it is missing or does not fit, a warning says so and the calls take the Python
-    path to the same library, at 11 to 21 us more of host time each."""
+    path to the same library, at 10 to 25 us more of host time each."""
     global _host
     if _host is None:
         load()

@@ -681,7 +681,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
 // multiplies.  The matrix pipe therefore always has eight MFMAs with their operands in registers
 // on either side of the barrier.
 //
-// Measured against the two-stage pipeline on 65536 routed rows x 128 experts (gate_up 4096 x 2048,
+// Measured against the two-stage pipeline that the wide tiles had before gemm_wide.hip, on 65536 routed rows x 128 experts (gate_up 4096 x 2048,
 // down 2048 x 2048): same results bit for bit, 7-10 % slower.  A lane's 16-byte load takes a
 // quarter of a 64-byte row, so every 128-byte line is requested from L2 twice (the request count
 // per launch doubles, the bytes fetched from HBM stay), and the path from L2 into LDS, not the

@@ -88,9 +88,9 @@ def test_gated_mlp(pra, oracle, variant, M, H, I):
 @pytest.mark.parametrize("m", [1, 7, 16])
 @pytest.mark.parametrize("H,I", [(2048, 768), (256, 128), (4096, 1024)])
 def test_gated_mlp_of_a_few_rows_equals_the_rows_of_a_larger_call(pra, H, I, m):
-    """Up to 16 rows the MLP runs as three launches (the down GEMM quantises its own input, ties to
-    even); rows are independent, so the result must be, bit for bit, what the same rows give inside a
-    larger call that takes the five-launch path."""
+    """A few rows run as two launches that quantise their own input (ties to even), more of them with quantisation
+    launches in front of the GEMMs; rows are independent, so the result must be, bit for bit, what the same rows give
+    inside a larger call."""
     g = torch.Generator().manual_seed(m + I)
     x = torch.randn(96, H, generator=g).to(torch.bfloat16).to(DEV)
     w13, s13 = _weights(2 * I, H, g)

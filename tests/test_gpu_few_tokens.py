@@ -1,6 +1,6 @@
-"""GPU parity of the streaming family's split-reduction kernel (a handful of tokens): one block and many, row
-counts up to its limit, ragged channels and reductions, self-quantising or not, on both sides of the hand-over to
-the streaming kernel; and of the top-k combine at every k that has its own variant."""
+"""GPU parity of the kernels for a handful of tokens: the streaming family's split-reduction kernel (one block and many,
+row counts up to its limit, ragged channels and reductions, self-quantising or not, both sides of the hand-over to the
+streaming kernel), the two-launch layer, the narrow tiles and the top-k combine at every k that has its own variant."""
 
 import pytest
 import torch
