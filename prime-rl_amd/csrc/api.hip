@@ -3,10 +3,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
-#include <algorithm>
 #include <condition_variable>
 #include <mutex>
-#include <vector>
 
 #include "../../include/moe_i8.h"
 #include "common.hpp"
@@ -30,20 +28,22 @@ int check_launch(hipError_t err, const char* what) {
 
 // A call's turn on its workspace, while it issues its launches.  Calls of several threads on one stream may share a
 // workspace, since the stream runs them one after the other, but only if their launches do not interleave.  A thread
-// that waits here waits for calls on the same workspace and for nothing else.
+// that waits here waits for calls on the same workspace and for nothing else.  The turns taken are a list through the
+// calls' own stack frames: nothing is allocated, nothing throws.
 class WorkspaceTurn {
  public:
   explicit WorkspaceTurn(const void* workspace) : workspace_(workspace) {
     std::unique_lock<std::mutex> lock(state().mutex);
-    while (std::find(state().busy.begin(), state().busy.end(), workspace_) != state().busy.end()) state().ended.wait(lock);
-    state().busy.push_back(workspace_);
+    while (taken()) state().ended.wait(lock);
+    next_ = state().first;
+    state().first = this;
   }
   ~WorkspaceTurn() {
     {
       std::lock_guard<std::mutex> lock(state().mutex);
-      std::vector<const void*>& busy = state().busy;
-      *std::find(busy.begin(), busy.end(), workspace_) = busy.back();
-      busy.pop_back();
+      WorkspaceTurn** at = &state().first;
+      while (*at != this) at = &(*at)->next_;
+      *at = next_;
     }
     state().ended.notify_all();
   }
@@ -53,13 +53,19 @@ class WorkspaceTurn {
   struct State {
     std::mutex mutex;
     std::condition_variable ended;
-    std::vector<const void*> busy;  // one entry per thread inside a call
+    WorkspaceTurn* first = nullptr;
   };
   static State& state() {
     static State* s = new State;  // never destroyed: threads may outlive static objects
     return *s;
   }
+  bool taken() const {
+    for (const WorkspaceTurn* t = state().first; t; t = t->next_)
+      if (t->workspace_ == workspace_) return true;
+    return false;
+  }
   const void* workspace_;
+  WorkspaceTurn* next_;
 };
 
 bool valid_block_size(int b) { return b == 16 || b == 32 || b == 64 || b == 128; }
