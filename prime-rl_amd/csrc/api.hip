@@ -5,6 +5,7 @@
 
 #include <condition_variable>
 #include <mutex>
+#include <new>
 
 #include "../../include/moe_i8.h"
 #include "common.hpp"
@@ -56,7 +57,8 @@ class WorkspaceTurn {
     WorkspaceTurn* first = nullptr;
   };
   static State& state() {
-    static State* s = new State;  // never destroyed: threads may outlive static objects
+    alignas(State) static char memory[sizeof(State)];
+    static State* s = new (memory) State;  // never destroyed: threads may outlive static objects
     return *s;
   }
   bool taken() const {
