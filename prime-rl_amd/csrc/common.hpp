@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace moe_i8 {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -24,6 +26,24 @@ inline int device_cu_count() {
   }();
   return count;
 }
+
+// A kernel's limit of dynamic LDS, raised on each device the first time a launch goes there (one object per kernel).
+class DynamicLds {
+ public:
+  hipError_t allow(const void* kernel, int bytes) {
+    int dev = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return err;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (dev < 64 && (done_.load(std::memory_order_acquire) & bit)) return hipSuccess;
+    err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (err == hipSuccess) done_.fetch_or(bit, std::memory_order_release);
+    return err;
+  }
+
+ private:
+  std::atomic<uint64_t> done_{0};
+};
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
 

@@ -123,9 +123,9 @@ hipError_t launch_rows(const DenseFewArgs& a, hipStream_t stream) {
   const int width = MODE == kGateUpSilu ? a.n / 2 : a.n;
   const size_t lds = (size_t)a.m * C * 1024;
   const int groups = (width + kOut - 1) / kOut, most = device_cu_count();  // a workgroup per compute unit: one quantisation each
-  static const hipError_t attr =
-      hipFuncSetAttribute((const void*)dense_few_kernel<MODE, C, R>, hipFuncAttributeMaxDynamicSharedMemorySize, kDenseFewRows * C * 1024);
-  if (attr != hipSuccess) return attr;
+  static DynamicLds limit;
+  const hipError_t err = limit.allow((const void*)dense_few_kernel<MODE, C, R>, kDenseFewRows * C * 1024);
+  if (err != hipSuccess) return err;
   hipLaunchKernelGGL((dense_few_kernel<MODE, C, R>), dim3((unsigned)(groups < most ? groups : most)), dim3(64 * kWaves), lds, stream, a);
   return hipGetLastError();
 }

@@ -244,9 +244,9 @@ hipError_t launch_config(const SplitParams& p0, int64_t blocks, hipStream_t stre
   constexpr int kRing = ring_bytes(TN, KS, S);
   p.ntiles = ((MODE == kGateUpSilu ? p.N / 2 : p.N) + kOut - 1) / kOut;
   const size_t bytes = kRing + (size_t)p.rows * (p.K + kRowPad);
-  static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_split_kernel<MODE, kFused, TN, KS, S>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds - 1024);
-  if (attr != hipSuccess) return attr;
+  static DynamicLds limit;
+  const hipError_t err = limit.allow((const void*)gemm_split_kernel<MODE, kFused, TN, KS, S>, kMaxLds - 1024);
+  if (err != hipSuccess) return err;
   hipLaunchKernelGGL((gemm_split_kernel<MODE, kFused, TN, KS, S>), dim3((unsigned)p.ntiles, (unsigned)blocks), dim3(64 * KS), bytes,
                      stream, p);
   return hipGetLastError();
