@@ -286,7 +286,9 @@ const Config kConfigs[] = {
     MOE_I8_DENSE(128, 128, 1, 2, 4, 4, 2, 1, 1.75f, 3.18f, 3.49f, 1.59f),
     MOE_I8_DENSE(128, 128, 1, 2, 2, 2, 2, 2, 0.71f, 3.66f, 5.59f, 1.72f),
 };
-// The 256-row tiles of the grouped family (one persistent workgroup per compute unit).
+// The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Over 216 problems of 500..8192 rows
+// the choice takes on average 0.5 %, at most 27 % (4032 x 12736 x 896: 88.5 against 69.6 us), longer than the faster of
+// both; constants fitted to the present wide tiles alone chose worse (0.7-1.0 %).
 const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, nullptr, nullptr};
 
 float estimate(const Config& c, int64_t m, int64_t n, int64_t k) {
