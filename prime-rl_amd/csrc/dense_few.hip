@@ -35,7 +35,7 @@ __global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) 
 
   // the row first: its loads are waited for first
   uint4 v[2 * C];
-  auto fetch = [&](int row) {
+  auto fetch = [&](int row) __attribute__((always_inline)) {
     const uint4* x = reinterpret_cast<const uint4*>(p.x + (int64_t)row * K);
 #pragma unroll
     for (int i = 0; i < 2 * C; ++i) v[i] = row < p.m && i * kWave + lane < K / kQuantVec ? x[i * kWave + lane] : make_uint4(0u, 0u, 0u, 0u);
@@ -60,8 +60,7 @@ __global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) 
   const int stride = gridDim.x * kWaves * kOut;
   fetch_weights(ch0);
 
-  for (int row = wave; row < p.m; row += kWaves) {
-    if (row != wave) fetch(row);
+  auto quantise = [&](int row) __attribute__((always_inline)) {
     float m = 0.0f;
 #pragma unroll
     for (int i = 0; i < 2 * C; ++i) m = fmaxf(m, absmax8(v[i]));
@@ -71,6 +70,13 @@ __global__ __launch_bounds__(64 * kWaves) void dense_few_kernel(DenseFewArgs p) 
 #pragma unroll
     for (int i = 0; i < 2 * C; ++i)
       *reinterpret_cast<uint2*>(xq + row * (C * 1024) + (i * kWave + lane) * kQuantVec) = quant8<true>(v[i], inv);
+  };
+  // The first row apart from the loop, in front of whose loads it would wait for the weights as well: 4 rows of 8192 on
+  // 2048 channels 8.2 us in the loop, 7.4 apart, of 5120 on 4096 6.9 / 6.8.
+  if (wave < p.m) quantise(wave);
+  for (int row = wave + kWaves; row < p.m; row += kWaves) {
+    fetch(row);
+    quantise(row);
   }
   __syncthreads();
 

@@ -179,9 +179,9 @@ __global__ __launch_bounds__(64 * (kOne ? 16 : down_waves(C))) void down_few_ker
     const float ws = p.w2_scale[(int64_t)e * p.hidden + n0 + (lane & (R - 1))];
     while (true) {
       const int at = pair;
-      float m = 0.0f;
+      float m = 0.0f;  // (with absmax8 131 registers at C = 2, not 115: 4 tokens on 256 experts of 7168 x 2048 193.5 us, not 188)
 #pragma unroll
-      for (int c = 0; c < 2 * C; ++c) m = fmaxf(m, absmax8(v[c]));
+      for (int c = 0; c < 2 * C; ++c) m = fmaxf(m, absmax8_skip_nan(v[c]));
       const float absmax = fmaxf(wave_max(m), 1e-10f);
       const float inv = 127.0f / absmax, a_scale = absmax / 127.0f;
       v4i q[C];

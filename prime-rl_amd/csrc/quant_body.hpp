@@ -46,10 +46,13 @@ __device__ __forceinline__ uint2 quant8(const uint4& v, float inv) {
   return make_uint2(pack_low_bytes(y), pack_low_bytes(y + 4));
 }
 
-// The same for finite values only (weights): without the sign bit, bf16 patterns order like unsigned integers, so the
-// maximum is taken on packed 16-bit lanes (two elements per operation).  A NaN would be the largest of its 8 elements
-// and hide them from the float maximum of the row.
+// The same on packed 16-bit lanes, two elements per operation: without the sign bit, bf16 patterns order like integers.
+// absmax8_packed is for finite values only (weights): a NaN is the largest pattern and hides the other seven from the
+// row's float maximum.  absmax8_skip_nan adds 0x7f, which makes an infinity the largest signed number and every NaN a
+// negative one (no carry leaves a lane: 0x7fff + 0x7f < 2^16); for kernels whose registers would not hold the elements that
+// absmax8 unpacks and quant8 then finds unpacked.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef short i16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float absmax8_packed(const uint4& v) {
   const uint32_t w[4] = {v.x & 0x7fff7fffu, v.y & 0x7fff7fffu, v.z & 0x7fff7fffu, v.w & 0x7fff7fffu};
   u16x2 m = __builtin_elementwise_max(
@@ -57,6 +60,15 @@ __device__ __forceinline__ float absmax8_packed(const uint4& v) {
       __builtin_elementwise_max(__builtin_bit_cast(u16x2, w[2]), __builtin_bit_cast(u16x2, w[3])));
   const uint32_t top = m[0] > m[1] ? m[0] : m[1];
   return __uint_as_float(top << 16);
+}
+__device__ __forceinline__ float absmax8_skip_nan(const uint4& v) {
+  constexpr uint32_t kAbs = 0x7fff7fffu, kUp = 0x007f007fu;
+  const uint32_t w[4] = {(v.x & kAbs) + kUp, (v.y & kAbs) + kUp, (v.z & kAbs) + kUp, (v.w & kAbs) + kUp};
+  const i16x2 m = __builtin_elementwise_max(
+      __builtin_elementwise_max(__builtin_bit_cast(i16x2, w[0]), __builtin_bit_cast(i16x2, w[1])),
+      __builtin_elementwise_max(__builtin_bit_cast(i16x2, w[2]), __builtin_bit_cast(i16x2, w[3])));
+  const int top = m[0] > m[1] ? m[0] : m[1];
+  return __uint_as_float((uint32_t)(top > 0x7f ? top - 0x7f : 0) << 16);
 }
 
 // Weight flavour of quant8: q = rint(x / scale) (ties to even, the correctly rounded fp32 quotient),
