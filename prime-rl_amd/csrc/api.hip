@@ -945,6 +945,7 @@ moe_i8::GemmArgs dense_group(int mode, const DenseCarve& c, char* ws, const int8
                            ? gate_up_args(a_q, a_scale, w, w_scale, sorted, eids, npp, m, 1, 1, k, n / 2, kDenseBlock, c.cap, out)
                            : down_args(a_q, a_scale, w, w_scale, nullptr, sorted, eids, npp, m, 1, n, k, kDenseBlock, c.cap, out);
   g.expert_ids_ascend = true;  // one expert
+  g.identity = true;
   return g;
 }
 

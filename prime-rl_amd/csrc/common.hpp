@@ -300,6 +300,7 @@ struct GemmArgs {
   void* out;  // bf16 [P, I] | bf16 [P, H] | int32 [P, N]
   int64_t max_rows_per_expert = 0;  // upper bound if the caller knows one (the token count), else 0
   bool expert_ids_ascend = false;   // expert_ids is known to come from moe_align (non-decreasing over the used blocks)
+  bool identity = false;            // ... and one expert owns all of them, every block is used: a dense layer
   int tile_geometry = 0;            // LDS-tiled family: kTileAuto, kTileWide (256-row tiles), kTileDeep (128-row tiles) or kTileRing (256-row tiles, four-stage ring; on demand only)
 };
 constexpr int kTileAuto = 0, kTileWide = 1, kTileDeep = 2, kTileRing = 3;

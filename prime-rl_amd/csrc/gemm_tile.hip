@@ -20,19 +20,19 @@
 // chunk) spread over all banks; because a load fills LDS linearly the swizzle is applied to the
 // global source address of each lane.
 //
-// The tile list is derived inside the kernel from expert_ids (block -> expert, ascending): every
-// workgroup scans it once into LDS.  Tasks (tile, channel tile) are numbered channel tile fastest
-// and split into 8 contiguous ranges, one per XCD (workgroup id % 8), so that the workgroups
-// running on one XCD at a time share token rows and expert weights in that XCD's L2.  The first
-// loads of the next task are issued before the epilogue of the current one.
+// The tile list is derived inside the kernel from expert_ids (tile_list.hpp).  Tasks (tile, channel tile) are numbered
+// channel tile fastest and split into 8 contiguous ranges, one per XCD (workgroup id % 8), so that the workgroups running
+// on one XCD at a time share token rows and expert weights in that XCD's L2.  The first loads of the next task are issued
+// before the epilogue of the current one.  GEMMs of 64 experts of 4096 x 1408 with 64 rows each, with the starting steps of
+// rotation_mask: 150 -> 132 us (gate_up, K = 4096).
 #include <type_traits>
 
-#include "common.hpp"
+#include "tile_list.hpp"
 
 namespace moe_i8 {
 namespace {
 
-constexpr int kThreads = 512;
+constexpr int kThreads = kTileThreads;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kBN = 256;       // weight rows per tile
 constexpr int kBK = 128;       // reduction bytes per step
@@ -41,10 +41,8 @@ constexpr int kTokOffset = kBN * kBK;
 constexpr int kTileTok = 128;                          // token rows per tile
 constexpr int kSlots = 3;                              // LDS stages
 constexpr int kStageBytes = (kBN + kTileTok) * kBK;    // 48 KB
-constexpr int kMaxTiles = 2048;                        // capacity of the in-LDS tile list
+constexpr int kMaxTiles = 2048;                        // of a launch
 constexpr int kTokLoads = kTileTok / 64;               // wave-level loads of 8 token rows per wavefront and step
-constexpr int kXcds = 8;
-constexpr int kGroupTiles = 8;  // token tiles of one expert whose tasks are interleaved per channel tile
 
 struct TileParams {
   const int8_t* a_q;
@@ -53,15 +51,14 @@ struct TileParams {
   const float* w_scale;
   const float* row_weight;
   const int32_t* sorted_ids;
-  const int32_t* expert_ids;
   const int32_t* npp;
   int64_t P;
   int row_div;
-  int E;
   int N;
   int K;
   int B;
-  int ntiles;  // channel tiles
+  TileListArgs tiles;
+  int rotate;  // mask of the reduction step that a task starts at (rotation_mask)
   int ascend;  // expert_ids is known to ascend over the used blocks (it comes from moe_align)
   void* out;
 };
@@ -110,152 +107,9 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 
 __device__ __forceinline__ int swizzle_of_row(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-// ---- block-wide scans over kThreads threads (used once per workgroup, for the tile list) ----
-template <bool kMax>
-__device__ __forceinline__ int scan_op(int a, int b) {
-  return kMax ? (a > b ? a : b) : a + b;
-}
-
-template <bool kMax>
-__device__ __forceinline__ void block_scan(int v, int* wave_part, int& incl, int& excl) {
-  const int ident = kMax ? -1 : 0;
-  const int lane = lane_id();
-  const int wave = threadIdx.x / kWave;
-  int x = v;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int n = __shfl_up(x, d);
-    if (lane >= d) x = scan_op<kMax>(n, x);
-  }
-  int prev = __shfl_up(x, 1);
-  if (lane == 0) prev = ident;
-  if (lane == kWave - 1) wave_part[wave] = x;
-  __syncthreads();
-  int carry = ident;
-  for (int i = 0; i < wave; ++i) carry = scan_op<kMax>(carry, wave_part[i]);
-  __syncthreads();
-  incl = scan_op<kMax>(carry, x);
-  excl = scan_op<kMax>(carry, prev);
-}
-
-// tile_desc[t] = first block | number of blocks << 16 | rank in group << 20 | group size << 24.
-// Tiles start at multiples of `per_tile` blocks inside each run of equal expert ids and never cross
-// a run; up to kGroupTiles consecutive tiles of a run form a group.  scratch holds nblocks ints.
-__device__ int build_tile_list(const int32_t* __restrict__ expert_ids, int nblocks, int per_tile, int* scratch,
-                               int* wave_part, uint32_t* tile_desc, int* total_out, int max_tiles) {
-  const int tid = threadIdx.x;
-  for (int j = tid; j < nblocks; j += kThreads) scratch[j] = expert_ids[j];
-  __syncthreads();
-  const int chunk = (nblocks + kThreads - 1) / kThreads;
-  const int j0 = tid * chunk < nblocks ? tid * chunk : nblocks;
-  const int j1 = j0 + chunk < nblocks ? j0 + chunk : nblocks;
-  // start of the run that contains block j = prefix max of (j if a run starts at j else -1)
-  int local_start = -1;
-  for (int j = j0; j < j1; ++j)
-    if (j == 0 || scratch[j] != scratch[j - 1]) local_start = j;
-  int incl, carry_start;
-  block_scan<true>(local_start, wave_part, incl, carry_start);
-  int leaders = 0;
-  int cur = carry_start;
-  for (int j = j0; j < j1; ++j) {
-    if (j == 0 || scratch[j] != scratch[j - 1]) cur = j;
-    if ((j - cur) % per_tile == 0) ++leaders;
-  }
-  int incl_leaders, t;
-  block_scan<false>(leaders, wave_part, incl_leaders, t);
-  cur = carry_start;
-  for (int j = j0; j < j1; ++j) {
-    if (j == 0 || scratch[j] != scratch[j - 1]) cur = j;
-    if ((j - cur) % per_tile == 0) {
-      int nb = 1;
-      while (nb < per_tile && j + nb < nblocks && scratch[j + nb] == scratch[j]) ++nb;
-      // bits 0-15 first block, 16-19 blocks, 20-22 rank of the tile inside its group, 24-27 group size
-      if (t < max_tiles)
-        tile_desc[t] = (uint32_t)j | ((uint32_t)nb << 16) | ((uint32_t)(((j - cur) / per_tile) % kGroupTiles) << 20);
-      ++t;
-    }
-  }
-  if (tid == kThreads - 1) *total_out = incl_leaders < max_tiles ? incl_leaders : max_tiles;
-  __syncthreads();
-  // Groups: up to kGroupTiles consecutive tiles of one expert.  The leader of a group counts its
-  // members and writes the size into all of them.
-  const int total = *total_out;
-  for (int g = tid; g < total; g += kThreads) {
-    if (((tile_desc[g] >> 20) & 7u) != 0) continue;
-    int count = 1;
-    while (count < kGroupTiles && g + count < total && ((tile_desc[g + count] >> 20) & 7u) == (uint32_t)count) ++count;
-    for (int i = 0; i < count; ++i) tile_desc[g + i] |= (uint32_t)count << 24;
-  }
-  __syncthreads();
-  return total;
-}
-
-// The same list when the expert ids are known to ascend over the used blocks (what moe_align writes):
-// every expert then owns at most one run of blocks, found by comparing a block with its neighbours, and
-// the number of tiles in front of an expert is one scan over the experts instead of two over the blocks
-// (a third of the time on a long list).  Runs of ids outside [0, E) get no tiles.  scratch holds
-// 2 * num_experts ints; per_tile is 1 << per_tile_log2.
-__device__ int build_tile_list_ascending(const int32_t* __restrict__ expert_ids, int nblocks, int num_experts,
-                                         int per_tile_log2, int* scratch, int* wave_part, uint32_t* tile_desc,
-                                         int* total_out, int max_tiles) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  int* first = scratch;               // first block of the expert's run
-  int* end = scratch + num_experts;   // one past its last block
-  for (int e = tid; e < 2 * num_experts; e += kThreads) scratch[e] = 0;
-  __syncthreads();
-  for (int j = tid; j < nblocks; j += kThreads) {
-    const int e = expert_ids[j];
-    const int prev = j > 0 ? expert_ids[j - 1] : -1;
-    const int next = j + 1 < nblocks ? expert_ids[j + 1] : -1;
-    if (e >= 0 && e < num_experts) {
-      if (j == 0 || e != prev) first[e] = j;
-      if (j + 1 == nblocks || e != next) end[e] = j + 1;
-    }
-  }
-  __syncthreads();
-  // thread t owns experts 2t and 2t + 1 (num_experts <= 2 * kThreads)
-  const int per_tile = 1 << per_tile_log2;
-  int f[2], nb[2], tiles[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int e = 2 * tid + i;
-    f[i] = e < num_experts ? first[e] : 0;
-    nb[i] = e < num_experts ? end[e] - f[i] : 0;
-    tiles[i] = (nb[i] + per_tile - 1) >> per_tile_log2;
-  }
-  const int mine = tiles[0] + tiles[1];
-  const int incl = wave_inclusive_scan_add(mine);
-  if (lane == kWave - 1) wave_part[wave] = incl;
-  __syncthreads();
-  int carry = 0, total = 0;
-#pragma unroll
-  for (int i = 0; i < kWaves; ++i) {
-    const int w = wave_part[i];
-    if (i < wave) carry += w;
-    total += w;
-  }
-  int t = carry + incl - mine;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    for (int r = 0; r < tiles[i]; ++r, ++t) {
-      if (t >= max_tiles) break;
-      const int left = nb[i] - (r << per_tile_log2);
-      const int in_group = tiles[i] - (r & ~(kGroupTiles - 1));
-      tile_desc[t] = (uint32_t)(f[i] + (r << per_tile_log2)) | ((uint32_t)(left < per_tile ? left : per_tile) << 16) |
-                     ((uint32_t)(r & (kGroupTiles - 1)) << 20) |
-                     ((uint32_t)(in_group < kGroupTiles ? in_group : kGroupTiles) << 24);
-    }
-  }
-  if (tid == 0) *total_out = total < max_tiles ? total : max_tiles;
-  __syncthreads();
-  return total < max_tiles ? total : max_tiles;
-}
-
 struct Task {
   int e;          // expert; -1 = no more work, -2 = tile of ignored expert ids
-  int nt;         // channel tile
+  int n0, n1;     // its channels (gate_up: gate channels)
   int64_t slot0;  // first slot of the tile in sorted_ids
   int nsub;       // active 64-row sub-blocks (1..4)
 };
@@ -264,7 +118,19 @@ struct TaskLoads {
   const int8_t* wbase;  // weights of the task's expert (wave-uniform)
   uint32_t woff[4];     // per lane: byte offset of its chunk of weight row i from wbase
   uint32_t xoff[4];     // per lane: byte offset of its chunk of token row i from a_q
+  int first;            // byte offset of the first reduction step
 };
+
+// The n-th weight row of a tile's 256; the last channel again behind the end of the task.
+template <int MODE>
+__device__ __forceinline__ int weight_row(const Task& tk, int N, int row) {
+  if constexpr (MODE == kGateUpSilu) {
+    const int inter = N / 2;
+    return min(tk.n0 + (row & 127), min(tk.n1, inter) - 1) + (row >= 128 ? inter : 0);
+  } else {
+    return min(tk.n0 + row, min(tk.n1, N) - 1);
+  }
+}
 
 // Weights: lane fills LDS slot (lane & 7) of row 32 * wave + 8 * i + (lane >> 3): it fetches the logical
 // chunk (lane & 7) ^ swizzle(row) of that row, and swizzle(row) = (lane >> 3) ^ (i & 1).  Token rows
@@ -272,19 +138,12 @@ struct TaskLoads {
 template <int MODE>
 __device__ __forceinline__ void setup_loads(const TileParams& p, const Task& tk, int wave, int lane, TaskLoads& ld) {
   const int K = p.K;
-  const int inter = p.N / 2;
+  ld.first = (tk.e & p.rotate) * kBK;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = 32 * wave + 8 * i + (lane >> 3);
     const int chunk = ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;
-    int n;
-    if constexpr (MODE == kGateUpSilu) {
-      const int ch = tk.nt * 128 + (row & 127);
-      n = (ch < inter ? ch : inter - 1) + (row >= 128 ? inter : 0);
-    } else {
-      const int ch = tk.nt * kBN + row;
-      n = ch < p.N ? ch : p.N - 1;
-    }
+    const int n = weight_row<MODE>(tk, p.N, row);
     ld.woff[i] = (uint32_t)n * (uint32_t)K + chunk;
     if (i < kTokLoads) {
       const int trow = 8 * kTokLoads * wave + 8 * i + (lane >> 3);
@@ -396,6 +255,7 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
   const int lrow = lane & 31;
   const int lhalf = lane >> 5;
   const int inter = p.N / 2;
+  const int limit = min(tk.n1, MODE == kGateUpSilu ? inter : p.N);  // behind the task's channels
   int32_t tok[2];
 #pragma unroll
   for (int tj = 0; tj < 2; ++tj) {
@@ -411,8 +271,8 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
       for (int ci = 0; ci < NCI; ++ci)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int n = tk.nt * kBN + cpart * (NCI * 32) + ci * 32 + 8 * q + 4 * lhalf;
-          if (n < p.N)
+          const int n = tk.n0 + cpart * (NCI * 32) + ci * 32 + 8 * q + 4 * lhalf;
+          if (n < limit)
             *reinterpret_cast<v4i*>(out + n) =
                 v4i{acc[ci][tj][4 * q], acc[ci][tj][4 * q + 1], acc[ci][tj][4 * q + 2], acc[ci][tj][4 * q + 3]};
         }
@@ -422,14 +282,14 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
     constexpr int CPR = NCI * 4;         // 16-byte chunks per staged row
     constexpr int kRowBytes = CPR * 16;
     const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
-    const int n0 = tk.nt * kBN + cpart * kChannels;  // first channel of this wavefront
+    const int n0 = tk.n0 + cpart * kChannels;  // first channel of this wavefront
     // The channel scales of this wavefront go through LDS: read from there they do not count
     // as vector-memory loads, so the second half's arithmetic does not have to wait for the first
     // half's stores (the vector-memory counter retires in order).
     if (2 * lane < kChannels) {
       const int n = n0 + 2 * lane;
       *reinterpret_cast<float2*>(wave_scales + 2 * lane) =
-          n < p.N ? *reinterpret_cast<const float2*>(wsc + n) : make_float2(0.0f, 0.0f);
+          n < limit ? *reinterpret_cast<const float2*>(wsc + n) : make_float2(0.0f, 0.0f);
     }
     float as[2], rw[2];
 #pragma unroll
@@ -462,7 +322,7 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
             *reinterpret_cast<const uint4*>(wave_lds + row * kRowBytes + ((chunk ^ staging_swizzle<CPR>(row)) * 16));
         const int32_t t = __shfl(tok[tj], row);
         const int n = n0 + chunk * 8;
-        if (t >= 0 && n < p.N)
+        if (t >= 0 && n < limit)
           __builtin_nontemporal_store(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}, reinterpret_cast<v4i*>(static_cast<uint16_t*>(p.out) + (int64_t)t * p.N + n));
       }
     }
@@ -471,7 +331,7 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
     constexpr int CPR = NCI * 2;
     constexpr int kRowBytes = CPR * 16;
     const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
-    const int n0 = tk.nt * 128 + cpart * kChannels;  // first gate channel of this wavefront
+    const int n0 = tk.n0 + cpart * kChannels;  // first gate channel of this wavefront
     // 64 token rows x kChannels channels
 #pragma unroll
     for (int tj = 0; tj < 2; ++tj) {
@@ -504,7 +364,7 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
           *reinterpret_cast<const uint4*>(wave_lds + row * kRowBytes + ((chunk ^ staging_swizzle<CPR>(row)) * 16));
       const int32_t t = __shfl(tok[(r * (64 / CPR)) >> 5], row & 31);
       const int n = n0 + chunk * 8;
-      if (t >= 0 && n < inter)
+      if (t >= 0 && n < limit)
         __builtin_nontemporal_store(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}, reinterpret_cast<v4i*>(static_cast<uint16_t*>(p.out) + (int64_t)t * inter + n));
     }
   }
@@ -513,29 +373,21 @@ __device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, in
 template <int MODE>
 __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
   __shared__ __align__(16) char stages[kSlots * kStageBytes];
-  __shared__ uint32_t tile_desc[kMaxTiles];
-  __shared__ int wave_part[kWaves];
+  __shared__ TileList<kMaxTiles> list;
   __shared__ __align__(16) float channel_scales[kWaves * 128];
-  __shared__ int total_tiles;
 
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int nk = p.K / kBK;
 
-  const int npp = *p.npp;
-  const int nblocks = npp / p.B;
-  const int sub_per_block = p.B / 64;
-  const int per_tile = kTileTok / p.B;  // 1 or 2 blocks
-  const int ntile =
-      p.ascend ? build_tile_list_ascending(p.expert_ids, nblocks, p.E, per_tile == 2 ? 1 : 0,
-                                           reinterpret_cast<int*>(stages), wave_part, tile_desc, &total_tiles,
-                                           kMaxTiles)
-               : build_tile_list(p.expert_ids, nblocks, per_tile, reinterpret_cast<int*>(stages), wave_part, tile_desc,
-                                 &total_tiles, kMaxTiles);
-  const int total = ntile * p.ntiles;
-  const int per_xcd = (total + kXcds - 1) / kXcds;
   const int xcd = blockIdx.x % kXcds;
+  const TileRange range = p.ascend ? build_ascending(p.tiles, xcd, reinterpret_cast<int*>(stages), list)
+                                   : build_any_order(p.tiles, *p.npp / p.B, xcd, reinterpret_cast<int*>(stages), list);
+  const int sub_per_block = p.B / 64;
+  const int total = range.tiles * p.tiles.ntiles;
+  const int per_xcd = (total + kXcds - 1) / kXcds;
+  const int my_tasks = min(per_xcd, max(total - xcd * per_xcd, 0));
   const int stride = gridDim.x / kXcds;
 
   // ---- MFMA operand reads: lane feeds row (lane & 31), 16-byte chunk 2 * kk + (lane >> 5) ----
@@ -550,35 +402,30 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
   auto decode = [&](int it) {
     Task tk;
     tk.e = -1;
-    tk.nt = 0;
+    tk.n0 = tk.n1 = 0;
     tk.slot0 = 0;
     tk.nsub = 0;
-    if (it < per_xcd && xcd * per_xcd + it < total) {
-      const int task = xcd * per_xcd + it;
-      // The tasks of a group of T token tiles of one expert run channel tile by channel tile: T
-      // consecutive tasks (on neighbouring compute units) stream the same weight tile.
-      const int tile0 = task / p.ntiles;
-      const uint32_t d0 = tile_desc[tile0];
-      const int first = tile0 - (int)((d0 >> 20) & 7u);
-      const int T = (int)((d0 >> 24) & 15u);
-      const int pos = task - first * p.ntiles;
-      const uint32_t d = tile_desc[first + pos % T];
-      tk.nt = pos / T;
-      const int blk = (int)(d & 0xffffu);
-      const int e = p.expert_ids[blk];
-      tk.slot0 = (int64_t)blk * p.B;
-      tk.nsub = (int)((d >> 16) & 15u) * sub_per_block;
-      tk.e = (e >= 0 && e < p.E) ? e : -2;
+    // a piece is a part of the tile's channels
+    const TaskPiece tp = piece_at(it, my_tasks, stride);
+    if (tp.task >= 0) {
+      constexpr int kOut = MODE == kGateUpSilu ? kBN / 2 : kBN;
+      const uint2 d = look_up_task(p.tiles, list, range, xcd * per_xcd + tp.task);
+      const int width = kOut / tp.pieces;
+      tk.n0 = (int)(d.y >> 16) * kOut + tp.piece * width;
+      tk.n1 = tk.n0 + width;
+      tk.slot0 = (int64_t)(d.x & 0xffffu) * p.B;
+      tk.nsub = (int)((d.x >> 16) & 15u) * sub_per_block;
+      tk.e = tk.nsub > 0 ? (int)(d.y & 0xffffu) : -2;
     }
     return tk;
   };
 
   // Does any run of blocks make more than one tile?  (A tile that is not the first of its group, or a
-  // group of more than one.)  If none does, every weight row is read by one workgroup only and is
-  // fetched with the non-temporal hint; the choice is made once per launch so that the step loop
+  // group of more than one.)  If none in this XCD's part does, every weight row is read by one workgroup only and is
+  // fetched with the non-temporal hint; the choice is made once per workgroup so that the step loop
   // carries no test.
   bool shared_local = false;
-  for (int g = t; g < ntile; g += kThreads) shared_local |= (tile_desc[g] >> 20) != (1u << 4);  // rank 0, group size 1
+  for (int g = t; g < range.hi - range.lo; g += kThreads) shared_local |= (list.desc[g] >> 20) != (1u << 4);  // rank 0, group size 1
   const bool weights_shared = __syncthreads_or(shared_local ? 1 : 0) != 0;
 
   auto run = [&](auto nt_tag) {
@@ -592,8 +439,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
   int slot = 0;  // stage of the step being multiplied
   // The scratch of the tile list lived in the stage memory; everybody is past it (the builder ends
   // with a barrier), so the first stages can be filled now.
-  issue_stage_loads<NT>(ld, p.a_q, stage0, wave, 0);
-  issue_stage_loads<NT>(ld, p.a_q, stage0 + kStageBytes, wave, kBK);
+  auto at = [&](const TaskLoads& ld, int s) {  // byte offset of step s
+    const int k = ld.first + s * kBK;
+    return k < p.K ? k : k - p.K;
+  };
+  issue_stage_loads<NT>(ld, p.a_q, stage0, wave, at(ld, 0));
+  issue_stage_loads<NT>(ld, p.a_q, stage0 + kStageBytes, wave, at(ld, 1));
   constexpr int kLoadsPerStep = 4 + kTokLoads;  // per wavefront
 
   bool stores_pending = false;
@@ -635,9 +486,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
         if (fill >= kSlots) fill -= kSlots;
         const uint32_t fill_addr = stage0 + fill * kStageBytes;
         if (s + kAhead < nk)
-          issue_stage_loads<NT>(ld, p.a_q, fill_addr, wave, (s + kAhead) * kBK);
+          issue_stage_loads<NT>(ld, p.a_q, fill_addr, wave, at(ld, s + kAhead));
         else if (nx.e >= 0)
-          issue_stage_loads<NT>(nld, p.a_q, fill_addr, wave, (s + kAhead - nk) * kBK);
+          issue_stage_loads<NT>(nld, p.a_q, fill_addr, wave, at(nld, s + kAhead - nk));
         multiply_stage<NCI>(rd, stages + slot * kStageBytes, acc);
         slot = slot + 1 == kSlots ? 0 : slot + 1;
       }
@@ -690,6 +541,7 @@ constexpr int kRingBK = 64;
 constexpr int kRingSlots = 4;
 constexpr int kRingHalf = kBN * kRingBK;    // 16 KB
 constexpr int kRingStage = 2 * kRingHalf;   // 32 KB
+constexpr int kRingMaxTiles = 6144;         // of a launch
 constexpr int kRingLoads = 4;               // wave-level loads per wavefront and step
 
 // chunk swizzle of a 64-byte LDS row: 16 consecutive rows reading one logical chunk, and 8 rows
@@ -706,19 +558,11 @@ struct RingLoads {
 template <int MODE>
 __device__ __forceinline__ void ring_setup_loads(const TileParams& p, const Task& tk, int wave, int lane, RingLoads& ld) {
   const int K = p.K;
-  const int inter = p.N / 2;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = 32 * wave + 16 * i + (lane >> 2);
     const int chunk = ((lane & 3) ^ swizzle_of_row64(row)) * 16;
-    int n;
-    if constexpr (MODE == kGateUpSilu) {
-      const int ch = tk.nt * 128 + (row & 127);
-      n = (ch < inter ? ch : inter - 1) + (row >= 128 ? inter : 0);
-    } else {
-      const int ch = tk.nt * kBN + row;
-      n = ch < p.N ? ch : p.N - 1;
-    }
+    const int n = weight_row<MODE>(tk, p.N, row);
     ld.woff[i] = (uint32_t)n * (uint32_t)K + chunk;
     uint32_t arow = 0;
     if ((row >> 6) < tk.nsub) {
@@ -790,7 +634,7 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
       for (int ci = 0; ci < 4; ++ci)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int n = tk.nt * kBN + cpart * 128 + ci * 32 + 8 * q + 4 * lhalf;
+          const int n = tk.n0 + cpart * 128 + ci * 32 + 8 * q + 4 * lhalf;
           if (n < p.N)
             *reinterpret_cast<v4i*>(out + n) =
                 v4i{acc[ci][tj][4 * q], acc[ci][tj][4 * q + 1], acc[ci][tj][4 * q + 2], acc[ci][tj][4 * q + 3]};
@@ -798,7 +642,7 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
     }
   } else if constexpr (MODE == kDown) {
     const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
-    const int n0 = tk.nt * kBN + cpart * 128;  // first channel of this wavefront
+    const int n0 = tk.n0 + cpart * 128;  // first channel of this wavefront
     // channel scales through LDS (see `epilogue`)
     {
       const int n = n0 + 2 * lane;
@@ -843,7 +687,7 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
     }
   } else {
     const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
-    const int n0 = tk.nt * 128 + cpart * 64;  // first gate channel of this wavefront
+    const int n0 = tk.n0 + cpart * 64;  // first gate channel of this wavefront
     float as[2];
 #pragma unroll
     for (int tj = 0; tj < 2; ++tj) as[tj] = tok[tj] >= 0 ? p.a_scale[tok[tj] / p.row_div] : 0.0f;
@@ -883,12 +727,9 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
 
 template <int MODE>
 __global__ __launch_bounds__(kThreads, 1) void gemm_ring_kernel(TileParams p) {
-  constexpr int kMaxTiles = 6144;
   __shared__ __align__(16) char stages[kRingSlots * kRingStage];
-  __shared__ uint32_t tile_desc[kMaxTiles];
-  __shared__ int wave_part[kWaves];
+  __shared__ TileList<kRingMaxTiles> list;
   __shared__ __align__(16) float channel_scales[kWaves * 128];
-  __shared__ int total_tiles;
 
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -896,18 +737,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_ring_kernel(TileParams p) {
   const int my_sub = wave / 2;  // token sub-block this wavefront multiplies
   const int nk = p.K / kRingBK;
 
-  const int npp = *p.npp;
-  const int nblocks = npp / p.B;
-  const int sub_per_block = p.B / 64;
-  const int per_tile = 256 / p.B;  // 2 or 4 blocks
-  const int ntile =
-      p.ascend ? build_tile_list_ascending(p.expert_ids, nblocks, p.E, per_tile == 4 ? 2 : 1, reinterpret_cast<int*>(stages),
-                                           wave_part, tile_desc, &total_tiles, kMaxTiles)
-               : build_tile_list(p.expert_ids, nblocks, per_tile, reinterpret_cast<int*>(stages), wave_part, tile_desc,
-                                 &total_tiles, kMaxTiles);
-  const int total = ntile * p.ntiles;
-  const int per_xcd = (total + kXcds - 1) / kXcds;
   const int xcd = blockIdx.x % kXcds;
+  const TileRange range = p.ascend ? build_ascending(p.tiles, xcd, reinterpret_cast<int*>(stages), list)
+                                   : build_any_order(p.tiles, *p.npp / p.B, xcd, reinterpret_cast<int*>(stages), list);
+  const int sub_per_block = p.B / 64;
+  const int total = range.tiles * p.tiles.ntiles;
+  const int per_xcd = (total + kXcds - 1) / kXcds;
   const int stride = gridDim.x / kXcds;
 
   const int lrow = lane & 31;
@@ -934,23 +769,17 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_ring_kernel(TileParams p) {
   auto decode = [&](int it) {
     Task tk;
     tk.e = -1;
-    tk.nt = 0;
+    tk.n0 = tk.n1 = 0;
     tk.slot0 = 0;
     tk.nsub = 0;
     if (it < per_xcd && xcd * per_xcd + it < total) {
-      const int task = xcd * per_xcd + it;
-      const int tile0 = task / p.ntiles;
-      const uint32_t d0 = tile_desc[tile0];
-      const int first = tile0 - (int)((d0 >> 20) & 7u);
-      const int T = (int)((d0 >> 24) & 15u);
-      const int pos = task - first * p.ntiles;
-      const uint32_t d = tile_desc[first + pos % T];
-      tk.nt = pos / T;
-      const int blk = (int)(d & 0xffffu);
-      const int e = p.expert_ids[blk];
-      tk.slot0 = (int64_t)blk * p.B;
-      tk.nsub = (int)((d >> 16) & 15u) * sub_per_block;
-      tk.e = (e >= 0 && e < p.E) ? e : -2;
+      constexpr int kOut = MODE == kGateUpSilu ? kBN / 2 : kBN;
+      const uint2 d = look_up_task(p.tiles, list, range, xcd * per_xcd + it);
+      tk.n0 = (int)(d.y >> 16) * kOut;
+      tk.n1 = tk.n0 + kOut;
+      tk.slot0 = (int64_t)(d.x & 0xffffu) * p.B;
+      tk.nsub = (int)((d.x >> 16) & 15u) * sub_per_block;
+      tk.e = tk.nsub > 0 ? (int)(d.y & 0xffffu) : -2;
     }
     return tk;
   };
@@ -1053,7 +882,7 @@ bool ring_supports(const GemmArgs& a) {
   const int64_t blocks = (a.sorted_cap + a.block_size - 1) / a.block_size;
   const int per_tile = 256 / a.block_size;
   const int64_t tiles = a.expert_ids_ascend ? (blocks + per_tile - 1) / per_tile + a.num_experts : blocks;
-  return tiles <= 6144 && blocks <= (int64_t)(kRingSlots * kRingStage / sizeof(int)) && blocks <= 65535;
+  return tiles <= kRingMaxTiles && blocks <= (int64_t)(kRingSlots * kRingStage / sizeof(int)) && blocks <= 65535;
 }
 
 template <int MODE, bool RING>
@@ -1065,15 +894,22 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.w_scale = a.w_scale;
   p.row_weight = a.row_weight;
   p.sorted_ids = a.sorted_token_ids;
-  p.expert_ids = a.expert_ids;
   p.npp = a.num_tokens_post_padded;
   p.P = a.num_pairs;
   p.row_div = a.row_div;
-  p.E = a.num_experts;
   p.N = a.n;
   p.K = a.k;
   p.B = a.block_size;
-  p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kBN - 1) / kBN;
+  p.tiles.expert_ids = a.expert_ids;
+  p.tiles.E = a.num_experts;
+  p.tiles.per_tile = (RING ? 256 : kTileTok) / a.block_size;
+  p.tiles.even = 0;
+  p.tiles.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kBN - 1) / kBN;
+  p.tiles.by_ntiles = divider(p.tiles.ntiles);
+  p.tiles.by_per_tile = divider(p.tiles.per_tile);
+  p.tiles.blocks = (int)(a.sorted_cap / a.block_size);
+  p.tiles.identity = a.identity ? 1 : 0;
+  p.rotate = RING ? 0 : rotation_mask(a.k);
   p.ascend = a.expert_ids_ascend && a.num_experts <= 2 * kThreads ? 1 : 0;
   p.out = a.out;
   const int grid = device_cu_count() / kXcds * kXcds;

@@ -28,18 +28,16 @@
 #include <type_traits>
 
 #include "lds_loads.hpp"
+#include "tile_list.hpp"
 
 namespace moe_i8 {
 namespace {
 
-constexpr int kThreads = 512;
+constexpr int kThreads = kTileThreads;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kTok = 256;   // token rows per tile
 constexpr int kCh = 256;    // weight rows per tile
-constexpr int kXcds = 8;
-constexpr int kGroupTiles = 8;   // token tiles of one expert whose tasks are interleaved per channel tile
 constexpr int kMaxTiles = 6144;  // of a launch
-constexpr int kMaxLocal = kMaxTiles / kXcds + 2 + 2 * kGroupTiles;  // ... that one XCD's workgroups look at
 constexpr int kX0 = kCh * kStepBytes;              // token rows 0..127 of a stage, behind the weight rows
 constexpr int kX1 = kX0 + kTok / 2 * kStepBytes;   // token rows 128..255
 constexpr int kStage = kX1 + kTok / 2 * kStepBytes;
@@ -53,180 +51,16 @@ struct WideParams {
   const float* w_scale;
   const float* row_weight;  // null = 1
   const int32_t* sorted_ids;
-  const int32_t* expert_ids;
   const int32_t* npp;
   int P;
-  int row_div;
-  uint32_t div_magic;  // id / row_div = (id * div_magic) >> (32 + div_shift) for row_div > 1
-  int div_shift;
-  int E;
+  Divider row_of;
   int N;
   int K;
   int B;
-  int per_tile;  // most blocks of a tile
-  int even;      // an expert's blocks are dealt evenly to its tiles, instead of full tiles and a rest
-  int ntiles;    // channel tiles
+  TileListArgs tiles;
   int ascend;  // expert_ids is known to ascend over the used blocks (it comes from moe_align)
   void* out;
 };
-
-struct TileList {
-  uint32_t desc[kMaxLocal];    // first block | blocks << 16 | rank in group << 20 | group size << 24
-  uint16_t expert[kMaxLocal];  // 0xffff: ids outside [0, E)
-  int wave_part[kWaves];
-  int total;
-};
-
-__device__ __forceinline__ int wave_scan_max(int v) {
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int n = __shfl_up(v, d);
-    if (lane_id() >= d) v = n > v ? n : v;
-  }
-  return v;
-}
-
-struct TileRange {
-  int lo, hi;  // tiles [lo, hi) of the launch are in the list, tile t at t - lo
-  int tiles;   // of the launch
-};
-
-// The tiles that the workgroups of one XCD look at: those of its range of tasks, and the rest of their groups.
-__device__ __forceinline__ TileRange range_of(int tiles, int ntiles, int xcd) {
-  const int total = tiles * ntiles;
-  const int per_xcd = (total + kXcds - 1) / kXcds;
-  const int first = xcd * per_xcd / ntiles, last = ((xcd + 1) * per_xcd - 1) / ntiles;
-  TileRange r;
-  r.lo = first - (kGroupTiles - 1) > 0 ? first - (kGroupTiles - 1) : 0;
-  r.hi = last + kGroupTiles < tiles ? last + kGroupTiles : tiles;
-  if (r.hi > r.lo + kMaxLocal) r.hi = r.lo + kMaxLocal;
-  r.tiles = tiles;
-  return r;
-}
-
-// Tiles start at multiples of `per_tile` blocks inside each run of equal expert ids and never cross a run; up
-// to kGroupTiles consecutive tiles of a run form a group.  scratch holds nblocks ints.
-__device__ TileRange build_any_order(const WideParams& p, int nblocks, int per_tile, int xcd, int* scratch, TileList& list) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  for (int j = tid; j < nblocks; j += kThreads) scratch[j] = p.expert_ids[j];
-  __syncthreads();
-  const int chunk = (nblocks + kThreads - 1) / kThreads;
-  const int j0 = tid * chunk < nblocks ? tid * chunk : nblocks;
-  const int j1 = j0 + chunk < nblocks ? j0 + chunk : nblocks;
-  // start of the run that contains block j = prefix max of (j if a run starts at j else -1)
-  int start = -1;
-  for (int j = j0; j < j1; ++j)
-    if (j == 0 || scratch[j] != scratch[j - 1]) start = j;
-  const int scan = wave_scan_max(start);
-  int before = __shfl_up(scan, 1);
-  if (lane == 0) before = -1;
-  if (lane == kWave - 1) list.wave_part[wave] = scan;
-  __syncthreads();
-  for (int i = 0; i < wave; ++i) before = list.wave_part[i] > before ? list.wave_part[i] : before;
-  __syncthreads();
-  int leaders = 0;
-  int cur = before;
-  for (int j = j0; j < j1; ++j) {
-    if (j == 0 || scratch[j] != scratch[j - 1]) cur = j;
-    if ((j - cur) % per_tile == 0) ++leaders;
-  }
-  const int incl = wave_inclusive_scan_add(leaders);
-  if (lane == kWave - 1) list.wave_part[wave] = incl;
-  __syncthreads();
-  int t = incl - leaders, tiles = 0;
-  for (int i = 0; i < kWaves; ++i) {
-    if (i < wave) t += list.wave_part[i];
-    tiles += list.wave_part[i];
-  }
-  const TileRange r = range_of(tiles < kMaxTiles ? tiles : kMaxTiles, p.ntiles, xcd);
-  cur = before;
-  for (int j = j0; j < j1; ++j) {
-    if (j == 0 || scratch[j] != scratch[j - 1]) cur = j;
-    if ((j - cur) % per_tile != 0) continue;
-    if (t >= r.lo && t < r.hi) {
-      int nb = 1;
-      while (nb < per_tile && j + nb < nblocks && scratch[j + nb] == scratch[j]) ++nb;
-      const int e = scratch[j];
-      list.desc[t - r.lo] = (uint32_t)j | ((uint32_t)nb << 16) | ((uint32_t)(((j - cur) / per_tile) % kGroupTiles) << 20);
-      list.expert[t - r.lo] = e >= 0 && e < p.E ? (uint16_t)e : (uint16_t)0xffff;
-    }
-    ++t;
-  }
-  __syncthreads();
-  // the leader of a group counts its members and writes the size into all of them
-  const int count = r.hi - r.lo;
-  for (int g = tid; g < count; g += kThreads) {
-    if (((list.desc[g] >> 20) & 7u) != 0) continue;
-    int size = 1;
-    while (size < kGroupTiles && g + size < count && ((list.desc[g + size] >> 20) & 7u) == (uint32_t)size) ++size;
-    for (int i = 0; i < size; ++i) list.desc[g + i] |= (uint32_t)size << 24;
-  }
-  __syncthreads();
-  return r;
-}
-
-// The same list when the expert ids are known to ascend over the used blocks (what moe_align writes): every
-// expert then owns at most one run of blocks, found by comparing a block with its neighbours, and the number of
-// tiles in front of an expert is one scan over the experts instead of two over the blocks.  Runs of ids
-// outside [0, E) get no tiles.  scratch holds 2 * E ints.
-__device__ TileRange build_ascending(const WideParams& p, int nblocks, int xcd, int* scratch, TileList& list) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  int* first = scratch;        // first block of the expert's run
-  int* end = scratch + p.E;    // one past its last block
-  for (int e = tid; e < 2 * p.E; e += kThreads) scratch[e] = 0;
-  __syncthreads();
-  for (int j = tid; j < nblocks; j += kThreads) {
-    const int e = p.expert_ids[j];
-    const int prev = j > 0 ? p.expert_ids[j - 1] : -1;
-    const int next = j + 1 < nblocks ? p.expert_ids[j + 1] : -1;
-    if (e >= 0 && e < p.E) {
-      if (j == 0 || e != prev) first[e] = j;
-      if (j + 1 == nblocks || e != next) end[e] = j + 1;
-    }
-  }
-  __syncthreads();
-  // thread t owns experts 2t and 2t + 1 (E <= 2 * kThreads)
-  int f[2], nb[2], tiles[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int e = 2 * tid + i;
-    f[i] = e < p.E ? first[e] : 0;
-    nb[i] = e < p.E ? end[e] - f[i] : 0;
-    tiles[i] = (nb[i] + p.per_tile - 1) / p.per_tile;
-  }
-  const int mine = tiles[0] + tiles[1];
-  const int incl = wave_inclusive_scan_add(mine);
-  if (lane == kWave - 1) list.wave_part[wave] = incl;
-  __syncthreads();
-  int t = incl - mine, total = 0;
-#pragma unroll
-  for (int i = 0; i < kWaves; ++i) {
-    const int w = list.wave_part[i];
-    if (i < wave) t += w;
-    total += w;
-  }
-  const TileRange range = range_of(total < kMaxTiles ? total : kMaxTiles, p.ntiles, xcd);
-  auto put = [&](int t, int e, int first_block, int blocks, int n, int r) {
-    if (t < range.lo || t >= range.hi) return;
-    const int in_group = n - (r & ~(kGroupTiles - 1));
-    const int from = p.even ? r * blocks / n : r * p.per_tile;
-    const int to = p.even ? (r + 1) * blocks / n : from + p.per_tile < blocks ? from + p.per_tile : blocks;
-    list.desc[t - range.lo] = (uint32_t)(first_block + from) | ((uint32_t)(to - from) << 16) | ((uint32_t)(r & (kGroupTiles - 1)) << 20) |
-                              ((uint32_t)(in_group < kGroupTiles ? in_group : kGroupTiles) << 24);
-    list.expert[t - range.lo] = (uint16_t)e;
-  };
-  if (p.E == 1) {  // a dense layer: all tiles are one expert's
-    for (int r = tid; r < total; r += kThreads) put(r, 0, first[0], end[0] - first[0], total, r);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      for (int r = 0; r < tiles[i]; ++r, ++t) put(t, 2 * tid + i, f[i], nb[i], tiles[i], r);
-  }
-  __syncthreads();
-  return range;
-}
 
 struct Task {
   int e;      // expert; -1 = no more work
@@ -280,7 +114,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
   __shared__ __align__(16) char staging[kWaves * kStaging];
   __shared__ __align__(16) int32_t ids[3][kTok];                          // slots of the current, the next and the task after it
   __shared__ __align__(16) float a_scales[2][kTok], row_weights[2][kTok], w_scales[2][kCh];
-  __shared__ TileList list;
+  __shared__ TileList<kMaxTiles> list;
   __shared__ uint2 table[kTable];                           // tasks it .. of this workgroup: block | blocks << 16, expert | channel tile << 16
 
   const int t = threadIdx.x;
@@ -291,37 +125,29 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
   const int nk = p.K / kStepBytes;
   const int inter = p.N / 2;
 
-  const int nblocks = __builtin_amdgcn_readfirstlane(*p.npp) / p.B;
   const int xcd = blockIdx.x % kXcds;
-  TileRange range = p.ascend ? build_ascending(p, nblocks, xcd, reinterpret_cast<int*>(stages), list)
-                                   : build_any_order(p, nblocks, p.per_tile, xcd, reinterpret_cast<int*>(stages), list);
+  TileRange range = p.ascend ? build_ascending(p.tiles, xcd, reinterpret_cast<int*>(stages), list)
+                             : build_any_order(p.tiles, __builtin_amdgcn_readfirstlane(*p.npp) / p.B, xcd, reinterpret_cast<int*>(stages), list);
   // (said to be wave-uniform: everything that follows from them then stays in scalar registers)
   range.lo = __builtin_amdgcn_readfirstlane(range.lo);
   range.hi = __builtin_amdgcn_readfirstlane(range.hi);
   range.tiles = __builtin_amdgcn_readfirstlane(range.tiles);
-  const int total = range.tiles * p.ntiles;
+  const int total = range.tiles * p.tiles.ntiles;
   const int per_xcd = __builtin_amdgcn_readfirstlane((total + kXcds - 1) / kXcds);
+  const int my_tasks = total - xcd * per_xcd < per_xcd ? max(total - xcd * per_xcd, 0) : per_xcd;  // of the XCD
   const int stride = gridDim.x / kXcds;
   int it = 0;  // tasks handed out
 
   // Looks up tasks n0 .. n0 + kTable - 1 of this workgroup.
   auto fill_table = [&](int n0) {
     if (t >= kTable) return;
-    const int at = blockIdx.x / kXcds + (n0 + t) * stride, task = xcd * per_xcd + at;
+    const TaskPiece tp = piece_at(blockIdx.x / kXcds + (n0 + t) * stride, my_tasks, stride);
     uint2 d = make_uint2(0u, 0xffffffffu);  // no more
-    if (at < per_xcd && task < total) {
-      // The tasks of a group of T token tiles of one expert run channel tile by channel tile: T consecutive tasks
-      // (on neighbouring compute units) stream the same weight tile.
-      const int tile0 = task / p.ntiles;
-      const uint32_t d0 = list.desc[tile0 - range.lo];
-      const int first = tile0 - (int)((d0 >> 20) & 7u);
-      const int T = (int)((d0 >> 24) & 15u);
-      const int pos = task - first * p.ntiles;
-      const int nt = pos / T;
-      const int tile = first + (pos - nt * T) - range.lo;
-      const int e = list.expert[tile];
-      // a tile of ids outside [0, E): no rows
-      d = make_uint2(list.desc[tile] & (e == 0xffff ? 0xffffu : 0xfffffu), (e == 0xffff ? 0u : (uint32_t)e) | ((uint32_t)nt << 16));
+    if (tp.task >= 0) {
+      const uint2 whole = look_up_task(p.tiles, list, range, xcd * per_xcd + tp.task);
+      // a piece is a part of the tile's blocks
+      const int blocks = (int)(whole.x >> 16) & 15, from = tp.piece * blocks / tp.pieces, to = (tp.piece + 1) * blocks / tp.pieces;
+      if (tp.pieces == 1 || to > from) d = make_uint2(((whole.x & 0xffffu) + from) | (uint32_t)(to - from) << 16, whole.y);
     }
     table[t] = d;
   };
@@ -343,19 +169,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
       load_to_lds_4(p.sorted_ids + tk.slot0 + (row < tk.rows ? row : 0), lds_address(&ids[buf][wave * 64]));
     }
   };
-  auto row_of = [&](int32_t id) { return p.row_div == 1 ? (uint32_t)id : __umulhi((uint32_t)id, p.div_magic) >> p.div_shift; };
-  // where the task's rows are (its ids have landed)
-  auto setup_loads = [&](const Task& tk, int buf, TaskLoads& ld) {
-    // lane l looks at rows 4l .. 4l + 3
-    const int4 four = *reinterpret_cast<const int4*>(&ids[buf][4 * lane]);
-    auto in_use = [&](int id) { return (uint32_t)id < (uint32_t)p.P; };
-    const uint64_t used = __ballot(4 * lane < tk.rows && (in_use(four.x) || in_use(four.y) || in_use(four.z) || in_use(four.w)));
-    ld.units = __builtin_amdgcn_readfirstlane(used ? (63 - __builtin_clzll(used)) / 8 + 1 : 0);
+  // Where the task's rows are.  Lane fills LDS slot (lane & 7) of row base + 8 * i + (lane >> 3) of a wavefront's load i: it
+  // fetches chunk (lane & 7) ^ swizzle.
+  auto chunk_of = [&](int i) { return ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16; };
+  auto setup_weights = [&](const Task& tk, TaskLoads& ld) {
     ld.wbase = p.w + (int64_t)tk.e * p.N * p.K;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      // lane fills LDS slot (lane & 7) of row 32 * wave + 8 * i + (lane >> 3): it fetches chunk (lane & 7) ^ swizzle
-      const int chunk = ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;
       const int row = 32 * wave + 8 * i + (lane >> 3);
       int n;
       if constexpr (MODE == kGateUpSilu) {
@@ -365,12 +185,23 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
         const int ch = tk.nt * kCh + row;
         n = ch < p.N ? ch : p.N - 1;
       }
-      ld.woff[i] = (uint32_t)n * (uint32_t)p.K + chunk;
+      ld.woff[i] = (uint32_t)n * (uint32_t)p.K + chunk_of(i);
+    }
+  };
+  // ... (its ids have landed)
+  auto setup_tokens = [&](const Task& tk, int buf, TaskLoads& ld) {
+    // lane l looks at rows 4l .. 4l + 3
+    const int4 four = *reinterpret_cast<const int4*>(&ids[buf][4 * lane]);
+    auto in_use = [&](int id) { return (uint32_t)id < (uint32_t)p.P; };
+    const uint64_t used = __ballot(4 * lane < tk.rows && (in_use(four.x) || in_use(four.y) || in_use(four.z) || in_use(four.w)));
+    ld.units = __builtin_amdgcn_readfirstlane(used ? (63 - __builtin_clzll(used)) / 8 + 1 : 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
       // rows behind the last one in use fetch the tile's first row again
       int trow = (i >> 1) * 128 + 16 * wave + 8 * (i & 1) + (lane >> 3);
       if (trow >= ld.units * 32) trow = 0;
       const int32_t id = ids[buf][trow];
-      ld.xoff[i >> 1][i & 1] = (in_use(id) ? row_of(id) : 0u) * (uint32_t)p.K + chunk;
+      ld.xoff[i >> 1][i & 1] = (in_use(id) ? p.row_of(id) : 0u) * (uint32_t)p.K + chunk_of(i);
     }
   };
   // inputs of the task's epilogue
@@ -380,7 +211,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
       int32_t id = ids[buf][row < tk.rows ? row : 0];
       if (id < 0 || id >= p.P) id = 0;
       if (wave < 4) {
-        load_to_lds_4(p.a_scale + row_of(id), lds_address(&a_scales[aux][wave * 64]));
+        load_to_lds_4(p.a_scale + p.row_of(id), lds_address(&a_scales[aux][wave * 64]));
       } else {
         if (MODE == kDown && p.row_weight) load_to_lds_4(p.row_weight + id, lds_address(&row_weights[aux][(wave & 3) * 64]));
         int n;
@@ -436,29 +267,34 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
     Task nx = next_task();
     fetch_ids(tk, 0);
     fetch_ids(nx, 1);
-    wait_vmcnt<0>();
-    __syncthreads();
     TaskLoads nld;  // of the next task; without one, of this one
-    setup_loads(tk, 0, nld);
-    int units = nld.units;
-    fetch_aux(tk, 0, 0);
+    setup_weights(tk, nld);
     // Load cursors: where the next weight-and-first-half and the next second-half loads come from.  They run ahead of
     // the multiplication, into the next task where there is one, else over this task's first steps again.
     const uint64_t aq = uniform_address(p.a_q);
     uint64_t wp = uniform_address(nld.wbase), xp = aq, x1p = aq;
-    uint32_t woff[4], x0off[2], x1off[2];
+    uint32_t woff[4], x0off[2] = {0, 0}, x1off[2] = {0, 0};
 #pragma unroll
     for (int i = 0; i < 4; ++i) woff[i] = nld.woff[i];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) x0off[i] = nld.xoff[0][i], x1off[i] = nld.xoff[1][i];
     const uint32_t at_w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(stage0 + wave * 4096));
     const uint32_t at_x0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(stage0 + wave * 2048));
-    issue_w(wp, xp, woff, x0off, at_w0, at_x0);
+    // The first step's weights are requested while the token ids are on their way.
+    unroll<4>([&](auto i) { load_w(i, wp, xp, woff, x0off, at_w0, at_x0); });
+    wait_vmcnt<4>();
+    __syncthreads();
+    setup_tokens(tk, 0, nld);
+    int units = nld.units;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x0off[i] = nld.xoff[0][i], x1off[i] = nld.xoff[1][i];
+    fetch_aux(tk, 0, 0);
+    load_w(std::integral_constant<int, 4>{}, wp, xp, woff, x0off, at_w0, at_x0);
+    load_w(std::integral_constant<int, 5>{}, wp, xp, woff, x0off, at_w0, at_x0);
     issue_x1(x1p, x1off, at_x0);
     issue_w(wp + kStepBytes, xp + kStepBytes, woff, x0off, at_w0 + kStage, at_x0 + kStage);
     wp += 2 * kStepBytes, xp += 2 * kStepBytes, x1p += kStepBytes;
-    wait_vmcnt<0>();
+    wait_vmcnt<8>();  // all but the second half of step 0 and step 1
     barrier();
+    bool fresh = true;  // the first step's waits are as in any other step; a later task's first step has landed as a whole
     int buf = 0, aux = 0, slot = 0;
 
     while (true) {
@@ -506,7 +342,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
       if (group == 1) barrier();
       for (int s = 0; s < nk; ++s) {
         const char* st = stages + slot * kStage;
-        const int waits = s > 0 ? group : 2;  // which group has loads to wait for: everything of step 0 has landed
+        const int waits = s > 0 || fresh ? group : 2;  // which group has loads to wait for
         // ---- read 0 ----
 #pragma unroll
         for (int ci = 0; ci < 4; ++ci) {
@@ -528,7 +364,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
         // ---- read 1 ----
         if (n1 > 0) read_x(st + kX1);
         if (s == 0 && has_next) {
-          setup_loads(nx, buf == 2 ? 0 : buf + 1, nld);
+          setup_weights(nx, nld);
+          setup_tokens(nx, buf == 2 ? 0 : buf + 1, nld);
           fetch_aux(nx, buf == 2 ? 0 : buf + 1, aux ^ 1);
           after = next_task();
           fetch_ids(after, buf == 0 ? 2 : buf - 1);
@@ -564,6 +401,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
           __builtin_nontemporal_store(x, reinterpret_cast<v4i*>(to));
       };
       wait_vmcnt<0>();
+      fresh = false;
       if constexpr (MODE == kAccI32) {
 #pragma unroll
         for (int ti = 0; ti < 8; ++ti) {
@@ -663,27 +501,26 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.w_scale = a.w_scale;
   p.row_weight = a.row_weight;
   p.sorted_ids = a.sorted_token_ids;
-  p.expert_ids = a.expert_ids;
   p.npp = a.num_tokens_post_padded;
   p.P = (int)a.num_pairs;
-  p.row_div = a.row_div;
-  // rounded-up reciprocal of 31 + l fraction bits, 2^(l-1) < row_div <= 2^l: exact for ids below 2^31
-  int l = 0;
-  while ((1ll << l) < a.row_div) ++l;
-  p.div_magic = a.row_div > 1 ? (uint32_t)(((uint64_t)1 << (31 + l)) / (uint64_t)a.row_div + 1) : 0;
-  p.div_shift = l - 1;
-  p.E = a.num_experts;
+  p.row_of = divider(a.row_div);
+  p.tiles.expert_ids = a.expert_ids;
+  p.tiles.E = a.num_experts;
   p.N = a.n;
   p.K = a.k;
   p.B = a.block_size;
-  p.per_tile = kTok / a.block_size;
+  p.tiles.per_tile = kTok / a.block_size;
   // Nine blocks as 3 + 3 + 3 instead of 4 + 4 + 1: a step of one block costs far more than a quarter of a full one (its weight
   // rows are the same).  Layer us, full tiles and a rest / even ones: 256 experts of 7168 x 2048 at 8192 / 16384 tokens 4229 / 3790,
   // 6360 / 6247, 129 of 4096 x 1408, evenly routed, at 4096 1066 / 933 (skewed routing: the same).  Below: no difference
   // at 2048 x 768 and 2048 x 1408, and even tiles lose at short reductions, where a task is mostly its epilogue: 32
   // experts of 1024 x 512 at 5000 tokens 101.6 / 103.3, 256 of 2048 x 512 at 4000 297.9 / 303.7.
-  p.even = a.k >= 4096;
-  p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kCh - 1) / kCh;
+  p.tiles.even = a.k >= 4096;
+  p.tiles.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kCh - 1) / kCh;
+  p.tiles.by_ntiles = divider(p.tiles.ntiles);
+  p.tiles.by_per_tile = divider(p.tiles.per_tile);
+  p.tiles.blocks = (int)(a.sorted_cap / a.block_size);
+  p.tiles.identity = a.identity ? 1 : 0;
   p.ascend = a.expert_ids_ascend && a.num_experts <= 2 * kThreads ? 1 : 0;
   // The next launch of a layer reads the results back from the last-level cache where they about fit it and the weights do
   // not sweep it.  Layer us with / without the hint: 128 experts of 2048 x 768 at 8192 tokens 488 / 480, of 4096 x 1536 at

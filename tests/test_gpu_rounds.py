@@ -1,0 +1,62 @@
+"""GPU parity of the kernels with LDS-staged tiles where an XCD's last round of tasks is cut into pieces (channels of the narrow
+and deep tiles, blocks of the wide ones), and where tasks start their reductions at different steps (a stride of 4096
+bytes): int32 accumulators against the oracle's, exactly."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _check(pra, oracle, variant, counts, N, K, B=64):
+    gen = torch.Generator().manual_seed(N + K + len(counts))
+    E, P = len(counts), sum(counts)
+    ids = torch.repeat_interleave(torch.arange(E, dtype=torch.int32), torch.tensor(counts))
+    ids = ids[torch.randperm(P, generator=gen)].view(P, 1)
+    a = torch.randint(-127, 128, (P, K), dtype=torch.int8, generator=gen)
+    w = torch.randint(-127, 128, (E, N, K), dtype=torch.int8, generator=gen)
+    s, e, npp = pra.moe_align_block_size(ids.to(DEV), B, E)
+    got = pra.gemm_acc_i32(a.to(DEV), w.to(DEV), s, e, npp, 1, B, P, variant).cpu()
+    want = oracle.grouped_int_gemm(a, w, ids, 1)
+    assert torch.equal(got, want.view_as(got)), int((got != want.view_as(got)).sum())
+
+
+# (an XCD has 32 workgroups: these are 8 * 32 * rounds + 8 * rest tasks of 128 channels, the last XCD's range a little shorter)
+@pytest.mark.parametrize("variant", ["narrow", "tile_deep", "tile_wide"])
+@pytest.mark.parametrize("tasks", [1, 63, 65, 127, 129, 135, 257, 256 + 64, 256 + 72, 256 + 130, 512 + 17])
+def test_rest_of_the_last_round(pra, oracle, variant, tasks):
+    channels = 128 if variant == "narrow" else 256
+    _check(pra, oracle, variant, [70], tasks * channels - 16 * (tasks % 3), 512)
+
+
+@pytest.mark.parametrize("variant", ["narrow", "tile_deep", "tile_wide"])
+@pytest.mark.parametrize("counts", [[260, 5, 0, 64, 129], [1] * 37])
+def test_pieces_of_tiles_of_several_sizes(pra, oracle, variant, counts):
+    _check(pra, oracle, variant, counts, 2 * 256 + 48, 768)
+    _check(pra, oracle, variant, counts, 256, 768, B=128)
+
+
+@pytest.mark.parametrize("variant", ["narrow", "tile_deep", "tile_wide"])
+@pytest.mark.parametrize("K", [4096, 8192])
+def test_tasks_that_start_at_different_steps(pra, oracle, variant, K):
+    # 70 experts: the starting step wraps around twice
+    _check(pra, oracle, variant, [(7 * i) % 40 for i in range(70)], 272, K)
+
+
+@pytest.mark.parametrize("steps", [4, 5, 6, 7, 8])
+@pytest.mark.parametrize("most", [20, 60])
+def test_narrow_reductions_around_the_depth_of_the_ring(pra, oracle, steps, most):
+    # tiles of 64 token rows have six stages; those of 32 (no expert with more rows) seven, in the layer only
+    _check(pra, oracle, "narrow", [most - i % 13 for i in range(24)], 1024 + 16, steps * 128)
+
+
+@pytest.mark.parametrize("H,I", [(512, 1024), (768, 512), (896, 896), (4096, 1024)])
+def test_narrow_layer_of_32_tokens(pra, H, I):
+    from _util import inputs_mod
+
+    im = inputs_mod()
+    d = im.make_inputs(im.LayerShape("n", E=24, k=4, H=H, I=I), 32, seed=H).to(DEV)
+    kw = d.fused_experts_kwargs()
+    got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="narrow")
+    assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream"))
