@@ -10,14 +10,12 @@
 //
 // A tile's loads and a step's work are kept off the stream's critical path: tasks are looked up 64 at a time,
 // token ids travel two tiles ahead, and a step reads its operands before it issues the loads of a later step
-// between its multiplications.  Against two workgroups of four wavefronts with three stages each (64 KB in
-// flight, a look-up of two dependent scalar reads per tile, loads first): same tiles, but half as long per tile
-// and twice as many per workgroup, which evens out the last round; 0.57 us per step = 7.3 TB/s of weights.
-// Layer us before -> after: 128 experts of 2048 x 768 at 17 / 100 / 203 / 400 / 512 tokens 80.6 / 112.3 / 117.1 / 128.1 /
-// 135.1 -> 78.0 / 109.0 / 113.1 / 126.1 / 135.3, 4096 x 1408 with skewed routing at 17 / 64 tokens 104.7 / 148.6 -> 99.8 /
-// 143.2, but at 200 / 300 tokens, where one expert holds several tiles of rows, 231.0 / 265.1 -> 235.5 / 271.2; 256 experts
-// of 7168 x 2048 at 17 / 64 / 128 / 256 tokens 544 / 909 / 1062 / 1226 -> 535 / 874 / 1033 / 1186.  Launches of
-// several tasks of four steps gain nothing: 256 experts of 2048 x 512 at 90 tokens 134 -> 139.5.
+// between its multiplications.  What does not change during a step is decided outside the loop over the steps, of which
+// there is one per kind of wavefront and of loads: with some twenty branches in it a step cost 0.5 us even where all of its
+// rows came from L2, now 0.42; where they come from memory, 0.51-0.55 us a step are 7.6 TB/s of weights.
+// Layer us, before that -> after, with the starting steps of rotation_mask and the divided last rounds of piece_at: 128 experts of
+// 2048 x 768 at 203 tokens 117.2 -> 116.1, 4096 x 1408 with skewed routing at 32 tokens 129 -> 125, 256 experts of 7168 x 2048 at
+// 64 tokens 851 -> 844; gate_up GEMM alone, 16 experts of 4096 x 1408 with 512 rows each 190 -> 160.
 //
 // A tile is TOK token rows (32 or 64: part of a moe_align block) x 128 weight rows; the reduction runs
 // in steps of 128 bytes and both operands reach LDS by global -> LDS loads (global_load_lds_dwordx4, no
@@ -37,15 +35,17 @@
 // LDS rows are 128 bytes; the 16-byte chunk index is XOR-swizzled with row bits so that the MFMA
 // operand reads spread over all banks; because a load fills LDS linearly the swizzle is applied to the
 // global source address of each lane.
+#include <type_traits>
+
 #include "lds_loads.hpp"
+#include "tile_list.hpp"
 
 namespace moe_i8 {
 namespace {
 
-constexpr int kThreads = 512;
+constexpr int kThreads = kTileThreads;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kCh = 128;    // weight rows per tile
-constexpr int kXcds = 8;
 constexpr int kMinSteps = 4;
 
 template <int TOK>
@@ -74,13 +74,14 @@ struct NarrowParams {
   const int32_t* sorted_ids;
   const int32_t* expert_ids;
   const int32_t* npp;
-  int64_t P;
-  int row_div;
+  int P;
+  Divider row_of;
   int E;
   int N;
   int K;
   int B;
   int ntiles;  // channel tiles
+  int rotate;  // mask of the reduction step that a task starts at (rotation_mask)
   void* out;
 };
 
@@ -93,7 +94,7 @@ __device__ __forceinline__ void load_to_lds_dword(const void* base, uint32_t off
 
 struct Task {
   int e;          // expert; -1 = no more work
-  int ct;         // channel tile
+  int n0, n1;     // its channels
   int64_t slot0;  // first slot of the tile in sorted_ids
   bool single;    // nothing else reads the expert's weight rows
 };
@@ -101,11 +102,13 @@ struct Task {
 struct TaskLoads {
   const int8_t* wbase;  // weights of the task's expert (wave-uniform)
   bool stream;          // fetch the weight rows with the non-temporal hint
+  int first;            // byte offset of the first reduction step
   uint32_t woff[2];     // per lane: byte offset of its chunk of weight row i from wbase
   uint32_t xoff;        // per lane: byte offset of its chunk of its token row from a_q
 };
 
-template <int MODE, int TOK>
+// FULL: the reduction has at least kStages steps, so that the ring is always full and every wait the same.
+template <int MODE, int TOK, bool FULL>
 __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p) {
   using S = Shape<TOK>;
   using F = Mfma<S::MF>;
@@ -113,6 +116,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   constexpr int kStageBytes = S::kStageBytes;
   constexpr int kTokOffset = kCh * kStepBytes;
   constexpr int NI = 32 / S::MF;  // MFMA tiles of a wavefront's 32 weight rows
+  constexpr int kOut = MODE == kGateUpSilu ? kCh / 2 : kCh;  // channels of a whole tile
   __shared__ __align__(16) char stages[kStages * kStageBytes];
   __shared__ __align__(16) TileAux aux[3];
 
@@ -125,10 +129,11 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   const int K = p.K;
   const int nk = K / kStepBytes;
   const int inter = p.N / 2;
-  const bool loads_tokens = wave < S::kTokWaves;
+  const int width = MODE == kGateUpSilu ? inter : p.N;
+  const bool loads_tokens = S::kTokWaves == kWaves || wave < S::kTokWaves;
   // Steps the loads run ahead of the multiplication: the ring's depth, less for very short reductions (the
   // rows of the next tile are set up in the first step of the current one).
-  const int ahead = nk - 1 < kStages - 1 ? nk - 1 : kStages - 1;
+  const int ahead = FULL || nk > kStages ? kStages - 1 : nk - 1;
 
   // ---- this workgroup's tasks: (block, channel tile), channel tile fastest, split into 8 contiguous
   // ranges, one per XCD (workgroup id % 8), so that workgroups that run side by side share token
@@ -142,21 +147,22 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   const int xcd = blockIdx.x % kXcds;
   const int stride = gridDim.x / kXcds;
   const int in_range = total - xcd * per_xcd < per_xcd ? total - xcd * per_xcd : per_xcd;
-  const int phase_len = (per_xcd + stride - 1) / stride * stride;
+  const int rounds = (per_xcd + stride - 1) / stride;  // of a phase
 
-  // Candidate tasks of this workgroup: `first_slot + i * stride` of its XCD's range, phase by phase.  Lane i
+  // Candidate tasks of this workgroup: its places in the rounds of its XCD's range, phase by phase (a task of a last round
+  // that leaves workgroups idle is cut into pieces of its channels).  Lane i
   // looks up candidate 64 * chunk + i, so that taking the next task is a bit scan and a few lane reads: looked
   // up one by one (two dependent scalar reads, about 1 us) they held up every tile, whose steps are 0.6 us.
   // A task needs a valid expert id and rows that are not all padding (valid rows are a prefix of a block).
-  const int candidates = phase_len / stride * sub_per_block;
+  const int candidates = rounds * sub_per_block;
   uint64_t open = 0;  // candidates of the current chunk not handed out yet
-  int chunk_base = 0, lane_e = 0, lane_blk = 0, lane_ct = 0, lane_flags = 0;
+  int chunk_base = 0, lane_e = 0, lane_blk = 0, lane_n0 = 0, lane_n1 = 0, lane_flags = 0;
   auto look_up = [&]() {
     const int i = chunk_base + lane;
-    const int sub = i / (phase_len / stride);
-    const int at = (int)(blockIdx.x / kXcds) + (i - sub * (phase_len / stride)) * stride;
-    bool ok = i < candidates && at < in_range;
-    const int task = xcd * per_xcd + (ok ? at : 0);
+    const int sub = i / rounds;
+    const TaskPiece tp = piece_at((int)(blockIdx.x / kXcds) + (i - sub * rounds) * stride, in_range, stride);
+    bool ok = i < candidates && tp.task >= 0;
+    const int task = xcd * per_xcd + (ok ? tp.task : 0);
     const int blk = ok ? task / p.ntiles : 0;
     const int64_t slot0 = (int64_t)blk * p.B + (int64_t)(ok ? sub : 0) * TOK;
     const int e = p.expert_ids[blk];
@@ -173,14 +179,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
                         (sub_per_block == 1 || !(other >= 0 && other < p.P));
     lane_e = e;
     lane_blk = blk;
-    lane_ct = task - blk * p.ntiles;
+    const int width = kOut / tp.pieces;
+    lane_n0 = (task - blk * p.ntiles) * kOut + tp.piece * width;
+    lane_n1 = lane_n0 + width;
     lane_flags = sub * 2 + (single ? 1 : 0);
     open = __ballot(ok);
   };
   auto next_task = [&]() {
     Task tk;
     tk.e = -1;
-    tk.ct = 0;
+    tk.n0 = tk.n1 = 0;
     tk.slot0 = 0;
     tk.single = false;
     while (open == 0 && chunk_base + kWave < candidates) {
@@ -192,7 +200,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
       open &= open - 1;
       const int flags = __builtin_amdgcn_readlane(lane_flags, i);
       tk.e = __builtin_amdgcn_readlane(lane_e, i);
-      tk.ct = __builtin_amdgcn_readlane(lane_ct, i);
+      tk.n0 = __builtin_amdgcn_readlane(lane_n0, i);
+      tk.n1 = __builtin_amdgcn_readlane(lane_n1, i);
       tk.slot0 = (int64_t)__builtin_amdgcn_readlane(lane_blk, i) * p.B + (flags >> 1) * TOK;
       tk.single = flags & 1;
     }
@@ -200,8 +209,11 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   };
 
   const uint32_t stage0 = lds_address(stages);
+  auto in_use = [&](int32_t id) { return (uint32_t)id < (uint32_t)p.P; };
 
   // ---- global -> LDS loads ----
+  // the task's channel c, the last one again behind its end
+  auto channel = [&](const Task& tk, int c) { return min(tk.n0 + c, min(tk.n1, width) - 1); };
   // Lane fills LDS slot (lane & 7) of row base + 8 * i + (lane >> 3): it fetches the logical chunk
   // (lane & 7) ^ swizzle(row) of that row.
   auto setup_weight_loads = [&](const Task& tk, TaskLoads& ld) {
@@ -212,22 +224,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
       int n;
       if constexpr (MODE == kGateUpSilu) {
         const int j = row & 31;
-        const int ch = tk.ct * 64 + (row >> 5) * 16 + (j & 15);
-        n = (ch < inter ? ch : inter - 1) + (j >= 16 ? inter : 0);
+        n = channel(tk, (row >> 5) * 16 + (j & 15)) + (j >= 16 ? inter : 0);
       } else {
-        const int ch = tk.ct * kCh + row;
-        n = ch < p.N ? ch : p.N - 1;
+        n = channel(tk, row);
       }
       ld.woff[i] = (uint32_t)n * (uint32_t)K + chunk;
     }
     ld.wbase = p.w + (int64_t)tk.e * p.N * K;
     ld.stream = tk.single;
+    ld.first = (tk.e & p.rotate) * kStepBytes;
   };
   auto setup_token_loads = [&](const TileAux& ax, TaskLoads& ld) {
     const int row = (8 * wave + (lane >> 3)) & (TOK - 1);
     const int chunk = ((lane & 7) ^ swizzle_of_row(row)) * 16;
     const int32_t tok = ax.ids[row];
-    const uint32_t arow = (tok >= 0 && tok < p.P) ? (uint32_t)(tok / p.row_div) : 0u;
+    const uint32_t arow = in_use(tok) ? p.row_of(tok) : 0u;
     ld.xoff = arow * (uint32_t)K + chunk;
   };
   auto issue_weights = [&](const TaskLoads& ld, int stage, int koff) {
@@ -249,8 +260,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   auto issue_scales = [&](const Task& tk, TileAux& ax) {
     if constexpr (MODE == kAccI32) return;
     const int32_t tok = ax.ids[lane & (TOK - 1)];
-    const uint32_t t = (tok >= 0 && tok < p.P) ? (uint32_t)tok : 0u;
-    load_to_lds_dword(p.a_scale, (t / (uint32_t)p.row_div) * 4u, lds_address(ax.a_scale));
+    const uint32_t t = in_use(tok) ? (uint32_t)tok : 0u;
+    load_to_lds_dword(p.a_scale, p.row_of((int)t) * 4u, lds_address(ax.a_scale));
     const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
     if constexpr (MODE == kDown) {
       // without routed weights the slot is filled with something readable and never used
@@ -260,12 +271,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
         load_to_lds_dword(p.a_scale, 0u, lds_address(ax.row_w));
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int n = tk.ct * kCh + 64 * j + lane;
-        load_to_lds_dword(wsc, (uint32_t)(n < p.N ? n : p.N - 1) * 4u, lds_address(ax.w_scale + 64 * j));
+        load_to_lds_dword(wsc, (uint32_t)channel(tk, 64 * j + lane) * 4u, lds_address(ax.w_scale + 64 * j));
       }
     } else {
-      const int ch = tk.ct * 64 + lane;
-      const uint32_t c = (uint32_t)(ch < inter ? ch : inter - 1);
+      const uint32_t c = (uint32_t)channel(tk, lane);
       load_to_lds_dword(wsc, c * 4u, lds_address(ax.w_scale));
       load_to_lds_dword(wsc, (c + (uint32_t)inter) * 4u, lds_address(ax.w_scale + 64));
     }
@@ -291,7 +300,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   auto epilogue = [&](const Task& tk, const TileAux& ax, typename F::Acc (&acc)[NI]) {
     const int row = th * S::MF + lrow;
     const int32_t tok = ax.ids[row];
-    if (tok < 0 || tok >= p.P) return;
+    if (!in_use(tok)) return;
+    const int limit = min(tk.n1, width);
     auto piece = [&](int j, int (&v)[4]) {  // weight rows 8 * j + 4 * lgrp + r (j = 0..3); 16-row tiles: 16 * j + 4 * lgrp + r
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] = S::MF == 32 ? acc[0][(4 * j + r) % F::kRegs] : acc[j % NI][r];
@@ -305,13 +315,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
 #pragma unroll
       for (int j = 0; j < kPieces / 2; ++j) {
         const int c = 16 * cg + kPieceRows * j + 4 * lgrp;
-        const int n = tk.ct * 64 + c;
+        const int n = tk.n0 + c;
         const float4 wg = *reinterpret_cast<const float4*>(ax.w_scale + c);
         const float4 wu = *reinterpret_cast<const float4*>(ax.w_scale + 64 + c);
         int g[4], u[4];
         piece(j, g);
         piece(j + kPieces / 2, u);
-        if (n < inter) *reinterpret_cast<uint2*>(out + n) = silu_mul_epilogue4(g, u, as, wg, wu);
+        if (n < limit) *reinterpret_cast<uint2*>(out + n) = silu_mul_epilogue4(g, u, as, wg, wu);
       }
     } else {
       const float as = MODE == kDown ? ax.a_scale[row] : 0.0f;
@@ -319,8 +329,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
 #pragma unroll
       for (int j = 0; j < kPieces; ++j) {
         const int c = 32 * cg + kPieceRows * j + 4 * lgrp;
-        const int n = tk.ct * kCh + c;
-        if (n >= p.N) continue;
+        const int n = tk.n0 + c;
+        if (n >= limit) continue;
         int v[4];
         piece(j, v);
         if constexpr (MODE == kAccI32) {
@@ -339,12 +349,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   look_up();
   Task tk = next_task();
   if (tk.e < 0) return;
-  TaskLoads ld, nld;
+  TaskLoads ld;
+  auto from = [&](const TaskLoads& ld, int s) {
+    const int at = ld.first + s * kStepBytes;
+    return at < K ? at : at - K;
+  };
   constexpr int kEarly = 2;  // steps whose weights are requested before the row ids are in
   issue_ids(tk, aux[0]);
   setup_weight_loads(tk, ld);
 #pragma unroll
-  for (int s = 0; s < kEarly; ++s) issue_weights(ld, s, s * kStepBytes);
+  for (int s = 0; s < kEarly; ++s) issue_weights(ld, s, from(ld, s));
   Task nx = next_task();
   issue_ids(nx.e >= 0 ? nx : tk, aux[1]);
   Task n2 = next_task();
@@ -352,95 +366,117 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   wait_vmcnt<2 * kEarly>();
   setup_token_loads(aux[0], ld);
 #pragma unroll
-  for (int s = 0; s < kEarly; ++s) issue_tokens(ld, s, s * kStepBytes);
+  for (int s = 0; s < kEarly; ++s) issue_tokens(ld, s, from(ld, s));
   issue_scales(tk, aux[0]);
   for (int s = kEarly; s < ahead; ++s) {
-    issue_weights(ld, s, s * kStepBytes);
-    issue_tokens(ld, s, s * kStepBytes);
+    issue_weights(ld, s, from(ld, s));
+    issue_tokens(ld, s, from(ld, s));
   }
-  nld = ld;
+  int next_at = from(ld, ahead);  // byte offset of the next step to fetch, of the task that `ld` is set up for
   wait_all_but(ahead - kEarly);  // steps 0 and 1 (their loads are not in the order of the steps)
 
-  int par = 0;    // aux of the current task; the next ones follow
-  int stage = 0;  // ring position of the step being multiplied
-  bool fresh = true;
+  int par = 0;                     // aux of the current task; the next ones follow
+  int read_at = 0;                 // ring offset of the step being multiplied
+  int fill_at = ahead * kStageBytes;  // ... of the step being fetched
+  const uint32_t wdst = stage0 + wave * 2048, xdst = stage0 + kTokOffset + wave * 1024;
+  // a wavefront whose half of the tile is padding (valid rows are a prefix) only loads
+  auto half_in_use = [&](const TileAux& ax) { return in_use(__builtin_amdgcn_readfirstlane(ax.ids[th * S::MF])); };
+  bool active = half_in_use(aux[0]), next_active = false;
   while (true) {
     typename F::Acc acc[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int r = 0; r < F::kRegs; ++r) acc[i][r] = 0;
-    // a wavefront whose half of the tile is padding (valid rows are a prefix) only loads
-    const int32_t half_first = __builtin_amdgcn_readfirstlane(aux[par].ids[th * S::MF]);
-    const bool active = half_first >= 0 && half_first < p.P;
     TileAux& ax_next = aux[par + 1 < 3 ? par + 1 : par - 2];
     TileAux& ax_n2 = aux[par + 2 < 3 ? par + 2 : par - 1];
-
-    for (int s = 0; s < nk; ++s) {
-      // this wavefront's loads of step s have landed ...
-      if (!fresh) wait_all_but(ahead - 1);
-      fresh = false;
-      // ... and so have everybody's; everybody is also done reading the stage that is filled next
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      int fill = stage + ahead;
-      if (fill >= kStages) fill -= kStages;
-      if (s == 0) {
-        // the next task's rows (their ids were fetched a task ago) and, for the one after it, the ids
-        const Task& t1 = nx.e >= 0 ? nx : tk;
-        setup_weight_loads(t1, nld);
-        setup_token_loads(nx.e >= 0 ? ax_next : aux[par], nld);
-        if (n2.e >= 0) issue_ids(n2, ax_n2);
-      }
-      // Operands first, then the loads of the step `ahead` of this one a piece at a time between the
-      // multiplications: the address unit takes 16 clocks per load and the whole workgroup's 20-24 of them in front
-      // of the operand reads made a step 0.45 us even where every load hit L2.
-      const char* st = stages + stage * kStageBytes;
-      v4i a[F::kSub][NI], b[F::kSub];
-      if (active) {
+    int advance = kStepBytes;
+    // Steps [s0, s1), during which the loads are those of one task.  This loop is what the kernel does all the time, and
+    // with few rows its instructions, not the memory, are what a step costs as soon as the rows come from L2: everything
+    // that does not change inside is decided outside.
+    auto steps = [&](auto active_tag, auto stream_tag, int s0, int s1) {
+      constexpr bool ACTIVE = decltype(active_tag)::value, STREAM = decltype(stream_tag)::value;
+      for (int s = s0; s < s1; ++s) {
+        // everybody's loads of step s have landed, and everybody is done reading the stage that is filled next
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // Operands first, then the loads of the step `ahead` of this one a piece at a time between the
+        // multiplications: the address unit takes 16 clocks per load and the whole workgroup's 20-24 of them in front
+        // of the operand reads made a step 0.45 us even where every load hit L2.
+        const char* st = stages + read_at;
+        v4i a[F::kSub][NI], b[F::kSub];
+        if constexpr (ACTIVE) {
 #pragma unroll
-        for (int kk = 0; kk < F::kSub; ++kk) {
-          b[kk] = *reinterpret_cast<const v4i*>(st + x_ld + chunk[kk]);
+          for (int kk = 0; kk < F::kSub; ++kk) {
+            b[kk] = *reinterpret_cast<const v4i*>(st + x_ld + chunk[kk]);
 #pragma unroll
-          for (int i = 0; i < NI; ++i) a[kk][i] = *reinterpret_cast<const v4i*>(st + w_ld[i] + chunk[kk]);
+            for (int i = 0; i < NI; ++i) a[kk][i] = *reinterpret_cast<const v4i*>(st + w_ld[i] + chunk[kk]);
+          }
+        }
+        const int8_t* wsrc = ld.wbase + next_at;
+        const int8_t* xsrc = p.a_q + next_at;
+        auto mul = [&](int kk) {
+          if constexpr (ACTIVE)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) acc[i] = F::mul(a[kk][i], b[kk], acc[i]);
+        };
+        auto one_weight = [&](int i) {
+          if constexpr (STREAM)
+            load_to_lds_16_stream(wsrc, ld.woff[i], wdst + fill_at + i * 1024);
+          else
+            load_to_lds_16(wsrc, ld.woff[i], wdst + fill_at + i * 1024);
+        };
+        mul(0);
+        one_weight(0);
+        if constexpr (F::kSub == 4) mul(1);
+        one_weight(1);
+        mul(F::kSub == 4 ? 2 : 1);
+        if (loads_tokens) load_to_lds_16(xsrc, ld.xoff, xdst + fill_at);
+        if constexpr (F::kSub == 4) mul(3);
+        if (s == 1) {
+          if (nx.e >= 0) issue_scales(nx, ax_next);
+          if (n2.e >= 0) issue_ids(n2, ax_n2);
+        }
+        next_at = next_at + advance < K ? next_at + advance : 0;
+        read_at = read_at + kStageBytes < kStages * kStageBytes ? read_at + kStageBytes : 0;
+        fill_at = fill_at + kStageBytes < kStages * kStageBytes ? fill_at + kStageBytes : 0;
+        // this wavefront's loads of the next step have landed; after a task's last step, before its stores
+        if constexpr (FULL) {
+          if (loads_tokens)
+            wait_vmcnt<3 * (kStages - 2)>();
+          else
+            wait_vmcnt<2 * (kStages - 2)>();
+        } else {
+          wait_all_but(ahead - 1);
         }
       }
-      // the step fetched: of this task, of the next one, or (nothing left) the last one again, which keeps the
-      // counts uniform
-      const bool in_task = s + ahead < nk || nx.e < 0;
-      const int fs = s + ahead < nk ? s + ahead : nx.e < 0 ? nk - 1 : s + ahead - nk;
-      const int8_t* wsrc = (in_task ? ld.wbase : nld.wbase) + fs * kStepBytes;
-      const bool nt = in_task ? ld.stream : nld.stream;
-      const uint32_t wdst = stage0 + fill * kStageBytes + wave * 2048;
-      const uint32_t w0 = in_task ? ld.woff[0] : nld.woff[0], w1 = in_task ? ld.woff[1] : nld.woff[1];
-      const uint32_t x0 = in_task ? ld.xoff : nld.xoff;
-      auto mul = [&](int kk) {
-        if (active)
-#pragma unroll
-          for (int i = 0; i < NI; ++i) acc[i] = F::mul(a[kk][i], b[kk], acc[i]);
-      };
-      auto one_weight = [&](uint32_t off, uint32_t dst) {
-        if (nt)
-          load_to_lds_16_stream(wsrc, off, dst);
-        else
-          load_to_lds_16(wsrc, off, dst);
-      };
-      mul(0);
-      one_weight(w0, wdst);
-      if constexpr (F::kSub == 4) mul(1);
-      one_weight(w1, wdst + 1024);
-      mul(F::kSub == 4 ? 2 : 1);
-      if (loads_tokens) load_to_lds_16(p.a_q + fs * kStepBytes, x0, stage0 + fill * kStageBytes + kTokOffset + wave * 1024);
-      if constexpr (F::kSub == 4) mul(3);
-      if (s == 1 && nx.e >= 0) issue_scales(nx, ax_next);
-      stage = stage + 1 < kStages ? stage + 1 : 0;
+    };
+    // The loads run `ahead` steps in front of the multiplication: into the next task, or (nothing left) this task's last
+    // step again and again, which keeps the counts uniform.
+    for (int part = 0; part < 2; ++part) {
+      const int s0 = part == 0 ? 0 : nk - ahead, s1 = part == 0 ? nk - ahead : nk;
+      if (part == 1 && nx.e >= 0) {
+        // the next task's rows (their ids were fetched a task ago)
+        setup_weight_loads(nx, ld);
+        setup_token_loads(ax_next, ld);
+        next_at = ld.first;
+        next_active = half_in_use(ax_next);
+      } else if (part == 1) {
+        next_at = (next_at > 0 ? next_at : K) - kStepBytes;
+        advance = 0;
+      }
+      if (active && ld.stream)
+        steps(std::true_type{}, std::true_type{}, s0, s1);
+      else if (active)
+        steps(std::true_type{}, std::false_type{}, s0, s1);
+      else if (ld.stream)
+        steps(std::false_type{}, std::true_type{}, s0, s1);
+      else
+        steps(std::false_type{}, std::false_type{}, s0, s1);
     }
-    // Before the stores the coming step's loads have landed, and the next wait need not get past them.
-    wait_all_but(ahead - 1);
-    fresh = true;
     if (active) epilogue(tk, aux[par], acc);
     if (nx.e < 0) break;
+    active = next_active;
     tk = nx;
-    ld = nld;
     nx = n2;
     n2 = next_task();
     par = par + 1 < 3 ? par + 1 : 0;
@@ -459,16 +495,20 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.sorted_ids = a.sorted_token_ids;
   p.expert_ids = a.expert_ids;
   p.npp = a.num_tokens_post_padded;
-  p.P = a.num_pairs;
-  p.row_div = a.row_div;
+  p.P = (int)a.num_pairs;
+  p.row_of = divider(a.row_div);
   p.E = a.num_experts;
   p.N = a.n;
   p.K = a.k;
   p.B = a.block_size;
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 63) / 64 : (a.n + kCh - 1) / kCh;
+  p.rotate = rotation_mask(a.k);
   p.out = a.out;
   const int grid = device_cu_count() / kXcds * kXcds;
-  hipLaunchKernelGGL((gemm_narrow_kernel<MODE, TOK>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
+  if (a.k >= Shape<TOK>::kStages * kStepBytes)
+    hipLaunchKernelGGL((gemm_narrow_kernel<MODE, TOK, true>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
+  else
+    hipLaunchKernelGGL((gemm_narrow_kernel<MODE, TOK, false>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
   return hipGetLastError();
 }
 
