@@ -64,6 +64,11 @@ struct StreamParams {
   int B;
   int64_t cap;        // entries of sorted_ids
   int wave_capacity;  // wavefronts of this kernel the device holds at a time
+  // Rows of a multiple of 4096 bytes have one window of all of them on a few memory channels: there the wavefronts of an
+  // expert start their reductions (int32 sums, exact in any order) at window expert & rotate and wrap around.  Layer us of 129
+  // experts of 4096 x 1408 (skewed routing) at 5 / 8 / 12 / 16 tokens 75.9 / 91.9 / 101.0 / 113.9 -> 72.0 / 89.4 / 98.1 /
+  // 109.8; with the tile pair in it too, half of that.
+  int rotate;
   int round_even;     // in-kernel quantisation: ties to even instead of away from zero
   void* out;
 };
@@ -118,10 +123,11 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
   const int st_base = ld_row * kWinBytes + ((ld_chunk ^ ld_row) * 16);  // ^ (j % 4) * 64, + j * 1024
   const int rd_base = col * kWinBytes + ((grp ^ col) * 16);             // ^ u * 64, + t * 4096
 
-  // The wavefront walks windows (pair 0, k 0), (pair 0, k 256), ..., (pair 1, k 0), ... ; `fq`/`fk`
+  // The wavefront walks windows (pair 0, k 0), (pair 0, k 256), ..., (pair 1, k 0), ... (from `start` on and around); `fq`/`fk`
   // track the window whose weights are being fetched (`fk` also the one whose activation rows are),
   // `cq`/`ck` the one being consumed.
-  int fq = 0, wk = 0, fk = 0;
+  const int start = (e & p.rotate) * kWinBytes;  // (see StreamParams)
+  int fq = 0, wk = start, fk = start;
   auto fetch_weights = [&](Window<NS>& win) {
     int wrow[kTiles];
     bool wok[kTiles];
@@ -133,10 +139,8 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
       win.w[j] = chunk_in ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(src)) : v4i{0, 0, 0, 0};
     }
     wk += kWinBytes;
-    if (wk >= K) {
-      wk = 0;
-      ++fq;
-    }
+    if (wk >= K) wk = 0;
+    if (wk == start) ++fq;
   };
 
   // The weights of the first two windows depend on nothing but the expert of the block: they are
@@ -421,6 +425,7 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.N = a.n;
   p.K = a.k;
   p.B = a.block_size;
+  p.rotate = a.k % 4096 == 0 ? 15 : 0;
   p.out = a.out;
   p.cap = a.sorted_cap;
   const int total_pairs = MODE == kGateUpSilu ? a.n / 2 / 16 : (a.n / 16 + kTiles - 1) / kTiles;

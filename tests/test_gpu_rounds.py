@@ -37,7 +37,7 @@ def test_pieces_of_tiles_of_several_sizes(pra, oracle, variant, counts):
     _check(pra, oracle, variant, counts, 256, 768, B=128)
 
 
-@pytest.mark.parametrize("variant", ["narrow", "tile_deep", "tile_wide"])
+@pytest.mark.parametrize("variant", ["narrow", "tile_deep", "tile_wide", "stream"])
 @pytest.mark.parametrize("K", [4096, 8192])
 def test_tasks_that_start_at_different_steps(pra, oracle, variant, K):
     # 70 experts: the starting step wraps around twice
