@@ -322,6 +322,8 @@ bool gemm_tile_prefers_deep(const GemmArgs& a);
 int gemm_tile_geometry(const GemmArgs& a);  // kTileWide or kTileDeep (kTileRing on demand): what a launch of the family would use
 bool gemm_wide_supports(const GemmArgs& a);
 hipError_t launch_gemm_wide(const GemmArgs& a, hipStream_t stream);
+bool gemm_deep_supports(const GemmArgs& a);
+hipError_t launch_gemm_deep(const GemmArgs& a, hipStream_t stream);
 hipError_t launch_gemm_narrow(const GemmArgs& a, hipStream_t stream);
 bool gemm_narrow_supports(const GemmArgs& a);
 

@@ -1,32 +1,31 @@
-// Grouped int8 GEMM for gfx950, LDS-tiled family: its deep tiles (around a hundred routed rows per expert), the
-// ring pipeline and the choice of the family's kernel; the wide tiles are in gemm_wide.hip.
+// Grouped int8 GEMM for gfx950, LDS-tiled family: the choice of the family's kernel (wide tiles in gemm_wide.hip, deep ones
+// in gemm_deep.hip) and the ring pipeline.
+//
+// Ring pipeline for the 256 x 256 tile (the geometry kTileRing; never chosen by itself, kept as a
+// measured alternative to the wide tiles): reduction steps of 64 bytes through a ring
+// of four 32 KB stages (16 KB of weight rows, then 16 KB of token rows), every stage filled three
+// steps before it is multiplied, so that up to 96 KB of loads are in flight per compute unit
+// against the 64 KB of a two-stage pipeline.  LDS rows are 64 bytes (four 16-byte chunks); a
+// wave-level load covers 16 rows.
 //
 // Persistent workgroups (one per CU, 512 threads = 8 wavefronts) walk a list of tiles.  A tile is
 // a run of 64-row moe_align sub-blocks of ONE expert (aligned to the start of the expert's segment)
-// x 256 weight rows (output channels); the reduction runs in steps of 128 bytes.  The MFMA
-// (v_mfma_i32_32x32x32_i8) is used "transposed" (A operand = weight rows, B operand = token rows),
-// so a lane ends up with runs of 4 consecutive channels of one token.
+// x 256 weight rows (output channels).  The MFMA (v_mfma_i32_32x32x32_i8) is used "transposed" (A operand =
+// weight rows, B operand = token rows), so a lane ends up with runs of 4 consecutive channels of one token.
 //
-// Deep tiles hold up to 128 token rows, with a ring of three 48 KB stages and loads two steps ahead.  With
-// few rows per expert a step holds little arithmetic and the kernel is bound by the weight stream
-// from HBM, i.e. by the bytes a compute unit keeps in flight.  All eight wavefronts multiply in
-// every task: with two active sub-blocks wavefront w owns sub-block w / 4 and a quarter of the
-// channels, with one an eighth of the channels.
+// One barrier per step, placed in the MIDDLE of the step: the operands of the step's second
+// 32-byte half are read while the first half multiplies; once they are in registers the whole
+// stage has been consumed, so the barrier both frees it for the loads four steps ahead and
+// publishes the next stage, whose first-half operands are then read while the second half
+// multiplies.  The matrix pipe therefore always has eight MFMAs with their operands in registers
+// on either side of the barrier.
 //
-// Both operands go global -> LDS directly (global_load_lds_dwordx4: no staging registers, no
-// ds_write), with one s_barrier per step and explicit vmcnt waits.  Every wavefront-level load
-// covers 8 rows x 128 contiguous bytes, i.e. whole cache lines.  LDS rows are 128 bytes; the 16-byte
-// chunk index is XOR-swizzled with row bits so that the MFMA-layout reads (32 consecutive rows, same
-// chunk) spread over all banks; because a load fills LDS linearly the swizzle is applied to the
-// global source address of each lane.
-//
-// The tile list is derived inside the kernel from expert_ids (tile_list.hpp).  Tasks (tile, channel tile) are numbered
-// channel tile fastest and split into 8 contiguous ranges, one per XCD (workgroup id % 8), so that the workgroups running
-// on one XCD at a time share token rows and expert weights in that XCD's L2.  The first loads of the next task are issued
-// before the epilogue of the current one.  GEMMs of 64 experts of 4096 x 1408 with 64 rows each, with the starting steps of
-// rotation_mask: 150 -> 132 us (gate_up, K = 4096).
-#include <type_traits>
-
+// Measured against the two-stage pipeline that the wide tiles had before gemm_wide.hip, on 65536 routed rows x 128 experts (gate_up 4096 x 2048,
+// down 2048 x 2048): same results bit for bit, 7-10 % slower.  A lane's 16-byte load takes a
+// quarter of a 64-byte row, so every 128-byte line is requested from L2 twice (the request count
+// per launch doubles, the bytes fetched from HBM stay), and the path from L2 into LDS, not the
+// depth of the pipeline, is what bounds the loads of this tile.
+#include "lds_loads.hpp"
 #include "tile_list.hpp"
 
 namespace moe_i8 {
@@ -35,14 +34,12 @@ namespace {
 constexpr int kThreads = kTileThreads;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kBN = 256;       // weight rows per tile
-constexpr int kBK = 128;       // reduction bytes per step
-constexpr int kTokOffset = kBN * kBK;
-
-constexpr int kTileTok = 128;                          // token rows per tile
-constexpr int kSlots = 3;                              // LDS stages
-constexpr int kStageBytes = (kBN + kTileTok) * kBK;    // 48 KB
-constexpr int kMaxTiles = 2048;                        // of a launch
-constexpr int kTokLoads = kTileTok / 64;               // wave-level loads of 8 token rows per wavefront and step
+constexpr int kRingBK = 64;
+constexpr int kRingSlots = 4;
+constexpr int kRingHalf = kBN * kRingBK;    // 16 KB
+constexpr int kRingStage = 2 * kRingHalf;   // 32 KB
+constexpr int kRingMaxTiles = 6144;         // of a launch
+constexpr int kRingLoads = 4;               // wave-level loads per wavefront and step
 
 struct TileParams {
   const int8_t* a_q;
@@ -58,67 +55,15 @@ struct TileParams {
   int K;
   int B;
   TileListArgs tiles;
-  int rotate;  // mask of the reduction step that a task starts at (rotation_mask)
   int ascend;  // expert_ids is known to ascend over the used blocks (it comes from moe_align)
   void* out;
 };
-
-// s_waitcnt with only the vector-memory counter constrained (gfx9 encoding: vmcnt = bits 3:0 and
-// 15:14; expcnt 6:4 and lgkmcnt 11:8 left at their maximum).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
-}
-
-// 16 bytes per lane from global memory straight into LDS: lane i lands at lds_addr + 16 * i
-// (lds_addr is wave-uniform and goes through M0).  Issued as inline assembly so that the waits are
-// the explicit vmcnt waits of the ring below and not a conservative vmcnt(0) before every LDS read.
-// The source is a wave-uniform base (SGPR pair) plus an unsigned 32-bit byte offset per lane.
-__device__ __forceinline__ void load_to_lds_16(const int8_t* base, uint32_t offset, uint32_t lds_addr) {
-  const uint64_t b = reinterpret_cast<uint64_t>(base);
-  // readfirstlane yields a signed int: go through uint32_t so that the low half is not sign-extended
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  const uint64_t ub = (uint64_t)lo | ((uint64_t)hi << 32);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(ub)
-               : "memory", "m0");
-}
-
-// The same with the non-temporal hint: for launches in which no expert holds more rows than one
-// tile, so that every weight row is read by exactly one workgroup.  Streamed that way the weights
-// do not displace the token rows from L2 (measured: 5-8 % on launches bound by the weight stream;
-// a loss as soon as a second tile of an expert would have found the rows in L2).
-__device__ __forceinline__ void load_to_lds_16_stream(const int8_t* base, uint32_t offset, uint32_t lds_addr) {
-  const uint64_t b = reinterpret_cast<uint64_t>(base);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  const uint64_t ub = (uint64_t)lo | ((uint64_t)hi << 32);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-               :
-               : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(ub)
-               : "memory", "m0");
-}
-
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-  return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)p);
-}
-
-__device__ __forceinline__ int swizzle_of_row(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
 struct Task {
   int e;          // expert; -1 = no more work, -2 = tile of ignored expert ids
   int n0, n1;     // its channels (gate_up: gate channels)
   int64_t slot0;  // first slot of the tile in sorted_ids
   int nsub;       // active 64-row sub-blocks (1..4)
-};
-
-struct TaskLoads {
-  const int8_t* wbase;  // weights of the task's expert (wave-uniform)
-  uint32_t woff[4];     // per lane: byte offset of its chunk of weight row i from wbase
-  uint32_t xoff[4];     // per lane: byte offset of its chunk of token row i from a_q
-  int first;            // byte offset of the first reduction step
 };
 
 // The n-th weight row of a tile's 256; the last channel again behind the end of the task.
@@ -132,417 +77,9 @@ __device__ __forceinline__ int weight_row(const Task& tk, int N, int row) {
   }
 }
 
-// Weights: lane fills LDS slot (lane & 7) of row 32 * wave + 8 * i + (lane >> 3): it fetches the logical
-// chunk (lane & 7) ^ swizzle(row) of that row, and swizzle(row) = (lane >> 3) ^ (i & 1).  Token rows
-// likewise, of row (8 * kTokLoads) * wave + 8 * i + (lane >> 3).
-template <int MODE>
-__device__ __forceinline__ void setup_loads(const TileParams& p, const Task& tk, int wave, int lane, TaskLoads& ld) {
-  const int K = p.K;
-  ld.first = (tk.e & p.rotate) * kBK;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = 32 * wave + 8 * i + (lane >> 3);
-    const int chunk = ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;
-    const int n = weight_row<MODE>(tk, p.N, row);
-    ld.woff[i] = (uint32_t)n * (uint32_t)K + chunk;
-    if (i < kTokLoads) {
-      const int trow = 8 * kTokLoads * wave + 8 * i + (lane >> 3);
-      uint32_t arow = 0;
-      if ((trow >> 6) < tk.nsub) {
-        const int32_t tok = p.sorted_ids[tk.slot0 + trow];
-        if (tok >= 0 && tok < p.P) arow = (uint32_t)(tok / p.row_div);
-      }
-      ld.xoff[i] = arow * (uint32_t)K + chunk;
-    }
-  }
-  ld.wbase = p.w + (int64_t)tk.e * p.N * K;
-}
-
-// The token loads are issued regardless of the active sub-blocks (rows of inactive ones fetch row 0), so that
-// every wavefront has the same number of loads in flight per step and the counted waits of the ring hold for all.
-template <bool NT>
-__device__ __forceinline__ void issue_stage_loads(const TaskLoads& ld, const int8_t* a_q, uint32_t stage_addr,
-                                                  int wave, int koff) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (NT)
-      load_to_lds_16_stream(ld.wbase + koff, ld.woff[i], stage_addr + (wave * 4 + i) * 1024);
-    else
-      load_to_lds_16(ld.wbase + koff, ld.woff[i], stage_addr + (wave * 4 + i) * 1024);
-  }
-#pragma unroll
-  for (int i = 0; i < kTokLoads; ++i)
-    load_to_lds_16(a_q + koff, ld.xoff[i], stage_addr + kTokOffset + (wave * kTokLoads + i) * 1024);
-}
-
-struct TileReads {
-  int w_ld[4];
-  int x_ld[2];
-  int chunk[4];  // swizzled byte offset of logical chunk 2 * kk + (lane >> 5)
-};
-
-// How the eight wavefronts share a task.  With two active sub-blocks (NCI = 2) wavefront w owns sub-block w / 4
-// and a quarter of the channels (two MFMA tiles of 32 weight rows, twice 32 token rows), with one (NCI = 1) an
-// eighth of the channels: every wavefront multiplies in every task, so a tile with few rows costs its loads
-// and not the serial MFMA chain of the one or two wavefronts its rows would otherwise belong to.
-template <int MODE, int NCI>
-__device__ __forceinline__ void make_reads(int wave, int lane, TileReads& rd) {
-  constexpr int kParts = 8 / NCI;
-  const int tg = wave / kParts;
-  const int cpart = wave % kParts;
-  const int lrow = lane & 31;
-#pragma unroll
-  for (int ci = 0; ci < NCI; ++ci) {
-    int row;
-    if constexpr (MODE == kGateUpSilu) {
-      // LDS rows 0..127 hold gate channels, 128..255 the matching up channels
-      if constexpr (NCI == 2)
-        row = ci * 128 + cpart * 32 + lrow;
-      else
-        row = (lrow < 16 ? 0 : 128 - 16) + cpart * 16 + lrow;  // 16 gate rows, then their 16 up rows
-    } else {
-      row = cpart * (NCI * 32) + ci * 32 + lrow;
-    }
-    rd.w_ld[ci] = row * kBK;
-  }
-#pragma unroll
-  for (int tj = 0; tj < 2; ++tj) rd.x_ld[tj] = kTokOffset + (tg * 64 + tj * 32 + lrow) * kBK;
-}
-
-template <int NCI>
-__device__ __forceinline__ void multiply_stage(const TileReads& rd, const char* stage, v16i (&acc)[NCI][2]) {
-  v4i a[4][NCI], b[4][2];
-  // reads in the order the MFMAs consume them: b0 a0 | b1 | a1 | a2 | a3 per 32-byte sub-step
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    b[kk][0] = *reinterpret_cast<const v4i*>(stage + rd.x_ld[0] + rd.chunk[kk]);
-    a[kk][0] = *reinterpret_cast<const v4i*>(stage + rd.w_ld[0] + rd.chunk[kk]);
-    b[kk][1] = *reinterpret_cast<const v4i*>(stage + rd.x_ld[1] + rd.chunk[kk]);
-#pragma unroll
-    for (int ci = 1; ci < NCI; ++ci) a[kk][ci] = *reinterpret_cast<const v4i*>(stage + rd.w_ld[ci] + rd.chunk[kk]);
-  }
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-    for (int ci = 0; ci < NCI; ++ci)
-#pragma unroll
-      for (int tj = 0; tj < 2; ++tj)
-        acc[ci][tj] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[kk][ci], b[kk][tj], acc[ci][tj], 0, 0, 0);
-}
-
-// acc[ci][tj][4q + r] is weight row 32 * ci + 8q + 4 * (lane >> 5) + r of the wavefront's MFMA tiles
-// and token row tg * 64 + tj * 32 + (lane & 31) of the tile.  The bf16 results are transposed through
-// an LDS region private to the wavefront (at most 8 KB) so that the global stores are 16 bytes per
-// lane and cover whole runs of an output row (rows of 16-byte chunks, chunk index XOR-swizzled with
-// the row so that neither the 8-byte writes nor the 16-byte reads pile up on a bank).
-template <int CPR>
-__device__ __forceinline__ int staging_swizzle(int row) {
-  // rows of CPR chunks: 16 / CPR rows span all banks, rows that far apart must differ in the swizzle
-  if constexpr (CPR >= 8)
-    return row & (CPR - 1);
-  else if constexpr (CPR == 4)
-    return (row >> 2) & 3;
-  else
-    return (row >> 3) & 1;
-}
-
-template <int MODE, int NCI>
-__device__ __forceinline__ void epilogue(const TileParams& p, const Task& tk, int wave, int lane, v16i (&acc)[NCI][2],
-                                         char* wave_lds, float* wave_scales) {
-  constexpr int kParts = 8 / NCI;
-  const int tg = wave / kParts;
-  const int cpart = wave % kParts;
-  const int lrow = lane & 31;
-  const int lhalf = lane >> 5;
-  const int inter = p.N / 2;
-  const int limit = min(tk.n1, MODE == kGateUpSilu ? inter : p.N);  // behind the task's channels
-  int32_t tok[2];
-#pragma unroll
-  for (int tj = 0; tj < 2; ++tj) {
-    tok[tj] = p.sorted_ids[tk.slot0 + tg * 64 + tj * 32 + lrow];
-    if (tok[tj] < 0 || tok[tj] >= p.P) tok[tj] = -1;
-  }
-  if constexpr (MODE == kAccI32) {
-#pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      if (tok[tj] < 0) continue;
-      int32_t* out = static_cast<int32_t*>(p.out) + (int64_t)tok[tj] * p.N;
-#pragma unroll
-      for (int ci = 0; ci < NCI; ++ci)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = tk.n0 + cpart * (NCI * 32) + ci * 32 + 8 * q + 4 * lhalf;
-          if (n < limit)
-            *reinterpret_cast<v4i*>(out + n) =
-                v4i{acc[ci][tj][4 * q], acc[ci][tj][4 * q + 1], acc[ci][tj][4 * q + 2], acc[ci][tj][4 * q + 3]};
-        }
-    }
-  } else if constexpr (MODE == kDown) {
-    constexpr int kChannels = NCI * 32;  // of this wavefront
-    constexpr int CPR = NCI * 4;         // 16-byte chunks per staged row
-    constexpr int kRowBytes = CPR * 16;
-    const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
-    const int n0 = tk.n0 + cpart * kChannels;  // first channel of this wavefront
-    // The channel scales of this wavefront go through LDS: read from there they do not count
-    // as vector-memory loads, so the second half's arithmetic does not have to wait for the first
-    // half's stores (the vector-memory counter retires in order).
-    if (2 * lane < kChannels) {
-      const int n = n0 + 2 * lane;
-      *reinterpret_cast<float2*>(wave_scales + 2 * lane) =
-          n < limit ? *reinterpret_cast<const float2*>(wsc + n) : make_float2(0.0f, 0.0f);
-    }
-    float as[2], rw[2];
-#pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      as[tj] = tok[tj] >= 0 ? p.a_scale[tok[tj] / p.row_div] : 0.0f;
-      rw[tj] = tok[tj] >= 0 ? (p.row_weight ? p.row_weight[tok[tj]] : 1.0f) : 0.0f;
-    }
-#pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      // 32 token rows x kChannels channels
-#pragma unroll
-      for (int ci = 0; ci < NCI; ++ci) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float4 ws = *reinterpret_cast<const float4*>(wave_scales + ci * 32 + 8 * q + 4 * lhalf);
-          const int v[4] = {acc[ci][tj][4 * q], acc[ci][tj][4 * q + 1], acc[ci][tj][4 * q + 2], acc[ci][tj][4 * q + 3]};
-          *reinterpret_cast<uint2*>(wave_lds + lrow * kRowBytes + (((ci * 4 + q) ^ staging_swizzle<CPR>(lrow)) * 16) +
-                                    lhalf * 8) = down_epilogue4(v, as[tj], ws, rw[tj]);
-        }
-      }
-      // Before the first stores everything this wavefront has in flight is complete (its share of
-      // the next tile's first stage, issued during the last step, and the loads above), so the
-      // stores are the only vector-memory work still pending when the next tile starts.
-      if (tj == 0) wait_vmcnt<0>();
-#pragma unroll
-      for (int r = 0; r < CPR / 2; ++r) {
-        const int row = r * (64 / CPR) + lane / CPR;
-        const int chunk = lane % CPR;
-        const uint4 v =
-            *reinterpret_cast<const uint4*>(wave_lds + row * kRowBytes + ((chunk ^ staging_swizzle<CPR>(row)) * 16));
-        const int32_t t = __shfl(tok[tj], row);
-        const int n = n0 + chunk * 8;
-        if (t >= 0 && n < limit)
-          __builtin_nontemporal_store(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}, reinterpret_cast<v4i*>(static_cast<uint16_t*>(p.out) + (int64_t)t * p.N + n));
-      }
-    }
-  } else {
-    constexpr int kChannels = NCI * 16;  // activation channels of this wavefront
-    constexpr int CPR = NCI * 2;
-    constexpr int kRowBytes = CPR * 16;
-    const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
-    const int n0 = tk.n0 + cpart * kChannels;  // first gate channel of this wavefront
-    // 64 token rows x kChannels channels
-#pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const float as = tok[tj] >= 0 ? p.a_scale[tok[tj] / p.row_div] : 0.0f;
-      const int row = tj * 32 + lrow;
-#pragma unroll
-      for (int c = 0; c < CPR; ++c) {
-        // gate rows sit in MFMA tile gi at 8 * gq, the matching up rows in tile ui at 8 * uq
-        constexpr int kHalfTiles = NCI >= 2 ? NCI / 2 : 1;
-        const int gi = NCI >= 2 ? c / 4 : 0;
-        const int gq = NCI >= 2 ? c % 4 : c;
-        const int ui = NCI >= 2 ? gi + kHalfTiles : 0;
-        const int uq = NCI >= 2 ? gq : c + 2;
-        const int n = n0 + c * 8 + 4 * lhalf;
-        const int ns = n < inter ? n : 0;
-        const float4 wg = *reinterpret_cast<const float4*>(wsc + ns);
-        const float4 wu = *reinterpret_cast<const float4*>(wsc + inter + ns);
-        const int g[4] = {acc[gi][tj][4 * gq], acc[gi][tj][4 * gq + 1], acc[gi][tj][4 * gq + 2], acc[gi][tj][4 * gq + 3]};
-        const int u[4] = {acc[ui][tj][4 * uq], acc[ui][tj][4 * uq + 1], acc[ui][tj][4 * uq + 2], acc[ui][tj][4 * uq + 3]};
-        *reinterpret_cast<uint2*>(wave_lds + row * kRowBytes + ((c ^ staging_swizzle<CPR>(row)) * 16) + lhalf * 8) =
-            silu_mul_epilogue4(g, u, as, wg, wu);
-      }
-    }
-    wait_vmcnt<0>();  // as in the down epilogue: only the stores below stay pending
-#pragma unroll
-    for (int r = 0; r < CPR; ++r) {
-      const int row = r * (64 / CPR) + lane / CPR;
-      const int chunk = lane % CPR;
-      const uint4 v =
-          *reinterpret_cast<const uint4*>(wave_lds + row * kRowBytes + ((chunk ^ staging_swizzle<CPR>(row)) * 16));
-      const int32_t t = __shfl(tok[(r * (64 / CPR)) >> 5], row & 31);
-      const int n = n0 + chunk * 8;
-      if (t >= 0 && n < limit)
-        __builtin_nontemporal_store(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}, reinterpret_cast<v4i*>(static_cast<uint16_t*>(p.out) + (int64_t)t * inter + n));
-    }
-  }
-}
-
-template <int MODE>
-__global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileParams p) {
-  __shared__ __align__(16) char stages[kSlots * kStageBytes];
-  __shared__ TileList<kMaxTiles> list;
-  __shared__ __align__(16) float channel_scales[kWaves * 128];
-
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int nk = p.K / kBK;
-
-  const int xcd = blockIdx.x % kXcds;
-  const TileRange range = p.ascend ? build_ascending(p.tiles, xcd, reinterpret_cast<int*>(stages), list)
-                                   : build_any_order(p.tiles, *p.npp / p.B, xcd, reinterpret_cast<int*>(stages), list);
-  const int sub_per_block = p.B / 64;
-  const int total = range.tiles * p.tiles.ntiles;
-  const int per_xcd = (total + kXcds - 1) / kXcds;
-  const int my_tasks = min(per_xcd, max(total - xcd * per_xcd, 0));
-  const int stride = gridDim.x / kXcds;
-
-  // ---- MFMA operand reads: lane feeds row (lane & 31), 16-byte chunk 2 * kk + (lane >> 5) ----
-  const int lsw = swizzle_of_row(lane & 31);
-  const int lhalf = lane >> 5;
-  TileReads rd;
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) rd.chunk[kk] = ((2 * kk + lhalf) ^ lsw) * 16;
-
-  const uint32_t stage0 = lds_address(stages);
-
-  auto decode = [&](int it) {
-    Task tk;
-    tk.e = -1;
-    tk.n0 = tk.n1 = 0;
-    tk.slot0 = 0;
-    tk.nsub = 0;
-    // a piece is a part of the tile's channels
-    const TaskPiece tp = piece_at(it, my_tasks, stride);
-    if (tp.task >= 0) {
-      constexpr int kOut = MODE == kGateUpSilu ? kBN / 2 : kBN;
-      const uint2 d = look_up_task(p.tiles, list, range, xcd * per_xcd + tp.task);
-      const int width = kOut / tp.pieces;
-      tk.n0 = (int)(d.y >> 16) * kOut + tp.piece * width;
-      tk.n1 = tk.n0 + width;
-      tk.slot0 = (int64_t)(d.x & 0xffffu) * p.B;
-      tk.nsub = (int)((d.x >> 16) & 15u) * sub_per_block;
-      tk.e = tk.nsub > 0 ? (int)(d.y & 0xffffu) : -2;
-    }
-    return tk;
-  };
-
-  // Does any run of blocks make more than one tile?  (A tile that is not the first of its group, or a
-  // group of more than one.)  If none in this XCD's part does, every weight row is read by one workgroup only and is
-  // fetched with the non-temporal hint; the choice is made once per workgroup so that the step loop
-  // carries no test.
-  bool shared_local = false;
-  for (int g = t; g < range.hi - range.lo; g += kThreads) shared_local |= (list.desc[g] >> 20) != (1u << 4);  // rank 0, group size 1
-  const bool weights_shared = __syncthreads_or(shared_local ? 1 : 0) != 0;
-
-  auto run = [&](auto nt_tag) {
-  constexpr bool NT = decltype(nt_tag)::value;
-  int it = blockIdx.x / kXcds;
-  Task tk = decode(it);
-  while (tk.e == -2) tk = decode(it += stride);
-  if (tk.e < 0) return;
-  TaskLoads ld;
-  setup_loads<MODE>(p, tk, wave, lane, ld);
-  int slot = 0;  // stage of the step being multiplied
-  // The scratch of the tile list lived in the stage memory; everybody is past it (the builder ends
-  // with a barrier), so the first stages can be filled now.
-  auto at = [&](const TaskLoads& ld, int s) {  // byte offset of step s
-    const int k = ld.first + s * kBK;
-    return k < p.K ? k : k - p.K;
-  };
-  issue_stage_loads<NT>(ld, p.a_q, stage0, wave, at(ld, 0));
-  issue_stage_loads<NT>(ld, p.a_q, stage0 + kStageBytes, wave, at(ld, 1));
-  constexpr int kLoadsPerStep = 4 + kTokLoads;  // per wavefront
-
-  bool stores_pending = false;
-  while (true) {
-    // look ahead: the first loads of the next task are issued during the last step(s) of this one
-    int nit = it + stride;
-    Task nx = decode(nit);
-    while (nx.e == -2) nx = decode(nit += stride);
-    TaskLoads nld = ld;
-    if (nx.e >= 0) setup_loads<MODE>(p, nx, wave, lane, nld);
-
-    // NCI = MFMA tiles of 32 weight rows per wavefront
-    auto run_task = [&](auto nci_tag) {
-      constexpr int NCI = decltype(nci_tag)::value;
-      v16i acc[NCI][2];
-#pragma unroll
-      for (int ci = 0; ci < NCI; ++ci)
-#pragma unroll
-        for (int tj = 0; tj < 2; ++tj)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[ci][tj][r] = 0;
-      make_reads<MODE, NCI>(wave, lane, rd);
-      for (int s = 0; s < nk; ++s) {
-        // This wavefront's loads of step s have landed ...  A wavefront that has just run an
-        // epilogue waited for all its loads there and only has the epilogue's stores pending: it
-        // lets them drain behind the first step instead of stalling on them.
-        // in flight behind step s: the loads of step s + 1 (issued one step ago), if there is one
-        if (s > 0 || !stores_pending) {
-          if (s + 1 < nk || nx.e >= 0)
-            wait_vmcnt<kLoadsPerStep>();
-          else
-            wait_vmcnt<0>();
-        }
-        // ... and so have everybody's; everybody is also done reading the stage of the step before,
-        // which is the one to fill next
-        __builtin_amdgcn_s_barrier();
-        constexpr int kAhead = kSlots - 1;
-        int fill = slot + kAhead;
-        if (fill >= kSlots) fill -= kSlots;
-        const uint32_t fill_addr = stage0 + fill * kStageBytes;
-        if (s + kAhead < nk)
-          issue_stage_loads<NT>(ld, p.a_q, fill_addr, wave, at(ld, s + kAhead));
-        else if (nx.e >= 0)
-          issue_stage_loads<NT>(nld, p.a_q, fill_addr, wave, at(nld, s + kAhead - nk));
-        multiply_stage<NCI>(rd, stages + slot * kStageBytes, acc);
-        slot = slot + 1 == kSlots ? 0 : slot + 1;
-      }
-      // everybody is done reading the stage of the last step: it becomes the epilogue's staging area
-      // (the next task's first loads went to the other stages)
-      __builtin_amdgcn_s_barrier();
-      const int last = slot == 0 ? kSlots - 1 : slot - 1;
-      epilogue<MODE, NCI>(p, tk, wave, lane, acc, stages + last * kStageBytes + wave * 8192 / (4 / NCI),
-                            channel_scales + wave * 128);
-      stores_pending = MODE != kAccI32;
-    };
-    if (tk.nsub >= 2)
-      run_task(std::integral_constant<int, 2>{});
-    else
-      run_task(std::integral_constant<int, 1>{});
-    if (nx.e < 0) break;
-    tk = nx;
-    ld = nld;
-    it = nit;
-  }
-  wait_vmcnt<0>();
-  };
-  if (weights_shared)
-    run(std::false_type{});
-  else
-    run(std::true_type{});
-}
-
-// ---------------------------------------------------------------------------------------------
-// Ring pipeline for the 256 x 256 tile (the geometry kTileRing; never chosen by itself, kept as a
-// measured alternative to the two-stage pipeline above): reduction steps of 64 bytes through a ring
-// of four 32 KB stages (16 KB of weight rows, then 16 KB of token rows), every stage filled three
-// steps before it is multiplied, so that up to 96 KB of loads are in flight per compute unit
-// against the 64 KB of the two-stage pipeline.  LDS rows are 64 bytes (four 16-byte chunks); a
-// wave-level load covers 16 rows.
-//
-// One barrier per step, placed in the MIDDLE of the step: the operands of the step's second
-// 32-byte half are read while the first half multiplies; once they are in registers the whole
-// stage has been consumed, so the barrier both frees it for the loads four steps ahead and
-// publishes the next stage, whose first-half operands are then read while the second half
-// multiplies.  The matrix pipe therefore always has eight MFMAs with their operands in registers
-// on either side of the barrier.
-//
-// Measured against the two-stage pipeline that the wide tiles had before gemm_wide.hip, on 65536 routed rows x 128 experts (gate_up 4096 x 2048,
-// down 2048 x 2048): same results bit for bit, 7-10 % slower.  A lane's 16-byte load takes a
-// quarter of a 64-byte row, so every 128-byte line is requested from L2 twice (the request count
-// per launch doubles, the bytes fetched from HBM stay), and the path from L2 into LDS, not the
-// depth of the pipeline, is what bounds the loads of this tile.
-constexpr int kRingBK = 64;
-constexpr int kRingSlots = 4;
-constexpr int kRingHalf = kBN * kRingBK;    // 16 KB
-constexpr int kRingStage = 2 * kRingHalf;   // 32 KB
-constexpr int kRingMaxTiles = 6144;         // of a launch
-constexpr int kRingLoads = 4;               // wave-level loads per wavefront and step
+// The chunk index of a staged row of eight 16-byte chunks is XOR-swizzled with the row so that neither the 8-byte writes nor the
+// 16-byte reads pile up on a bank.
+__device__ __forceinline__ int staging_swizzle(int row) { return row & 7; }
 
 // chunk swizzle of a 64-byte LDS row: 16 consecutive rows reading one logical chunk, and 8 rows
 // reading two neighbouring chunks, both spread over all banks
@@ -609,8 +146,10 @@ __device__ __forceinline__ void ring_multiply(const RingOperands& o, v16i (&acc)
 
 __device__ __forceinline__ void wait_lds_reads() { __builtin_amdgcn_s_waitcnt(0xC07F); }  // lgkmcnt(0), others free
 
-// The epilogue of the ring pipeline: the same arithmetic as `epilogue` with four MFMA tiles per
-// wavefront, staged through 4 KB per wavefront (32 token rows x 64 channels of bf16 at a time).
+// acc[ci][tj][4q + r] is weight row 32 * ci + 8q + 4 * (lane >> 5) + r of the wavefront's MFMA tiles
+// and token row tg * 64 + tj * 32 + (lane & 31) of the tile.  The bf16 results are transposed through
+// 4 KB of LDS per wavefront (32 token rows x 64 channels at a time) so that the global stores are 16 bytes per
+// lane and cover whole runs of an output row.
 template <int MODE>
 __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& tk, int wave, int lane, v16i (&acc)[4][2],
                                               char* wave_lds, float* wave_scales) {
@@ -643,7 +182,9 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
   } else if constexpr (MODE == kDown) {
     const float* wsc = p.w_scale + (int64_t)tk.e * p.N;
     const int n0 = tk.n0 + cpart * 128;  // first channel of this wavefront
-    // channel scales through LDS (see `epilogue`)
+    // The channel scales of this wavefront go through LDS: read from there they do not count
+    // as vector-memory loads, so the second half's arithmetic does not have to wait for the first
+    // half's stores (the vector-memory counter retires in order).
     {
       const int n = n0 + 2 * lane;
       *reinterpret_cast<float2*>(wave_scales + 2 * lane) =
@@ -666,7 +207,7 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
           const int q = c % 4;
           const float4 ws = *reinterpret_cast<const float4*>(wave_scales + ci * 32 + 8 * q + 4 * lhalf);
           const int v[4] = {acc[ci][tj][4 * q], acc[ci][tj][4 * q + 1], acc[ci][tj][4 * q + 2], acc[ci][tj][4 * q + 3]};
-          *reinterpret_cast<uint2*>(wave_lds + lrow * 128 + ((c ^ staging_swizzle<8>(lrow)) * 16) + lhalf * 8) =
+          *reinterpret_cast<uint2*>(wave_lds + lrow * 128 + ((c ^ staging_swizzle(lrow)) * 16) + lhalf * 8) =
               down_epilogue4(v, as[tj], ws, rw[tj]);
         }
         // everything this wavefront has in flight is complete before its first stores, which
@@ -676,7 +217,7 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
         for (int r = 0; r < 4; ++r) {
           const int row = r * 8 + lane / 8;
           const int chunk = lane % 8;
-          const uint4 v = *reinterpret_cast<const uint4*>(wave_lds + row * 128 + ((chunk ^ staging_swizzle<8>(row)) * 16));
+          const uint4 v = *reinterpret_cast<const uint4*>(wave_lds + row * 128 + ((chunk ^ staging_swizzle(row)) * 16));
           const int32_t t = __shfl(tok[tj], row);
           const int n = n0 + h * 64 + chunk * 8;
           if (t >= 0 && n < p.N)
@@ -706,7 +247,7 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
         const float4 wu = *reinterpret_cast<const float4*>(wsc + inter + ns);
         const int g[4] = {acc[gi][tj][4 * gq], acc[gi][tj][4 * gq + 1], acc[gi][tj][4 * gq + 2], acc[gi][tj][4 * gq + 3]};
         const int u[4] = {acc[ui][tj][4 * gq], acc[ui][tj][4 * gq + 1], acc[ui][tj][4 * gq + 2], acc[ui][tj][4 * gq + 3]};
-        *reinterpret_cast<uint2*>(wave_lds + lrow * 128 + ((c ^ staging_swizzle<8>(lrow)) * 16) + lhalf * 8) =
+        *reinterpret_cast<uint2*>(wave_lds + lrow * 128 + ((c ^ staging_swizzle(lrow)) * 16) + lhalf * 8) =
             silu_mul_epilogue4(g, u, as[tj], wg, wu);
       }
       if (tj == 0) wait_vmcnt<0>();  // as in the down epilogue: only the stores below stay pending
@@ -714,7 +255,7 @@ __device__ __forceinline__ void ring_epilogue(const TileParams& p, const Task& t
       for (int r = 0; r < 4; ++r) {
         const int row = r * 8 + lane / 8;
         const int chunk = lane % 8;
-        const uint4 v = *reinterpret_cast<const uint4*>(wave_lds + row * 128 + ((chunk ^ staging_swizzle<8>(row)) * 16));
+        const uint4 v = *reinterpret_cast<const uint4*>(wave_lds + row * 128 + ((chunk ^ staging_swizzle(row)) * 16));
         const int32_t t = __shfl(tok[tj], row);
         const int n = n0 + chunk * 8;
         if (t >= 0 && n < inter)
@@ -885,8 +426,8 @@ bool ring_supports(const GemmArgs& a) {
   return tiles <= kRingMaxTiles && blocks <= (int64_t)(kRingSlots * kRingStage / sizeof(int)) && blocks <= 65535;
 }
 
-template <int MODE, bool RING>
-hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
+template <int MODE>
+hipError_t launch_ring(const GemmArgs& a, hipStream_t stream) {
   TileParams p;
   p.a_q = a.a_q;
   p.a_scale = a.a_scale;
@@ -902,38 +443,18 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.B = a.block_size;
   p.tiles.expert_ids = a.expert_ids;
   p.tiles.E = a.num_experts;
-  p.tiles.per_tile = (RING ? 256 : kTileTok) / a.block_size;
+  p.tiles.per_tile = 256 / a.block_size;
   p.tiles.even = 0;
   p.tiles.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kBN - 1) / kBN;
   p.tiles.by_ntiles = divider(p.tiles.ntiles);
   p.tiles.by_per_tile = divider(p.tiles.per_tile);
   p.tiles.blocks = (int)(a.sorted_cap / a.block_size);
   p.tiles.identity = a.identity ? 1 : 0;
-  p.rotate = RING ? 0 : rotation_mask(a.k);
   p.ascend = a.expert_ids_ascend && a.num_experts <= 2 * kThreads ? 1 : 0;
   p.out = a.out;
   const int grid = device_cu_count() / kXcds * kXcds;
-  if constexpr (RING)
-    hipLaunchKernelGGL((gemm_ring_kernel<MODE>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
-  else
-    hipLaunchKernelGGL((gemm_tile_kernel<MODE>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
+  hipLaunchKernelGGL((gemm_ring_kernel<MODE>), dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
   return hipGetLastError();
-}
-
-bool deep_supports(const GemmArgs& a) {
-  // per-lane source offsets are 32-bit: one expert's weights and the activation matrix must each
-  // span less than 4 GiB
-  const int64_t act_rows = (a.num_pairs + a.row_div - 1) / a.row_div;
-  if (!((a.block_size == 64 || a.block_size == 128) && a.k % kBK == 0 && a.k >= kSlots * kBK && a.n % 16 == 0 &&
-        (int64_t)a.n * a.k < (1ll << 32) && act_rows * a.k < (1ll << 32)))
-    return false;
-  // The tile list lives in LDS.  A run of equal expert ids of L blocks makes ceil(L / blocks per
-  // tile) tiles; moe_align's ids ascend, so there is one run per expert.  Ids of unknown order could
-  // make every block a tile of its own.  While the list is built the block ids sit in the stages.
-  const int64_t blocks = (a.sorted_cap + a.block_size - 1) / a.block_size;
-  const int per_tile = kTileTok / a.block_size;
-  const int64_t tiles = a.expert_ids_ascend ? (blocks + per_tile - 1) / per_tile + a.num_experts : blocks;
-  return tiles <= kMaxTiles && blocks <= (int64_t)(kSlots * kStageBytes / sizeof(int)) && blocks <= 65535;
 }
 
 }  // namespace
@@ -941,9 +462,9 @@ bool deep_supports(const GemmArgs& a) {
 bool gemm_tile_supports(const GemmArgs& a) {
   switch (a.tile_geometry) {
     case kTileWide: return gemm_wide_supports(a);
-    case kTileDeep: return deep_supports(a);
+    case kTileDeep: return gemm_deep_supports(a);
     case kTileRing: return ring_supports(a);
-    default: return gemm_wide_supports(a) || deep_supports(a);
+    default: return gemm_wide_supports(a) || gemm_deep_supports(a);
   }
 }
 
@@ -962,27 +483,20 @@ int gemm_tile_geometry(const GemmArgs& a) {
   if (a.tile_geometry == kTileWide) return kTileWide;
   if (a.tile_geometry == kTileDeep) return kTileDeep;
   if (a.tile_geometry == kTileRing) return kTileRing;
-  return deep_supports(a) && (gemm_tile_prefers_deep(a) || !gemm_wide_supports(a)) ? kTileDeep : kTileWide;
+  return gemm_deep_supports(a) && (gemm_tile_prefers_deep(a) || !gemm_wide_supports(a)) ? kTileDeep : kTileWide;
 }
 
 hipError_t launch_gemm_tile(const GemmArgs& a, hipStream_t stream) {
   const int geometry = gemm_tile_geometry(a);
   if (geometry == kTileRing) {
     switch (a.mode) {
-      case kGateUpSilu: return launch_mode<kGateUpSilu, true>(a, stream);
-      case kDown: return launch_mode<kDown, true>(a, stream);
-      case kAccI32: return launch_mode<kAccI32, true>(a, stream);
+      case kGateUpSilu: return launch_ring<kGateUpSilu>(a, stream);
+      case kDown: return launch_ring<kDown>(a, stream);
+      case kAccI32: return launch_ring<kAccI32>(a, stream);
       default: return hipErrorInvalidValue;
     }
   }
-  if (geometry == kTileDeep) {
-    switch (a.mode) {
-      case kGateUpSilu: return launch_mode<kGateUpSilu, false>(a, stream);
-      case kDown: return launch_mode<kDown, false>(a, stream);
-      case kAccI32: return launch_mode<kAccI32, false>(a, stream);
-      default: return hipErrorInvalidValue;
-    }
-  }
+  if (geometry == kTileDeep) return launch_gemm_deep(a, stream);
   return launch_gemm_wide(a, stream);
 }
 

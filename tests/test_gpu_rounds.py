@@ -60,3 +60,16 @@ def test_narrow_layer_of_32_tokens(pra, H, I):
     kw = d.fused_experts_kwargs()
     got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="narrow")
     assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream"))
+
+
+@pytest.mark.parametrize("H", [384, 512, 640])
+@pytest.mark.parametrize("tokens", [120, 300, 1500])
+def test_deep_layer_around_the_depth_of_the_ring(pra, H, tokens):
+    # 3 to 5 steps in the first GEMM; several tasks per workgroup, so that a task's first steps run behind stores
+    from _util import inputs_mod
+
+    im = inputs_mod()
+    d = im.make_inputs(im.LayerShape("d", E=40, k=4, H=H, I=2560), tokens, seed=H + tokens).to(DEV)
+    kw = d.fused_experts_kwargs()
+    got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="tile_deep")
+    assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream"))
