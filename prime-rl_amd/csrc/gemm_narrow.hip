@@ -19,11 +19,14 @@
 //
 // A tile is TOK token rows (32 or 64: part of a moe_align block) x 128 weight rows; the reduction runs
 // in steps of 128 bytes and both operands reach LDS by global -> LDS loads (global_load_lds_dwordx4, no
-// staging registers).  Wavefront w multiplies weight rows [32 * (w % 4), + 32) of the tile with token half
-// w / 4, used "transposed" (A operand = weight rows), so a lane ends up with runs of 4 consecutive
-// channels of one token and stores its results straight from registers, 16 bytes at a time.  For the
-// gate_up GEMM the 32 weight rows of a wavefront are 16 gate rows and the 16 matching up rows, which
-// puts a gate value and its up value into the same lane.
+// staging registers).  Wavefront w multiplies weight rows [64 * (w % 2), + 64) of the tile with token rows
+// [16 * (w / 2), + 16), used "transposed" (A operand = weight rows), so a lane ends up with runs of 4 consecutive
+// channels of one token; after an exchange between lanes a store covers 64 bytes of 16 rows.  For the
+// gate_up GEMM the 64 weight rows of a wavefront are 16 gate rows, the 16 matching up rows and once more, which
+// puts a gate value and its up value into the same lane.  (32 weight rows x 32 token rows per wavefront read a fifth less
+// from LDS, which made steps whose rows come from L2 5 % faster, but their stores were pieces of 32 bytes: 128 experts of
+// 2048 x 768 with 14 / 32 / 64 rows each, gate_up + down, 61 + 37.7 / 66 + 43.5 / 79.5 + 54 -> 61 + 36.4 / 64.6 + 41.4 /
+// 70.5 + 51.8 us.)
 //
 // Nothing in the steady state is a compiler-visible vector load: token ids, activation scales,
 // routed weights and channel scales of later tiles also travel global -> LDS (4 bytes per lane) while
@@ -47,13 +50,13 @@ constexpr int kThreads = kTileThreads;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kCh = 128;    // weight rows per tile
 constexpr int kMinSteps = 4;
+constexpr int64_t kThroughBytes = 8 << 20;  // results of a launch from which on they are written through (see launch_mode)
 
 template <int TOK>
 struct Shape {
   static constexpr int kStages = TOK == 64 ? 6 : 7;
   static constexpr int kStageBytes = (kCh + TOK) * kStepBytes;  // 24 | 20 KB
   static constexpr int kTokWaves = TOK / 8;                     // wavefronts that load token rows (8 rows each)
-  static constexpr int MF = TOK / 2;                            // MFMA edge: 32 or 16
 };
 
 // Inputs of one tile's epilogue (and of the loads of its token rows), filled by 4-byte global -> LDS
@@ -82,6 +85,7 @@ struct NarrowParams {
   int B;
   int ntiles;  // channel tiles
   int rotate;  // mask of the reduction step that a task starts at (rotation_mask)
+  bool through;  // results are written through to memory (see launch_mode)
   void* out;
 };
 
@@ -90,6 +94,16 @@ __device__ __forceinline__ void load_to_lds_dword(const void* base, uint32_t off
                :
                : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(uniform_address(base))
                : "memory", "m0");
+}
+
+// through: written through to memory instead of left in the L2.  (The two wait states behind that store: a store of more than
+// 8 bytes reads its data that late, and the compiler, which keeps a write of them away from its own stores, does not know of
+// this one.)
+__device__ __forceinline__ void store16(void* to, const v4i& v, bool through) {
+  if (through)
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" :: "v"(reinterpret_cast<uint64_t>(to)), "v"(v) : "memory");
+  else
+    *reinterpret_cast<v4i*>(to) = v;
 }
 
 struct Task {
@@ -111,21 +125,20 @@ struct TaskLoads {
 template <int MODE, int TOK, bool FULL>
 __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p) {
   using S = Shape<TOK>;
-  using F = Mfma<S::MF>;
+  using F = Mfma<16>;
   constexpr int kStages = S::kStages;
   constexpr int kStageBytes = S::kStageBytes;
   constexpr int kTokOffset = kCh * kStepBytes;
-  constexpr int NI = 32 / S::MF;  // MFMA tiles of a wavefront's 32 weight rows
   constexpr int kOut = MODE == kGateUpSilu ? kCh / 2 : kCh;  // channels of a whole tile
   __shared__ __align__(16) char stages[kStages * kStageBytes];
   __shared__ __align__(16) TileAux aux[3];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int cg = wave & 3;   // channel quarter
-  const int th = wave >> 2;  // token half
-  const int lrow = lane % S::MF;
-  const int lgrp = lane / S::MF;
+  const int cg = wave & 1;            // channel half
+  const int tok0 = (wave >> 1) * 16;  // first of its 16 token rows
+  const int lrow = lane & 15;
+  const int lgrp = lane >> 4;
   const int K = p.K;
   const int nk = K / kStepBytes;
   const int inter = p.N / 2;
@@ -219,7 +232,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   auto setup_weight_loads = [&](const Task& tk, TaskLoads& ld) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int row = 16 * wave + 8 * i + (lane >> 3);  // LDS weight row; wavefront row / 32 (mod 4) multiplies it
+      const int row = 16 * wave + 8 * i + (lane >> 3);  // LDS weight row; the wavefronts of channel half row / 64 multiply it
       const int chunk = ((lane & 7) ^ swizzle_of_row(row)) * 16;
       int n;
       if constexpr (MODE == kGateUpSilu) {
@@ -288,87 +301,63 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   };
 
   // ---- MFMA operand reads ----
-  int w_ld[NI], chunk[F::kSub];
+  int w_ld[4], chunk[2];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) w_ld[i] = (32 * cg + S::MF * i + lrow) * kStepBytes;
-  const int x_ld = kTokOffset + (th * S::MF + lrow) * kStepBytes;
+  for (int i = 0; i < 4; ++i) w_ld[i] = (64 * cg + 16 * i + lrow) * kStepBytes;
+  const int x_ld = kTokOffset + (tok0 + lrow) * kStepBytes;
 #pragma unroll
-  for (int kk = 0; kk < F::kSub; ++kk) chunk[kk] = ((kk * (64 / S::MF) + lgrp) ^ swizzle_of_row(lrow)) * 16;
+  for (int kk = 0; kk < 2; ++kk) chunk[kk] = ((4 * kk + lgrp) ^ swizzle_of_row(lrow)) * 16;
 
-  // Token row th * MF + lrow of the tile; acc[i][4q + r] is weight row MF * i + 8q + 4 * lgrp + r (q = 0 for
-  // the 16-row tiles) of this wavefront's 32.
-  auto epilogue = [&](const Task& tk, const TileAux& ax, typename F::Acc (&acc)[NI]) {
-    const int row = th * S::MF + lrow;
+  // Token row tok0 + lrow of the tile; acc[i][r] is weight row 16 * i + 4 * lgrp + r of this wavefront's 64.
+  auto epilogue = [&](const Task& tk, const TileAux& ax, typename F::Acc (&acc)[4]) {
+    const int row = tok0 + lrow;
     const int32_t tok = ax.ids[row];
     if (!in_use(tok)) return;
     const int limit = min(tk.n1, width);
-    auto piece = [&](int j, int (&v)[4]) {  // weight rows 8 * j + 4 * lgrp + r (j = 0..3); 16-row tiles: 16 * j + 4 * lgrp + r
+    auto piece = [&](int j, int (&v)[4]) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = S::MF == 32 ? acc[0][(4 * j + r) % F::kRegs] : acc[j % NI][r];
+      for (int r = 0; r < 4; ++r) v[r] = acc[j][r];
     };
-    constexpr int kPieces = S::MF == 32 ? 4 : 2;
-    constexpr int kPieceRows = S::MF == 32 ? 8 : 16;
-    // Two pieces' results: the lanes of a row trade halves, so that each holds 8 consecutive channels of one piece and a tile
-    // takes half as many stores (down GEMM of 128 experts of 2048 x 768 with 60 rows each 56.7 -> 55 us, of 16 of 4096 x 1408
-    // with 512 119.5 -> 113.5).
-    auto pair = [&](const uint2& a, const uint2& b) {
-      if constexpr (S::MF == 32) {
-        const auto x = __builtin_amdgcn_permlane32_swap(a.x, b.x, false, false), y = __builtin_amdgcn_permlane32_swap(a.y, b.y, false, false);
-        return make_uint4(x[0], y[0], x[1], y[1]);
-      } else {
-        const auto x = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false), y = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
-        return make_uint4(x[0], y[0], x[1], y[1]);
-      }
+    // Results of 16 + 16 channels: the lanes of a row trade halves, so that each holds 8 consecutive channels and a store
+    // covers 64 bytes of 16 rows.
+    auto store = [&](uint16_t* line, int n, const uint2& a, const uint2& b) {
+      const auto x = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false), y = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
+      n += 16 * (lgrp & 1) + 8 * (lgrp >> 1);
+      if (n < limit) store16(line + n, v4i{(int)x[0], (int)y[0], (int)x[1], (int)y[1]}, p.through);
     };
-    const int paired = kPieceRows * (lgrp & 1) + 8 * (lgrp >> 1);  // channel of a lane's first result of a pair
     if constexpr (MODE == kGateUpSilu) {
-      // weight rows 0..15 of the wavefront are gate channels, 16..31 the matching up channels
-      uint16_t* out = static_cast<uint16_t*>(p.out) + (int64_t)tok * inter;
+      // weight rows 0..15 and 32..47 of the wavefront are gate channels, 16..31 and 48..63 the matching up channels
       const float as = ax.a_scale[row];
-      uint2 h[kPieces / 2];
+      uint2 h[2];
 #pragma unroll
-      for (int j = 0; j < kPieces / 2; ++j) {
-        const int c = 16 * cg + kPieceRows * j + 4 * lgrp;
-        const float4 wg = *reinterpret_cast<const float4*>(ax.w_scale + c);
-        const float4 wu = *reinterpret_cast<const float4*>(ax.w_scale + 64 + c);
+      for (int j = 0; j < 2; ++j) {
+        const int c = 32 * cg + 16 * j + 4 * lgrp;
         int g[4], u[4];
-        piece(j, g);
-        piece(j + kPieces / 2, u);
-        h[j] = silu_mul_epilogue4(g, u, as, wg, wu);
+        piece(2 * j, g);
+        piece(2 * j + 1, u);
+        h[j] = silu_mul_epilogue4(g, u, as, *reinterpret_cast<const float4*>(ax.w_scale + c), *reinterpret_cast<const float4*>(ax.w_scale + 64 + c));
       }
-      if constexpr (S::MF == 32) {
-        const int n = tk.n0 + 16 * cg + paired;
-        const uint4 v = pair(h[0], h[1]);
-        if (n < limit) *reinterpret_cast<uint4*>(out + n) = v;
-      } else {
-        const int n = tk.n0 + 16 * cg + 4 * lgrp;
-        if (n < limit) *reinterpret_cast<uint2*>(out + n) = h[0];
-      }
+      store(static_cast<uint16_t*>(p.out) + (int64_t)tok * inter, tk.n0 + 32 * cg, h[0], h[1]);
     } else {
       const float as = MODE == kDown ? ax.a_scale[row] : 0.0f;
       const float rw = MODE == kDown && p.row_weight ? ax.row_w[row] : 1.0f;
-      if constexpr (MODE == kAccI32) {
+      uint2 h[4];
 #pragma unroll
-        for (int j = 0; j < kPieces; ++j) {
-          const int n = tk.n0 + 32 * cg + kPieceRows * j + 4 * lgrp;
-          int v[4];
-          piece(j, v);
-          if (n < limit) *reinterpret_cast<v4i*>(static_cast<int32_t*>(p.out) + (int64_t)tok * p.N + n) = v4i{v[0], v[1], v[2], v[3]};
+      for (int j = 0; j < 4; ++j) {
+        const int c = 64 * cg + 16 * j + 4 * lgrp;
+        int v[4];
+        piece(j, v);
+        if constexpr (MODE == kAccI32) {
+          if (tk.n0 + c < limit)
+            *reinterpret_cast<v4i*>(static_cast<int32_t*>(p.out) + (int64_t)tok * p.N + tk.n0 + c) = v4i{v[0], v[1], v[2], v[3]};
+        } else {
+          h[j] = down_epilogue4(v, as, *reinterpret_cast<const float4*>(ax.w_scale + c), rw);
         }
-      } else {
-        uint2 h[kPieces];
-#pragma unroll
-        for (int j = 0; j < kPieces; ++j) {
-          int v[4];
-          piece(j, v);
-          h[j] = down_epilogue4(v, as, *reinterpret_cast<const float4*>(ax.w_scale + 32 * cg + kPieceRows * j + 4 * lgrp), rw);
-        }
-#pragma unroll
-        for (int j = 0; j < kPieces; j += 2) {
-          const int n = tk.n0 + 32 * cg + kPieceRows * j + paired;
-          const uint4 v = pair(h[j], h[j + 1]);
-          if (n < limit) *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.out) + (int64_t)tok * p.N + n) = v;
-        }
+      }
+      if constexpr (MODE == kDown) {
+        uint16_t* line = static_cast<uint16_t*>(p.out) + (int64_t)tok * p.N;
+        store(line, tk.n0 + 64 * cg, h[0], h[1]);
+        store(line, tk.n0 + 64 * cg + 32, h[2], h[3]);
       }
     }
   };
@@ -409,13 +398,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   int read_at = 0;                 // ring offset of the step being multiplied
   int fill_at = ahead * kStageBytes;  // ... of the step being fetched
   const uint32_t wdst = stage0 + wave * 2048, xdst = stage0 + kTokOffset + wave * 1024;
-  // a wavefront whose half of the tile is padding (valid rows are a prefix) only loads
-  auto half_in_use = [&](const TileAux& ax) { return in_use(__builtin_amdgcn_readfirstlane(ax.ids[th * S::MF])); };
-  bool active = half_in_use(aux[0]), next_active = false;
+  // a wavefront whose part of the tile is padding (valid rows are a prefix) only loads
+  auto part_in_use = [&](const TileAux& ax) { return tok0 < TOK && in_use(__builtin_amdgcn_readfirstlane(ax.ids[tok0])); };
+  bool active = part_in_use(aux[0]), next_active = false;
   while (true) {
-    typename F::Acc acc[NI];
+    typename F::Acc acc[4];
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int r = 0; r < F::kRegs; ++r) acc[i][r] = 0;
     TileAux& ax_next = aux[par + 1 < 3 ? par + 1 : par - 2];
@@ -433,21 +422,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
         // multiplications: the address unit takes 16 clocks per load and the whole workgroup's 20-24 of them in front
         // of the operand reads made a step 0.45 us even where every load hit L2.
         const char* st = stages + read_at;
-        v4i a[F::kSub][NI], b[F::kSub];
+        v4i a[2][4], b[2];
         if constexpr (ACTIVE) {
 #pragma unroll
-          for (int kk = 0; kk < F::kSub; ++kk) {
+          for (int kk = 0; kk < 2; ++kk) {
             b[kk] = *reinterpret_cast<const v4i*>(st + x_ld + chunk[kk]);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) a[kk][i] = *reinterpret_cast<const v4i*>(st + w_ld[i] + chunk[kk]);
+            for (int i = 0; i < 4; ++i) a[kk][i] = *reinterpret_cast<const v4i*>(st + w_ld[i] + chunk[kk]);
           }
         }
         const int8_t* wsrc = ld.wbase + next_at;
         const int8_t* xsrc = p.a_q + next_at;
-        auto mul = [&](int kk) {
+        auto mul = [&](int kk, int half) {
           if constexpr (ACTIVE)
 #pragma unroll
-            for (int i = 0; i < NI; ++i) acc[i] = F::mul(a[kk][i], b[kk], acc[i]);
+            for (int i = 2 * half; i < 2 * half + 2; ++i) acc[i] = F::mul(a[kk][i], b[kk], acc[i]);
         };
         auto one_weight = [&](int i) {
           if constexpr (STREAM)
@@ -455,13 +444,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
           else
             load_to_lds_16(wsrc, ld.woff[i], wdst + fill_at + i * 1024);
         };
-        mul(0);
+        mul(0, 0);
         one_weight(0);
-        if constexpr (F::kSub == 4) mul(1);
+        mul(0, 1);
         one_weight(1);
-        mul(F::kSub == 4 ? 2 : 1);
+        mul(1, 0);
         if (loads_tokens) load_to_lds_16(xsrc, ld.xoff, xdst + fill_at);
-        if constexpr (F::kSub == 4) mul(3);
+        mul(1, 1);
         if (s == 1) {
           if (nx.e >= 0) issue_scales(nx, ax_next);
           if (n2.e >= 0) issue_ids(n2, ax_n2);
@@ -489,7 +478,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
         setup_weight_loads(nx, ld);
         setup_token_loads(ax_next, ld);
         next_at = ld.first;
-        next_active = half_in_use(ax_next);
+        next_active = part_in_use(ax_next);
       } else if (part == 1) {
         next_at = (next_at > 0 ? next_at : K) - kStepBytes;
         advance = 0;
@@ -533,6 +522,13 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.B = a.block_size;
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 63) / 64 : (a.n + kCh - 1) / kCh;
   p.rotate = rotation_mask(a.k);
+  // Results left in the L2s are written back when they are displaced by the weight stream, line by line, and the rest when
+  // the launch ends.  Up to some megabytes that costs less than a write to memory per store, beyond it more.  Left / written
+  // through: down GEMM of 128 experts of 2048 x 768 with 8 / 14 / 20 / 32 / 64 rows each (4 / 7 / 10 / 17 / 34 MB) 35.3 / 36.4 /
+  // 39.4 / 43.2 / 53.0 and 36.3 / 36.9 / 38.4 / 41.4 / 51.8 us, gate_up with 14 / 20 / 32 / 64 rows (3 / 4 / 6 / 13 MB) 60.9 / 63.0 /
+  // 66.7 / 80.4 and 61.2 / 62.5 / 64.6 / 70.5; 64 of 4096 x 1408 with 8 / 20 / 32 / 64 rows, down (4 / 10 / 17 / 34 MB) 57.7 / 63.8 /
+  // 69.6 / 82.2 and 59.5 / 62.8 / 66.2 / 75.6, gate_up (1 / 4 / 6 / 12 MB) 118 / 119.5 / 121 / 142 and 118 / 120 / 123 / 133.5.
+  p.through = a.num_pairs * (MODE == kGateUpSilu ? a.n / 2 : a.n) * 2 >= kThroughBytes;
   p.out = a.out;
   const int grid = device_cu_count() / kXcds * kXcds;
   if (a.k >= Shape<TOK>::kStages * kStepBytes)
