@@ -16,10 +16,10 @@
 //    flight, the stores of the last epilogue included.  With scalar decisions in every step, tasks set up by dependent
 //    loads and an epilogue that drained everything, 16 experts of 4096 x 1408 with 512 rows each took 114 + 63 us
 //    (gate_up + down), 103 + 61 now; 78 experts with 12 to 517 rows 206 + 113, now 173 + 99.
-//  * Results are staged in the last step's stage, 4 KB per wavefront, and stored 64 or 128 bytes of a row at a time with
-//    the non-temporal hint.  64 experts of 4096 x 1408 with 96 rows each: 133 + 79 us; without the hint 146 + 88, with it
-//    but stored straight from registers in pieces of 32 bytes 138 + 113.  (The hint on stores of experts of one tile only
-//    loses part of it.)
+//  * Results are staged in the last step's stage, 4 KB per wavefront, and stored 64 or 128 bytes of a row at a time, through
+//    to memory.  64 experts of 4096 x 1408 with 96 rows each: 132 + 79 us; left in the L2s, where the weight stream displaces
+//    them, 146 + 88.  With the non-temporal hint instead 133 + 80, and 78 experts with 12 to 517 rows 0.7 % of the layer
+//    slower; with it and straight from registers in pieces of 32 bytes 138 + 113.
 //  * Weight rows that nothing else reads are fetched with the non-temporal hint, so that they do not displace token rows from
 //    L2: 64 experts of 4096 x 1408 with 40 rows each 139 + 84 us without, 132 + 76 with.  It is chosen per task: where only
 //    some experts have several tiles the others still profit.
@@ -91,12 +91,12 @@ struct TaskLoads {
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// A store that is issued whatever its mask, so that the waits can count it.  (The two wait states behind it: a store of more
+// A store through to memory, issued whatever its mask, so that the waits can count it.  (The two wait states behind it: a store of more
 // than 8 bytes reads its data that late, and the compiler, which keeps a write of them away from its own stores, does not know
 // of this one.)
-__device__ __forceinline__ void store16_stream(void* to, const uint4& v, uint64_t lanes) {
+__device__ __forceinline__ void store16_through(void* to, const uint4& v, uint64_t lanes) {
   lanes = uniform_address(reinterpret_cast<const void*>(lanes));
-  asm volatile("s_mov_b64 exec, %2\n\tglobal_store_dwordx4 %0, %1, off nt\n\ts_mov_b64 exec, -1\n\ts_nop 1"
+  asm volatile("s_mov_b64 exec, %2\n\tglobal_store_dwordx4 %0, %1, off sc1\n\ts_mov_b64 exec, -1\n\ts_nop 1"
                :: "v"(reinterpret_cast<uint64_t>(to)), "v"(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}), "s"(lanes) : "memory");
 }
 
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
         const uint4 v = *reinterpret_cast<const uint4*>(staging + r * 64 + ((lane & 3) ^ ((r >> 1) & 3)) * 16);
         const int tok = ax.ids[row0 + r], n = tk.n0 + 32 * cg + 8 * (lane & 3);
         const bool ok = in_use(tok);
-        store16_stream(static_cast<uint16_t*>(p.out) + (int64_t)(ok ? tok : 0) * inter + n, v, __ballot(ok && n < limit));
+        store16_through(static_cast<uint16_t*>(p.out) + (int64_t)(ok ? tok : 0) * inter + n, v, __ballot(ok && n < limit));
       }
     } else if constexpr (MODE == kDown) {
       const float as = ax.a_scale[row];
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
         const uint4 v = *reinterpret_cast<const uint4*>(staging + r * 128 + ((lane & 7) ^ (r & 7)) * 16);
         const int tok = ax.ids[row0 + r], n = tk.n0 + 64 * cg + 8 * (lane & 7);
         const bool ok = in_use(tok);
-        store16_stream(static_cast<uint16_t*>(p.out) + (int64_t)(ok ? tok : 0) * p.N + n, v, __ballot(ok && n < limit));
+        store16_through(static_cast<uint16_t*>(p.out) + (int64_t)(ok ? tok : 0) * p.N + n, v, __ballot(ok && n < limit));
       }
     } else {
       const int32_t tok = ax.ids[row];
