@@ -99,8 +99,10 @@ int check_gemm_common(const void* a_q, const void* w, const int32_t* sorted, con
 // while every block fits one such pass, and loses badly as soon as a few experts hold more (a
 // shared expert that every token visits, skewed routing), which the host cannot see.  It is
 // therefore picked where no expert can hold more than 16 rows (it holds at most one per token),
-// or where there is at most one routed row per expert on average.
-constexpr int kStreamMaxRows = 16;
+// or where there is at most one routed row per expert on average.  Launches with 2 GB of weights and more run long enough
+// for the narrow tiles' slower start not to count, and their deeper prefetch wins earlier: layer us, streaming / narrow, of
+// DeepSeek-V3 at 9 / 16 / 32 tokens 338 / 332, 476 / 469, 656 / 642 (0.2-0.4 GB, Qwen3-30B-A3B at 10 / 16: 60 / 62, 75 / 78.5).
+constexpr int kStreamMaxRows = 16, kStreamMaxRowsLongStream = 8;
 constexpr int kStreamRowsPerExpert = 1;
 constexpr int kSelfQuantMaxInter = 1024;  // longest reduction moe_i8_gemm_down_bf16 takes for any routing
 
@@ -115,12 +117,13 @@ int tile_geometry_of(int variant) {
 // The narrow tiles (64 x 128 tasks) start up faster and balance better; the deep tiles stream an
 // expert's weights once for up to 128 rows, which counts the more the longer a launch runs and the
 // more the routing is skewed.  Layer us, narrow / deep, by the weight bytes of the launch and rows per expert: 0.2-0.4 GB
-// (Qwen3-30B-A3B, even routing) 24 rows 125 / 130, 32 135 / 134, 40 142 / 139, 48 159 / 144; 0.7-1.5 GB (GLM-4.5-Air,
-// Zipf routing and a shared expert) 24 289 / 300, 28 317 / 317, 32 338 / 337, 36 366 / 347; 3.8-7.5 GB (DeepSeek-V3)
-// 16 1406 / 1456, 20 1545 / 1577, 24 1627 / 1604, 32 1766 / 1632.
+// (Qwen3-30B-A3B, even routing) 24 rows 121 / 124, 32 129 / 130, 36 132 / 132, 40 136 / 134, 44 140 / 136; 0.7-1.5 GB
+// (GLM-4.5-Air) with Zipf routing and a shared expert 9 194 / 203, 11 213 / 210, 17 248 / 244, 20 266 / 252, 28 305 / 269,
+// evenly routed 11 378 / 390, 17 391 / 402, 21 397 / 404, 32 418 / 420: between the two; 3.8-7.5 GB (DeepSeek-V3) 4 985 /
+// 986, 8 1151 / 1153, 10 1228 / 1222, 12 1289 / 1258, 16 1392 / 1344, 24 1548 / 1450.
 int narrow_rows_per_expert(const moe_i8::GemmArgs& g) {
   const int64_t weight_bytes = (int64_t)g.num_experts * g.n * g.k;
-  return weight_bytes < (512ll << 20) ? 40 : weight_bytes < (2048ll << 20) ? 28 : 16;
+  return weight_bytes < (512ll << 20) ? 40 : weight_bytes < moe_i8::kLongStreamBytes ? 20 : 10;
 }
 
 // Which family a launch goes to (MOE_I8_GEMM_STREAM, _TILE or _NARROW); -1 with the error set if a
@@ -148,7 +151,9 @@ int picks_family(const moe_i8::GemmArgs& g0, int variant) {
   const int64_t rows_x_experts = g.num_pairs;
   const int64_t most_rows = g.max_rows_per_expert > 0 && g.max_rows_per_expert < g.num_pairs ? g.max_rows_per_expert
                                                                                              : g.num_pairs;
-  if (most_rows <= kStreamMaxRows || rows_x_experts <= (int64_t)kStreamRowsPerExpert * g.num_experts)
+  const bool long_stream = (int64_t)g.num_experts * g.n * g.k >= moe_i8::kLongStreamBytes && moe_i8::gemm_narrow_supports(g);
+  if (long_stream ? most_rows <= kStreamMaxRowsLongStream
+                  : most_rows <= kStreamMaxRows || rows_x_experts <= (int64_t)kStreamRowsPerExpert * g.num_experts)
     return MOE_I8_GEMM_STREAM;
   if (rows_x_experts <= (int64_t)narrow_rows_per_expert(g) * g.num_experts && moe_i8::gemm_narrow_supports(g))
     return MOE_I8_GEMM_NARROW;

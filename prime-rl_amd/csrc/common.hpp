@@ -305,7 +305,8 @@ struct GemmArgs {
 };
 constexpr int kTileAuto = 0, kTileWide = 1, kTileDeep = 2, kTileRing = 3;
 // The LDS-tiled family picks its deep geometry up to this many routed rows per expert (launches with 2 GB of weights and more: fewer).
-constexpr int kTileDeepRowsPerExpert = 96, kTileDeepRowsLongStream = 64;
+constexpr int kTileDeepRowsPerExpert = 104, kTileDeepRowsLongStream = 80;
+constexpr int64_t kLongStreamBytes = 2048ll << 20;  // weights of a launch
 hipError_t launch_gemm_stream(const GemmArgs& a, hipStream_t stream);
 // register-only int8 MFMA loop (measurement aid): sink holds mfma_probe_sink_bytes(workgroups)
 int64_t mfma_probe_sink_bytes(int workgroups);

@@ -468,13 +468,13 @@ bool gemm_tile_supports(const GemmArgs& a) {
   }
 }
 
-// Measured on three layer shapes (Qwen3-30B-A3B, GLM-4.5-Air, DeepSeek-V3): the deep tiles win where a 256-row
-// tile would be mostly padding and the kernel is bound by the weight stream.  Layer us at 64 / 80 / 96 / 107 routed
-// rows per expert, deep against wide: 155 / 165 / 171 / - against 162 / 170 / 177 / - with 0.2-0.4 GB of weights per
-// launch, 471 / - / - / 570 against 485 / - / - / 541 with 0.7-1.5 GB; with 3.8-7.5 GB 2040 / - / 2339 against 2015 / - /
-// 2234.
+// Measured on three layer shapes (Qwen3-30B-A3B, GLM-4.5-Air, DeepSeek-V3): the deep tiles win as long as few experts hold
+// more rows than one of them, and a little less far where a launch streams so many weights that a step is bound by them in
+// either.  Layer us, deep / wide, by routed rows per expert: 64 147 / 160, 96 162 / 174, 104 175.5 / 179, 108 190 / 180 with
+// 0.2-0.4 GB of weights per launch; 63 395 / 436, 97 492 / 514, 112 551 / 562 (evenly routed 509 / 531), 133 609 / 587 (649 / 556)
+// with 0.7-1.5 GB; 48 1770 / 1842, 64 1939 / 1979, 78 2094 / 2109, 94 2238 / 2234, 109 2368 / 2352 with 3.8-7.5 GB.
 bool gemm_tile_prefers_deep(const GemmArgs& a) {
-  const bool long_stream = (int64_t)a.num_experts * a.n * a.k >= (2048ll << 20);
+  const bool long_stream = (int64_t)a.num_experts * a.n * a.k >= kLongStreamBytes;
   return a.num_pairs <= (int64_t)(long_stream ? kTileDeepRowsLongStream : kTileDeepRowsPerExpert) * a.num_experts;
 }
 
