@@ -238,7 +238,13 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
         o[h] = down_epilogue4(v, as, ws, 1.0f);
       }
     }
-    *reinterpret_cast<uint4*>(p.out + (int64_t)m * width + n) = make_uint4(o[0].x, o[0].y, o[1].x, o[1].y);
+    // Through to memory: left in the L2s all results are written back when the launch ends, in one go (linear layers with their
+    // quantisation, 333 x 4096 x 2048 11.6 -> 11.3 us, 1024 x 4096 x 4096 29.5 -> 29.1, 700 x 7168 x 2048 23.0 -> 21.9, 64 x
+    // 4096 x 4096 the same).  (The two wait states: the store reads its data that late, and the compiler, which keeps a write of
+    // them away from its own stores, does not know of this one.)
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1"
+                 :: "v"(reinterpret_cast<uint64_t>(p.out + (int64_t)m * width + n)), "v"(v4i{(int)o[0].x, (int)o[0].y, (int)o[1].x, (int)o[1].y})
+                 : "memory");
   }
 }
 
