@@ -73,3 +73,15 @@ def test_deep_layer_around_the_depth_of_the_ring(pra, H, tokens):
     kw = d.fused_experts_kwargs()
     got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="tile_deep")
     assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream"))
+
+
+@pytest.mark.parametrize("tokens", [255, 256, 300])
+def test_narrow_results_around_the_size_that_is_written_through(pra, tokens):
+    # 4 * tokens rows of 4096 bf16 from the second GEMM: 8 MB at 256 tokens
+    from _util import inputs_mod
+
+    im = inputs_mod()
+    d = im.make_inputs(im.LayerShape("t", E=24, k=4, H=4096, I=512), tokens, seed=tokens).to(DEV)
+    kw = d.fused_experts_kwargs()
+    got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="narrow")
+    assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream"))
