@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   __shared__ __align__(16) char stages[kStages * kStage];
   __shared__ __align__(16) TileAux aux[3];
   __shared__ TileList<kMaxTiles> list;
-  // tasks it .. of this workgroup: block | blocks << 16 | piece << 20 | log2(pieces) << 22 | single << 31, expert | channel tile << 16
+  // tasks it .. of this workgroup: block | blocks << 16 | piece << 20 | log2(pieces) << 22 | single << 31, task_word
   __shared__ uint2 table[kTable];
   constexpr int kOut = MODE == kGateUpSilu ? kCh / 2 : kCh;  // channels of a whole tile
   // counted stores of a wavefront and unit in an epilogue (the int32 results' are the compiler's and not counted)
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   auto fill_table = [&](int n0) {
     if (t >= kTable) return;
     const TaskPiece tp = piece_at(blockIdx.x / kXcds + (n0 + t) * stride, my_tasks, stride);
-    uint2 d = make_uint2(0u, 0xffffffffu);  // no more
+    uint2 d = make_uint2(0u, kNoTask);
     if (tp.task >= 0) {
       d = look_up_task(p.tiles, list, range, xcd * per_xcd + tp.task);
       const bool single = (d.x >> 20) == (1u << 4);  // rank 0 of a group of one
@@ -152,16 +152,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   auto next_task = [&]() {
     const uint2 d = table[it % kTable];
     const uint32_t d0 = (uint32_t)uniform((int)d.x);
-    const int d1 = uniform((int)d.y);
+    const uint32_t d1 = (uint32_t)uniform((int)d.y);
     const int shift = (int)(d0 >> 22) & 3;  // 1, 2 or 4 pieces
     Task tk;
     tk.slot0 = (int)(d0 & 0xffffu) * p.B;
     tk.rows = (int)((d0 >> 16) & 15u) * p.B;
     tk.single = d0 >> 31;
-    tk.n0 = (d1 >> 16) * kOut + ((int)(d0 >> 20) & 3) * (kOut >> shift);
+    tk.n0 = task_channel_tile(d1) * kOut + ((int)(d0 >> 20) & 3) * (kOut >> shift);
     tk.n1 = tk.n0 + (kOut >> shift);
-    tk.e = d1 < 0 ? -1 : d1 & 0xffff;
-    if (d1 >= 0) ++it;
+    tk.e = task_expert(d1);
+    if (tk.e >= 0) ++it;
     return tk;
   };
   auto in_use = [&](int id) { return (uint32_t)id < (uint32_t)p.P; };

@@ -316,11 +316,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_ring_kernel(TileParams p) {
     if (it < per_xcd && xcd * per_xcd + it < total) {
       constexpr int kOut = MODE == kGateUpSilu ? kBN / 2 : kBN;
       const uint2 d = look_up_task(p.tiles, list, range, xcd * per_xcd + it);
-      tk.n0 = (int)(d.y >> 16) * kOut;
+      tk.n0 = task_channel_tile(d.y) * kOut;
       tk.n1 = tk.n0 + kOut;
       tk.slot0 = (int64_t)(d.x & 0xffffu) * p.B;
       tk.nsub = (int)((d.x >> 16) & 15u) * sub_per_block;
-      tk.e = tk.nsub > 0 ? (int)(d.y & 0xffffu) : -2;
+      tk.e = tk.nsub > 0 ? task_expert(d.y) : -2;
     }
     return tk;
   };

@@ -115,7 +115,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
   __shared__ __align__(16) int32_t ids[3][kTok];                          // slots of the current, the next and the task after it
   __shared__ __align__(16) float a_scales[2][kTok], row_weights[2][kTok], w_scales[2][kCh];
   __shared__ TileList<kMaxTiles> list;
-  __shared__ uint2 table[kTable];                           // tasks it .. of this workgroup: block | blocks << 16, expert | channel tile << 16
+  __shared__ uint2 table[kTable];                           // tasks it .. of this workgroup: block | blocks << 16, task_word
 
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
   auto fill_table = [&](int n0) {
     if (t >= kTable) return;
     const TaskPiece tp = piece_at(blockIdx.x / kXcds + (n0 + t) * stride, my_tasks, stride);
-    uint2 d = make_uint2(0u, 0xffffffffu);  // no more
+    uint2 d = make_uint2(0u, kNoTask);
     if (tp.task >= 0) {
       const uint2 whole = look_up_task(p.tiles, list, range, xcd * per_xcd + tp.task);
       // a piece is a part of the tile's blocks
@@ -154,13 +154,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
   auto next_task = [&]() {
     const uint2 d = table[it % kTable];
     const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.x);
-    const int d1 = __builtin_amdgcn_readfirstlane((int)d.y);
+    const uint32_t d1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.y);
     Task tk;
     tk.slot0 = (int)(d0 & 0xffffu) * p.B;
     tk.rows = (int)(d0 >> 16) * p.B;
-    tk.nt = d1 >> 16;
-    tk.e = d1 < 0 ? -1 : d1 & 0xffff;
-    if (d1 >= 0) ++it;
+    tk.nt = task_channel_tile(d1);
+    tk.e = task_expert(d1);
+    if (tk.e >= 0) ++it;
     return tk;
   };
   auto fetch_ids = [&](const Task& tk, int buf) {

@@ -229,7 +229,16 @@ __device__ TileRange build_ascending(const TileListArgs& p, int xcd, int* scratc
   return range;
 }
 
-// Task `task` of a launch: its tile's entry (0 blocks where the expert id is out of range) and expert | channel tile << 16.
+// A task's second word: expert | channel tile << 16.  Both halves are full ranges (a matrix of less than 2^32 bytes in rows of at
+// least 256 has up to 65536 channel tiles), so no bit is left for "no more tasks": that is the word with all bits set, whose
+// expert no layer has.
+constexpr uint32_t kNoTask = 0xffffffffu;
+__host__ __device__ constexpr uint32_t task_word(uint32_t expert, uint32_t channel_tile) { return expert | channel_tile << 16; }
+__host__ __device__ constexpr int task_expert(uint32_t word) { return word == kNoTask ? -1 : (int)(word & 0xffffu); }
+__host__ __device__ constexpr int task_channel_tile(uint32_t word) { return (int)(word >> 16); }
+static_assert(kMaxExperts <= 0xffff, "an expert's half of a task word is never all ones");
+
+// Task `task` of a launch: its tile's entry (0 blocks where the expert id is out of range) and its task_word.
 // The tasks of a group of T token tiles of one expert run channel tile by channel tile: T consecutive tasks (on
 // neighbouring compute units) stream the same weight tile.
 template <int MAX>
@@ -243,7 +252,7 @@ __device__ __forceinline__ uint2 look_up_task(const TileListArgs& p, const TileL
   const int nt = (int)(((float)pos + 0.5f) * __builtin_amdgcn_rcpf((float)T));
   const int tile = first + (pos - nt * T) - range.lo;
   const int e = list.expert[tile];
-  return make_uint2(e == 0xffff ? list.desc[tile] & 0xff00ffffu : list.desc[tile], (e == 0xffff ? 0u : (uint32_t)e) | ((uint32_t)nt << 16));
+  return make_uint2(e == 0xffff ? list.desc[tile] & 0xff00ffffu : list.desc[tile], task_word(e == 0xffff ? 0u : (uint32_t)e, (uint32_t)nt));
 }
 
 // The last round of an XCD's tasks is rarely full: where its tasks leave at least half of the workgroups idle, each is cut

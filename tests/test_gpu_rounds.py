@@ -30,6 +30,20 @@ def test_rest_of_the_last_round(pra, oracle, variant, tasks):
     _check(pra, oracle, variant, [70], tasks * channels - 16 * (tasks % 3), 512)
 
 
+@pytest.mark.parametrize("variant,K", [("tile_deep", 384), ("tile_wide", 256)])
+def test_more_channel_tiles_than_fifteen_bits_count(pra, variant, K):
+    N, P = 32768 * 256 + 5 * 256 + 16, 40
+    gen = torch.Generator(device=DEV).manual_seed(K)
+    a = torch.randint(-127, 128, (P, K), dtype=torch.int8, device=DEV, generator=gen)
+    w = torch.randint(-127, 128, (1, N, K), dtype=torch.int8, device=DEV, generator=gen)
+    s, e, npp = pra.moe_align_block_size(torch.zeros((P, 1), dtype=torch.int32, device=DEV), 64, 1)
+    got = pra.gemm_acc_i32(a, w, s, e, npp, 1, 64, P, variant).view(P, N)
+    # (the magnitude of every partial sum is below 384 * 127 * 127 < 2^24: exact in float32)
+    for at in range(0, N, 1 << 20):
+        want = a.float() @ w[0, at:at + (1 << 20)].float().T
+        assert torch.equal(got[:, at:at + (1 << 20)].float(), want), at
+
+
 @pytest.mark.parametrize("variant", ["narrow", "tile_deep", "tile_wide"])
 @pytest.mark.parametrize("counts", [[260, 5, 0, 64, 129], [1] * 37])
 def test_pieces_of_tiles_of_several_sizes(pra, oracle, variant, counts):
