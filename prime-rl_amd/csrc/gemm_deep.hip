@@ -91,15 +91,6 @@ struct TaskLoads {
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// A store through to memory, issued whatever its mask, so that the waits can count it.  (The two wait states behind it: a store of more
-// than 8 bytes reads its data that late, and the compiler, which keeps a write of them away from its own stores, does not know
-// of this one.)
-__device__ __forceinline__ void store16_through(void* to, const uint4& v, uint64_t lanes) {
-  lanes = uniform_address(reinterpret_cast<const void*>(lanes));
-  asm volatile("s_mov_b64 exec, %2\n\tglobal_store_dwordx4 %0, %1, off sc1\n\ts_mov_b64 exec, -1\n\ts_nop 1"
-               :: "v"(reinterpret_cast<uint64_t>(to)), "v"(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}), "s"(lanes) : "memory");
-}
-
 template <int MODE>
 __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   using F = Mfma<kUnit>;

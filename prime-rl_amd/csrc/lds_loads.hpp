@@ -1,4 +1,5 @@
-// Global -> LDS loads, counted waits and MFMA shapes shared by the dense and the split-reduction GEMM.
+// Global -> LDS loads, counted waits, counted stores and MFMA shapes shared by the GEMM kernels that stage through LDS (dense,
+// split reduction, narrow, deep, wide and ring tiles).
 #pragma once
 
 #include "common.hpp"
@@ -57,6 +58,19 @@ __device__ __forceinline__ void load_to_lds_4(const void* addr, uint32_t lds_add
                :
                : "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(reinterpret_cast<uint64_t>(addr))
                : "memory", "m0");
+}
+// A store through to memory by those of the active lanes that are in `lanes`, issued even if that is none of them, so that the
+// waits can count it (where the branches around it are the same for all lanes: a branch that no lane takes is jumped over as
+// a whole).  The lanes that were active before are active again afterwards.  (The two wait states behind it: a store of more
+// than 8 bytes reads its data that late, and the compiler, which keeps a write of them away from its own stores, does not know
+// of this one.)
+__device__ __forceinline__ void store16_through(void* to, const uint4& v, uint64_t lanes) {
+  uint64_t active;
+  lanes = uniform_address(reinterpret_cast<const void*>(lanes));
+  asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_dwordx4 %1, %2, off sc1\n\ts_mov_b64 exec, %0\n\ts_nop 1"
+               : "=&s"(active)
+               : "v"(reinterpret_cast<uint64_t>(to)), "v"(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}), "s"(lanes)
+               : "memory", "scc");
 }
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)p);

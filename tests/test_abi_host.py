@@ -224,6 +224,20 @@ def test_task_words_hold_every_expert_and_channel_tile(pra, tmp_path):
     assert run.returncode == 0 and run.stdout.strip() == "ok", run.stdout + run.stderr
 
 
+def test_masked_store_leaves_the_active_lanes_as_they_were(pra, tmp_path):
+    """The store that sets its own lane mask, inside a branch that only some lanes take: behind it, the mask is what it was and
+    not all lanes (read from the assembly; the kernel is not run)."""
+    import subprocess
+
+    asm = tmp_path / "masked_store.s"
+    subprocess.run([pra.build._hipcc(), *pra.build.HIPCC_FLAGS, "--offload-device-only", "-S", "-I", str(pra.build.CSRC),
+                    str(ROOT / "tests" / "c" / "masked_store.hip"), "-o", str(asm)], check=True, capture_output=True, text=True)
+    text = asm.read_text()
+    saved = re.search(r"s_and_saveexec_b64 (s\[\d+:\d+\]), s\[\d+:\d+\]\s+global_store_dwordx4 .*? sc1\s+s_mov_b64 exec, (\S+)", text)
+    assert saved and saved[1] == saved[2], text
+    assert not re.search(r"exec, -1\b", text)
+
+
 # Which kernels the library picks by itself for the chain of stages at every benchmark point (shape, tokens) and how
 # many launches the chain makes there (calls of a few tokens run without it: test_launches_of_a_call).  These are the kernels the committed measurements were taken on: a retune of the
 # hand-over points between the GEMM families must change this table knowingly.
