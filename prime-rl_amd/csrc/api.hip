@@ -116,14 +116,24 @@ int tile_geometry_of(int variant) {
 // Routed rows per expert up to which the narrow tiles beat the deep geometry of the LDS-tiled family.
 // The narrow tiles (64 x 128 tasks) start up faster and balance better; the deep tiles stream an
 // expert's weights once for up to 128 rows, which counts the more the longer a launch runs and the
-// more the routing is skewed.  Layer us, narrow / deep, by the weight bytes of the launch and rows per expert: 0.2-0.4 GB
-// (Qwen3-30B-A3B, even routing) 24 rows 121 / 124, 32 129 / 130, 36 132 / 132, 40 136 / 134, 44 140 / 136; 0.7-1.5 GB
-// (GLM-4.5-Air) with Zipf routing and a shared expert 9 194 / 203, 11 213 / 210, 17 248 / 244, 20 266 / 252, 28 305 / 269,
-// evenly routed 11 378 / 390, 17 391 / 402, 21 397 / 404, 32 418 / 420: between the two; 3.8-7.5 GB (DeepSeek-V3) 4 985 /
-// 986, 8 1151 / 1153, 10 1228 / 1222, 12 1289 / 1258, 16 1392 / 1344, 24 1548 / 1450.
+// more the routing is skewed.  Where evenly spread and Zipf routing (expert popularity falling with rank^-1.2) disagree, which
+// the host cannot see, the line takes the smaller loss.  Measured on launches of 0.16 to 7 GB of 13 layer shapes; us of the
+// launch, narrow / deep, at rows per expert, evenly | Zipf:
+//   0.38 GB (128 experts of 2048 x 768, gate_up)  32: 66.1 / 68.6 | 57.8 / 60.4   40: 69.6 / 69.7 | 60.4 / 59.0
+//   0.56 GB (96 of 3072 x 1024, gate_up)  20: 93.3 / 99.9 | 75.5 / 87.5   28: 96.3 / 101 | 88.0 / 88.8   36: 102 / 102 | 96.6 / 91.9
+//   0.69 GB (129 of 4096 x 1408, down)  16: 128 / 131 | 75.3 / 74.0   20: 131 / 132 | 85.0 / 82.9   24: 135 / 133 | 96.9 / 90.4
+//   1.4 GB (the same, gate_up)  16: 239 / 244 | 139 / 139   20: 244 / 248 | 155 / 148   24: 243 / 251 | 175 / 164
+//   1.9 GB (128 of 5120 x 1536, gate_up)  16: 305 / 305 | 179 / 189   20: 310 / 307 | 212 / 195
+//   2.8 GB (96 of 6144 x 2560, gate_up)  10: 442 / 450 | 285 / 296   12: 444 / 452 | 301 / 294   20: 448 / 459 | 369 / 330
+//   3.5 GB (256 of 7168 x 2048, down)  8: 575 / 581 | 195 / 186   12: 598 / 600 | 221 / 201   16: 617 / 610 | 274 / 236
+//   7.0 GB (the same, gate_up)  8: 1071 / 1072 | 362 / 325   12: 1083 / 1085 | 430 / 357
+// Below 0.4 GB the two cross between 26 and more than 44 rows.  From 0.5 to 0.56 GB (four shapes) the deep tiles take 1 to 7 %
+// longer at 20-28 rows evenly spread, -8 to +16 %, on average 2, with Zipf routing, and win from 28-36 on; the step from there to 20
+// lies between the largest launch measured that wants 28 (0.56 GB) and the smallest that wants 20 (0.69).  Given away: up to 4 %
+// of an evenly spread gate_up launch of 1.4-1.5 GB at 20-28 rows (where Zipf routing wins 4-12 %), 2 % of one of 2.8 GB at 10-28.
 int narrow_rows_per_expert(const moe_i8::GemmArgs& g) {
   const int64_t weight_bytes = (int64_t)g.num_experts * g.n * g.k;
-  return weight_bytes < (512ll << 20) ? 40 : weight_bytes < moe_i8::kLongStreamBytes ? 20 : 10;
+  return weight_bytes < (512ll << 20) ? 40 : weight_bytes < (640ll << 20) ? 28 : weight_bytes < moe_i8::kLongStreamBytes ? 20 : 10;
 }
 
 // Which family a launch goes to (MOE_I8_GEMM_STREAM, _TILE or _NARROW); -1 with the error set if a

@@ -25,6 +25,14 @@ import pytest
         (321, 8, 128, 4096, 1408, "tile_deep"),
         (1664, 8, 128, 4096, 1408, "tile_deep"),
         (1665, 8, 128, 4096, 1408, "tile_wide"),
+        # 512 MiB, 576 MiB and 608 MiB: 28; from 640 MiB on 20
+        (224, 8, 64, 4096, 1024, "narrow"),
+        (225, 8, 64, 4096, 1024, "tile_deep"),
+        (336, 8, 96, 3072, 1024, "narrow"),
+        (337, 8, 96, 3072, 1024, "tile_deep"),
+        (224, 8, 64, 4096, 1216, "narrow"),
+        (160, 8, 64, 4096, 1280, "narrow"),
+        (161, 8, 64, 4096, 1280, "tile_deep"),
         # 0.2 and 0.4 GB: 40 and 104
         (640, 8, 128, 2048, 768, "narrow"),
         (641, 8, 128, 2048, 768, "tile_deep"),
