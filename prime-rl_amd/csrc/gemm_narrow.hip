@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   const bool loads_tokens = S::kTokWaves == kWaves || wave < S::kTokWaves;
   // Steps the loads run ahead of the multiplication: the ring's depth, less for very short reductions (the
   // rows of the next tile are set up in the first step of the current one).
-  const int ahead = FULL || nk > kStages ? kStages - 1 : nk - 1;
+  const int ahead = FULL ? kStages - 1 : nk - 1;
 
   // ---- this workgroup's tasks: (block, channel tile), channel tile fastest, split into 8 contiguous
   // ranges, one per XCD (workgroup id % 8), so that workgroups that run side by side share token
