@@ -30,6 +30,24 @@ def test_rest_of_the_last_round(pra, oracle, variant, tasks):
     _check(pra, oracle, variant, [70], tasks * channels - 16 * (tasks % 3), 512)
 
 
+# The layer's task list is built from ids that are known to ascend.  Eight tiles: an XCD gets as many tasks as there are channel
+# tiles; the other routings put several tiles of an expert into a group (deep tiles 9 and 8, wide ones 5 and 4).
+@pytest.mark.parametrize("variant", ["tile_deep", "tile_wide"])
+@pytest.mark.parametrize("counts", [[100, 0, 1, 64, 65, 128, 33, 7, 90], [700, 0, 130, 40], [1000]])
+@pytest.mark.parametrize("ntiles", [3, 8, 9, 16, 17, 31, 32, 33, 40, 41, 48, 49, 65])
+def test_layer_tasks_around_a_round(pra, variant, counts, ntiles):
+    from _util import inputs_mod
+
+    im, M = inputs_mod(), sum(counts)
+    for H, I in ((512, 128 * ntiles), (256 * ntiles, 512)):  # the first GEMM's channel tiles, the second one's
+        d = im.make_inputs(im.LayerShape("r", E=len(counts), k=1, H=H, I=I), M, seed=ntiles, device=DEV, weights_on_device=True)
+        ids = torch.repeat_interleave(torch.arange(len(counts), dtype=torch.int32), torch.tensor(counts))
+        d.topk_ids.copy_(ids[torch.randperm(M, generator=torch.Generator().manual_seed(ntiles))].view(M, 1))
+        kw = d.fused_experts_kwargs()
+        got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant=variant)
+        assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream")), (H, I)
+
+
 @pytest.mark.parametrize("variant,K", [("tile_deep", 384), ("tile_wide", 256)])
 def test_more_channel_tiles_than_fifteen_bits_count(pra, variant, K):
     N, P = 32768 * 256 + 5 * 256 + 16, 40
