@@ -102,6 +102,9 @@ int check_gemm_common(const void* a_q, const void* w, const int32_t* sorted, con
 // or where there is at most one routed row per expert on average.  Launches with 2 GB of weights and more run long enough
 // for the narrow tiles' slower start not to count, and their deeper prefetch wins earlier: layer us, streaming / narrow, of
 // DeepSeek-V3 at 9 / 16 / 32 tokens 338 / 332, 476 / 469, 656 / 642 (0.2-0.4 GB, Qwen3-30B-A3B at 10 / 16: 60 / 62, 75 / 78.5).
+// The line at 2 GB, from both sides, at 9-16 tokens of evenly spread | Zipf routing: launches of 2.5 GB (128 experts of 4096 x
+// 2560) narrow 0.6-4.7 % ahead | 1-4 % behind, of 2.8 GB (96 of 6144 x 2560) 1.9-2.8 | 3.6-4.6 ahead; of 1.9 GB (128 of 5120 x
+// 1536) 0.1-2.0 | 5-11 ahead, of 1.4 GB between 3.6 ahead and 8 behind.
 constexpr int kStreamMaxRows = 16, kStreamMaxRowsLongStream = 8;
 constexpr int kStreamRowsPerExpert = 1;
 constexpr int kSelfQuantMaxInter = 1024;  // longest reduction moe_i8_gemm_down_bf16 takes for any routing

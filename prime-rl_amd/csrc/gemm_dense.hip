@@ -10,15 +10,14 @@
 // workgroup is the rate at which its operands arrive (about 50 bytes per clock and compute unit), so up
 // to 150 KB of loads stay in flight (S stages) and 128 bytes of every row are fetched at a time.
 //
-// Measured against the grouped families' choice on the same operands (us, rows x channels x reduction):
-// 5x2816x4096 23.9 -> 4.1, 64x4096x4096 30.2 -> 5.9, 333x4096x2048 30.5 -> 8.0, 1115x1792x1536 26.5 -> 7.4,
-// 8170x2384x3200 89.8 -> 74; from a few thousand rows and channels on the 256 x 256 tiles win again
-// (8192x8192x2048 154 against 139): see kConfigs.
+// Kernel durations in a trace, the fastest grouped family (narrow tiles) / this kernel, rows x channels x reduction, us:
+// 64x4096x4096 18.0 / 6.2, 333x4096x2048 14.0 / 8.5, 1115x1792x1536 11.6 / 7.7 (about 3 of each are what the trace shows for
+// a kernel that does nothing); from a few thousand rows and channels on the 256 x 256 tiles win: see kConfigs.
 //
 // Loads go global -> LDS (16 bytes per lane, 8 rows x 128 bytes each) with the 16-byte chunk index
 // XOR-swizzled with the row, as in the grouped families.  They are issued a few at a time between the
 // multiplications of a step: all of them at its start hold up the wavefront until the address unit has
-// taken them (333x4096x2048 8.8 -> 8.0 us).  Activation rows are padded with zeros to a multiple of 128
+// taken them (333x4096x2048 9.0 -> 8.5 us, 333x4096x4096 14.2 -> 13.0, 1000x2384x3200 16.7 -> 15.7).  Activation rows are padded with zeros to a multiple of 128
 // bytes (the quantiser writes them), which lets a reduction of any multiple of 64 run on the same path.
 #include "lds_loads.hpp"
 
@@ -239,8 +238,8 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
       }
     }
     // Through to memory: left in the L2s all results are written back when the launch ends, in one go (linear layers with their
-    // quantisation, 333 x 4096 x 2048 11.6 -> 11.3 us, 1024 x 4096 x 4096 29.5 -> 29.1, 700 x 7168 x 2048 23.0 -> 21.9, 64 x
-    // 4096 x 4096 the same).  (The two wait states: the store reads its data that late, and the compiler, which keeps a write of
+    // quantisation, medians of three runs in turn, us: 700 x 7168 x 2048 23.0 -> 22.3, 1000 x 2384 x 3200 22.7 -> 22.2, 2000 x 4096 x
+    // 4096 46.5 -> 45.8, 1024 x 4096 x 4096 29.7 -> 29.3, 333 x 4096 x 2048 11.7 -> 11.5, 64 x 4096 x 4096 the same).  (The two wait states: the store reads its data that late, and the compiler, which keeps a write of
     // them away from its own stores, does not know of this one.)
     asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1"
                  :: "v"(reinterpret_cast<uint64_t>(p.out + (int64_t)m * width + n)), "v"(v4i{(int)o[0].x, (int)o[0].y, (int)o[1].x, (int)o[1].y})

@@ -13,9 +13,11 @@
 // between its multiplications.  What does not change during a step is decided outside the loop over the steps, of which
 // there is one per kind of wavefront and of loads: with some twenty branches in it a step cost 0.5 us even where all of its
 // rows came from L2, now 0.42; where they come from memory, 0.51-0.55 us a step are 7.6 TB/s of weights.
-// Layer us, before that -> after, with the starting steps of rotation_mask and the divided last rounds of piece_at: 128 experts of
-// 2048 x 768 at 203 tokens 117.2 -> 116.1, 4096 x 1408 with skewed routing at 32 tokens 129 -> 125, 256 experts of 7168 x 2048 at
-// 64 tokens 851 -> 844; gate_up GEMM alone, 16 experts of 4096 x 1408 with 512 rows each 190 -> 160.
+// Before that -> after, with the starting steps of rotation_mask, the divided last rounds of piece_at and the stores described
+// below, in turn on one box, us: the layer of 128 experts of 2048 x 768 at 203 tokens 117.4 -> 115.7, 4096 x 1408 with skewed
+// routing at 32 tokens 128 -> 122, 256 experts of 7168 x 2048 at 64 tokens 874 -> 866 (on another box no difference); gate_up +
+// down, 64 experts of 4096 x 1408 with 20 / 40 rows each 128.5 + 65.9 / 142 + 78.1 -> 118 + 64.1 / 126 + 69.7, 96 of 3072 x 1024
+// 95.0 + 57.0 / 108.9 + 68.3 -> 94.3 + 52.5 / 106.0 + 59.5.
 //
 // A tile is TOK token rows (32 or 64: part of a moe_align block) x 128 weight rows; the reduction runs
 // in steps of 128 bytes and both operands reach LDS by global -> LDS loads (global_load_lds_dwordx4, no

@@ -473,6 +473,10 @@ bool gemm_tile_supports(const GemmArgs& a) {
 // either.  Layer us, deep / wide, by routed rows per expert: 64 147 / 160, 96 162 / 174, 104 175.5 / 179, 108 190 / 180 with
 // 0.2-0.4 GB of weights per launch; 63 395 / 436, 97 492 / 514, 112 551 / 562 (evenly routed 509 / 531), 133 609 / 587 (649 / 556)
 // with 0.7-1.5 GB; 48 1770 / 1842, 64 1939 / 1979, 78 2094 / 2109, 94 2238 / 2234, 109 2368 / 2352 with 3.8-7.5 GB.
+// On launches of 13 layer shapes, by how many per cent the wide tiles take longer at 96 / 104 / 112 rows, evenly spread | Zipf
+// routing: up to 0.56 GB 5..41 / -6..15 / -17..6 | 7..44 / 8..31 / 0..16; 0.69-1.9 GB 7..19 / -7..9 / -8..3 | -1..21 / 1..14 /
+// -1..12.  Beyond, at 64 / 80 / 96 rows: 2.5-2.8 GB 9..13 / 7..15 / 9..16 | 6..7 / 2..4 / -2..5, 3.5 GB 0.5 / -2 / -3.5 | -4 / -4 / -5,
+// 7 GB 8 / 8 / 8 | 4 / 0 / -3: the lower line is for the largest launches, those of 2 to 3 GB could go further.
 bool gemm_tile_prefers_deep(const GemmArgs& a) {
   const bool long_stream = (int64_t)a.num_experts * a.n * a.k >= kLongStreamBytes;
   return a.num_pairs <= (int64_t)(long_stream ? kTileDeepRowsLongStream : kTileDeepRowsPerExpert) * a.num_experts;

@@ -257,8 +257,10 @@ __device__ __forceinline__ uint2 look_up_task(const TileListArgs& p, const TileL
 
 // The last round of an XCD's tasks is rarely full: where its tasks leave at least half of the workgroups idle, each is cut
 // into two or four pieces that run side by side.  A piece does not cost its share (its steps are shorter, not fewer), so
-// nothing is cut where more than half are busy.  Narrow tiles, 34 experts of 4096 x 1408 (3.2 rounds) 76.7 -> 74.2 us; wide
-// tiles, 128 of 2048 x 768 at 8192 tokens (7.2 and 9.7 rounds), the layer 481 -> 478.
+// nothing is cut where more than half are busy.  Whole / in pieces, us: narrow tiles, gate_up, experts of 4096 x 1408 with 20
+// rows each: 24 (2.06 rounds) 54.3 / 51.9, 40 (3.44) 78.4 / 76.3, 64 (5.5) 121.3 / 118.3; 34 (2.92: nothing to cut) 65.5 / 65.4;
+// deep tiles, 4096 x 1408 with skewed routing at 517 tokens, the layer 315.8 / 314.4; wide tiles, 128 of 2048 x 768 at 8192
+// tokens (7.2 and 9.7 rounds), the layer 469.4 / 468.7.
 // Task and piece of place `at` (= workgroup of the XCD + round * stride), of `tasks` of the XCD.
 struct TaskPiece {
   int task;    // -1: none
