@@ -102,9 +102,15 @@ int check_gemm_common(const void* a_q, const void* w, const int32_t* sorted, con
 // or where there is at most one routed row per expert on average.  Launches with 2 GB of weights and more run long enough
 // for the narrow tiles' slower start not to count, and their deeper prefetch wins earlier: layer us, streaming / narrow, of
 // DeepSeek-V3 at 9 / 16 / 32 tokens 338 / 332, 476 / 469, 656 / 642 (0.2-0.4 GB, Qwen3-30B-A3B at 10 / 16: 60 / 62, 75 / 78.5).
-// The line at 2 GB, from both sides, at 9-16 tokens of evenly spread | Zipf routing: launches of 2.5 GB (128 experts of 4096 x
-// 2560) narrow 0.6-4.7 % ahead | 1-4 % behind, of 2.8 GB (96 of 6144 x 2560) 1.9-2.8 | 3.6-4.6 ahead; of 1.9 GB (128 of 5120 x
-// 1536) 0.1-2.0 | 5-11 ahead, of 1.4 GB between 3.6 ahead and 8 behind.
+// Why not lower: 8 rows from 0.5 GB on would cost evenly spread layers of 0.56 and 1.4 GB 1-2 %, 4 rows from 2 GB on
+// layers of 2.5 GB 1-4 %, and which routing a call has the host cannot see.  By how many per cent narrow takes longer, at 5 / 8 /
+// 12 / 16 tokens, evenly spread | Zipf routing, by the weight bytes of the gate_up launch:
+//   0.4 GB (128 experts of 2048 x 768)  8 / 8 / 2 / 6 | 9 / 6 / 4 / -2        0.56 (96 of 3072 x 1024)  2 / -1 / 1 / -2 | 2 / 3 / 2 / -2
+//   1.4 (128 of 4096 x 1408)  1 / 1 / 2 / 2 | -1 / 0 / -5 / -6, with a shared expert -1 / 0 / 1 / 1 | 0 / -1 / -6 / -8
+//   1.9 (128 of 5120 x 1536)  -4 / -2 / -2 / -1 | -7 / -5 / -4 / -5           2.5 (128 of 4096 x 2560)  1 / 2 / 0 / -2 | -4 / 4 / -1 / 0
+//   2.8 (96 of 6144 x 2560)  -1 / -1 / -1 / 0 | -5 / -4 / -2 / -4             7 (256 of 7168 x 2048)  -2 / -2 / -1 / -1 | -5 / -4 / -4 / -6
+// Given away: the negative figures of 0.56 to 1.9 GB at all and of 2.8 and 7 GB at up to 8 tokens.  A launch of 2.5 GB whose down
+// GEMM (1.25) keeps streaming is 2 % slower than with both streaming under Zipf routing, up to 2 % faster evenly routed.
 constexpr int kStreamMaxRows = 16, kStreamMaxRowsLongStream = 8;
 constexpr int kStreamRowsPerExpert = 1;
 constexpr int kSelfQuantMaxInter = 1024;  // longest reduction moe_i8_gemm_down_bf16 takes for any routing

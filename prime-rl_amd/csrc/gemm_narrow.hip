@@ -525,11 +525,14 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 63) / 64 : (a.n + kCh - 1) / kCh;
   p.rotate = rotation_mask(a.k);
   // Results left in the L2s are written back when they are displaced by the weight stream, line by line, and the rest when
-  // the launch ends.  Up to some megabytes that costs less than a write to memory per store, beyond it more.  Left / written
-  // through: down GEMM of 128 experts of 2048 x 768 with 8 / 14 / 20 / 32 / 64 rows each (4 / 7 / 10 / 17 / 34 MB) 35.3 / 36.4 /
-  // 39.4 / 43.2 / 53.0 and 36.3 / 36.9 / 38.4 / 41.4 / 51.8 us, gate_up with 14 / 20 / 32 / 64 rows (3 / 4 / 6 / 13 MB) 60.9 / 63.0 /
-  // 66.7 / 80.4 and 61.2 / 62.5 / 64.6 / 70.5; 64 of 4096 x 1408 with 8 / 20 / 32 / 64 rows, down (4 / 10 / 17 / 34 MB) 57.7 / 63.8 /
-  // 69.6 / 82.2 and 59.5 / 62.8 / 66.2 / 75.6, gate_up (1 / 4 / 6 / 12 MB) 118 / 119.5 / 121 / 142 and 118 / 120 / 123 / 133.5.
+  // the launch ends: with few of them that costs less than a write to memory per store, with many more.  Where the two cross
+  // depends on the shape, and neither the bytes, the rows per expert nor the weights alone say where; 8 MB is the size from
+  // which on writing through won for all shapes but one.  Left / written through, us, at the size where they are even and at 8 MB:
+  // gate_up, 32 experts of 4096 x 1536 below 2 MB, at 6 69.9 / 66.2; 128 of 2048 x 512 2.5 MB, 52.2 / 48.9; 96 of 3072 x 1024
+  // 3.5 MB, 108.5 / 105.2; 128 of 2048 x 768 4.5 MB, 72.1 / 68.0; 64 of 4096 x 1408 6.5 MB, 131.5 / 129.6; down, 32 of 4096 x 1536
+  // 5 MB, 39.6 / 38.0; 64 of 4096 x 1408 5 MB, 64.2 / 62.1; 128 of 2048 x 768 5.5 MB, 39.2 / 38.2; 128 of 2048 x 512 6.5 MB, 31.2 /
+  // 30.1; 96 of 3072 x 1024 10 MB, 50.8 / 52.0.  Below 8 MB the line so gives away up to 6 % (128 of 2048 x 512, gate_up), beyond
+  // up to 2 (the last one); at 2 to 4 MB writing through would cost a down GEMM 1 to 5 %.
   p.through = a.num_pairs * (MODE == kGateUpSilu ? a.n / 2 : a.n) * 2 >= kThroughBytes;
   p.out = a.out;
   const int grid = device_cu_count() / kXcds * kXcds;

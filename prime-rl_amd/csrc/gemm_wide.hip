@@ -227,6 +227,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wide_kernel(WideParams p) {
     }
   };
 
+  // (A last round in pieces makes up to four workgroups read one expert's rows as well, and the hint stays on there: the rounds
+  // before it need it.  gate_up + down us of experts with 256 rows each, hint as it is / off for a range with such a round / last
+  // round whole: 48 of 4096 x 1408 173 + 93 / 194 + 92 / 182 + 92, 136 of 2048 x 512 99 + 75 / 107 + 77 / 104 + 77, 24 of 4096 x
+  // 1408 105 + 53.8 / 112 + 53.8 / 117 + 56; without a full round before it, 8 of 4096 x 1408 43.7 + 24.8 / 44.9 + 24.9 / 50.5 + 26.8,
+  // 4 of them 39.9 + 22.0 / 39.4 + 20.2 / 49.6 + 25.0.)
   bool shared_local = false;
   for (int g = t; g < range.hi - range.lo; g += kThreads) shared_local |= (list.desc[g] >> 20) != (1u << 4);  // rank 0, group size 1
   const bool weights_shared = __builtin_amdgcn_readfirstlane(__syncthreads_or(shared_local ? 1 : 0)) != 0;

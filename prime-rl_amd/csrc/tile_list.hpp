@@ -248,7 +248,8 @@ __device__ __forceinline__ uint2 look_up_task(const TileListArgs& p, const TileL
   const int first = tile0 - (int)((d0 >> 20) & 7u);
   const int T = (int)((d0 >> 24) & 15u);
   const int pos = task - first * p.ntiles;
-  // pos / T: the quotient is below 2^16 (channel tiles) and a half off any integer's edge, the reciprocal good to 1 ulp
+  // pos / T: (pos + 0.5) / T is at least 1 / (2 * kGroupTiles) = 2^-4 away from any integer; with a quotient below 2^16 (channel
+  // tiles), the reciprocal's 1 ulp and the product's rounding are an error below 2^-6
   const int nt = (int)(((float)pos + 0.5f) * __builtin_amdgcn_rcpf((float)T));
   const int tile = first + (pos - nt * T) - range.lo;
   const int e = list.expert[tile];
