@@ -86,7 +86,6 @@ struct NarrowParams {
   int K;
   int B;
   int ntiles;  // channel tiles
-  int rotate;  // mask of the reduction step that a task starts at (rotation_mask)
   bool through;  // results are written through to memory (see launch_mode)
   void* out;
 };
@@ -163,6 +162,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   const int stride = gridDim.x / kXcds;
   const int in_range = total - xcd * per_xcd < per_xcd ? total - xcd * per_xcd : per_xcd;
   const int rounds = (per_xcd + stride - 1) / stride;  // of a phase
+  const int rotate = rotation_mask(K, min(total, p.E * p.ntiles), kCh);
 
   // Candidate tasks of this workgroup: its places in the rounds of its XCD's range, phase by phase (a task of a last round
   // that leaves workgroups idle is cut into pieces of its channels).  Lane i
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
     }
     ld.wbase = p.w + (int64_t)tk.e * p.N * K;
     ld.stream = tk.single;
-    ld.first = (tk.e & p.rotate) * kStepBytes;
+    ld.first = (tk.e & rotate) * kStepBytes;
   };
   auto setup_token_loads = [&](const TileAux& ax, TaskLoads& ld) {
     const int row = (8 * wave + (lane >> 3)) & (TOK - 1);
@@ -523,7 +523,6 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.K = a.k;
   p.B = a.block_size;
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 63) / 64 : (a.n + kCh - 1) / kCh;
-  p.rotate = rotation_mask(a.k);
   // Results left in the L2s are written back when they are displaced by the weight stream, line by line, and the rest when
   // the launch ends: with few of them that costs less than a write to memory per store, with many more.  Where the two cross
   // depends on the shape, and neither the bytes, the rows per expert nor the weights alone say where; 8 MB is the size from

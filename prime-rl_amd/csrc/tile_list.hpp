@@ -278,12 +278,22 @@ __device__ __forceinline__ TaskPiece piece_at(int at, int tasks, int stride) {
 }
 
 // Rows whose stride is a multiple of 4096 bytes have one reduction step of all of them on a few memory channels, and
-// workgroups that start together stay together.  There a task starts its reduction (int32 sums, exact in any order) at step
-// expert & mask and wraps around; all channel tiles of an expert at the same one, so that they still share its token rows (with
-// the channel tile in it too, the wide tiles lost up to 8 %).  gate_up us without / with it, 64 experts, narrow tiles of 16
-// rows each and deep tiles of 64: K = 4096 122 / 116, 144 / 128; 8192 115 / 105, 155 / 139; 12288 137 / 127, 153 / 136; of 1024,
-// 2048, 2560, 3072, 3584, 5120, 6144 and 7168 none moves by more than 1 %.  The wide tiles do not use it: with many rows
-// per expert it changes nothing.
-inline int rotation_mask(int k) { return k % 4096 == 0 ? 31 : 0; }
+// workgroups that start together stay together for a while.  There a task starts its reduction (int32 sums, exact in any order)
+// at step expert & mask and wraps around; all channel tiles of an expert at the same one, so that they still share its token rows
+// (with the channel tile in it too, the wide tiles lost up to 8 %).  Long launches spread by themselves, and it then depends on
+// how far apart the XCDs' ranges lie, and even on where the weights lie, whether it helps: with rows of 8192 bytes and more it
+// costs more than it gives.  gate_up of 92 layer shapes, several allocations each, both sides on the same buffers: by how many per
+// cent it is faster with it, by the weights that the launch reads, mean (worst .. best).  Evenly routed, up to 0.65 GiB 12 (-2 .. 24)
+// with narrow tiles of 16 rows, 13 (-8 .. 32) with deep ones of 64, 0.65-0.8 GiB 6 (-1 .. 19) and 10 (2 .. 27); beyond, K = 4096
+// 0 to 1 (-8 .. 14) and 1 to 3 (-5 .. 19), K = 8192 0.85-1.2 GiB -6 (-13 .. 5) and -2 (-15 .. 15), 1.2-1.7 2 and 2, 1.7-2.2 -1 (-10 .. 5)
+// and -1 (-16 .. 8), 12288 1.7-2.2 -3 and -8.  64 experts of 8192 x 1024 (1 GiB), narrow, 161 us without and 179 with it, of 8192 x
+// 2048, deep, 335 and 385; given away with K = 4096: 64 experts of 2048 channels (1 GiB), narrow, 7 %, 96 of 1408, deep, 4.  Zipf
+// routing: 4 and 6 up to 0.8 GiB, beyond -1 to 1.  Of K = 1024, 2048, 2560, 3072, 3584, 5120, 6144 and 7168 none moves by more than
+// 1 %.  The wide tiles do not use it: with many rows per expert it changes nothing.
+constexpr int64_t kRotateBytes = 819ll << 20;  // 0.8 GiB
+// tasks: of the launch, one for every time that weight_rows rows are read
+__host__ __device__ constexpr int rotation_mask(int k, int tasks, int weight_rows) {
+  return k == 4096 || (k % 4096 == 0 && (int64_t)tasks * weight_rows * k <= kRotateBytes) ? 31 : 0;
+}
 
 }  // namespace moe_i8

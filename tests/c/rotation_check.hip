@@ -1,0 +1,26 @@
+// Host check of which launches start their tasks at different reduction steps.
+#include <cstdio>
+
+#include "tile_list.hpp"
+
+using namespace moe_i8;
+
+int main() {
+  int wrong = 0;
+  auto check = [&](int experts, int k, int inter, bool rotates) {  // gate_up, one tile per expert and channel tile
+    for (int rows : {128, 256})  // narrow and deep tiles
+      if ((rotation_mask(k, experts * (2 * inter / rows), rows) != 0) != rotates)
+        ++wrong, printf("%d experts of %d x %d, tiles of %d rows\n", experts, k, inter, rows);
+  };
+  check(32, 8192, 1024, true);    // 0.5 GiB: 15 and 27 % faster
+  check(64, 8192, 768, true);     // 0.75 GiB
+  check(64, 8192, 1024, false);   // 1 GiB: 10 % slower with narrow tiles
+  check(64, 8192, 2048, false);   // 2 GiB: 8 and 15 % slower
+  check(256, 8192, 2048, false);  // 8 GiB: the product needs 64 bits
+  check(64, 4096, 1024, true);
+  check(256, 4096, 2048, true);   // 4 GiB
+  check(64, 2048, 1024, false);   // no multiple of 4096 bytes
+  check(64, 7168, 1024, false);
+  if (!wrong) printf("ok\n");
+  return wrong != 0;
+}

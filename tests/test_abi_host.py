@@ -238,6 +238,16 @@ def test_masked_store_leaves_the_active_lanes_as_they_were(pra, tmp_path):
     assert not re.search(r"exec, -1\b", text)
 
 
+def test_starting_steps_by_the_length_of_a_launch(pra, tmp_path):
+    import subprocess
+
+    exe = tmp_path / "rotation_check"
+    subprocess.run([pra.build._hipcc(), "--offload-host-only", "-std=c++17", "-I", str(pra.build.CSRC),
+                    str(ROOT / "tests" / "c" / "rotation_check.hip"), "-o", str(exe)], check=True, capture_output=True, text=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0 and run.stdout.strip() == "ok", run.stdout + run.stderr
+
+
 # Which kernels the library picks by itself for the chain of stages at every benchmark point (shape, tokens) and how
 # many launches the chain makes there (calls of a few tokens run without it: test_launches_of_a_call).  These are the kernels the committed measurements were taken on: a retune of the
 # hand-over points between the GEMM families must change this table knowingly.

@@ -78,6 +78,23 @@ def test_tasks_that_start_at_different_steps(pra, oracle, variant, K):
     _check(pra, oracle, variant, [(7 * i) % 40 for i in range(70)], 272, K)
 
 
+@pytest.mark.parametrize("variant", ["narrow", "tile_deep"])
+@pytest.mark.parametrize("inter", [768, 1024])
+@pytest.mark.parametrize("skewed", [False, True])
+def test_starting_steps_of_long_launches(pra, variant, inter, skewed):
+    # 0.75 GiB and 1 GiB of weights in the first GEMM: on either side of the line
+    from _util import inputs_mod
+
+    im = inputs_mod()
+    E, rows = 64, 24
+    d = im.make_inputs(im.LayerShape("s", E=E, k=1, H=8192, I=inter), E * rows, seed=inter, device=DEV, weights_on_device=True)
+    ids = torch.arange(E * rows) % E if not skewed else torch.cat([torch.arange(E), torch.full((400,), 5), torch.arange(E * (rows - 1) - 400) % 50])
+    d.topk_ids.copy_(ids.to(torch.int32).view(-1, 1))
+    kw = d.fused_experts_kwargs()
+    got = pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant=variant)
+    assert torch.equal(got, pra.fused_experts(*d.fused_experts_args(), **kw, gemm_variant="stream"))
+
+
 @pytest.mark.parametrize("steps", [4, 5, 6, 7, 8])
 @pytest.mark.parametrize("most", [20, 60])
 def test_narrow_reductions_around_the_depth_of_the_ring(pra, oracle, steps, most):
