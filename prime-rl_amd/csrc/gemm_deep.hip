@@ -5,7 +5,7 @@
 // 128 bytes through a ring of three 48 KB LDS stages filled by global -> LDS loads two steps ahead.  The MFMA
 // (v_mfma_i32_32x32x32_i8) is used "transposed" (A operand = weight rows): a lane ends up with 4 consecutive channels of a
 // token, a wavefront with a quarter of the channels of the 32-row units th and th + 2.  The tasks are cut into ranges of XCDs
-// and last rounds into pieces of channels as tile_list.hpp says, and start at the steps of rotation_mask.
+// and last rounds into pieces of channels as tile_list.hpp says, and start at the steps of start_step.
 //
 // What bounds it: the weight stream from memory where an expert has one tile (5.2-5.9e12 bytes per second of weights), the
 // path from L2 into LDS (about 1 us a step of 48 KB) where it has several.  Hence:
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   const int per_xcd = uniform((total + kXcds - 1) / kXcds);
   const int my_tasks = min(per_xcd, max(total - xcd * per_xcd, 0));  // of the XCD
   const int stride = gridDim.x / kXcds;
-  const int rotate = rotation_mask(K, min(total, p.tiles.E * p.tiles.ntiles), kCh);
+  const int rotate = rotation(K, min(total, p.tiles.E * p.tiles.ntiles), kCh, p.tiles.E);
   int it = 0;  // tasks handed out
 
   // Looks up tasks n0 .. n0 + kTable - 1 of this workgroup.
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   auto setup_weights = [&](const Task& tk, TaskLoads& ld) {
     ld.wbase = p.w + (int64_t)tk.e * p.N * K;
     ld.stream = tk.single;
-    ld.first = (tk.e & rotate) * kStepBytes;
+    ld.first = start_step(tk.e, rotate) * kStepBytes;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       ld.woff[i] = (uint32_t)weight_row(tk, 32 * wave + 8 * i + (lane >> 3)) * (uint32_t)K + ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;

@@ -13,7 +13,7 @@
 // between its multiplications.  What does not change during a step is decided outside the loop over the steps, of which
 // there is one per kind of wavefront and of loads: with some twenty branches in it a step cost 0.5 us even where all of its
 // rows came from L2, now 0.42; where they come from memory, 0.51-0.55 us a step are 7.6 TB/s of weights.
-// Before that -> after, with the starting steps of rotation_mask, the divided last rounds of piece_at and the stores described
+// Before that -> after, with the starting steps of start_step, the divided last rounds of piece_at and the stores described
 // below, in turn on one box, us: the layer of 128 experts of 2048 x 768 at 203 tokens 117.4 -> 115.7, 4096 x 1408 with skewed
 // routing at 32 tokens 128 -> 122, 256 experts of 7168 x 2048 at 64 tokens 874 -> 866 (on another box no difference); gate_up +
 // down, 64 experts of 4096 x 1408 with 20 / 40 rows each 128.5 + 65.9 / 142 + 78.1 -> 118 + 64.1 / 126 + 69.7, 96 of 3072 x 1024
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   const int stride = gridDim.x / kXcds;
   const int in_range = total - xcd * per_xcd < per_xcd ? total - xcd * per_xcd : per_xcd;
   const int rounds = (per_xcd + stride - 1) / stride;  // of a phase
-  const int rotate = rotation_mask(K, min(total, p.E * p.ntiles), kCh);
+  const int rotate = rotation(K, min(total, p.E * p.ntiles), kCh, p.E);
 
   // Candidate tasks of this workgroup: its places in the rounds of its XCD's range, phase by phase (a task of a last round
   // that leaves workgroups idle is cut into pieces of its channels).  Lane i
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
     }
     ld.wbase = p.w + (int64_t)tk.e * p.N * K;
     ld.stream = tk.single;
-    ld.first = (tk.e & rotate) * kStepBytes;
+    ld.first = start_step(tk.e, rotate) * kStepBytes;
   };
   auto setup_token_loads = [&](const TileAux& ax, TaskLoads& ld) {
     const int row = (8 * wave + (lane >> 3)) & (TOK - 1);

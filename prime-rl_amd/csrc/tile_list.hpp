@@ -279,7 +279,7 @@ __device__ __forceinline__ TaskPiece piece_at(int at, int tasks, int stride) {
 
 // Rows whose stride is a multiple of 4096 bytes have one reduction step of all of them on a few memory channels, and
 // workgroups that start together stay together for a while.  There a task starts its reduction (int32 sums, exact in any order)
-// at step expert & mask and wraps around; all channel tiles of an expert at the same one, so that they still share its token rows
+// at start_step and wraps around; all channel tiles of an expert at the same one, so that they still share its token rows
 // (with the channel tile in it too, the wide tiles lost up to 8 %).  Long launches spread by themselves, and it then depends on
 // how far apart the XCDs' ranges lie, and even on where the weights lie, whether it helps: with rows of 8192 bytes and more it
 // costs more than it gives.  gate_up of 92 layer shapes, several allocations each, both sides on the same buffers: by how many per
@@ -290,10 +290,17 @@ __device__ __forceinline__ TaskPiece piece_at(int at, int tasks, int stride) {
 // 2048, deep, 335 and 385; given away with K = 4096: 64 experts of 2048 channels (1 GiB), narrow, 7 %, 96 of 1408, deep, 4.  Zipf
 // routing: 4 and 6 up to 0.8 GiB, beyond -1 to 1.  Of K = 1024, 2048, 2560, 3072, 3584, 5120, 6144 and 7168 none moves by more than
 // 1 %.  The wide tiles do not use it: with many rows per expert it changes nothing.
+// The starts of few experts are spread over all 4096 bytes: next to each other, one step apart, they share channels again.  One
+// step apart / spread, us, narrow tiles: 8 experts of 8192 x 1536 40 / 36 (all at the first step: 38.5), of 8192 x 2048 53 / 45, 16
+// of 4096 x 1536 39 / 35, of 8192 x 1024 48 / 44; deep: 16 of 4096 x 2048 57 / 49, of 8192 x 2048 107 / 92; of 17 layer shapes none slower.
 constexpr int64_t kRotateBytes = 819ll << 20;  // 0.8 GiB
-// tasks: of the launch, one for every time that weight_rows rows are read
-__host__ __device__ constexpr int rotation_mask(int k, int tasks, int weight_rows) {
-  return k == 4096 || (k % 4096 == 0 && (int64_t)tasks * weight_rows * k <= kRotateBytes) ? 31 : 0;
+constexpr int kStartSteps = 32;                // of 128 bytes
+// Steps between the starts of two experts that follow each other; 0: all tasks start at the first one.  tasks: of the launch, one
+// for every time that weight_rows rows are read.
+__host__ __device__ constexpr int rotation(int k, int tasks, int weight_rows, int experts) {
+  if (k % 4096 != 0 || (k > 4096 && (int64_t)tasks * weight_rows * k > kRotateBytes)) return 0;
+  return experts < kStartSteps ? kStartSteps / experts : 1;
 }
+__host__ __device__ constexpr int start_step(int expert, int rotation) { return expert * rotation % kStartSteps; }
 
 }  // namespace moe_i8

@@ -9,7 +9,7 @@ int main() {
   int wrong = 0;
   auto check = [&](int experts, int k, int inter, bool rotates) {  // gate_up, one tile per expert and channel tile
     for (int rows : {128, 256})  // narrow and deep tiles
-      if ((rotation_mask(k, experts * (2 * inter / rows), rows) != 0) != rotates)
+      if ((rotation(k, experts * (2 * inter / rows), rows, experts) != 0) != rotates)
         ++wrong, printf("%d experts of %d x %d, tiles of %d rows\n", experts, k, inter, rows);
   };
   check(32, 8192, 1024, true);    // 0.5 GiB: 15 and 27 % faster
@@ -21,6 +21,16 @@ int main() {
   check(256, 4096, 2048, true);   // 4 GiB
   check(64, 2048, 1024, false);   // no multiple of 4096 bytes
   check(64, 7168, 1024, false);
+  // the starts of up to 32 experts: all different, and as far apart as they can be
+  for (int experts = 1; experts <= 300; ++experts) {
+    const int r = rotation(4096, experts * 8, 256, experts);
+    bool used[kStartSteps] = {};
+    for (int e = 0; e < experts; ++e) {
+      const int s = start_step(e, r);
+      if (s < 0 || s >= kStartSteps || (experts <= kStartSteps && (used[s] || s < e * (kStartSteps / experts)))) ++wrong, printf("start of %d of %d\n", e, experts);
+      else used[s] = true;
+    }
+  }
   if (!wrong) printf("ok\n");
   return wrong != 0;
 }

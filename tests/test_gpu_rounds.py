@@ -73,9 +73,10 @@ def test_pieces_of_tiles_of_several_sizes(pra, oracle, variant, counts):
 
 @pytest.mark.parametrize("variant", ["narrow", "tile_deep", "tile_wide", "stream"])
 @pytest.mark.parametrize("K", [4096, 8192])
-def test_tasks_that_start_at_different_steps(pra, oracle, variant, K):
-    # 70 experts: the starting step wraps around twice
-    _check(pra, oracle, variant, [(7 * i) % 40 for i in range(70)], 272, K)
+@pytest.mark.parametrize("experts", [1, 5, 8, 31, 33, 70])
+def test_tasks_that_start_at_different_steps(pra, oracle, variant, K, experts):
+    # 70 experts: the starting step wraps around twice; below 32 the starts are several steps apart
+    _check(pra, oracle, variant, [(7 * i + 3) % 40 for i in range(experts)], 272, K)
 
 
 @pytest.mark.parametrize("variant", ["narrow", "tile_deep"])
