@@ -40,7 +40,17 @@ struct DenseParams {
   int ntiles;
 };
 
-template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int WPE>
+// Results of a launch up to which they are written through to memory: left in the L2s all of them are written back when the launch
+// ends, in one go.  Beyond, the L2s have written most of them back by then, and stores to memory cost more.  Linear layers with
+// their quantisation, 270 problems of 20..8192 rows, 512..14336 channels and a reduction of 512 / 1024 / 2048 / 4096 / 7168, by how
+// many per cent faster on average through to memory, by the size of the results: up to 1 MB 0, 1-2 MB 0 / 1 / 1 / 1 / 1, 2-4 MB 4 /
+// 4 / 3 / 2 / 1, 4-8 MB 7 / 6 / 4 / 2 / 1, 8-16 MB 13 / 11 / 5 / 2 / 0, 16-32 MB 9 / 6 for the first two (from here on the others run on
+// the wide tiles), 32-64 MB 3; of 512 and 640, 68 MB 2, 94 MB 0, 109 MB -1, 128 MB and more -3 (8192 x 512 x 8192 66.6 us left in
+// the L2s, 70.0 through to memory).
+constexpr int64_t kThroughBytes = 96 << 20;
+
+// THROUGH: results are written through to memory.  (A template argument: decided at run time it cost the smallest launches 0.2 of 7 us.)
+template <int MODE, bool THROUGH, int TM, int TN, int KS, int WM, int WN, int S, int WPE>
 __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(DenseParams p) {
   constexpr int G = WM * WN;                   // wavefronts of a group: they share the group's stages
   constexpr int kThreads = 64 * KS * G;
@@ -237,17 +247,11 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
         o[h] = down_epilogue4(v, as, ws, 1.0f);
       }
     }
-    // Through to memory: left in the L2s all results are written back when the launch ends, in one go (linear layers with their
-    // quantisation, medians of three runs in turn, us: 700 x 7168 x 2048 23.0 -> 22.3, 1000 x 2384 x 3200 22.7 -> 22.2, 2000 x 4096 x
-    // 4096 46.5 -> 45.8, 1024 x 4096 x 4096 29.7 -> 29.3, 333 x 4096 x 2048 11.7 -> 11.5, 64 x 4096 x 4096 the same).  (The two wait states: the store reads its data that late, and the compiler, which keeps a write of
-    // them away from its own stores, does not know of this one.)
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1"
-                 :: "v"(reinterpret_cast<uint64_t>(p.out + (int64_t)m * width + n)), "v"(v4i{(int)o[0].x, (int)o[0].y, (int)o[1].x, (int)o[1].y})
-                 : "memory");
+    store16(p.out + (int64_t)m * width + n, v4i{(int)o[0].x, (int)o[0].y, (int)o[1].x, (int)o[1].y}, THROUGH);
   }
 }
 
-template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int WPE>
+template <int MODE, bool THROUGH, int TM, int TN, int KS, int WM, int WN, int S, int WPE>
 hipError_t launch_config(const DenseParams& p0, hipStream_t stream) {
   DenseParams p = p0;
   constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;
@@ -255,7 +259,7 @@ hipError_t launch_config(const DenseParams& p0, hipStream_t stream) {
   p.mtiles = (p.M + TM - 1) / TM;
   p.ntiles = (width + kOut - 1) / kOut;
   const int per_xcd = (p.mtiles * p.ntiles + kXcds - 1) / kXcds;
-  hipLaunchKernelGGL((gemm_dense_kernel<MODE, TM, TN, KS, WM, WN, S, WPE>), dim3((unsigned)(per_xcd * kXcds)),
+  hipLaunchKernelGGL((gemm_dense_kernel<MODE, THROUGH, TM, TN, KS, WM, WN, S, WPE>), dim3((unsigned)(per_xcd * kXcds)),
                      dim3(64 * KS * WM * WN), 0, stream, p);
   return hipGetLastError();
 }
@@ -272,12 +276,14 @@ struct Config {
   float per_round;  // us
   float per_k;      // us per 1024 reduction bytes
   float rate;       // 1e15 operations per second
-  hipError_t (*gate_up)(const DenseParams&, hipStream_t);
-  hipError_t (*down)(const DenseParams&, hipStream_t);
+  hipError_t (*gate_up[2])(const DenseParams&, hipStream_t);  // more than kThroughBytes of results, up to that
+  hipError_t (*down[2])(const DenseParams&, hipStream_t);
 };
-#define MOE_I8_DENSE(TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, RATE)                 \
-  {TM, TN, PER_CU, START, ROUND, PER_K, RATE, launch_config<kGateUpSilu, TM, TN, KS, WM, WN, S, WPE>, \
-   launch_config<kDown, TM, TN, KS, WM, WN, S, WPE>}
+// (so many results in tiles of fewer rows and channels are no launch that the estimates would choose: they are always written through)
+#define MOE_I8_DENSE(TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, RATE)                              \
+  {TM, TN, PER_CU, START, ROUND, PER_K, RATE,                                                                     \
+   {launch_config<kGateUpSilu, TM * TN < 128 * 128, TM, TN, KS, WM, WN, S, WPE>, launch_config<kGateUpSilu, true, TM, TN, KS, WM, WN, S, WPE>}, \
+   {launch_config<kDown, TM * TN < 128 * 128, TM, TN, KS, WM, WN, S, WPE>, launch_config<kDown, true, TM, TN, KS, WM, WN, S, WPE>}}
 // The constants are least-squares fits to 150 problems drawn over 1..8192 rows, 512..16384 channels and
 // 512..8192 reduction bytes (rms error of a fit 6-14 %).  The configuration the estimates pick takes on
 // average 0.8 % longer than the fastest one of the table.
@@ -294,7 +300,7 @@ const Config kConfigs[] = {
 // The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Over 216 problems of 500..8192 rows
 // the choice takes on average 0.5 %, at most 27 % (4032 x 12736 x 896: 88.5 against 69.6 us), longer than the faster of
 // both; constants fitted to the present wide tiles alone chose worse (0.7-1.0 %).
-const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, nullptr, nullptr};
+const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, {}, {}};
 
 float estimate(const Config& c, int64_t m, int64_t n, int64_t k) {
   const int64_t tiles = ((m + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn);
@@ -337,7 +343,8 @@ hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream) {
   p.K = a.k;
   p.lda = dense_row_stride(a.k);
   const Config* c = pick(a.m, a.n, a.k, false);
-  return a.mode == kGateUpSilu ? c->gate_up(p, stream) : c->down(p, stream);
+  const bool through = a.m * (a.mode == kGateUpSilu ? a.n / 2 : a.n) * 2 <= kThroughBytes;
+  return (a.mode == kGateUpSilu ? c->gate_up : c->down)[through](p, stream);
 }
 
 }  // namespace moe_i8

@@ -97,16 +97,6 @@ __device__ __forceinline__ void load_to_lds_dword(const void* base, uint32_t off
                : "memory", "m0");
 }
 
-// through: written through to memory instead of left in the L2.  (The two wait states behind that store: a store of more than
-// 8 bytes reads its data that late, and the compiler, which keeps a write of them away from its own stores, does not know of
-// this one.)
-__device__ __forceinline__ void store16(void* to, const v4i& v, bool through) {
-  if (through)
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" :: "v"(reinterpret_cast<uint64_t>(to)), "v"(v) : "memory");
-  else
-    *reinterpret_cast<v4i*>(to) = v;
-}
-
 struct Task {
   int e;          // expert; -1 = no more work
   int n0, n1;     // its channels

@@ -72,6 +72,15 @@ __device__ __forceinline__ void store16_through(void* to, const uint4& v, uint64
                : "v"(reinterpret_cast<uint64_t>(to)), "v"(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}), "s"(lanes)
                : "memory", "scc");
 }
+// through: written through to memory instead of left in the L2.  (The two wait states behind that store: a store of more than
+// 8 bytes reads its data that late, and the compiler, which keeps a write of them away from its own stores, does not know of
+// this one.)
+__device__ __forceinline__ void store16(void* to, const v4i& v, bool through) {
+  if (through)
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" :: "v"(reinterpret_cast<uint64_t>(to)), "v"(v) : "memory");
+  else
+    *reinterpret_cast<v4i*>(to) = v;
+}
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)p);
 }

@@ -101,6 +101,17 @@ def test_gated_mlp_of_a_few_rows_equals_the_rows_of_a_larger_call(pra, H, I, m):
     assert torch.equal(small, big[:m]), int((small != big[:m]).sum())
 
 
+@pytest.mark.parametrize("m", [6144, 6145, 8192])
+def test_results_around_the_size_that_is_written_through(pra, m):
+    # 96 MB of results at 6144 rows; rows are independent
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, 512, generator=g).to(torch.bfloat16).to(DEV)
+    w, s = (t.to(DEV) for t in _weights(8192, 512, g))
+    big = pra.apply_int8_linear(x, w, s)
+    for at in (0, 2000, m - 200):
+        assert torch.equal(big[at:at + 200], pra.apply_int8_linear(x[at:at + 200].contiguous(), w, s)), at
+
+
 def test_caller_owned_workspace_for_the_dense_ops(pra):
     """``workspace=`` of ``apply_int8_linear`` and ``w8a8_mlp``: the caller's buffer is used (bit-equal to the
     default call, also when the buffer starts out as garbage) and one that is too small is refused."""
