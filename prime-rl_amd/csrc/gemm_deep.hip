@@ -59,6 +59,7 @@ struct DeepParams {
   int B;
   TileListArgs tiles;
   int ascend;  // expert_ids is known to ascend over the used blocks (it comes from moe_align)
+  int rotate;  // steps between the starts of two experts that follow each other (rotation)
   void* out;
 };
 
@@ -125,7 +126,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   const int per_xcd = uniform((total + kXcds - 1) / kXcds);
   const int my_tasks = min(per_xcd, max(total - xcd * per_xcd, 0));  // of the XCD
   const int stride = gridDim.x / kXcds;
-  const int rotate = rotation(K, min(total, p.tiles.E * p.tiles.ntiles), kCh, p.tiles.E);
   int it = 0;  // tasks handed out
 
   // Looks up tasks n0 .. n0 + kTable - 1 of this workgroup.
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_deep_kernel(DeepParams p) {
   auto setup_weights = [&](const Task& tk, TaskLoads& ld) {
     ld.wbase = p.w + (int64_t)tk.e * p.N * K;
     ld.stream = tk.single;
-    ld.first = start_step(tk.e, rotate) * kStepBytes;
+    ld.first = start_step(tk.e, p.rotate) * kStepBytes;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       ld.woff[i] = (uint32_t)weight_row(tk, 32 * wave + 8 * i + (lane >> 3)) * (uint32_t)K + ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;
@@ -483,6 +483,7 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.tiles.blocks = (int)(a.sorted_cap / a.block_size);
   p.tiles.identity = a.identity ? 1 : 0;
   p.ascend = a.expert_ids_ascend && a.num_experts <= 2 * kThreads ? 1 : 0;
+  p.rotate = rotation(a.k, (int64_t)a.num_experts * a.n * a.k, a.num_experts);
   p.out = a.out;
   const dim3 grid((unsigned)(device_cu_count() / kXcds * kXcds));
   hipLaunchKernelGGL((gemm_deep_kernel<MODE>), grid, dim3(kThreads), 0, stream, p);

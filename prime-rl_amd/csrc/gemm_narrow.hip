@@ -86,6 +86,7 @@ struct NarrowParams {
   int K;
   int B;
   int ntiles;  // channel tiles
+  int rotate;  // steps between the starts of two experts that follow each other (rotation)
   bool through;  // results are written through to memory (see launch_mode)
   void* out;
 };
@@ -152,7 +153,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
   const int stride = gridDim.x / kXcds;
   const int in_range = total - xcd * per_xcd < per_xcd ? total - xcd * per_xcd : per_xcd;
   const int rounds = (per_xcd + stride - 1) / stride;  // of a phase
-  const int rotate = rotation(K, min(total, p.E * p.ntiles), kCh, p.E);
 
   // Candidate tasks of this workgroup: its places in the rounds of its XCD's range, phase by phase (a task of a last round
   // that leaves workgroups idle is cut into pieces of its channels).  Lane i
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_narrow_kernel(NarrowParams p
     }
     ld.wbase = p.w + (int64_t)tk.e * p.N * K;
     ld.stream = tk.single;
-    ld.first = start_step(tk.e, rotate) * kStepBytes;
+    ld.first = start_step(tk.e, p.rotate) * kStepBytes;
   };
   auto setup_token_loads = [&](const TileAux& ax, TaskLoads& ld) {
     const int row = (8 * wave + (lane >> 3)) & (TOK - 1);
@@ -513,6 +513,7 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.K = a.k;
   p.B = a.block_size;
   p.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 63) / 64 : (a.n + kCh - 1) / kCh;
+  p.rotate = rotation(a.k, (int64_t)a.num_experts * a.n * a.k, a.num_experts);
   // Results left in the L2s are written back when they are displaced by the weight stream, line by line, and the rest when
   // the launch ends: with few of them that costs less than a write to memory per store, with many more.  Where the two cross
   // depends on the shape, and neither the bytes, the rows per expert nor the weights alone say where; 8 MB is the size from

@@ -281,24 +281,24 @@ __device__ __forceinline__ TaskPiece piece_at(int at, int tasks, int stride) {
 // workgroups that start together stay together for a while.  There a task starts its reduction (int32 sums, exact in any order)
 // at start_step and wraps around; all channel tiles of an expert at the same one, so that they still share its token rows
 // (with the channel tile in it too, the wide tiles lost up to 8 %).  Long launches spread by themselves, and it then depends on
-// how far apart the XCDs' ranges lie, and even on where the weights lie, whether it helps: with rows of 8192 bytes and more it
-// costs more than it gives.  gate_up of 92 layer shapes, several allocations each, both sides on the same buffers: by how many per
-// cent it is faster with it, by the weights that the launch reads, mean (worst .. best).  Evenly routed, up to 0.65 GiB 12 (-2 .. 24)
-// with narrow tiles of 16 rows, 13 (-8 .. 32) with deep ones of 64, 0.65-0.8 GiB 6 (-1 .. 19) and 10 (2 .. 27); beyond, K = 4096
-// 0 to 1 (-8 .. 14) and 1 to 3 (-5 .. 19), K = 8192 0.85-1.2 GiB -6 (-13 .. 5) and -2 (-15 .. 15), 1.2-1.7 2 and 2, 1.7-2.2 -1 (-10 .. 5)
-// and -1 (-16 .. 8), 12288 1.7-2.2 -3 and -8.  64 experts of 8192 x 1024 (1 GiB), narrow, 161 us without and 179 with it, of 8192 x
-// 2048, deep, 335 and 385; given away with K = 4096: 64 experts of 2048 channels (1 GiB), narrow, 7 %, 96 of 1408, deep, 4.  Zipf
-// routing: 4 and 6 up to 0.8 GiB, beyond -1 to 1.  Of K = 1024, 2048, 2560, 3072, 3584, 5120, 6144 and 7168 none moves by more than
-// 1 %.  The wide tiles do not use it: with many rows per expert it changes nothing.
+// how far apart the XCDs' ranges lie, and even on where the weights lie, whether it helps.  gate_up of 92 layer shapes, several
+// allocations each, both sides on the same buffers: by how many per cent it is faster with it, by the weights of all experts, mean
+// (worst .. best).  Evenly routed, up to 0.65 GiB 12 (-2 .. 24) with narrow tiles of 16 rows, 13 (-8 .. 32) with deep ones of 64,
+// 0.65-0.8 GiB 6 (-1 .. 19) and 10 (2 .. 27); beyond, narrow, K = 4096 0 to 1 (-8 .. 14), 8192 0.85-1.2 GiB -6 (-13 .. 5), 1.2-1.7 2,
+// 1.7-2.2 -1 (-10 .. 5), 12288 -3 to 1; deep, K = 4096 1 to 3 (-5 .. 19), 8192 -2 (-15 .. 15), 2, -1 (-16 .. 8), 12288 -8 to 3.  64
+// experts of 8192 x 1024 (1 GiB), narrow, 161 us without and 179 with it, of 8192 x 2048, deep, 335 and 385.  Zipf routing: 4 and 6 up
+// to 0.8 GiB, beyond -1 to 1, but layers of 17 to 80 tokens, whose launches read a part of the experts, 1 to 4 (128 experts of 4096 x
+// 1408, 1536 and 2560), -3 (64 of 8192 x 1024) and -4 (32 of 8192 x 2048).  Hence up to 0.8 GiB, K = 4096 at any size.  Given away:
+// 64 experts of 4096 x 2048 (1 GiB), narrow, 5 to 7 %, 96 of 4096 x 1408, deep, 4.  Of K = 1024, 2048, 2560, 3072, 3584, 5120, 6144
+// and 7168 none moves by more than 1 %.  The wide tiles do not use it: with many rows per expert it changes nothing.
 // The starts of few experts are spread over all 4096 bytes: next to each other, one step apart, they share channels again.  One
 // step apart / spread, us, narrow tiles: 8 experts of 8192 x 1536 40 / 36 (all at the first step: 38.5), of 8192 x 2048 53 / 45, 16
 // of 4096 x 1536 39 / 35, of 8192 x 1024 48 / 44; deep: 16 of 4096 x 2048 57 / 49, of 8192 x 2048 107 / 92; of 17 layer shapes none slower.
 constexpr int64_t kRotateBytes = 819ll << 20;  // 0.8 GiB
 constexpr int kStartSteps = 32;                // of 128 bytes
-// Steps between the starts of two experts that follow each other; 0: all tasks start at the first one.  tasks: of the launch, one
-// for every time that weight_rows rows are read.
-__host__ __device__ constexpr int rotation(int k, int tasks, int weight_rows, int experts) {
-  if (k % 4096 != 0 || (k > 4096 && (int64_t)tasks * weight_rows * k > kRotateBytes)) return 0;
+// Steps between the starts of two experts that follow each other; 0: all tasks start at the first one.
+__host__ __device__ constexpr int rotation(int k, int64_t weight_bytes, int experts) {
+  if (k % 4096 != 0 || (k > 4096 && weight_bytes > kRotateBytes)) return 0;
   return experts < kStartSteps ? kStartSteps / experts : 1;
 }
 __host__ __device__ constexpr int start_step(int expert, int rotation) { return expert * rotation % kStartSteps; }
