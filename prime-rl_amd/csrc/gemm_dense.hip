@@ -276,14 +276,13 @@ struct Config {
   float per_round;  // us
   float per_k;      // us per 1024 reduction bytes
   float rate;       // 1e15 operations per second
-  hipError_t (*gate_up[2])(const DenseParams&, hipStream_t);  // more than kThroughBytes of results, up to that
-  hipError_t (*down[2])(const DenseParams&, hipStream_t);
+  hipError_t (*gate_up)(const DenseParams&, hipStream_t);
+  hipError_t (*down)(const DenseParams&, hipStream_t);
 };
-// (so many results in tiles of fewer rows and channels are no launch that the estimates would choose: they are always written through)
-#define MOE_I8_DENSE(TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, RATE)                              \
-  {TM, TN, PER_CU, START, ROUND, PER_K, RATE,                                                                     \
-   {launch_config<kGateUpSilu, TM * TN < 128 * 128, TM, TN, KS, WM, WN, S, WPE>, launch_config<kGateUpSilu, true, TM, TN, KS, WM, WN, S, WPE>}, \
-   {launch_config<kDown, TM * TN < 128 * 128, TM, TN, KS, WM, WN, S, WPE>, launch_config<kDown, true, TM, TN, KS, WM, WN, S, WPE>}}
+#define MOE_I8_DENSE_STORES(THROUGH, TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, RATE)          \
+  {TM, TN, PER_CU, START, ROUND, PER_K, RATE, launch_config<kGateUpSilu, THROUGH, TM, TN, KS, WM, WN, S, WPE>, \
+   launch_config<kDown, THROUGH, TM, TN, KS, WM, WN, S, WPE>}
+#define MOE_I8_DENSE(...) MOE_I8_DENSE_STORES(true, __VA_ARGS__)
 // The constants are least-squares fits to 150 problems drawn over 1..8192 rows, 512..16384 channels and
 // 512..8192 reduction bytes (rms error of a fit 6-14 %).  The configuration the estimates pick takes on
 // average 0.8 % longer than the fastest one of the table.
@@ -300,7 +299,14 @@ const Config kConfigs[] = {
 // The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Over 216 problems of 500..8192 rows
 // the choice takes on average 0.5 %, at most 27 % (4032 x 12736 x 896: 88.5 against 69.6 us), longer than the faster of
 // both; constants fitted to the present wide tiles alone chose worse (0.7-1.0 %).
-const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, {}, {}};
+const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, nullptr, nullptr};
+
+// The largest tiles of kConfigs for results of more than kThroughBytes (no launch that the estimates would choose has so many in
+// smaller ones).
+const Config kLarge[] = {
+    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 4, 4, 2, 1, 1.75f, 3.18f, 3.49f, 1.59f),
+    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 2, 2, 2, 2, 0.71f, 3.66f, 5.59f, 1.72f),
+};
 
 float estimate(const Config& c, int64_t m, int64_t n, int64_t k) {
   const int64_t tiles = ((m + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn);
@@ -343,8 +349,10 @@ hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream) {
   p.K = a.k;
   p.lda = dense_row_stride(a.k);
   const Config* c = pick(a.m, a.n, a.k, false);
-  const bool through = a.m * (a.mode == kGateUpSilu ? a.n / 2 : a.n) * 2 <= kThroughBytes;
-  return (a.mode == kGateUpSilu ? c->gate_up : c->down)[through](p, stream);
+  if (a.m * (a.mode == kGateUpSilu ? a.n / 2 : a.n) * 2 > kThroughBytes)
+    for (const Config& l : kLarge)
+      if (l.tm == c->tm && l.tn == c->tn && l.per_cu == c->per_cu) c = &l;
+  return a.mode == kGateUpSilu ? c->gate_up(p, stream) : c->down(p, stream);
 }
 
 }  // namespace moe_i8
