@@ -14,7 +14,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libmoe_i8.so"
 SOURCES = ["align.hip", "quant.hip", "sum.hip", "router.hip", "gemm_stream.hip", "gemm_tile.hip", "gemm_wide.hip",
-           "gemm_deep.hip", "gemm_narrow.hip", "gemm_dense.hip", "gemm_split.hip", "few_tokens.hip", "dense_few.hip", "api.hip"]
+           "gemm_deep.hip", "gemm_narrow.hip", "gemm_dense.hip", "gemm_dense_rows.hip", "gemm_split.hip", "few_tokens.hip", "dense_few.hip", "api.hip"]
 HOST_PATH = PKG_DIR / "_host.so"  # the Python entry points' native call path (CPython extension, no device code)
 PROBE_LIB_PATH = PKG_DIR / "libmoe_i8_probe.so"  # the benchmark's MFMA rate probe, a library of its own
 

@@ -1005,17 +1005,24 @@ bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
   return a0 < b0 + (uintptr_t)b_bytes && b0 < a0 + (uintptr_t)a_bytes;
 }
 
-// A few rows: the launch quantises them itself.  Whether it runs, unless a family is demanded or the output overlaps
-// the rows: every workgroup reads them all, while others already write.  (The other kernels read a copy of the rows
-// that a launch of its own has quantised.)
-bool takes_dense_few(const void* x, const moe_i8::GemmArgs& g, int variant) {
+// How a GEMM of a dense entry point runs: a few rows, or some tens to hundreds of them, are quantised by the product's own launch,
+// unless a family is demanded or the output overlaps the rows: every workgroup reads rows that others need while some already
+// write.  (The other kernels read a copy of the rows that a launch of its own has quantised.)
+enum DenseWay { kQuantised, kFew, kRows };
+DenseWay dense_way(const void* x, moe_i8::GemmArgs g, int variant) {
   const int64_t width = g.mode == moe_i8::kGateUpSilu ? g.n / 2 : g.n;
-  return variant == MOE_I8_GEMM_AUTO && moe_i8::dense_few_takes(g.num_pairs, g.n, g.k) && aligned16(x) && aligned16(g.w) &&
-         !overlap(x, 2 * g.num_pairs * g.k, g.out, 2 * g.num_pairs * width);
+  if (variant != MOE_I8_GEMM_AUTO || !aligned16(x) || !aligned16(g.w) || overlap(x, 2 * g.num_pairs * g.k, g.out, 2 * g.num_pairs * width))
+    return kQuantised;
+  const bool few = moe_i8::dense_few_takes(g.num_pairs, g.n, g.k);
+  g.tile_geometry = moe_i8::kTileWide;
+  if (moe_i8::dense_rows_takes(g.num_pairs, g.n, g.k, few, moe_i8::gemm_tile_supports(g))) return kRows;
+  return few ? kFew : kQuantised;
 }
-int run_dense_few(const void* x, const moe_i8::GemmArgs& g, hipStream_t stream) {
+int run_unquantised(DenseWay way, const void* x, const moe_i8::GemmArgs& g, hipStream_t stream) {
+  if (int rc = check_dense_gemm(g, MOE_I8_GEMM_AUTO)) return rc;
   const moe_i8::DenseFewArgs d{g.mode, static_cast<const uint16_t*>(x), g.w, g.w_scale, static_cast<uint16_t*>(g.out), (int)g.num_pairs, g.n, g.k};
-  return check_launch(moe_i8::launch_dense_few(d, stream), "dense_few");
+  return way == kFew ? check_launch(moe_i8::launch_dense_few(d, stream), "dense_few")
+                     : check_launch(moe_i8::launch_dense_rows(d, stream), "dense_rows");
 }
 
 // The ties-to-even row quantiser of the dense path; `padded`: rows for the dense kernel; `route`: its
@@ -1073,10 +1080,7 @@ int moe_i8_w8a8_linear(const void* x, const int8_t* w, const float* w_scale, voi
   float* a1 = reinterpret_cast<float*>(ws + c.a1);
   const moe_i8::GemmArgs g = dense_group(moe_i8::kDown, c, ws, x_q, a1, w, w_scale, out, m, n, k);
   const WorkspaceTurn turn(workspace);
-  if (takes_dense_few(x, g, variant)) {
-    if (int rc = check_dense_gemm(g, variant)) return rc;
-    return run_dense_few(x, g, s);
-  }
+  if (const DenseWay way = dense_way(x, g, variant)) return run_unquantised(way, x, g, s);
   const bool dense = takes_dense_kernel(g, variant);
   if (int rc = dense_quant(x, m, k, x_q, a1, dense, !dense, c, ws, s)) return rc;
   return run_dense(g, variant, s);
@@ -1100,15 +1104,18 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   const moe_i8::GemmArgs gu = dense_group(moe_i8::kGateUpSilu, c, ws, x_q, a1, w13, w13_scale, ws + c.act, m, 2 * inter, hidden);
   moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, ws, act_q, a2, w2, w2_scale, out, m, hidden, inter);
   const WorkspaceTurn turn(workspace);
-  if (takes_dense_few(x, gu, variant) && takes_dense_few(ws + c.act, dg, variant)) {
-    if (int rc = check_dense_gemm(gu, variant)) return rc;
-    if (int rc = check_dense_gemm(dg, variant)) return rc;
-    if (int rc = run_dense_few(x, gu, s)) return rc;
-    return run_dense_few(ws + c.act, dg, s);
-  }
+  const DenseWay way_gu = dense_way(x, gu, variant), way_dg = dense_way(ws + c.act, dg, variant);
+  if (way_gu)
+    if (int rc = check_dense_gemm(dg, variant)) return rc;  // before anything is launched
   const bool dense_gu = takes_dense_kernel(gu, variant), dense_dg = takes_dense_kernel(dg, variant);
-  if (int rc = dense_quant(x, m, hidden, x_q, a1, dense_gu, !dense_gu || !dense_dg, c, ws, s)) return rc;
-  if (int rc = run_dense(gu, variant, s)) return rc;
+  const bool route_dg = !way_dg && !dense_dg;  // the down GEMM reads the routing that a quantiser's launch writes
+  if (way_gu) {
+    if (int rc = run_unquantised(way_gu, x, gu, s)) return rc;
+  } else {
+    if (int rc = dense_quant(x, m, hidden, x_q, a1, dense_gu, !dense_gu || route_dg, c, ws, s)) return rc;
+    if (int rc = run_dense(gu, variant, s)) return rc;
+  }
+  if (way_dg) return run_unquantised(way_dg, ws + c.act, dg, s);
   // Few rows on the streaming family: its down GEMM quantises them itself (ties to even here), one
   // launch less.
   if (variant == MOE_I8_GEMM_STREAM && m <= kDenseSelfQuantRows && inter <= kSelfQuantMaxInter) {
@@ -1122,7 +1129,7 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
     dg.a_round_even = true;
     return check_launch(moe_i8::launch_gemm_stream(dg, s), "gemm_stream");
   }
-  if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, false, c, ws, s)) return rc;
+  if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, way_gu && route_dg, c, ws, s)) return rc;
   return run_dense(dg, variant, s);
 }
 

@@ -344,6 +344,7 @@ int dense_row_stride(int k);
 // Whether the dense kernel is the one for this problem; `wide_allowed`: the 256-row tiles of the LDS-tiled
 // family can run it too and are preferred where they are expected to be faster.
 bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed);
+float gemm_dense_estimate(int64_t m, int n, int k, bool wide_allowed);  // us of the product
 hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream);
 
 // The same for a few rows, which the launch quantises itself (ties to even).
@@ -360,6 +361,10 @@ struct DenseFewArgs {
 constexpr int kDenseFewRows = 16;
 bool dense_few_takes(int64_t m, int n, int k);
 hipError_t launch_dense_few(const DenseFewArgs& a, hipStream_t stream);
+// The dense kernel that quantises its own rows (ties to even): whether it is the one for this problem.  `few`: the kernel of a few
+// rows would run it otherwise; `wide_allowed` as in gemm_dense_takes.
+bool dense_rows_takes(int64_t m, int n, int k, bool few, bool wide_allowed);
+hipError_t launch_dense_rows(const DenseFewArgs& a, hipStream_t stream);
 
 // The whole layer of a few tokens in two launches: act holds tokens * top_k rows of inter bf16.
 struct FewTokensArgs {

@@ -337,6 +337,8 @@ bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed) {
   return pick(m, n, k, wide_allowed) != &kWide;
 }
 
+float gemm_dense_estimate(int64_t m, int n, int k, bool wide_allowed) { return estimate(*pick(m, n, k, wide_allowed), m, n, k); }
+
 hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream) {
   DenseParams p{};
   p.a_q = a.a_q;

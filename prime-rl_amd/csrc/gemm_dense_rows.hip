@@ -1,0 +1,341 @@
+// Dense int8 GEMM that quantises its own rows, for gfx950: linear layers and gated MLPs of about ten to some hundreds of rows.
+//
+// At this size a dense layer is two dependent launches, quantisation and product, and little else: 100 rows x 1000 channels x 1024
+// took 7.7 us for 0.1 us of bytes and 0.3 of operations.  Here a workgroup quantises the token rows of its tile itself, into
+// LDS, where they stay for the whole reduction; the weights run through a ring of stages as in the dense kernel, whose split of
+// the reduction, swizzle and epilogue it shares.  What bounds it: one latency for the rows, the vector units' work on them (about
+// 5 operations per element, 1 us for 32 rows of 1024), which hides the latency of the first weights, then the steps of the ring.
+// Repeating the quantisation per channel tile is what limits it: 64 rows per workgroup cost as much as the launch that they save
+// (64 x 64 tiles 6.9-7.7 us, never faster), and reductions beyond 4096 do not fit.
+// us per call, quantisation launch and dense kernel / here: 17 rows x 2672 channels x 896 6.75 / 3.9, 103 x 992 x 1024 7.7 / 4.2,
+// 309 x 512 x 896 7.2 / 4.9, 54 x 1248 x 1152 7.1 / 4.4, 122 x 8448 x 704 7.5 / 6.2, 45 x 624 x 2880 7.3 / 5.7; over 343 problems of
+// 17..1000 rows x 512..14336 channels x 192..4200, taken where the estimates say so, 22 % faster on average.
+#include "lds_loads.hpp"
+#include "quant_body.hpp"
+
+namespace moe_i8 {
+namespace {
+
+constexpr int kXcds = 8;
+constexpr int kWaves = 8;
+
+struct DenseRowsParams {
+  const uint16_t* x;     // [M, K] bf16
+  const int8_t* w;       // [N, K]
+  const float* w_scale;  // [N]
+  uint16_t* out;         // [M, N] (down) or [M, N / 2] (gate_up)
+  int M;
+  int N;
+  int K;
+  int mtiles;
+  int ntiles;
+};
+
+// TM x TN: tile; KS: groups of wavefronts that split the reduction; WM x WN: wavefronts of a group; S: stages; V: 1 KB vectors of a
+// bf16 row (K <= 512 * V).
+template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int V>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRowsParams p) {
+  constexpr int G = WM * WN;
+  static_assert(KS * G == kWaves && TM % kWaves == 0 && S >= 2);
+  constexpr int kThreads = 64 * kWaves;
+  constexpr int L = TN / 8 / G;                // 1 KB loads per wavefront and step
+  static_assert(TN % (8 * G) == 0 && (S - 2) * L <= 63);
+  constexpr int R = TM / kWaves;               // rows that a wavefront quantises
+  constexpr int kGroupBytes = TN * kStepBytes;
+  constexpr int kStage = KS * kGroupBytes;
+  constexpr int kPiece = TM * kStepBytes;      // 128 reduction bytes of all rows
+  constexpr int kRowsAt = S * kStage;          // quantised rows, behind the stages: [piece][row][128]
+  constexpr int MT = TM / WM, NT = TN / WN;
+  constexpr int MF = MT % 32 == 0 && NT % 32 == 0 ? 32 : 16;
+  constexpr int MI = MT / MF, NI = NT / MF;
+  using F = Mfma<MF>;
+  constexpr int kPartRow = TN * 4 + 16;        // bytes of a token's row of partial sums
+  constexpr int kPart = TM * kPartRow;
+  constexpr int kUsed = kRowsAt + V * 4 * kPiece;
+  constexpr int kLds = kUsed > KS * kPart ? kUsed : KS * kPart;
+  static_assert(kLds + 4 * (TM + TN) <= 160 * 1024, "LDS");
+  __shared__ __align__(16) char lds[kLds];
+  __shared__ __align__(16) float scales[(TN + 63) / 64 * 64 + TM];
+  constexpr int kRowScales = (TN + 63) / 64 * 64;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = wave / G, wg = wave % G;
+  const int wm = wg / WN, wn = wg % WN;
+
+  // tile of this workgroup: the workgroups of one XCD (id % 8) take neighbouring tiles, token tiles fastest
+  const int total = p.mtiles * p.ntiles;
+  const int per_xcd = (total + kXcds - 1) / kXcds;
+  const int tile = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+  if (tile >= total || (int)(blockIdx.x / kXcds) >= per_xcd) return;
+  const int m0 = tile % p.mtiles * TM;
+  const int nt = tile / p.mtiles;
+  const int inter = p.N / 2;
+  const int K = p.K;
+
+  // ---- the tile's rows, the first things in flight (rows behind the last one: that one again) ----
+  const int vectors = (K + 511) / 512;
+  uint4 v[R][V];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int row = m0 + wave * R + r;
+    const uint4* x = reinterpret_cast<const uint4*>(p.x + (int64_t)(row < p.M ? row : p.M - 1) * K);
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (i < vectors) v[r][i] = i * kWave + lane < K / kQuantVec ? x[i * kWave + lane] : make_uint4(0u, 0u, 0u, 0u);
+  }
+
+  auto weight_row = [&](int r) {  // LDS weight row r of the tile -> row of w
+    if constexpr (MODE == kGateUpSilu) {
+      const int half = TN / 2;
+      const int ch = nt * half + (r < half ? r : r - half);
+      return (ch < inter ? ch : inter - 1) + (r < half ? 0 : inter);
+    } else {
+      const int n = nt * TN + r;
+      return n < p.N ? n : p.N - 1;
+    }
+  };
+  const uint32_t lds0 = lds_address(lds);
+  uint32_t off[L];
+  bool hi[L];  // chunk in the upper 64 bytes of the step
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int r = (wg * L + i) * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ swizzle_of_row(r);
+    off[i] = (uint32_t)weight_row(r) * (uint32_t)K + chunk * 16;
+    hi[i] = chunk >= 4;
+  }
+  const int nk = (K + kStepBytes - 1) / kStepBytes;  // 128-byte pieces of the reduction; piece s * KS + g is this group's step s
+  const int steps = (nk + KS - 1) / KS;
+  const int mine = (nk - g + KS - 1) / KS;
+  const bool ragged = K % kStepBytes != 0;
+  auto issue = [&](int s, int slot, int from, int to) {
+    const int piece = s * KS + g;
+    const uint32_t base = lds0 + slot * kStage + g * kGroupBytes + wg * L * 1024;
+    // Last 64 bytes of a ragged reduction: the rows are zero there, so the weights may be anything readable: the lower half
+    // again (the next row would lie past the end of the matrix for the last one).
+    const uint32_t back = ragged && piece == nk - 1 ? 64u : 0u;
+#pragma unroll
+    for (int i = 0; i < L; ++i)
+      if (i >= from && i < to) load_to_lds_16(p.w + piece * kStepBytes, off[i] - (hi[i] ? back : 0u), base + i * 1024);
+  };
+
+  float top[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    top[r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (i < vectors) top[r] = fmaxf(top[r], absmax8(v[r][i]));
+    asm volatile("" ::"v"(top[r]));  // the rows are waited for here, in front of the loads that follow
+  }
+  for (int j0 = wave * 64; j0 < TN; j0 += kThreads)
+    load_to_lds_4(p.w_scale + weight_row(j0 + lane < TN ? j0 + lane : TN - 1), lds_address(scales + j0));
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < mine) issue(s, s, 0, L);
+
+  // ---- quantisation, while the first weights are on their way ----
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int row = wave * R + r;
+    const float absmax = fmaxf(wave_max(top[r]), 1e-10f);
+    const float inv = 127.0f / absmax;
+    if (lane == 0) scales[kRowScales + row] = absmax / 127.0f;
+    char* to = lds + kRowsAt + row * kStepBytes + (((lane >> 1) & 7) ^ swizzle_of_row(row)) * 16 + (lane & 1) * 8;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (i < vectors) *reinterpret_cast<uint2*>(to + (4 * i + (lane >> 4)) * kPiece) = quant8<true>(v[r][i], inv);
+  }
+
+  int w_ld[NI], x_ld[MI], chunk[F::kSub];
+  const int lrow = lane % MF;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) w_ld[i] = (wn * NT + i * MF + lrow) * kStepBytes;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) x_ld[i] = kRowsAt + (wm * MT + i * MF + lrow) * kStepBytes;
+#pragma unroll
+  for (int kk = 0; kk < F::kSub; ++kk) chunk[kk] = ((kk * (64 / MF) + lane / MF) ^ swizzle_of_row(lrow)) * 16;
+
+  typename F::Acc acc[NI][MI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+#pragma unroll
+      for (int r = 0; r < F::kRegs; ++r) acc[i][j][r] = 0;
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (not __syncthreads: the loads stay in flight)
+
+  int slot = 0;
+  for (int s = 0; s < steps; ++s) {
+    // this wavefront's loads of step s are in (those of the next S - 2 steps, as far as there are any, stay in flight)
+    const int later = mine - 1 - s;
+    wait_groups<L, S - 2>(later < 0 ? 0 : later);
+    if constexpr (G > 1)
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int fill = slot == 0 ? S - 1 : slot - 1;  // the slot of step s - 1: everybody is done reading it
+    const bool more = s + S - 1 < mine;
+    if (s < mine) {
+      const char* st = lds + slot * kStage + g * kGroupBytes;
+      const char* rows = lds + (s * KS + g) * kPiece;
+      v4i a[2][NI], b[2][MI];
+      auto read = [&](int kk) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) a[kk & 1][i] = *reinterpret_cast<const v4i*>(st + w_ld[i] + chunk[kk]);
+#pragma unroll
+        for (int j = 0; j < MI; ++j) b[kk & 1][j] = *reinterpret_cast<const v4i*>(rows + x_ld[j] + chunk[kk]);
+      };
+      read(0);
+#pragma unroll
+      for (int kk = 0; kk < F::kSub; ++kk) {
+        if (kk + 1 < F::kSub) read(kk + 1);
+        // the loads of the step S - 1 ahead go out a few at a time between the multiplications
+        // (with two stages they have only this step to arrive in: all of them first)
+        if (more && (S > 2 || kk == 0)) issue(s + S - 1, fill, S > 2 ? kk * L / F::kSub : 0, S > 2 ? (kk + 1) * L / F::kSub : L);
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < MI; ++j) acc[i][j] = F::mul(a[kk & 1][i], b[kk & 1][j], acc[i][j]);
+      }
+    }
+    slot = slot + 1 == S ? 0 : slot + 1;
+  }
+  wait_vmcnt<0>();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // ---- partial sums of the KS groups meet in LDS, [group][token][channel] ----
+  char* part = lds + g * kPart;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+#pragma unroll
+      for (int q = 0; q < F::kRegs / 4; ++q) {
+        const int tok = wm * MT + j * MF + lrow;
+        const int ch = wn * NT + i * MF + (MF == 32 ? 8 * q : 0) + 4 * (lane / MF);
+        *reinterpret_cast<v4i*>(part + tok * kPartRow + ch * 4) =
+            v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+      }
+  __syncthreads();
+
+  constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;  // output channels of the tile
+  constexpr int kPieces = kOut / 8;                        // 16-byte pieces of an output row
+  const int width = MODE == kGateUpSilu ? inter : p.N;
+  auto total4 = [&](int tok, int ch, int (&v)[4]) {
+    v4i s = *reinterpret_cast<const v4i*>(lds + tok * kPartRow + ch * 4);
+#pragma unroll
+    for (int k = 1; k < KS; ++k) s += *reinterpret_cast<const v4i*>(lds + k * kPart + tok * kPartRow + ch * 4);
+    v[0] = s[0], v[1] = s[1], v[2] = s[2], v[3] = s[3];
+  };
+  for (int u = threadIdx.x; u < TM * kPieces; u += kThreads) {
+    const int tok = u / kPieces, c = u % kPieces * 8;
+    const int m = m0 + tok, n = nt * kOut + c;
+    if (m >= p.M || n >= width) continue;
+    const float as = scales[kRowScales + tok];
+    uint2 o[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int ch = c + 4 * h;
+      int v[4];
+      total4(tok, ch, v);
+      const float4 ws = *reinterpret_cast<const float4*>(scales + ch);
+      if constexpr (MODE == kGateUpSilu) {
+        int up[4];
+        total4(tok, ch + kOut, up);
+        o[h] = silu_mul_epilogue4(v, up, as, ws, *reinterpret_cast<const float4*>(scales + ch + kOut));
+      } else {
+        o[h] = down_epilogue4(v, as, ws, 1.0f);
+      }
+    }
+    store16(p.out + (int64_t)m * width + n, v4i{(int)o[0].x, (int)o[0].y, (int)o[1].x, (int)o[1].y}, true);
+  }
+}
+
+template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int V>
+hipError_t launch_config(const DenseRowsParams& p0, hipStream_t stream) {
+  DenseRowsParams p = p0;
+  constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;
+  const int width = MODE == kGateUpSilu ? p.N / 2 : p.N;
+  p.mtiles = (p.M + TM - 1) / TM;
+  p.ntiles = (width + kOut - 1) / kOut;
+  const int per_xcd = (p.mtiles * p.ntiles + kXcds - 1) / kXcds;
+  hipLaunchKernelGGL((gemm_dense_rows_kernel<MODE, TM, TN, KS, WM, WN, S, V>), dim3((unsigned)(per_xcd * kXcds)), dim3(64 * kWaves), 0,
+                     stream, p);
+  return hipGetLastError();
+}
+
+// One way to cut the problem up and what it costs: a launch takes about
+//   start + rounds * (per_round + per_k * K / 1024) + waves * (per_wave + per_wave_k * K / 1024)
+// where a round is as many workgroups as the device holds at a time and a wave as many as it has compute units (the same, where a
+// unit holds one: then the second term is 0).  Least-squares fits to 540 problems of 2..1000 rows x 512..24576 channels x 192..4200
+// (rms error of a fit 4-7 %).  The choice between these and the launches they replace takes on average 0.6 % longer than the fastest
+// way, 1.9 % with up to 16 rows.
+struct Config {
+  int tm, tn;   // tile
+  int longest;  // reduction
+  int per_cu;   // workgroups a compute unit holds at a time
+  float start, per_round, per_k, per_wave, per_wave_k;  // us
+  hipError_t (*gate_up)(const DenseRowsParams&, hipStream_t);
+  hipError_t (*down)(const DenseRowsParams&, hipStream_t);
+};
+#define MOE_I8_ROWS(TM, TN, KS, WM, WN, S, V, PER_CU, START, ROUND, PER_K, WAVE, WAVE_K)                                          \
+  {TM, TN, 512 * V, PER_CU, START, ROUND, PER_K, WAVE, WAVE_K, launch_config<kGateUpSilu, TM, TN, KS, WM, WN, S, V>, \
+   launch_config<kDown, TM, TN, KS, WM, WN, S, V>}
+const Config kConfigs[] = {
+    MOE_I8_ROWS(16, 32, 4, 1, 2, 3, 2, 2, 1.97f, 1.87f, -1.06f, -0.06f, 1.37f),
+    MOE_I8_ROWS(16, 64, 2, 1, 4, 3, 2, 2, 1.89f, 1.94f, -0.87f, -0.11f, 1.62f),
+    MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 2, 1, 1.23f, 2.27f, 1.54f, 0.0f, 0.0f),
+    MOE_I8_ROWS(32, 128, 2, 1, 4, 3, 2, 1, 0.76f, 3.27f, 2.32f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 32, 8, 1, 1, 3, 4, 1, 1.12f, 2.41f, 0.83f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 64, 4, 1, 2, 3, 4, 1, 1.02f, 2.57f, 1.18f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 4, 1, 0.78f, 2.70f, 1.83f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 32, 8, 1, 1, 2, 8, 1, 0.17f, 2.82f, 1.12f, 0.0f, 0.0f),
+};
+
+const Config* pick(int64_t m, int n, int k, float* us) {
+  const Config* best = nullptr;
+  const float kb = (float)k / 1024.0f, cus = (float)device_cu_count();
+  for (const Config& c : kConfigs) {
+    if (k > c.longest || (c.longest > 1024 && k <= c.longest / 2)) continue;  // (fitted to reductions between the two)
+    const float tiles = (float)(((m + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn));
+    const float t = c.start + ceilf(tiles / (cus * c.per_cu)) * (c.per_round + c.per_k * kb) + ceilf(tiles / cus) * (c.per_wave + c.per_wave_k * kb);
+    if (!best || t < *us) best = &c, *us = t;
+  }
+  return best;
+}
+
+}  // namespace
+
+// A row more costs the kernel of a few rows a pass over its registers' weights, this one nothing up to 16: us there / here at 8 rows
+// 9168 x 1280 8.5 / 5.0, 11376 x 640 6.7 / 4.3, 2928 x 1408 4.5 / 4.5, 1776 x 3584 6.0 / 6.6; at 5 9264 x 1024 5.4 / 4.5, 3024 x 1024
+// 3.9 / 4.1.  Its time is about 3.48 + 0.0603 W + 0.0262 m W + 0.05 m us with W = n * k / 10^6 (rms error 9 %); it keeps what is within
+// 7 % of that (5 rows of 4096 x 1408, 4.83 by the estimates against 4.67: the gated MLP 10.0 / 10.75) and up to 4 rows everything,
+// where it is the faster one or even on all but the widest matrices.  A quantisation launch adds about 3.06 us + 0.69 per 5 MB that it moves to the
+// dense kernels' estimate.
+bool dense_rows_takes(int64_t m, int n, int k, bool few, bool wide_allowed) {
+  if (m < 5 || (int64_t)n * k >= (1ll << 32) || n % 16 != 0 || k % 64 != 0) return false;
+  float us = 0.0f;
+  if (!pick(m, n, k, &us)) return false;
+  const float w = (float)n * (float)k * 1e-6f;
+  return us < (few ? 0.93f * (3.48f + 0.0603f * w + 0.0262f * (float)m * w + 0.05f * (float)m)
+                   : gemm_dense_estimate(m, n, k, wide_allowed) + 3.06f + 0.69f * (float)m * (float)k * (3.0f / 5e6f));
+}
+
+hipError_t launch_dense_rows(const DenseFewArgs& a, hipStream_t stream) {
+  DenseRowsParams p{};
+  p.x = a.x;
+  p.w = a.w;
+  p.w_scale = a.w_scale;
+  p.out = a.out;
+  p.M = a.m;
+  p.N = a.n;
+  p.K = a.k;
+  float us;
+  const Config* c = pick(a.m, a.n, a.k, &us);
+  if (!c) return hipErrorInvalidValue;
+  return a.mode == kGateUpSilu ? c->gate_up(p, stream) : c->down(p, stream);
+}
+
+}  // namespace moe_i8

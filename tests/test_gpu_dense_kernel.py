@@ -49,3 +49,28 @@ def test_few_rows_in_one_launch(pra, oracle, M, N, K):
         w2 = torch.randint(-127, 128, (K, inter), generator=g, dtype=torch.int8).to(DEV)
         args = (x.to(DEV), w[: 2 * inter].to(DEV), (s[: 2 * inter] * 0.1).to(DEV), w2, (torch.rand(K, generator=g) * 1e-3).to(DEV))
         assert torch.equal(pra.w8a8_mlp(*args), pra.w8a8_mlp(*args, gemm_variant="stream"))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (16, 16, 64), (17, 560, 576), (33, 1040, 1024), (64, 864, 384), (5, 10880, 384), (100, 2064, 960), (500, 272, 1024),
+    (13, 11568, 256), (31, 8208, 512), (43, 11616, 640), (65, 8464, 192), (245, 2752, 1024), (600, 1552, 448), (54, 1248, 1152),
+    (16, 4112, 2048), (28, 8208, 1088), (30, 8176, 2048), (47, 5008, 1984), (9, 16912, 1344), (45, 624, 2880), (17, 1040, 4096),
+    (15, 528, 2112), (16, 2544, 3968),
+])
+def test_rows_quantised_by_their_tiles(pra, oracle, M, N, K):
+    """Rows quantised by the workgroups whose tiles they are in: every tile and length of its registers, rows and channels
+    that fill no tile, reductions of odd multiples of 64 and shorter than a workgroup's split, one round and several."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    x[0, : K // 2] = torch.arange(K // 2) % 255 - 127  # exact ties and the largest values
+    x[M // 2] = 0
+    x[M - 1, K - 1] = float("nan")  # skipped in the maximum, 0 as a value
+    clean = x.nan_to_num(0.0)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    s = torch.rand(N, generator=g) * 0.008 + 0.002
+    assert torch.equal(pra.apply_int8_linear(x.to(DEV), w.to(DEV), s.to(DEV)).cpu(), oracle.w8a8_linear(clean, w, s))
+    inter = N // 2 // 64 * 64
+    if inter:
+        w2 = torch.randint(-127, 128, (K, inter), generator=g, dtype=torch.int8).to(DEV)
+        args = (w[: 2 * inter].to(DEV), (s[: 2 * inter] * 0.1).to(DEV), w2, (torch.rand(K, generator=g) * 1e-3).to(DEV))
+        assert torch.equal(pra.w8a8_mlp(x.to(DEV), *args), pra.w8a8_mlp(clean.to(DEV), *args, gemm_variant="stream"))
