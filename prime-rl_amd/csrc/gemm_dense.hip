@@ -285,7 +285,11 @@ struct Config {
 #define MOE_I8_DENSE(...) MOE_I8_DENSE_STORES(true, __VA_ARGS__)
 // The constants are least-squares fits to 150 problems drawn over 1..8192 rows, 512..16384 channels and
 // 512..8192 reduction bytes (rms error of a fit 6-14 %).  The configuration the estimates pick takes on
-// average 0.8 % longer than the fastest one of the table.
+// average 0.8 % longer than the fastest one of the table.  (192 x 192, fitted later to 432 problems of 40..8192 rows, for those
+// that are one round of it and more than one of 128 x 128, us with the fastest of the others / with it: 930 rows x 9776 channels x
+// 3776 65.7 / 49.5, 1096 x 7232 x 1472 32.4 / 25.4, 2634 x 3392 x 2112 44.1 / 35.0, 2060 x 4192 x 704 21.3 / 17.5.  Of 128 x 192,
+// 192 x 128, 64 x 256, 128 x 256, 256 x 128, 64 x 192 and 128 x 64 each is the fastest here and there, by up to 15 %, but where the
+// estimates, which are off by 5-8 %, would choose them they lose as often.)
 const Config kConfigs[] = {
     MOE_I8_DENSE(16, 16, 8, 1, 1, 2, 4, 1, 2.45f, 0.53f, 0.38f, 1e9f),
     MOE_I8_DENSE(16, 32, 8, 1, 1, 3, 2, 1, 1.49f, 1.46f, 0.58f, 1e9f),
@@ -295,6 +299,7 @@ const Config kConfigs[] = {
     MOE_I8_DENSE(64, 128, 2, 2, 2, 3, 2, 1, 0.55f, 3.15f, 2.15f, 1.58f),
     MOE_I8_DENSE(128, 128, 1, 2, 4, 4, 2, 1, 1.75f, 3.18f, 3.49f, 1.59f),
     MOE_I8_DENSE(128, 128, 1, 2, 2, 2, 2, 2, 0.71f, 3.66f, 5.59f, 1.72f),
+    MOE_I8_DENSE(192, 192, 1, 2, 4, 3, 2, 1, 0.0f, 4.84f, 8.71f, 1.58f),
 };
 // The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Over 216 problems of 500..8192 rows
 // the choice takes on average 0.5 %, at most 27 % (4032 x 12736 x 896: 88.5 against 69.6 us), longer than the faster of
@@ -306,6 +311,7 @@ const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, nullptr, nullptr}
 const Config kLarge[] = {
     MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 4, 4, 2, 1, 1.75f, 3.18f, 3.49f, 1.59f),
     MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 2, 2, 2, 2, 0.71f, 3.66f, 5.59f, 1.72f),
+    MOE_I8_DENSE_STORES(false, 192, 192, 1, 2, 4, 3, 2, 1, 0.0f, 4.84f, 8.71f, 1.58f),
 };
 
 float estimate(const Config& c, int64_t m, int64_t n, int64_t k) {
