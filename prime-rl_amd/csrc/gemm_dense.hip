@@ -60,12 +60,19 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
   constexpr int kGroupBytes = (TM + TN) * kStepBytes;
   constexpr int kStage = KS * kGroupBytes;
   constexpr int MT = TM / WM, NT = TN / WN;
+  constexpr int kPartRow = TN * 4 + 16;        // bytes of a token's row of partial sums
+  constexpr int kPart = TM * kPartRow;
+  // Sums that are not partial, of tiles whose int32 sums would not fit or that are pairs of half as many results: finished in registers,
+  // they meet in LDS as bf16 (gate_up of 128 x 128: 1-1.4 % of an MLP; plain results of it, 1-3 % slower, stay below).
+  // For gate_up 16 weight rows of 32 are then gate rows and 16 the matching up rows: a lane has both in its registers.
+  constexpr bool kFinished = KS == 1 && (TM * TN > 128 * 128 || MODE == kGateUpSilu);
+  constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;  // output channels of the tile
+  constexpr int kOutRow = kOut * 2 + 16;
   constexpr int MF = MT % 32 == 0 && NT % 32 == 0 ? 32 : 16;
   constexpr int MI = MT / MF, NI = NT / MF;
   using F = Mfma<MF>;
-  constexpr int kPartRow = TN * 4 + 16;        // bytes of a token's row of partial sums
-  constexpr int kPart = TM * kPartRow;
-  constexpr int kLds = S * kStage > KS * kPart ? S * kStage : KS * kPart;
+  constexpr int kResults = kFinished ? TM * kOutRow : KS * kPart;
+  constexpr int kLds = S * kStage > kResults ? S * kStage : kResults;
   static_assert(kLds + 4 * (TM + TN) <= 160 * 1024, "LDS");
   __shared__ __align__(16) char lds[kLds];
   __shared__ __align__(16) float scales[(TM + TN + 63) / 64 * 64];
@@ -89,7 +96,10 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
   const int inter = p.N / 2;
 
   auto weight_row = [&](int r) {  // LDS weight row r of the tile -> row of w
-    if constexpr (MODE == kGateUpSilu) {
+    if constexpr (MODE == kGateUpSilu && kFinished) {
+      const int ch = nt * kOut + r / 32 * 16 + r % 16;
+      return (ch < inter ? ch : inter - 1) + (r % 32 < 16 ? 0 : inter);
+    } else if constexpr (MODE == kGateUpSilu) {
       const int half = TN / 2;
       const int ch = nt * half + (r < half ? r : r - half);
       return (ch < inter ? ch : inter - 1) + (r < half ? 0 : inter);
@@ -203,6 +213,46 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
   wait_vmcnt<0>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
+  constexpr int kPieces = kOut / 8;                        // 16-byte pieces of an output row
+  const int width = MODE == kGateUpSilu ? inter : p.N;
+  if constexpr (kFinished) {
+    static_assert(MODE != kGateUpSilu || NT % 32 == 0, "gate and up rows in turns of 16");
+    constexpr int kSets = MODE == kGateUpSilu ? NI * F::kRegs / 8 : NI * F::kRegs / 4;  // of 4 channels of a lane and token
+#pragma unroll
+    for (int j = 0; j < MI; ++j) {
+      const int tok = wm * MT + j * MF + lrow;
+      const float as = scales[TN + tok];
+#pragma unroll
+      for (int t = 0; t < kSets; ++t) {
+        // set t: registers 4 * q .. of block i; of gate_up the up rows are the ones 16 weight rows on
+        const int i = MF == 32 ? t / (MODE == kGateUpSilu ? 2 : 4) : MODE == kGateUpSilu ? 2 * t : t;
+        const int q = MF == 32 ? t % (MODE == kGateUpSilu ? 2 : 4) : 0;
+        const int at = wn * NT + i * MF + 8 * q + 4 * (lane / MF);  // row of the tile
+        const float4 ws = *reinterpret_cast<const float4*>(scales + at);
+        int v[4], up[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[r] = acc[i][j][4 * q + r];
+          if constexpr (MODE == kGateUpSilu) up[r] = MF == 32 ? acc[i][j][(4 * q + 8 + r) % F::kRegs] : acc[(i + 1) % NI][j][r];
+        }
+        uint2 o;
+        if constexpr (MODE == kGateUpSilu)
+          o = silu_mul_epilogue4(v, up, as, ws, *reinterpret_cast<const float4*>(scales + at + 16));
+        else
+          o = down_epilogue4(v, as, ws, 1.0f);
+        const int c = MODE == kGateUpSilu ? at / 32 * 16 + at % 16 : at;
+        *reinterpret_cast<uint2*>(lds + tok * kOutRow + c * 2) = o;
+      }
+    }
+    __syncthreads();
+    for (int u = threadIdx.x; u < TM * kPieces; u += kThreads) {
+      const int tok = u / kPieces, c = u % kPieces * 8;
+      const int m = m0 + tok, n = nt * kOut + c;
+      if (m < p.M && n < width) store16(p.out + (int64_t)m * width + n, *reinterpret_cast<const v4i*>(lds + tok * kOutRow + c * 2), THROUGH);
+    }
+    return;
+  }
+
   // ---- partial sums of the KS groups meet in LDS, [group][token][channel] ----
   char* part = lds + g * kPart;
 #pragma unroll
@@ -218,9 +268,6 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
       }
   __syncthreads();
 
-  constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;  // output channels of the tile
-  constexpr int kPieces = kOut / 8;                        // 16-byte pieces of an output row
-  const int width = MODE == kGateUpSilu ? inter : p.N;
   auto total4 = [&](int tok, int ch, int (&v)[4]) {
     v4i s = *reinterpret_cast<const v4i*>(lds + tok * kPartRow + ch * 4);
 #pragma unroll
@@ -265,7 +312,9 @@ hipError_t launch_config(const DenseParams& p0, hipStream_t stream) {
 }
 
 // One way to cut the problem up and what it costs.  A launch takes about
-//   start + rounds * per_round + max(rounds * per_k * K / 1024, padded operations / rate)
+//   start + rounds * per_round + max((full rounds * per_k + the last one's share) * K / 1024, padded operations / rate),
+// where a last round of a few tiles takes per_k_few and one of many up to per_k (the chip's power is the limit: its clock falls as
+// more matrix cores work)
 // where a round is as many workgroups as the device holds at a time: small tiles are bound by a round's
 // latency and by how fast a compute unit takes in its two operands, large ones by the matrix pipes at the
 // clock the power limit allows.
@@ -274,58 +323,72 @@ struct Config {
   int per_cu;       // workgroups a compute unit holds at a time
   float start;      // us
   float per_round;  // us
-  float per_k;      // us per 1024 reduction bytes
+  float per_k;      // us per 1024 reduction bytes of a full round
+  float per_k_few;  // ... of a nearly empty one
   float rate;       // 1e15 operations per second
   hipError_t (*gate_up)(const DenseParams&, hipStream_t);
   hipError_t (*down)(const DenseParams&, hipStream_t);
 };
-#define MOE_I8_DENSE_STORES(THROUGH, TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, RATE)          \
-  {TM, TN, PER_CU, START, ROUND, PER_K, RATE, launch_config<kGateUpSilu, THROUGH, TM, TN, KS, WM, WN, S, WPE>, \
+#define MOE_I8_DENSE_STORES(THROUGH, TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, PER_K_FEW, RATE)         \
+  {TM, TN, PER_CU, START, ROUND, PER_K, PER_K_FEW, RATE, launch_config<kGateUpSilu, THROUGH, TM, TN, KS, WM, WN, S, WPE>, \
    launch_config<kDown, THROUGH, TM, TN, KS, WM, WN, S, WPE>}
 #define MOE_I8_DENSE(...) MOE_I8_DENSE_STORES(true, __VA_ARGS__)
-// The constants are least-squares fits to 150 problems drawn over 1..8192 rows, 512..16384 channels and
-// 512..8192 reduction bytes (rms error of a fit 6-14 %).  The configuration the estimates pick takes on
-// average 0.8 % longer than the fastest one of the table.  (192 x 192, fitted later to 432 problems of 40..8192 rows, for those
-// that are one round of it and more than one of 128 x 128, us with the fastest of the others / with it: 930 rows x 9776 channels x
-// 3776 65.7 / 49.5, 1096 x 7232 x 1472 32.4 / 25.4, 2634 x 3392 x 2112 44.1 / 35.0, 2060 x 4192 x 704 21.3 / 17.5.  Of 128 x 192,
-// 192 x 128, 64 x 256, 128 x 256, 256 x 128, 64 x 192 and 128 x 64 each is the fastest here and there, by up to 15 %, but where the
-// estimates, which are off by 5-8 %, would choose them they lose as often.)
+// The constants are least-squares fits: those of the tiles up to 64 x 64 to 150 problems drawn over 1..8192 rows, 512..16384
+// channels and 512..8192 reduction bytes (rms error of a fit 6-14 %), the others' to 320 problems of 250..8192 rows (5-6 %, the
+// grouped family's 11 %), over which the configuration that the estimates pick takes on average 0.2 % longer than the fastest one of
+// the table (with the same cost for each round, and a rate, it took 1.1 % longer).
+// The four largest are for problems that fill the chip badly in 128 x 128 tiles (more rounds of less) and in 256 x 256 ones (half a
+// round): linear layers, us without / with them, 1818 rows x 4384 channels x 3008 54.0 / 39.1, 4868 x 3456 x 7680 164 / 138, 6508 x
+// 3984 x 6592 231 / 193, 5755 x 1488 x 1536 33.6 / 28.1.  192 x 192, 192 x 256, 256 x 256, 320 x 192, 128 x 256, 256 x 128, 64 x 192,
+// 64 x 256 and 128 x 64 beside them add nothing.
 const Config kConfigs[] = {
-    MOE_I8_DENSE(16, 16, 8, 1, 1, 2, 4, 1, 2.45f, 0.53f, 0.38f, 1e9f),
-    MOE_I8_DENSE(16, 32, 8, 1, 1, 3, 2, 1, 1.49f, 1.46f, 0.58f, 1e9f),
-    MOE_I8_DENSE(32, 32, 8, 1, 1, 2, 2, 1, 1.35f, 1.64f, 0.70f, 1e9f),
-    MOE_I8_DENSE(32, 64, 4, 1, 2, 3, 2, 1, 1.27f, 2.03f, 1.06f, 0.98f),
-    MOE_I8_DENSE(64, 64, 2, 2, 2, 4, 2, 1, 1.56f, 2.08f, 1.38f, 1.12f),
-    MOE_I8_DENSE(64, 128, 2, 2, 2, 3, 2, 1, 0.55f, 3.15f, 2.15f, 1.58f),
-    MOE_I8_DENSE(128, 128, 1, 2, 4, 4, 2, 1, 1.75f, 3.18f, 3.49f, 1.59f),
-    MOE_I8_DENSE(128, 128, 1, 2, 2, 2, 2, 2, 0.71f, 3.66f, 5.59f, 1.72f),
-    MOE_I8_DENSE(192, 192, 1, 2, 4, 3, 2, 1, 0.0f, 4.84f, 8.71f, 1.58f),
+    MOE_I8_DENSE(16, 16, 8, 1, 1, 2, 4, 1, 2.45f, 0.53f, 0.38f, 0.38f, 1e9f),
+    MOE_I8_DENSE(16, 32, 8, 1, 1, 3, 2, 1, 1.49f, 1.46f, 0.58f, 0.58f, 1e9f),
+    MOE_I8_DENSE(32, 32, 8, 1, 1, 2, 2, 1, 1.35f, 1.64f, 0.70f, 0.70f, 1e9f),
+    MOE_I8_DENSE(32, 64, 4, 1, 2, 3, 2, 1, 1.27f, 2.03f, 1.06f, 1.06f, 0.98f),
+    MOE_I8_DENSE(64, 64, 2, 2, 2, 4, 2, 1, 1.56f, 2.08f, 1.38f, 1.38f, 1.12f),
+    MOE_I8_DENSE(64, 128, 2, 2, 2, 3, 2, 1, 1.10f, 2.42f, 2.65f, 2.41f, 1e9f),
+    MOE_I8_DENSE(128, 128, 1, 2, 4, 4, 2, 1, 0.77f, 3.27f, 4.54f, 3.74f, 1e9f),
+    MOE_I8_DENSE(128, 128, 1, 2, 2, 2, 2, 2, 0.22f, 4.29f, 7.73f, 5.34f, 1e9f),
+    MOE_I8_DENSE(128, 192, 1, 4, 2, 3, 2, 1, 0.35f, 4.31f, 6.18f, 4.63f, 1e9f),
+    MOE_I8_DENSE(256, 192, 1, 4, 2, 2, 2, 1, 0.0f, 7.04f, 10.80f, 7.67f, 1e9f),
+    MOE_I8_DENSE(192, 320, 1, 4, 2, 2, 2, 1, 0.0f, 7.86f, 12.92f, 10.01f, 1e9f),
+    MOE_I8_DENSE(192, 384, 1, 2, 4, 2, 2, 1, 0.0f, 8.42f, 15.58f, 11.33f, 1e9f),
 };
-// The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Over 216 problems of 500..8192 rows
-// the choice takes on average 0.5 %, at most 27 % (4032 x 12736 x 896: 88.5 against 69.6 us), longer than the faster of
-// both; constants fitted to the present wide tiles alone chose worse (0.7-1.0 %).
-const Config kWide = {256, 256, 1, 2.97f, 9.03f, 9.38f, 2.13f, nullptr, nullptr};
+// The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Their stores are not hidden behind another
+// round's product: 0.21 us per MB, 0.32 where rows of the result begin inside 64 bytes (5780 rows x 2672 channels x 512: 24.8 us, in
+// 192 x 384 tiles 19.4).
+const Config kWide = {256, 256, 1, 5.61f, 0.95f, 10.70f, 7.08f, 1e9f, nullptr, nullptr};
 
 // The largest tiles of kConfigs for results of more than kThroughBytes (no launch that the estimates would choose has so many in
 // smaller ones).
 const Config kLarge[] = {
-    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 4, 4, 2, 1, 1.75f, 3.18f, 3.49f, 1.59f),
-    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 2, 2, 2, 2, 0.71f, 3.66f, 5.59f, 1.72f),
-    MOE_I8_DENSE_STORES(false, 192, 192, 1, 2, 4, 3, 2, 1, 0.0f, 4.84f, 8.71f, 1.58f),
+    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 4, 4, 2, 1, 0.77f, 3.27f, 4.54f, 3.74f, 1e9f),
+    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 2, 2, 2, 2, 0.22f, 4.29f, 7.73f, 5.34f, 1e9f),
+    MOE_I8_DENSE_STORES(false, 128, 192, 1, 4, 2, 3, 2, 1, 0.35f, 4.31f, 6.18f, 4.63f, 1e9f),
+    MOE_I8_DENSE_STORES(false, 256, 192, 1, 4, 2, 2, 2, 1, 0.0f, 7.04f, 10.80f, 7.67f, 1e9f),
+    MOE_I8_DENSE_STORES(false, 192, 320, 1, 4, 2, 2, 2, 1, 0.0f, 7.86f, 12.92f, 10.01f, 1e9f),
+    MOE_I8_DENSE_STORES(false, 192, 384, 1, 2, 4, 2, 2, 1, 0.0f, 8.42f, 15.58f, 11.33f, 1e9f),
 };
 
 float estimate(const Config& c, int64_t m, int64_t n, int64_t k) {
   const int64_t tiles = ((m + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn);
   const int64_t room = (int64_t)device_cu_count() * c.per_cu;
-  const float rounds = (float)((tiles + room - 1) / room);
-  const float latency = rounds * c.per_k * (float)k / 1024.0f;
+  const float full = (float)(tiles / room), last = (float)(tiles % room) / (float)room;
+  const float rounds = last > 0.0f ? full + 1.0f : full;
+  const float turns = full * c.per_k + (last > 0.0f ? c.per_k_few + last * (c.per_k - c.per_k_few) : 0.0f);
+  const float latency = turns * (float)k / 1024.0f;
   const float ops = (float)(tiles * c.tm * c.tn) * (float)k * 2.0f / (c.rate * 1e9f);
   return c.start + rounds * c.per_round + (latency > ops ? latency : ops);
 }
 
+float estimate_wide(int64_t m, int64_t n, int64_t k) {
+  return estimate(kWide, m, n, k) + (float)(m * n) * 2e-6f * (n % 32 ? 0.32f : 0.21f);
+}
+
 const Config* pick(int64_t m, int64_t n, int64_t k, bool wide_allowed) {
   const Config* best = wide_allowed ? &kWide : nullptr;
-  float least = wide_allowed ? estimate(kWide, m, n, k) : 0.0f;
+  float least = wide_allowed ? estimate_wide(m, n, k) : 0.0f;
   for (const Config& c : kConfigs) {
     const float t = estimate(c, m, n, k);
     if (!best || t < least) least = t, best = &c;
@@ -343,7 +406,10 @@ bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed) {
   return pick(m, n, k, wide_allowed) != &kWide;
 }
 
-float gemm_dense_estimate(int64_t m, int n, int k, bool wide_allowed) { return estimate(*pick(m, n, k, wide_allowed), m, n, k); }
+float gemm_dense_estimate(int64_t m, int n, int k, bool wide_allowed) {
+  const Config* c = pick(m, n, k, wide_allowed);
+  return c == &kWide ? estimate_wide(m, n, k) : estimate(*c, m, n, k);
+}
 
 hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream) {
   DenseParams p{};

@@ -74,3 +74,27 @@ def test_rows_quantised_by_their_tiles(pra, oracle, M, N, K):
         w2 = torch.randint(-127, 128, (K, inter), generator=g, dtype=torch.int8).to(DEV)
         args = (w[: 2 * inter].to(DEV), (s[: 2 * inter] * 0.1).to(DEV), w2, (torch.rand(K, generator=g) * 1e-3).to(DEV))
         assert torch.equal(pra.w8a8_mlp(x.to(DEV), *args), pra.w8a8_mlp(clean.to(DEV), *args, gemm_variant="stream"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (673, 5552, 576), (643, 5392, 192), (1421, 5584, 576), (1300, 5904, 64), (2051, 5616, 576), (1800, 6176, 192),  # 128 x 192,
+    (2315, 6176, 576), (4804, 2912, 64), (2309, 6192, 1088),                            # 256 x 192, 192 x 320, 192 x 384
+    (11398, 4416, 576), (18529, 2720, 64), (21775, 2592, 576), (21327, 2368, 576),      # more than 96 MB of results
+])
+def test_large_tiles(pra, oracle, M, N, K):
+    """The tiles whose results are finished in registers, one round of them and several: rows and channels that fill no tile,
+    reductions of odd multiples of 64 and of one step, plain results and gate_up's."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    s = torch.rand(N, generator=g) * 0.008 + 0.002
+    dx, dw, ds = x.to(DEV), w.to(DEV), s.to(DEV)
+    out = pra.apply_int8_linear(dx, dw, ds)
+    assert torch.equal(out, pra.apply_int8_linear(dx, dw, ds, gemm_variant="stream"))
+    rows = torch.cat([torch.arange(0, M, 97), torch.arange(M - 40, M)])
+    assert torch.equal(out[rows.to(DEV)].cpu(), oracle.w8a8_linear(x[rows], w, s))
+    inter = N // 2 // 64 * 64
+    w2 = torch.randint(-127, 128, (K, inter), generator=g, dtype=torch.int8).to(DEV)
+    args = (dw[: 2 * inter], ds[: 2 * inter] * 0.1, w2, (torch.rand(K, generator=g) * 1e-3).to(DEV))
+    assert torch.equal(pra.w8a8_mlp(dx, *args), pra.w8a8_mlp(dx, *args, gemm_variant="stream"))
