@@ -72,6 +72,19 @@ __device__ __forceinline__ void store16_through(void* to, const uint4& v, uint64
                : "v"(reinterpret_cast<uint64_t>(to)), "v"(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}), "s"(lanes)
                : "memory", "scc");
 }
+// The same into the caches, or past them with the non-temporal hint.
+template <bool NT>
+__device__ __forceinline__ void store16_lanes(void* to, const uint4& v, uint64_t lanes) {
+  uint64_t active;
+  lanes = uniform_address(reinterpret_cast<const void*>(lanes));
+  const v4i x{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+  if constexpr (NT)
+    asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_dwordx4 %1, %2, off nt\n\ts_mov_b64 exec, %0\n\ts_nop 1"
+                 : "=&s"(active) : "v"(reinterpret_cast<uint64_t>(to)), "v"(x), "s"(lanes) : "memory", "scc");
+  else
+    asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_dwordx4 %1, %2, off\n\ts_mov_b64 exec, %0\n\ts_nop 1"
+                 : "=&s"(active) : "v"(reinterpret_cast<uint64_t>(to)), "v"(x), "s"(lanes) : "memory", "scc");
+}
 // through: written through to memory instead of left in the L2.  (The two wait states behind that store: a store of more than
 // 8 bytes reads its data that late, and the compiler, which keeps a write of them away from its own stores, does not know of
 // this one.)
