@@ -539,11 +539,13 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   p.B = a.block_size;
   p.tiles.per_tile = kTok / a.block_size;
   // Nine blocks as 3 + 3 + 3 instead of 4 + 4 + 1: a step of one block costs far more than a quarter of a full one (its weight
-  // rows are the same).  Layer us, full tiles and a rest / even ones: 256 experts of 7168 x 2048 at 8192 / 16384 tokens 4229 / 3790,
-  // 6360 / 6247, 129 of 4096 x 1408, evenly routed, at 4096 1066 / 933 (skewed routing: the same).  Below: no difference
-  // at 2048 x 768 and 2048 x 1408, and even tiles lose at short reductions, where a task is mostly its epilogue: 32
-  // experts of 1024 x 512 at 5000 tokens 101.6 / 103.3, 256 of 2048 x 512 at 4000 297.9 / 303.7.
-  p.tiles.even = a.k >= 4096;
+  // rows are the same, and it runs ahead of the others, so that they come from memory twice: 757 MB instead of 419 for experts of
+  // 264 rows).  Layer us, full tiles and a rest / even ones.  Reductions of 2048 and more: 256 experts of 7168 x 2048 at 8192 / 8800 /
+  // 12000 tokens 3768 / 3601, 4458 / 4099, 5018 / 4794 (its down GEMM alone), at 16384 the same; 128 of 2048 x 768 at 4300 / 5000 / 8192
+  // / 9000 320 / 315, 356 / 345, 481 / 475, 523 / 520; 64 of 2048 x 1408 at 3000 293 / 281; 256 of 2048 x 512 at 9000 506 / 480.  Below,
+  // where a task is mostly its epilogue, nothing or a loss: down GEMMs of 768 and 1408 +-1 %, 32 experts of 1024 x 512, Zipf
+  // routing, at 1500 / 5000 56.6 / 58.2, 97.2 / 99.3.
+  p.tiles.even = a.k >= 2048;
   p.tiles.ntiles = MODE == kGateUpSilu ? (a.n / 2 + 127) / 128 : (a.n + kCh - 1) / kCh;
   p.tiles.by_ntiles = divider(p.tiles.ntiles);
   p.tiles.by_per_tile = divider(p.tiles.per_tile);
