@@ -35,6 +35,15 @@ constexpr int kSub = 16;      // token rows per sub-tile (MFMA N)
 // Qwen3-30B-A3B shape: about 10 routed rows per expert.
 constexpr int kPairRowsPerExpert = 10;
 constexpr int kStepK = 64;    // reduction bytes per MFMA
+// Two wavefronts halve the reduction of a tile pair: workgroups of half the length and twice as many, so that a compute unit that
+// holds one more than another does not hold up the launch by as much.  Layer us, whole / halved: 129 experts of 4096 x 1408 with
+// skewed routing at 5 / 7 / 8 / 10 / 14 tokens 75.5 / 76.1, 71.1 / 71.6, 94.1 / 83.7, 94.5 / 83.7, 94.4 / 87.1, 128 of them
+// evenly routed at 5 / 8 / 12 105 / 103, 162 / 159, 197 / 193; 256 of 7168 x 2048 at 6 / 8 314 / 312, 388 / 377; 64 of 2048 x 1408,
+// skewed, at 6 / 12 43.9 / 38.5, 47.9 / 46.4, even, at 6 / 8 56.4 / 58.7, 67.9 / 65.0; 16 of 4096 x 4096 at 6 / 10 96.7 / 86.3, 117 /
+// 104.  A gate_up launch with fewer bytes per expert stays whole: 128 of 2048 x 768 at 9 to 16 tokens 0.6 % slower on average
+// (55.9 / 57.1 .. 69.3 / 67.1).  Quarters, or workgroups of two wavefronts: less, and losses of up to 4 % where halves have none.
+constexpr int kParts = 2;
+constexpr int64_t kSplitBytes = 4 << 20;
 constexpr int kTiles = 2;     // 16-row weight tiles per wavefront
 constexpr int kWinBytes = 256;                              // bytes of every weight row per window
 constexpr int kWinSteps = kWinBytes / kStepK;               // MFMA steps per window
@@ -99,6 +108,8 @@ __device__ __forceinline__ void pair_rows(const StreamParams& p, int q, int (&wr
   }
 }
 
+// KS: wavefronts that share a tile pair's reduction (npairs is 1 or 0 then); all of a workgroup must call this, for its barriers.
+//
 // `count_valid`: first pass over a block; the number of valid rows of the block is counted here,
 // after the first weight window has been requested, and returned.
 //
@@ -106,7 +117,7 @@ __device__ __forceinline__ void pair_rows(const StreamParams& p, int q, int (&wr
 // `a_lds` (int8) and `s_lds` (row scales) with the arithmetic of the stand-alone quantiser and the
 // operand reads come from there.  Every wavefront of the workgroup must call this, also those with
 // no weight rows left (`npairs` == 0): they take part in the quantisation and its two barriers.
-template <int MODE, int NS, bool kFused>
+template <int MODE, int NS, bool kFused, int KS>
 __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e, int sub0, int first_pair,
                                            int npairs, char* wave_lds, bool count_valid, char* a_lds,
                                            float* s_lds, int32_t top_id) {
@@ -126,7 +137,12 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
   // The wavefront walks windows (pair 0, k 0), (pair 0, k 256), ..., (pair 1, k 0), ... (from `start` on and around); `fq`/`fk`
   // track the window whose weights are being fetched (`fk` also the one whose activation rows are),
   // `cq`/`ck` the one being consumed.
-  const int start = (e & p.rotate) * kWinBytes;  // (see StreamParams)
+  const int all_windows = (K + kWinBytes - 1) / kWinBytes;
+  // the wavefront's part of the reduction
+  const int part = KS > 1 ? (int)(threadIdx.x / kWave) % KS : 0;
+  const int k0 = all_windows * part / KS * kWinBytes, k1 = KS == 1 || part + 1 == KS ? K : all_windows * (part + 1) / KS * kWinBytes;
+  const int nwin = (k1 - k0 + kWinBytes - 1) / kWinBytes;
+  const int start = KS == 1 ? (e & p.rotate) * kWinBytes : k0 + (p.rotate ? e % (nwin > 0 ? nwin : 1) * kWinBytes : 0);  // (see StreamParams)
   int fq = 0, wk = start, fk = start;
   auto fetch_weights = [&](Window<NS>& win) {
     int wrow[kTiles];
@@ -139,14 +155,13 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
       win.w[j] = chunk_in ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(src)) : v4i{0, 0, 0, 0};
     }
     wk += kWinBytes;
-    if (wk >= K) wk = 0;
+    if (wk >= k1) wk = k0;
     if (wk == start) ++fq;
   };
 
   // The weights of the first two windows depend on nothing but the expert of the block: they are
   // requested from HBM before the chain of dependent reads (row list -> token -> activation row,
   // or the quantisation of the rows) that the rest of the set-up is.
-  const int nwin = (K + kWinBytes - 1) / kWinBytes;
   const int total = npairs * nwin;
   Window<NS> w0, w1;
   if (total > 0) fetch_weights(w0);
@@ -237,7 +252,7 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
                                              : v4i{0, 0, 0, 0};
       }
     fk += kWinBytes;
-    if (fk >= K) fk = 0;
+    if (fk >= k1) fk = k0;
   };
   auto fetch = [&](Window<NS>& win) {
     fetch_weights(win);
@@ -311,6 +326,7 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
         for (int s = 0; s < NS; ++s)
           acc[t][s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(frag[t], win.a[s][u], acc[t][s], 0, 0, 0);
     }
+    if constexpr (KS > 1) return;
     ck += kWinBytes;
     if (ck >= K) {
       finish_pair(cq);
@@ -330,12 +346,30 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
     if (i + 2 < total) fetch(w0);
     consume(w1);
   }
+  if constexpr (KS > 1) {
+    // the parts' int32 sums meet in LDS, each in its wavefront's own area
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) *reinterpret_cast<v4i*>(wave_lds + ((t * NS + s) * kWave + lane) * 16) = acc[t][s];
+    __syncthreads();
+    if (part == 0 && npairs > 0) {
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+          for (int i = 1; i < KS; ++i) acc[t][s] += *reinterpret_cast<const v4i*>(wave_lds + i * kWaveLds + ((t * NS + s) * kWave + lane) * 16);
+      finish_pair(0);
+    }
+    __syncthreads();
+  }
   return nvalid;
 }
 
 // grid.x * grid.y: one workgroup of kWaves wavefronts per kWaves tile pairs and per block of the
 // row list's capacity (grid.z: see below).  NS = sub-tiles per pass.
-template <int MODE, bool kFused, int NS>
+template <int MODE, bool kFused, int NS, int KS>
 __global__ __launch_bounds__(kThreads, NS == 1 ? 3 : 2) void gemm_stream_kernel(StreamParams p) {
   __shared__ __align__(16) char lds[kWaves * kWaveLds];
   __shared__ __align__(16) char a_lds[kFused ? kSub * (kFusedMaxK + kFusedRowPad) : 16];
@@ -381,9 +415,9 @@ __global__ __launch_bounds__(kThreads, NS == 1 ? 3 : 2) void gemm_stream_kernel(
   }
   const int e = kFused ? p.expert_ids[blk] : e_entry;
   if (e < 0 || e >= p.E) return;
-  const int first_pair = (group * kWaves + threadIdx.x / kWave) * ppw;
-  // a wavefront past the last weight rows leaves, unless the workgroup needs it for the quantisation
-  if (!kFused && first_pair >= total_pairs) return;
+  const int first_pair = KS > 1 ? group * (kWaves / KS) + (int)(threadIdx.x / kWave) / KS : (group * kWaves + threadIdx.x / kWave) * ppw;
+  // a wavefront past the last weight rows leaves, unless the workgroup needs it for the quantisation or at the barriers
+  if (!kFused && KS == 1 && first_pair >= total_pairs) return;
   const int left = total_pairs - first_pair;
   const int npairs = left < 0 ? 0 : left < ppw ? left : ppw;
 
@@ -396,15 +430,15 @@ __global__ __launch_bounds__(kThreads, NS == 1 ? 3 : 2) void gemm_stream_kernel(
     if (sub0 * kSub >= p.B) return;
     const int32_t t = p.sorted_ids[(int64_t)blk * p.B + sub0 * kSub];
     if (t < 0 || t >= p.P) return;
-    stream_pass<MODE, NS, kFused>(p, blk, e, sub0, first_pair, npairs, wave_lds, false, a_lds, s_lds, top_id);
+    stream_pass<MODE, NS, kFused, KS>(p, blk, e, sub0, first_pair, npairs, wave_lds, false, a_lds, s_lds, top_id);
     return;
   }
   // One workgroup walks all passes; the first one counts the valid rows (a prefix of the block, at
   // least one: the block is in use) to know how many sub-tiles there are.
-  const int nvalid = stream_pass<MODE, NS, kFused>(p, blk, e, 0, first_pair, npairs, wave_lds, true, a_lds, s_lds, top_id);
+  const int nvalid = stream_pass<MODE, NS, kFused, KS>(p, blk, e, 0, first_pair, npairs, wave_lds, true, a_lds, s_lds, top_id);
   const int nsub = (nvalid + kSub - 1) / kSub;
   for (int sub0 = NS; sub0 < nsub; sub0 += NS)
-    stream_pass<MODE, NS, kFused>(p, blk, e, sub0, first_pair, npairs, wave_lds, false, a_lds, s_lds, top_id);
+    stream_pass<MODE, NS, kFused, KS>(p, blk, e, sub0, first_pair, npairs, wave_lds, false, a_lds, s_lds, top_id);
 }
 
 template <int MODE, bool kFused = false>
@@ -434,6 +468,8 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   if (blocks == 0 || waves == 0) return hipSuccess;
   if (blocks > 65535 || blocks * ((waves + kWaves - 1) / kWaves) >= (1ll << 31)) return hipErrorInvalidValue;
   const bool two = !kFused && a.num_pairs > (int64_t)kPairRowsPerExpert * a.num_experts;
+  const bool split = MODE != kAccI32 && !kFused && !two && a.k > kWinBytes &&
+                     (MODE == kDown || (int64_t)a.n * a.k >= kSplitBytes);
   // Passes per block that can be needed: no expert holds more rows than there are tokens (or pairs,
   // when the caller did not say).  One workgroup per pass once there can be more than one.
   const int ns = two ? 2 : 1;
@@ -441,13 +477,19 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
                                                                                              : a.num_pairs;
   const int64_t rows = most_rows < a.block_size ? most_rows : a.block_size;
   const int passes = kFused ? 1 : (int)((rows + kSub * ns - 1) / (kSub * ns));
-  const dim3 grid((unsigned)((waves + kWaves - 1) / kWaves), (unsigned)blocks, (unsigned)(passes > 1 ? passes : 1));
+  const int per_group = split ? kWaves / kParts : kWaves;  // tile pairs of a workgroup
+  const dim3 grid((unsigned)((waves + per_group - 1) / per_group), (unsigned)blocks, (unsigned)(passes > 1 ? passes : 1));
   p.wave_capacity = device_cu_count() * kWaves * (two ? 2 : 3);
   p.round_even = a.a_round_even ? 1 : 0;
+  if constexpr (MODE != kAccI32 && !kFused)
+    if (split) {
+      hipLaunchKernelGGL((gemm_stream_kernel<MODE, false, 1, kParts>), grid, dim3(kThreads), 0, stream, p);
+      return hipGetLastError();
+    }
   if (two)
-    hipLaunchKernelGGL((gemm_stream_kernel<MODE, kFused, kFused ? 1 : 2>), grid, dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((gemm_stream_kernel<MODE, kFused, kFused ? 1 : 2, 1>), grid, dim3(kThreads), 0, stream, p);
   else
-    hipLaunchKernelGGL((gemm_stream_kernel<MODE, kFused, 1>), grid, dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((gemm_stream_kernel<MODE, kFused, 1, 1>), grid, dim3(kThreads), 0, stream, p);
   return hipGetLastError();
 }
 

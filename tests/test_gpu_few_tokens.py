@@ -138,3 +138,29 @@ def test_layer_quantises_long_rows_as_the_row_quantiser_does(pra, H, M):
     pra.moe_sum(pra.gemm_down(h_q, a2, d.w2, d.w2_scale, d.topk_weights, s, e, npp, B, "stream").view(M, k, H), want)
     got = pra.fused_experts(*d.fused_experts_args(), **d.fused_experts_kwargs(), block_size_m=B, gemm_variant="stream")
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("E,k,H,I,M,B", [
+    (66, 8, 4160, 576, 9, 64),    # 17 windows and 3, the last of 64 bytes
+    (40, 4, 4096, 1088, 16, 16),  # starting windows; 5 windows
+    (33, 2, 7168, 320, 40, 64),   # up to 40 rows of an expert: several passes; 2 windows
+    (70, 4, 1088, 2064, 5, 32),   # an odd number of tile pairs (gate_up alone takes it)
+])
+def test_reductions_halved_between_wavefronts(pra, oracle, E, k, H, I, M, B):
+    """The streaming kernel with a tile pair's reduction in two wavefronts: windows that do not halve evenly, a last
+    window that is partial, a workgroup with one tile pair of two, starting windows, blocks of one and of several passes."""
+    im = inputs_mod()
+    inp = im.make_inputs(im.LayerShape("h", E=E, k=k, H=H, I=I), M, seed=E + M + H)
+    inp.topk_ids[:, 0] = 0  # an expert that every token visits
+    inp.topk_ids[:, 1:] = inp.topk_ids[:, 1:].clamp(min=1)
+    st = oracle.fused_experts_staged(inp.hidden_states, inp.w1, inp.w2, inp.topk_weights, inp.topk_ids, inp.w1_scale,
+                                     inp.w2_scale, B)
+    d = inp.to(DEV)
+    s, e, npp = pra.moe_align_block_size(d.topk_ids, B, E)
+    act = pra.gemm_gate_up_silu(st["x_q"].to(DEV), st["a1_scale"].to(DEV), d.w1, d.w1_scale, s, e, npp, k, B, M * k, "stream")
+    diff = (act.float().cpu() - st["cache2"].float()).abs() > 0.02 * st["cache2"].float().abs() + 1e-6  # (the exponential)
+    assert not bool(diff.any())
+    if I % 64:
+        return
+    down = pra.gemm_down(st["h_q"].to(DEV), st["a2_scale"].to(DEV), d.w2, d.w2_scale, d.topk_weights, s, e, npp, B, "stream")
+    assert torch.equal(down.cpu(), st["cache3"].reshape(M * k, H))
