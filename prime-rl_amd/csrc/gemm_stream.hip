@@ -8,7 +8,8 @@
 // and the loads of the next window are issued before the current one is consumed.  The registers
 // are then transposed into the MFMA operand layout through an 8 KB LDS area private to the
 // wavefront (16-byte chunks XOR-swizzled with the row, so that neither the row-linear writes nor
-// the 16-rows-same-chunk reads collide on a bank); no barrier is ever needed.  The few activation
+// the 16-rows-same-chunk reads collide on a bank); no barrier is needed on the way (two wavefronts that
+// share a reduction, see kParts, meet once at its end).  The few activation
 // rows of the block are read from global memory (vector cache) directly in the operand layout.
 //
 // v_mfma_i32_16x16x64_i8 is used "transposed": the A operand carries 16 weight rows (output
