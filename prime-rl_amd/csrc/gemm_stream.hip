@@ -36,8 +36,8 @@ constexpr int kSub = 16;      // token rows per sub-tile (MFMA N)
 // Qwen3-30B-A3B shape: about 10 routed rows per expert.
 constexpr int kPairRowsPerExpert = 10;
 constexpr int kStepK = 64;    // reduction bytes per MFMA
-// Two wavefronts halve the reduction of a tile pair: workgroups of half the length and twice as many, so that a compute unit that
-// holds one more than another does not hold up the launch by as much.  Layer us, whole / halved: 129 experts of 4096 x 1408 with
+// Two wavefronts halve the reduction of a tile pair: workgroups of half the length and twice as many.  With whole ones a launch takes
+// 5 to 25 % longer from 513 and from 769 workgroups on, two and three to a compute unit.  Layer us, whole / halved: 129 experts of 4096 x 1408 with
 // skewed routing at 5 / 7 / 8 / 10 / 14 tokens 75.5 / 76.1, 71.1 / 71.6, 94.1 / 83.7, 94.5 / 83.7, 94.4 / 87.1, 128 of them
 // evenly routed at 5 / 8 / 12 105 / 103, 162 / 159, 197 / 193; 256 of 7168 x 2048 at 6 / 8 314 / 312, 388 / 377; 64 of 2048 x 1408,
 // skewed, at 6 / 12 43.9 / 38.5, 47.9 / 46.4, even, at 6 / 8 56.4 / 58.7, 67.9 / 65.0; 16 of 4096 x 4096 at 6 / 10 96.7 / 86.3, 117 /
