@@ -98,3 +98,10 @@ def test_large_tiles(pra, oracle, M, N, K):
     w2 = torch.randint(-127, 128, (K, inter), generator=g, dtype=torch.int8).to(DEV)
     args = (dw[: 2 * inter], ds[: 2 * inter] * 0.1, w2, (torch.rand(K, generator=g) * 1e-3).to(DEV))
     assert torch.equal(pra.w8a8_mlp(dx, *args), pra.w8a8_mlp(dx, *args, gemm_variant="stream"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(570, 3824, 1600), (1400, 1600, 576), (1921, 1040, 4160), (1913, 1072, 4096), (560, 3776, 2560)])
+def test_tiles_of_96(pra, oracle, M, N, K):
+    """96 x 96 tiles, their reduction halved: rows and channels that fill no tile, an odd number of pieces and one of 64 bytes."""
+    test_large_tiles(pra, oracle, M, N, K)
