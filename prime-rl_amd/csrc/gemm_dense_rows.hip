@@ -272,6 +272,12 @@ hipError_t launch_config(const DenseRowsParams& p0, hipStream_t stream) {
 // unit holds one: then the second term is 0).  Least-squares fits to 540 problems of 2..1000 rows x 512..24576 channels x 192..4200
 // (rms error of a fit 4-7 %).  The choice between these and the launches they replace takes on average 0.6 % longer than the fastest
 // way, 1.9 % with up to 16 rows.
+// The 256 and 512 channel tiles are one round where the 128 channel ones are two, and a workgroup's rows serve twice as many channels; no
+// split of the reduction is left, and none is missed: 16 x 256 is faster than 32 x 128, which was here, also where both are one round
+// (170 rows x 4112 channels x 256 4.7 / 4.2 us).  Without / with the three of them, 60 drawn linear layers that they are picked for:
+// 13 % faster on average (two 5 % slower); 67 x 12848 x 192 6.9 / 4.2, 396 x 2544 x 704 8.5 / 6.0, 135 x 6640 x 1024 8.8 / 6.3, 1073 x 960
+// x 384 7.3 / 5.4, 146 x 17392 x 512 9.0 / 7.3.  Beside them 32 x 64, 48 x 64, 48 x 128, 48 x 256, 64 x 128 and 64 x 256 up to 1024,
+// 32 x 64, 32 x 128, 16 x 256 and 32 x 256 up to 2048 and 16 x 64 and 16 x 128 up to 4096 gain 0.2 % or nothing.
 struct Config {
   int tm, tn;   // tile
   int longest;  // reduction
@@ -287,7 +293,9 @@ const Config kConfigs[] = {
     MOE_I8_ROWS(16, 32, 4, 1, 2, 3, 2, 2, 1.97f, 1.87f, -1.06f, -0.06f, 1.37f),
     MOE_I8_ROWS(16, 64, 2, 1, 4, 3, 2, 2, 1.89f, 1.94f, -0.87f, -0.11f, 1.62f),
     MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 2, 1, 1.23f, 2.27f, 1.54f, 0.0f, 0.0f),
-    MOE_I8_ROWS(32, 128, 2, 1, 4, 3, 2, 1, 0.76f, 3.27f, 2.32f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 256, 1, 1, 8, 3, 2, 1, 0.98f, 2.44f, 2.91f, 0.0f, 0.0f),
+    MOE_I8_ROWS(32, 256, 1, 1, 8, 3, 2, 1, 0.75f, 3.59f, 3.33f, 0.0f, 0.0f),
+    MOE_I8_ROWS(32, 512, 1, 1, 8, 2, 1, 1, 0.53f, 4.37f, 4.63f, 0.0f, 0.0f),
     MOE_I8_ROWS(16, 32, 8, 1, 1, 3, 4, 1, 1.12f, 2.41f, 0.83f, 0.0f, 0.0f),
     MOE_I8_ROWS(16, 64, 4, 1, 2, 3, 4, 1, 1.02f, 2.57f, 1.18f, 0.0f, 0.0f),
     MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 4, 1, 0.78f, 2.70f, 1.83f, 0.0f, 0.0f),

@@ -105,3 +105,13 @@ def test_large_tiles(pra, oracle, M, N, K):
 def test_tiles_of_96(pra, oracle, M, N, K):
     """96 x 96 tiles, their reduction halved: rows and channels that fill no tile, an odd number of pieces and one of 64 bytes."""
     test_large_tiles(pra, oracle, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (250, 3632, 960), (14, 50000, 448), (45, 11600, 1024), (33, 21760, 64),              # 16 x 256
+    (97, 10512, 64), (700, 1968, 576), (209, 4624, 1024), (481, 4080, 512), (1690, 768, 960),  # 32 x 256
+    (250, 8208, 448), (449, 8176, 512), (1000, 4096, 192),                               # 32 x 512
+])
+def test_rows_quantised_by_wide_tiles(pra, oracle, M, N, K):
+    """Tiles whose wavefronts do not split the reduction: rows and channels that fill no tile, reductions of one step and up to the longest."""
+    test_rows_quantised_by_their_tiles(pra, oracle, M, N, K)
