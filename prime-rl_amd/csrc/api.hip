@@ -973,14 +973,6 @@ moe_i8::GemmArgs dense_group(int mode, const DenseCarve& c, char* ws, const int8
   return g;
 }
 
-// Whether one GEMM of a dense entry point runs on the dense kernel (which needs no routing arrays): unless
-// a family is demanded or the 256-row tiles of the LDS-tiled family are expected to be faster.
-bool takes_dense_kernel(moe_i8::GemmArgs g, int variant) {
-  if (variant != MOE_I8_GEMM_AUTO) return false;
-  g.tile_geometry = moe_i8::kTileWide;
-  return moe_i8::gemm_dense_takes(g.num_pairs, g.n, g.k, moe_i8::gemm_tile_supports(g));
-}
-
 int check_dense_gemm(const moe_i8::GemmArgs& g, int variant) {
   if (int rc = check_gemm_common(g.a_q, g.w, g.sorted_token_ids, g.expert_ids, g.num_tokens_post_padded, g.out, g.num_pairs,
                                  1, g.n, g.k, g.block_size, g.sorted_cap, variant))
@@ -988,41 +980,64 @@ int check_dense_gemm(const moe_i8::GemmArgs& g, int variant) {
   return aligned16(g.w_scale) ? MOE_I8_OK : fail(MOE_I8_EINVAL, "weight scales must be 16-byte aligned");
 }
 
-int run_dense(const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
+bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+  const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+  return a0 < b0 + (uintptr_t)b_bytes && b0 < a0 + (uintptr_t)a_bytes;
+}
+
+// How a GEMM of a dense entry point runs, decided once per GEMM.
+enum DenseWay {
+  kGrouped,  // quantised by a launch of its own, then the 256-row tiles or a demanded family, which read that launch's routing
+  kDense,    // quantised by a launch of its own, then the dense kernel, which needs no routing
+  kRows,     // the product's own launch quantises some tens to hundreds of rows
+  kFew,      // ... a few rows
+};
+struct DenseChoice {
+  DenseWay way;
+  int entry;  // tile of the dense kernel or of the one that quantises its rows
+};
+// `own`: the product's launch may quantise the rows.
+DenseChoice dense_choice(moe_i8::GemmArgs g, int variant, bool own) {
+  if (variant != MOE_I8_GEMM_AUTO) return {kGrouped, -1};
+  const bool few = own && moe_i8::dense_few_takes(g.num_pairs, g.n, g.k);
+  if (few && g.num_pairs < moe_i8::kDenseRowsFrom) return {kFew, -1};
+  moe_i8::DensePick quantised{-1, 0.0f};
+  if (!few) {
+    g.tile_geometry = moe_i8::kTileWide;
+    quantised = moe_i8::gemm_dense_pick(g.num_pairs, g.n, g.k, moe_i8::gemm_tile_supports(g));
+  }
+  if (own) {
+    const int entry = moe_i8::dense_rows_pick(g.num_pairs, g.n, g.k, few, quantised.us);
+    if (entry >= 0) return {kRows, entry};
+    if (few) return {kFew, -1};
+  }
+  return {quantised.entry < 0 ? kGrouped : kDense, quantised.entry};
+}
+// Whether the product's launch may quantise the rows at `x`: not where the output overlaps them, as every workgroup reads rows that
+// others need while some already write.  (The other kernels read a copy that a launch of its own has quantised.)
+bool may_quantise(const void* x, const moe_i8::GemmArgs& g) {
+  const int64_t width = g.mode == moe_i8::kGateUpSilu ? g.n / 2 : g.n;
+  return aligned16(x) && aligned16(g.w) && !overlap(x, 2 * g.num_pairs * g.k, g.out, 2 * g.num_pairs * width);
+}
+
+// The product of a quantised problem.
+int run_quantised(const DenseChoice& choice, const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
   if (int rc = check_dense_gemm(g, variant)) return rc;
-  if (takes_dense_kernel(g, variant)) {
+  if (choice.way == kDense) {
     const moe_i8::DenseArgs d{g.mode, g.a_q, g.a_scale, g.w, g.w_scale, g.out, g.num_pairs, g.n, g.k};
-    return check_launch(moe_i8::launch_gemm_dense(d, stream), "gemm_dense");
+    return check_launch(moe_i8::launch_gemm_dense(d, choice.entry, stream), "gemm_dense");
   }
   moe_i8::GemmArgs wide = g;
   wide.tile_geometry = moe_i8::kTileWide;
   if (variant == MOE_I8_GEMM_AUTO && moe_i8::gemm_tile_supports(wide)) variant = MOE_I8_GEMM_TILE_WIDE;
   return run_gemm(g, variant, stream);
 }
-
-bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
-  const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
-  return a0 < b0 + (uintptr_t)b_bytes && b0 < a0 + (uintptr_t)a_bytes;
-}
-
-// How a GEMM of a dense entry point runs: a few rows, or some tens to hundreds of them, are quantised by the product's own launch,
-// unless a family is demanded or the output overlaps the rows: every workgroup reads rows that others need while some already
-// write.  (The other kernels read a copy of the rows that a launch of its own has quantised.)
-enum DenseWay { kQuantised, kFew, kRows };
-DenseWay dense_way(const void* x, moe_i8::GemmArgs g, int variant) {
-  const int64_t width = g.mode == moe_i8::kGateUpSilu ? g.n / 2 : g.n;
-  if (variant != MOE_I8_GEMM_AUTO || !aligned16(x) || !aligned16(g.w) || overlap(x, 2 * g.num_pairs * g.k, g.out, 2 * g.num_pairs * width))
-    return kQuantised;
-  const bool few = moe_i8::dense_few_takes(g.num_pairs, g.n, g.k);
-  g.tile_geometry = moe_i8::kTileWide;
-  if (moe_i8::dense_rows_takes(g.num_pairs, g.n, g.k, few, moe_i8::gemm_tile_supports(g))) return kRows;
-  return few ? kFew : kQuantised;
-}
-int run_unquantised(DenseWay way, const void* x, const moe_i8::GemmArgs& g, hipStream_t stream) {
+// A problem whose rows the product's launch quantises.
+int run_unquantised(const DenseChoice& choice, const void* x, const moe_i8::GemmArgs& g, hipStream_t stream) {
   if (int rc = check_dense_gemm(g, MOE_I8_GEMM_AUTO)) return rc;
   const moe_i8::DenseFewArgs d{g.mode, static_cast<const uint16_t*>(x), g.w, g.w_scale, static_cast<uint16_t*>(g.out), (int)g.num_pairs, g.n, g.k};
-  return way == kFew ? check_launch(moe_i8::launch_dense_few(d, stream), "dense_few")
-                     : check_launch(moe_i8::launch_dense_rows(d, stream), "dense_rows");
+  return choice.way == kFew ? check_launch(moe_i8::launch_dense_few(d, stream), "dense_few")
+                            : check_launch(moe_i8::launch_dense_rows(d, choice.entry, stream), "dense_rows");
 }
 
 // The ties-to-even row quantiser of the dense path; `padded`: rows for the dense kernel; `route`: its
@@ -1080,10 +1095,11 @@ int moe_i8_w8a8_linear(const void* x, const int8_t* w, const float* w_scale, voi
   float* a1 = reinterpret_cast<float*>(ws + c.a1);
   const moe_i8::GemmArgs g = dense_group(moe_i8::kDown, c, ws, x_q, a1, w, w_scale, out, m, n, k);
   const WorkspaceTurn turn(workspace);
-  if (const DenseWay way = dense_way(x, g, variant)) return run_unquantised(way, x, g, s);
-  const bool dense = takes_dense_kernel(g, variant);
+  const DenseChoice choice = dense_choice(g, variant, may_quantise(x, g));
+  if (choice.way >= kRows) return run_unquantised(choice, x, g, s);
+  const bool dense = choice.way == kDense;
   if (int rc = dense_quant(x, m, k, x_q, a1, dense, !dense, c, ws, s)) return rc;
-  return run_dense(g, variant, s);
+  return run_quantised(choice, g, variant, s);
 }
 
 int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, const int8_t* w2,
@@ -1104,18 +1120,18 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   const moe_i8::GemmArgs gu = dense_group(moe_i8::kGateUpSilu, c, ws, x_q, a1, w13, w13_scale, ws + c.act, m, 2 * inter, hidden);
   moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, ws, act_q, a2, w2, w2_scale, out, m, hidden, inter);
   const WorkspaceTurn turn(workspace);
-  const DenseWay way_gu = dense_way(x, gu, variant), way_dg = dense_way(ws + c.act, dg, variant);
-  if (way_gu)
+  const DenseChoice choice_dg = dense_choice(dg, variant, may_quantise(ws + c.act, dg));
+  const DenseChoice choice_gu = dense_choice(gu, variant, may_quantise(x, gu));
+  const bool dense_dg = choice_dg.way == kDense, route_dg = choice_dg.way == kGrouped;
+  if (choice_gu.way >= kRows) {
     if (int rc = check_dense_gemm(dg, variant)) return rc;  // before anything is launched
-  const bool dense_gu = takes_dense_kernel(gu, variant), dense_dg = takes_dense_kernel(dg, variant);
-  const bool route_dg = !way_dg && !dense_dg;  // the down GEMM reads the routing that a quantiser's launch writes
-  if (way_gu) {
-    if (int rc = run_unquantised(way_gu, x, gu, s)) return rc;
+    if (int rc = run_unquantised(choice_gu, x, gu, s)) return rc;
   } else {
+    const bool dense_gu = choice_gu.way == kDense;
     if (int rc = dense_quant(x, m, hidden, x_q, a1, dense_gu, !dense_gu || route_dg, c, ws, s)) return rc;
-    if (int rc = run_dense(gu, variant, s)) return rc;
+    if (int rc = run_quantised(choice_gu, gu, variant, s)) return rc;
   }
-  if (way_dg) return run_unquantised(way_dg, ws + c.act, dg, s);
+  if (choice_dg.way >= kRows) return run_unquantised(choice_dg, ws + c.act, dg, s);
   // Few rows on the streaming family: its down GEMM quantises them itself (ties to even here), one
   // launch less.
   if (variant == MOE_I8_GEMM_STREAM && m <= kDenseSelfQuantRows && inter <= kSelfQuantMaxInter) {
@@ -1129,8 +1145,8 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
     dg.a_round_even = true;
     return check_launch(moe_i8::launch_gemm_stream(dg, s), "gemm_stream");
   }
-  if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, way_gu && route_dg, c, ws, s)) return rc;
-  return run_dense(dg, variant, s);
+  if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, choice_gu.way >= kRows && route_dg, c, ws, s)) return rc;
+  return run_quantised(choice_dg, dg, variant, s);
 }
 
 }  // extern "C"

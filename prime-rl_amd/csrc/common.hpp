@@ -341,11 +341,15 @@ struct DenseArgs {
   int k;
 };
 int dense_row_stride(int k);
-// Whether the dense kernel is the one for this problem; `wide_allowed`: the 256-row tiles of the LDS-tiled
-// family can run it too and are preferred where they are expected to be faster.
-bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed);
-float gemm_dense_estimate(int64_t m, int n, int k, bool wide_allowed);  // us of the product
-hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream);
+// How a dense GEMM is cut up, chosen once per GEMM and launched with: an entry of the kernel's table of tiles.
+struct DensePick {
+  int entry;  // -1: the dense kernel is not the one for this problem
+  float us;   // what the product is expected to take, by whichever kernel
+};
+// `wide_allowed`: the 256-row tiles of the LDS-tiled family can run the problem too and are preferred where they are expected to
+// be faster.
+DensePick gemm_dense_pick(int64_t m, int n, int k, bool wide_allowed);
+hipError_t launch_gemm_dense(const DenseArgs& a, int entry, hipStream_t stream);
 
 // The same for a few rows, which the launch quantises itself (ties to even).
 struct DenseFewArgs {
@@ -361,10 +365,11 @@ struct DenseFewArgs {
 constexpr int kDenseFewRows = 16;
 bool dense_few_takes(int64_t m, int n, int k);
 hipError_t launch_dense_few(const DenseFewArgs& a, hipStream_t stream);
-// The dense kernel that quantises its own rows (ties to even): whether it is the one for this problem.  `few`: the kernel of a few
-// rows would run it otherwise; `wide_allowed` as in gemm_dense_takes.
-bool dense_rows_takes(int64_t m, int n, int k, bool few, bool wide_allowed);
-hipError_t launch_dense_rows(const DenseFewArgs& a, hipStream_t stream);
+// The dense kernel that quantises its own rows (ties to even): the entry of its table for this problem, -1 if it is not the one.
+// `few`: the kernel of a few rows would run it otherwise; if not, `us`: what the quantised product is expected to take.
+constexpr int kDenseRowsFrom = 5;  // rows
+int dense_rows_pick(int64_t m, int n, int k, bool few, float us);
+hipError_t launch_dense_rows(const DenseFewArgs& a, int entry, hipStream_t stream);
 
 // The whole layer of a few tokens in two launches: act holds tokens * top_k rows of inter bf16.
 struct FewTokensArgs {

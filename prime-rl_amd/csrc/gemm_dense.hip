@@ -19,6 +19,8 @@
 // multiplications of a step: all of them at its start hold up the wavefront until the address unit has
 // taken them (333x4096x2048 9.0 -> 8.5 us, 333x4096x4096 14.2 -> 13.0, 1000x2384x3200 16.7 -> 15.7).  Activation rows are padded with zeros to a multiple of 128
 // bytes (the quantiser writes them), which lets a reduction of any multiple of 64 run on the same path.
+#include <iterator>
+
 #include "lds_loads.hpp"
 
 namespace moe_i8 {
@@ -392,32 +394,23 @@ float estimate_wide(int64_t m, int64_t n, int64_t k) {
   return estimate(kWide, m, n, k) + (float)(m * n) * 2e-6f * (n % 32 ? 0.32f : 0.21f);
 }
 
-const Config* pick(int64_t m, int64_t n, int64_t k, bool wide_allowed) {
-  const Config* best = wide_allowed ? &kWide : nullptr;
-  float least = wide_allowed ? estimate_wide(m, n, k) : 0.0f;
-  for (const Config& c : kConfigs) {
-    const float t = estimate(c, m, n, k);
-    if (!best || t < least) least = t, best = &c;
-  }
-  return best;
-}
-
 }  // namespace
 
 int dense_row_stride(int k) { return (k + kStepBytes - 1) / kStepBytes * kStepBytes; }
 
-bool gemm_dense_takes(int64_t m, int n, int k, bool wide_allowed) {
+DensePick gemm_dense_pick(int64_t m, int n, int k, bool wide_allowed) {
+  DensePick best{-1, wide_allowed ? estimate_wide(m, n, k) : 0.0f};
+  for (int i = 0; i < (int)std::size(kConfigs); ++i) {
+    const float us = estimate(kConfigs[i], m, n, k);
+    if (us < best.us || (i == 0 && !wide_allowed)) best = {i, us};
+  }
   // per-lane source offsets are 32-bit: the weights and the activation matrix must each span less than 4 GiB
-  if (m < 1 || (int64_t)n * k >= (1ll << 32) || m * dense_row_stride(k) >= (1ll << 32)) return false;
-  return pick(m, n, k, wide_allowed) != &kWide;
+  if (m < 1 || (int64_t)n * k >= (1ll << 32) || m * dense_row_stride(k) >= (1ll << 32)) best.entry = -1;
+  return best;
 }
 
-float gemm_dense_estimate(int64_t m, int n, int k, bool wide_allowed) {
-  const Config* c = pick(m, n, k, wide_allowed);
-  return c == &kWide ? estimate_wide(m, n, k) : estimate(*c, m, n, k);
-}
-
-hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream) {
+hipError_t launch_gemm_dense(const DenseArgs& a, int entry, hipStream_t stream) {
+  if (entry < 0 || entry >= (int)std::size(kConfigs)) return hipErrorInvalidValue;
   DenseParams p{};
   p.a_q = a.a_q;
   p.a_scale = a.a_scale;
@@ -428,7 +421,7 @@ hipError_t launch_gemm_dense(const DenseArgs& a, hipStream_t stream) {
   p.N = a.n;
   p.K = a.k;
   p.lda = dense_row_stride(a.k);
-  const Config* c = pick(a.m, a.n, a.k, false);
+  const Config* c = kConfigs + entry;
   if (a.m * (a.mode == kGateUpSilu ? a.n / 2 : a.n) * 2 > kThroughBytes)
     for (const Config& l : kLarge)
       if (l.tm == c->tm && l.tn == c->tn && l.per_cu == c->per_cu) c = &l;

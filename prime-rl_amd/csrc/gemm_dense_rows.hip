@@ -10,6 +10,8 @@
 // us per call, quantisation launch and dense kernel / here: 17 rows x 2672 channels x 896 6.75 / 3.9, 103 x 992 x 1024 7.7 / 4.2,
 // 309 x 512 x 896 7.2 / 4.9, 54 x 1248 x 1152 7.1 / 4.4, 122 x 8448 x 704 7.5 / 6.2, 45 x 624 x 2880 7.3 / 5.7; over 343 problems of
 // 17..1000 rows x 512..14336 channels x 192..4200, taken where the estimates say so, 22 % faster on average.
+#include <iterator>
+
 #include "lds_loads.hpp"
 #include "quant_body.hpp"
 
@@ -302,18 +304,6 @@ const Config kConfigs[] = {
     MOE_I8_ROWS(16, 32, 8, 1, 1, 2, 8, 1, 0.17f, 2.82f, 1.12f, 0.0f, 0.0f),
 };
 
-const Config* pick(int64_t m, int n, int k, float* us) {
-  const Config* best = nullptr;
-  const float kb = (float)k / 1024.0f, cus = (float)device_cu_count();
-  for (const Config& c : kConfigs) {
-    if (k > c.longest || (c.longest > 1024 && k <= c.longest / 2)) continue;  // (fitted to reductions between the two)
-    const float tiles = (float)(((m + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn));
-    const float t = c.start + ceilf(tiles / (cus * c.per_cu)) * (c.per_round + c.per_k * kb) + ceilf(tiles / cus) * (c.per_wave + c.per_wave_k * kb);
-    if (!best || t < *us) best = &c, *us = t;
-  }
-  return best;
-}
-
 }  // namespace
 
 // A row more costs the kernel of a few rows a pass over its registers' weights, this one nothing up to 16: us there / here at 8 rows
@@ -322,16 +312,25 @@ const Config* pick(int64_t m, int n, int k, float* us) {
 // 7 % of that (5 rows of 4096 x 1408, 4.83 by the estimates against 4.67: the gated MLP 10.0 / 10.75) and up to 4 rows everything,
 // where it is the faster one or even on all but the widest matrices.  A quantisation launch adds about 3.06 us + 0.69 per 5 MB that it moves to the
 // dense kernels' estimate.
-bool dense_rows_takes(int64_t m, int n, int k, bool few, bool wide_allowed) {
-  if (m < 5 || (int64_t)n * k >= (1ll << 32) || n % 16 != 0 || k % 64 != 0) return false;
-  float us = 0.0f;
-  if (!pick(m, n, k, &us)) return false;
+int dense_rows_pick(int64_t m, int n, int k, bool few, float us) {
+  if (m < kDenseRowsFrom || (int64_t)n * k >= (1ll << 32) || n % 16 != 0 || k % 64 != 0) return -1;
   const float w = (float)n * (float)k * 1e-6f;
-  return us < (few ? 0.93f * (3.48f + 0.0603f * w + 0.0262f * (float)m * w + 0.05f * (float)m)
-                   : gemm_dense_estimate(m, n, k, wide_allowed) + 3.06f + 0.69f * (float)m * (float)k * (3.0f / 5e6f));
+  float least = few ? 0.93f * (3.48f + 0.0603f * w + 0.0262f * (float)m * w + 0.05f * (float)m)
+                    : us + 3.06f + 0.69f * (float)m * (float)k * (3.0f / 5e6f);
+  int best = -1;
+  const float kb = (float)k / 1024.0f, cus = (float)device_cu_count();
+  for (int i = 0; i < (int)std::size(kConfigs); ++i) {
+    const Config& c = kConfigs[i];
+    if (k > c.longest || (c.longest > 1024 && k <= c.longest / 2)) continue;  // (fitted to reductions between the two)
+    const float tiles = (float)(((m + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn));
+    const float t = c.start + ceilf(tiles / (cus * c.per_cu)) * (c.per_round + c.per_k * kb) + ceilf(tiles / cus) * (c.per_wave + c.per_wave_k * kb);
+    if (t < least) best = i, least = t;
+  }
+  return best;
 }
 
-hipError_t launch_dense_rows(const DenseFewArgs& a, hipStream_t stream) {
+hipError_t launch_dense_rows(const DenseFewArgs& a, int entry, hipStream_t stream) {
+  if (entry < 0 || entry >= (int)std::size(kConfigs) || a.k > kConfigs[entry].longest) return hipErrorInvalidValue;
   DenseRowsParams p{};
   p.x = a.x;
   p.w = a.w;
@@ -340,10 +339,7 @@ hipError_t launch_dense_rows(const DenseFewArgs& a, hipStream_t stream) {
   p.M = a.m;
   p.N = a.n;
   p.K = a.k;
-  float us;
-  const Config* c = pick(a.m, a.n, a.k, &us);
-  if (!c) return hipErrorInvalidValue;
-  return a.mode == kGateUpSilu ? c->gate_up(p, stream) : c->down(p, stream);
+  return a.mode == kGateUpSilu ? kConfigs[entry].gate_up(p, stream) : kConfigs[entry].down(p, stream);
 }
 
 }  // namespace moe_i8
