@@ -297,6 +297,24 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
                     const float* w2_scale, void* out, int64_t m, int hidden, int inter, void* workspace,
                     int64_t workspace_bytes, int variant, void* stream);
 
+/*
+ * The kernel of each GEMM of the two, decided on the host from the sizes alone (no GPU call) as the call itself decides, for
+ * pointers that are aligned and an output that does not overlap the input.  A diagnostic like moe_i8_layer_plan: it lets a test
+ * say which kernel and tile its sizes run on.  Any output pointer may be null.  Returns MOE_I8_EUNSUPPORTED when `variant`
+ * demands a family that does not handle the shape.
+ */
+#define MOE_I8_DENSE_FEW 16   /* a few rows, quantised by every workgroup */
+#define MOE_I8_DENSE_ROWS 17  /* some tens to hundreds of rows, quantised by the workgroups whose tiles they are in */
+#define MOE_I8_DENSE_TILES 18 /* rows quantised by a launch of their own */
+typedef struct moe_i8_dense_kernel {
+  int kernel;                    /* MOE_I8_DENSE_*, or MOE_I8_GEMM_* where a grouped family runs it */
+  int tile_rows, tile_channels;  /* weight rows of a tile for gate_up; 0 where the kernel has no such tiles */
+  int entry;                     /* place in the kernel's table of tiles, some of which differ in more than their size; -1: none */
+  int through;                   /* results are written through to memory */
+} moe_i8_dense_kernel;
+int moe_i8_linear_plan(int64_t m, int n, int k, int variant, moe_i8_dense_kernel* product);
+int moe_i8_mlp_plan(int64_t m, int hidden, int inter, int variant, moe_i8_dense_kernel* gate_up, moe_i8_dense_kernel* down);
+
 #ifdef __cplusplus
 }
 #endif

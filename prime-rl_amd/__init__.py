@@ -13,6 +13,8 @@ from .api import (  # noqa: F401
     fused_topk,
     layer_launches,
     layer_plan,
+    linear_plan,
+    mlp_plan,
     grouped_topk,
     route_topk,
     routed_experts_payload,
@@ -40,6 +42,8 @@ __all__ = [
     "fused_moe",
     "layer_launches",
     "layer_plan",
+    "linear_plan",
+    "mlp_plan",
     "moe_align_block_size",
     "per_token_quant_int8",
     "quantize_weights_per_channel",

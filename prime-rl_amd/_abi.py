@@ -21,8 +21,17 @@ OK = 0
 EINVAL, EWORKSPACE, ELAUNCH, EUNSUPPORTED = -1, -2, -3, -4
 DTYPE_BF16 = 0
 GEMM_AUTO, GEMM_STREAM, GEMM_TILE, GEMM_NARROW, GEMM_TILE_WIDE, GEMM_TILE_DEEP, GEMM_TILE_RING = 0, 1, 2, 3, 4, 5, 6
+DENSE_FEW, DENSE_ROWS, DENSE_TILES = 16, 17, 18
 SCORE_SOFTMAX, SCORE_SIGMOID, SCORE_TOPK_SOFTMAX = 0, 1, 2
 MAX_EXPERTS = 1024
+
+
+
+class DenseKernel(ctypes.Structure):
+    """``moe_i8_dense_kernel``"""
+
+    _fields_ = [("kernel", c_int), ("tile_rows", c_int), ("tile_channels", c_int), ("entry", c_int), ("through", c_int)]
+
 
 _P = c_void_p
 # name -> (restype, argtypes); mirrors include/moe_i8.h one to one
@@ -71,6 +80,8 @@ SIGNATURES = {
         [_P, _P, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, _P, c_int, c_int, c_int, c_int,
          c_float, _P, _P, _P, c_int, c_int64, c_int64, _P, c_int64, c_int, _P],
     ),
+    "moe_i8_linear_plan": (c_int, [c_int64, c_int, c_int, c_int, _P]),
+    "moe_i8_mlp_plan": (c_int, [c_int64, c_int, c_int, c_int, _P, _P]),
     "moe_i8_layer_plan": (c_int, [c_int64, c_int, c_int, c_int, c_int, c_int, c_int, _P, _P, _P]),
     "moe_i8_layer_launches": (c_int, [c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P]),
     "moe_i8_fused_experts_static": (

@@ -115,7 +115,8 @@ def workspace_bytes(m: int, top_k: int, num_experts: int, hidden: int, inter: in
 
 
 _KERNEL_NAMES = {_abi.GEMM_STREAM: "stream", _abi.GEMM_NARROW: "narrow", _abi.GEMM_TILE_WIDE: "tile_wide",
-                 _abi.GEMM_TILE_DEEP: "tile_deep", _abi.GEMM_TILE_RING: "tile_ring"}
+                 _abi.GEMM_TILE_DEEP: "tile_deep", _abi.GEMM_TILE_RING: "tile_ring", _abi.DENSE_FEW: "dense_few",
+                 _abi.DENSE_ROWS: "dense_rows", _abi.DENSE_TILES: "dense"}
 
 
 def layer_plan(m: int, top_k: int, num_experts: int, hidden: int, inter: int,
@@ -142,6 +143,31 @@ def layer_launches(m: int, top_k: int, num_experts: int, hidden: int, inter: int
     _abi.check(_abi.load().moe_i8_layer_launches(m, top_k, num_experts, hidden, inter, block_size, _variant(gemm_variant),
                                                  1 if routed else 0, ctypes.byref(n)))
     return n.value
+
+
+def _dense_kernel(k: _abi.DenseKernel) -> dict:
+    return {"kernel": _KERNEL_NAMES[k.kernel], "tile": (k.tile_rows, k.tile_channels) if k.tile_rows else None,
+            "entry": k.entry if k.entry >= 0 else None, "through": bool(k.through)}
+
+
+def linear_plan(m: int, n: int, k: int, gemm_variant: str | int = "auto") -> dict:
+    """The kernel of an ``apply_int8_linear`` call, decided on the host from the sizes alone as the call itself decides:
+    ``{"kernel": name, "tile": (rows, channels) or None, "entry": place in the kernel's table of tiles or None, "through":
+    results are written through to memory}``."""
+    import ctypes
+
+    out = _abi.DenseKernel()
+    _abi.check(_abi.load().moe_i8_linear_plan(m, n, k, _variant(gemm_variant), ctypes.byref(out)))
+    return _dense_kernel(out)
+
+
+def mlp_plan(m: int, hidden: int, inter: int, gemm_variant: str | int = "auto") -> dict:
+    """The same for the two GEMMs of a ``w8a8_mlp`` call: ``{"gate_up": {...}, "down": {...}}``."""
+    import ctypes
+
+    gate_up, down = _abi.DenseKernel(), _abi.DenseKernel()
+    _abi.check(_abi.load().moe_i8_mlp_plan(m, hidden, inter, _variant(gemm_variant), ctypes.byref(gate_up), ctypes.byref(down)))
+    return {"gate_up": _dense_kernel(gate_up), "down": _dense_kernel(down)}
 
 
 # --------------------------------------------------------------------------------------------- #

@@ -1020,6 +1020,19 @@ bool may_quantise(const void* x, const moe_i8::GemmArgs& g) {
   return aligned16(x) && aligned16(g.w) && !overlap(x, 2 * g.num_pairs * g.k, g.out, 2 * g.num_pairs * width);
 }
 
+struct MlpChoice {
+  DenseChoice gate_up, down;
+};
+MlpChoice mlp_choice(const moe_i8::GemmArgs& gu, const moe_i8::GemmArgs& dg, int variant, bool own_gu, bool own_dg) {
+  return {dense_choice(gu, variant, own_gu), dense_choice(dg, variant, own_dg)};
+}
+
+// The 256-row tiles of the LDS-tiled family for what the dense kernel leaves to the grouped families, where they can run it.
+int grouped_variant(moe_i8::GemmArgs g, int variant) {
+  g.tile_geometry = moe_i8::kTileWide;
+  return variant == MOE_I8_GEMM_AUTO && moe_i8::gemm_tile_supports(g) ? MOE_I8_GEMM_TILE_WIDE : variant;
+}
+
 // The product of a quantised problem.
 int run_quantised(const DenseChoice& choice, const moe_i8::GemmArgs& g, int variant, hipStream_t stream) {
   if (int rc = check_dense_gemm(g, variant)) return rc;
@@ -1027,10 +1040,7 @@ int run_quantised(const DenseChoice& choice, const moe_i8::GemmArgs& g, int vari
     const moe_i8::DenseArgs d{g.mode, g.a_q, g.a_scale, g.w, g.w_scale, g.out, g.num_pairs, g.n, g.k};
     return check_launch(moe_i8::launch_gemm_dense(d, choice.entry, stream), "gemm_dense");
   }
-  moe_i8::GemmArgs wide = g;
-  wide.tile_geometry = moe_i8::kTileWide;
-  if (variant == MOE_I8_GEMM_AUTO && moe_i8::gemm_tile_supports(wide)) variant = MOE_I8_GEMM_TILE_WIDE;
-  return run_gemm(g, variant, stream);
+  return run_gemm(g, grouped_variant(g, variant), stream);
 }
 // A problem whose rows the product's launch quantises.
 int run_unquantised(const DenseChoice& choice, const void* x, const moe_i8::GemmArgs& g, hipStream_t stream) {
@@ -1038,6 +1048,27 @@ int run_unquantised(const DenseChoice& choice, const void* x, const moe_i8::Gemm
   const moe_i8::DenseFewArgs d{g.mode, static_cast<const uint16_t*>(x), g.w, g.w_scale, static_cast<uint16_t*>(g.out), (int)g.num_pairs, g.n, g.k};
   return choice.way == kFew ? check_launch(moe_i8::launch_dense_few(d, stream), "dense_few")
                             : check_launch(moe_i8::launch_dense_rows(d, choice.entry, stream), "dense_rows");
+}
+
+int dense_shape_args(int64_t m, int n, int k, int variant) {
+  if (m < 1 || m > INT32_MAX - kDenseBlock) return fail(MOE_I8_EINVAL, "m out of range");
+  if (n < 16 || n % 16) return fail(MOE_I8_EINVAL, "output channels (%d) must be a positive multiple of 16", n);
+  if (k < 64 || k % 64) return fail(MOE_I8_EINVAL, "reduction length (%d) must be a positive multiple of 64", k);
+  if (variant < MOE_I8_GEMM_AUTO || variant > MOE_I8_GEMM_TILE_RING) return fail(MOE_I8_EINVAL, "unknown GEMM variant %d", variant);
+  return MOE_I8_OK;
+}
+int dense_plan(const DenseChoice& choice, const moe_i8::GemmArgs& g, int variant, moe_i8_dense_kernel* out) {
+  moe_i8_dense_kernel plan{MOE_I8_DENSE_FEW, 0, 0, choice.entry, 0};
+  if (choice.way == kGrouped) {
+    plan.kernel = picks_kernel(g, grouped_variant(g, variant));
+    if (plan.kernel < 0) return MOE_I8_EUNSUPPORTED;
+  } else if (choice.way != kFew) {
+    const moe_i8::DenseTile tile = choice.way == kDense ? moe_i8::gemm_dense_tile(choice.entry) : moe_i8::dense_rows_tile(choice.entry);
+    plan = {choice.way == kDense ? MOE_I8_DENSE_TILES : MOE_I8_DENSE_ROWS, tile.rows, tile.channels, choice.entry,
+            choice.way == kRows || moe_i8::gemm_dense_through(g.mode, g.num_pairs, g.n)};
+  }
+  if (out) *out = plan;
+  return MOE_I8_OK;
 }
 
 // The ties-to-even row quantiser of the dense path; `padded`: rows for the dense kernel; `route`: its
@@ -1120,8 +1151,7 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   const moe_i8::GemmArgs gu = dense_group(moe_i8::kGateUpSilu, c, ws, x_q, a1, w13, w13_scale, ws + c.act, m, 2 * inter, hidden);
   moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, ws, act_q, a2, w2, w2_scale, out, m, hidden, inter);
   const WorkspaceTurn turn(workspace);
-  const DenseChoice choice_dg = dense_choice(dg, variant, may_quantise(ws + c.act, dg));
-  const DenseChoice choice_gu = dense_choice(gu, variant, may_quantise(x, gu));
+  const auto [choice_gu, choice_dg] = mlp_choice(gu, dg, variant, may_quantise(x, gu), may_quantise(ws + c.act, dg));
   const bool dense_dg = choice_dg.way == kDense, route_dg = choice_dg.way == kGrouped;
   if (choice_gu.way >= kRows) {
     if (int rc = check_dense_gemm(dg, variant)) return rc;  // before anything is launched
@@ -1147,6 +1177,24 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   }
   if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, choice_gu.way >= kRows && route_dg, c, ws, s)) return rc;
   return run_quantised(choice_dg, dg, variant, s);
+}
+
+int moe_i8_linear_plan(int64_t m, int n, int k, int variant, moe_i8_dense_kernel* product) {
+  if (int rc = dense_shape_args(m, n, k, variant)) return rc;
+  const DenseCarve c = dense_carve(m, k, 0);
+  const moe_i8::GemmArgs g = dense_group(moe_i8::kDown, c, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, m, n, k);
+  return dense_plan(dense_choice(g, variant, true), g, variant, product);
+}
+
+int moe_i8_mlp_plan(int64_t m, int hidden, int inter, int variant, moe_i8_dense_kernel* gate_up, moe_i8_dense_kernel* down) {
+  if (inter < 64 || inter % 64) return fail(MOE_I8_EINVAL, "inter (%d) must be a positive multiple of 64", inter);
+  if (int rc = dense_shape_args(m, hidden, hidden, variant)) return rc;
+  const DenseCarve c = dense_carve(m, hidden, inter);
+  const moe_i8::GemmArgs gu = dense_group(moe_i8::kGateUpSilu, c, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, m, 2 * inter, hidden);
+  const moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, m, hidden, inter);
+  const MlpChoice choice = mlp_choice(gu, dg, variant, true, true);
+  if (int rc = dense_plan(choice.gate_up, gu, variant, gate_up)) return rc;
+  return dense_plan(choice.down, dg, variant, down);
 }
 
 }  // extern "C"

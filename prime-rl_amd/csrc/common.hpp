@@ -349,6 +349,12 @@ struct DensePick {
 // `wide_allowed`: the 256-row tiles of the LDS-tiled family can run the problem too and are preferred where they are expected to
 // be faster.
 DensePick gemm_dense_pick(int64_t m, int n, int k, bool wide_allowed);
+struct DenseTile {
+  int rows;
+  int channels;  // weight rows
+};
+DenseTile gemm_dense_tile(int entry);
+bool gemm_dense_through(int mode, int64_t m, int n);  // results are written through to memory
 hipError_t launch_gemm_dense(const DenseArgs& a, int entry, hipStream_t stream);
 
 // The same for a few rows, which the launch quantises itself (ties to even).
@@ -369,6 +375,7 @@ hipError_t launch_dense_few(const DenseFewArgs& a, hipStream_t stream);
 // `few`: the kernel of a few rows would run it otherwise; if not, `us`: what the quantised product is expected to take.
 constexpr int kDenseRowsFrom = 5;  // rows
 int dense_rows_pick(int64_t m, int n, int k, bool few, float us);
+DenseTile dense_rows_tile(int entry);
 hipError_t launch_dense_rows(const DenseFewArgs& a, int entry, hipStream_t stream);
 
 // The whole layer of a few tokens in two launches: act holds tokens * top_k rows of inter bf16.

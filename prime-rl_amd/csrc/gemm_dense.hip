@@ -409,6 +409,10 @@ DensePick gemm_dense_pick(int64_t m, int n, int k, bool wide_allowed) {
   return best;
 }
 
+DenseTile gemm_dense_tile(int entry) { return {kConfigs[entry].tm, kConfigs[entry].tn}; }
+
+bool gemm_dense_through(int mode, int64_t m, int n) { return m * (mode == kGateUpSilu ? n / 2 : n) * 2 <= kThroughBytes; }
+
 hipError_t launch_gemm_dense(const DenseArgs& a, int entry, hipStream_t stream) {
   if (entry < 0 || entry >= (int)std::size(kConfigs)) return hipErrorInvalidValue;
   DenseParams p{};
@@ -422,7 +426,7 @@ hipError_t launch_gemm_dense(const DenseArgs& a, int entry, hipStream_t stream) 
   p.K = a.k;
   p.lda = dense_row_stride(a.k);
   const Config* c = kConfigs + entry;
-  if (a.m * (a.mode == kGateUpSilu ? a.n / 2 : a.n) * 2 > kThroughBytes)
+  if (!gemm_dense_through(a.mode, a.m, a.n))
     for (const Config& l : kLarge)
       if (l.tm == c->tm && l.tn == c->tn && l.per_cu == c->per_cu) c = &l;
   return a.mode == kGateUpSilu ? c->gate_up(p, stream) : c->down(p, stream);

@@ -329,6 +329,8 @@ int dense_rows_pick(int64_t m, int n, int k, bool few, float us) {
   return best;
 }
 
+DenseTile dense_rows_tile(int entry) { return {kConfigs[entry].tm, kConfigs[entry].tn}; }
+
 hipError_t launch_dense_rows(const DenseFewArgs& a, int entry, hipStream_t stream) {
   if (entry < 0 || entry >= (int)std::size(kConfigs) || a.k > kConfigs[entry].longest) return hipErrorInvalidValue;
   DenseRowsParams p{};

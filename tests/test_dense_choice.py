@@ -1,0 +1,51 @@
+"""Which kernel and tile a dense call is given, and that the GPU tests of the dense kernels run every one of them."""
+
+import pytest
+
+import test_gpu_dense_kernel as gpu
+
+
+def _cases(*tests):
+    return [c for t in tests for mark in t.pytestmark if mark.name == "parametrize" for c in mark.args[1]]
+
+
+def _reached(pra, cases):
+    """The kernels and table entries of the linear layer and of the gated MLP's gate_up that the GPU tests run for these sizes."""
+    linear, gate_up = set(), set()
+    for m, n, k in cases:
+        p = pra.linear_plan(m, n, k)
+        linear.add((p["kernel"], p["entry"]))
+        inter = n // 2 // 64 * 64
+        if inter:
+            p = pra.mlp_plan(m, k, inter)["gate_up"]
+            gate_up.add((p["kernel"], p["entry"]))
+    return linear, gate_up
+
+
+def test_every_tile_of_rows_that_their_workgroups_quantise_is_run(pra):
+    linear, gate_up = _reached(pra, _cases(gpu.test_rows_quantised_by_their_tiles, gpu.test_rows_quantised_by_wide_tiles))
+    assert linear == {("dense_rows", i) for i in range(10)}
+    assert gate_up >= linear
+
+
+def test_the_kernel_of_a_few_rows_is_run_with_every_number_of_rows_a_wavefront_can_have(pra):
+    few = [(m, n, k) for m, n, k in _cases(gpu.test_few_rows_in_one_launch, gpu.test_most_rows_in_one_launch)
+           if pra.linear_plan(m, n, k)["kernel"] == "dense_few"]
+    assert {1, 2, 8, 13, 16} <= {m for m, _, _ in few}  # one row a wavefront, the second one of some and of all of them
+    assert {(k + 1023) // 1024 for _, _, k in few} == set(range(1, 9))
+
+
+def test_plans_follow_a_demanded_family_and_reject_what_a_call_rejects(pra):
+    assert pra.linear_plan(333, 4096, 2048, gemm_variant="stream") == {"kernel": "stream", "tile": None, "entry": None, "through": False}
+    assert pra.mlp_plan(333, 4096, 2048, gemm_variant="tile_wide")["down"]["kernel"] == "tile_wide"
+    assert pra.linear_plan(333, 4096, 2048)["tile"] == (64, 128)
+    assert pra.linear_plan(17, 2672, 896)["kernel"] == "dense_rows"
+    assert pra.mlp_plan(5, 4096, 1408) == {w: {"kernel": "dense_few", "tile": None, "entry": None, "through": False} for w in ("gate_up", "down")}
+    for sizes in ((0, 4096, 2048), (8, 4090, 2048), (8, 4096, 2016)):
+        with pytest.raises(pra._abi.MoeI8Error):
+            pra.linear_plan(*sizes)
+    with pytest.raises(pra._abi.MoeI8Error):
+        pra.mlp_plan(8, 4096, 1400)
+    with pytest.raises(pra._abi.MoeI8Error):
+        pra.linear_plan(8, 4096, 2048 + 64, gemm_variant="tile_wide")  # a reduction of no whole 128 bytes
+    assert pra._abi.load().moe_i8_mlp_plan(8, 4096, 1408, pra._abi.GEMM_AUTO, None, None) == pra._abi.OK

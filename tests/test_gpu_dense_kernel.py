@@ -115,3 +115,11 @@ def test_tiles_of_96(pra, oracle, M, N, K):
 def test_rows_quantised_by_wide_tiles(pra, oracle, M, N, K):
     """Tiles whose wavefronts do not split the reduction: rows and channels that fill no tile, reductions of one step and up to the longest."""
     test_rows_quantised_by_their_tiles(pra, oracle, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 128, 8192), (16, 240, 4224), (15, 128, 6016), (14, 144, 7168), (6, 8192, 4160), (6, 4096, 8192)])
+def test_most_rows_in_one_launch(pra, oracle, M, N, K):
+    """As many rows as one launch of the kernel of a few rows takes, where no other kernel that quantises its rows can run."""
+    assert pra.linear_plan(M, N, K)["kernel"] == "dense_few"
+    assert pra.mlp_plan(M, K, N // 2 // 64 * 64)["gate_up"]["kernel"] == "dense_few"
+    test_few_rows_in_one_launch(pra, oracle, M, N, K)
