@@ -1023,8 +1023,10 @@ bool may_quantise(const void* x, const moe_i8::GemmArgs& g) {
 struct MlpChoice {
   DenseChoice gate_up, down;
 };
+// Where a grouped family runs the down GEMM the first quantisation has a launch of its own, which also writes that family's routing.
 MlpChoice mlp_choice(const moe_i8::GemmArgs& gu, const moe_i8::GemmArgs& dg, int variant, bool own_gu, bool own_dg) {
-  return {dense_choice(gu, variant, own_gu), dense_choice(dg, variant, own_dg)};
+  const DenseChoice down = dense_choice(dg, variant, own_dg);
+  return {dense_choice(gu, variant, own_gu && down.way != kGrouped), down};
 }
 
 // The 256-row tiles of the LDS-tiled family for what the dense kernel leaves to the grouped families, where they can run it.
@@ -1152,13 +1154,13 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
   moe_i8::GemmArgs dg = dense_group(moe_i8::kDown, c, ws, act_q, a2, w2, w2_scale, out, m, hidden, inter);
   const WorkspaceTurn turn(workspace);
   const auto [choice_gu, choice_dg] = mlp_choice(gu, dg, variant, may_quantise(x, gu), may_quantise(ws + c.act, dg));
-  const bool dense_dg = choice_dg.way == kDense, route_dg = choice_dg.way == kGrouped;
+  const bool dense_dg = choice_dg.way == kDense;
   if (choice_gu.way >= kRows) {
     if (int rc = check_dense_gemm(dg, variant)) return rc;  // before anything is launched
     if (int rc = run_unquantised(choice_gu, x, gu, s)) return rc;
   } else {
     const bool dense_gu = choice_gu.way == kDense;
-    if (int rc = dense_quant(x, m, hidden, x_q, a1, dense_gu, !dense_gu || route_dg, c, ws, s)) return rc;
+    if (int rc = dense_quant(x, m, hidden, x_q, a1, dense_gu, !dense_gu || choice_dg.way == kGrouped, c, ws, s)) return rc;
     if (int rc = run_quantised(choice_gu, gu, variant, s)) return rc;
   }
   if (choice_dg.way >= kRows) return run_unquantised(choice_dg, ws + c.act, dg, s);
@@ -1175,7 +1177,7 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
     dg.a_round_even = true;
     return check_launch(moe_i8::launch_gemm_stream(dg, s), "gemm_stream");
   }
-  if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, choice_gu.way >= kRows && route_dg, c, ws, s)) return rc;
+  if (int rc = dense_quant(ws + c.act, m, inter, act_q, a2, dense_dg, false, c, ws, s)) return rc;
   return run_quantised(choice_dg, dg, variant, s);
 }
 

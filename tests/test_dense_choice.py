@@ -49,3 +49,11 @@ def test_plans_follow_a_demanded_family_and_reject_what_a_call_rejects(pra):
     with pytest.raises(pra._abi.MoeI8Error):
         pra.linear_plan(8, 4096, 2048 + 64, gemm_variant="tile_wide")  # a reduction of no whole 128 bytes
     assert pra._abi.load().moe_i8_mlp_plan(8, 4096, 1408, pra._abi.GEMM_AUTO, None, None) == pra._abi.OK
+
+
+def test_a_grouped_down_gemm_finds_the_routing_that_the_first_quantisation_writes(pra):
+    """Weights of 4 GiB, which the dense kernels do not take: the kernel of a few rows writes no routing, so it does not run the
+    gate_up in front of them, though it could."""
+    plan = pra.mlp_plan(2, 8192, 1 << 19)
+    assert plan["down"]["kernel"] == plan["gate_up"]["kernel"] == "stream"
+    assert pra.linear_plan(2, 1 << 20, 8192)["kernel"] == "dense_few"
