@@ -1004,7 +1004,7 @@ DenseChoice dense_choice(moe_i8::GemmArgs g, int variant, bool own) {
   moe_i8::DensePick quantised{-1, 0.0f};
   if (!few) {
     g.tile_geometry = moe_i8::kTileWide;
-    quantised = moe_i8::gemm_dense_pick(g.num_pairs, g.n, g.k, moe_i8::gemm_tile_supports(g));
+    quantised = moe_i8::gemm_dense_pick(g.mode, g.num_pairs, g.n, g.k, moe_i8::gemm_tile_supports(g));
   }
   if (own) {
     const int entry = moe_i8::dense_rows_pick(g.num_pairs, g.n, g.k, few, quantised.us);

@@ -348,7 +348,7 @@ struct DensePick {
 };
 // `wide_allowed`: the 256-row tiles of the LDS-tiled family can run the problem too and are preferred where they are expected to
 // be faster.
-DensePick gemm_dense_pick(int64_t m, int n, int k, bool wide_allowed);
+DensePick gemm_dense_pick(int mode, int64_t m, int n, int k, bool wide_allowed);
 struct DenseTile {
   int rows;
   int channels;  // weight rows

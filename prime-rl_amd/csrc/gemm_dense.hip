@@ -365,7 +365,12 @@ const Config kConfigs[] = {
 };
 // The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Their stores are not hidden behind another
 // round's product: 0.21 us per MB, 0.32 where rows of the result begin inside 64 bytes (5780 rows x 2672 channels x 512: 24.8 us, in
-// 192 x 384 tiles 19.4).
+// 192 x 384 tiles 19.4).  gate_up stores half as many results as it has weight rows and takes 0.32 us per MB
+// of them, with the SiLU that is not hidden either: over 1220 gate_up GEMMs of 100..16384 rows, 512..16384 weight rows and a reduction of
+// 512..7168 the choice takes on average 0.23 % longer than the fastest tile, 0.28 % at 0.21 us, 0.40 % at 0.21 us for twice the results.  us,
+// the dense tiles taken then / the wide ones: 2048 x 7936 x 1024 30.4 / 26.6, 6510 x 11264 x 640 81.4 / 72.0, 8052 x 8448 x 512 71.7 / 63.3, 4096 x
+// 2816 x 4096 58.5 / 58.6; left to the dense tiles: 5047 x 1920 x 2304 37.7 / 40.2; wrong by most: 5485 x 4480 x
+// 768 36.2 / 39.2.
 const Config kWide = {256, 256, 1, 5.61f, 0.95f, 10.70f, 7.08f, 1e9f, nullptr, nullptr};
 
 // The largest tiles of kConfigs for results of more than kThroughBytes (no launch that the estimates would choose has so many in
@@ -390,16 +395,17 @@ float estimate(const Config& c, int64_t m, int64_t n, int64_t k) {
   return c.start + rounds * c.per_round + (latency > ops ? latency : ops);
 }
 
-float estimate_wide(int64_t m, int64_t n, int64_t k) {
-  return estimate(kWide, m, n, k) + (float)(m * n) * 2e-6f * (n % 32 ? 0.32f : 0.21f);
+float estimate_wide(int mode, int64_t m, int64_t n, int64_t k) {
+  const int64_t width = mode == kGateUpSilu ? n / 2 : n;
+  return estimate(kWide, m, n, k) + (float)(m * width) * 2e-6f * (mode == kGateUpSilu || width % 32 ? 0.32f : 0.21f);
 }
 
 }  // namespace
 
 int dense_row_stride(int k) { return (k + kStepBytes - 1) / kStepBytes * kStepBytes; }
 
-DensePick gemm_dense_pick(int64_t m, int n, int k, bool wide_allowed) {
-  DensePick best{-1, wide_allowed ? estimate_wide(m, n, k) : 0.0f};
+DensePick gemm_dense_pick(int mode, int64_t m, int n, int k, bool wide_allowed) {
+  DensePick best{-1, wide_allowed ? estimate_wide(mode, m, n, k) : 0.0f};
   for (int i = 0; i < (int)std::size(kConfigs); ++i) {
     const float us = estimate(kConfigs[i], m, n, k);
     if (us < best.us || (i == 0 && !wide_allowed)) best = {i, us};

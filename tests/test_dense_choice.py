@@ -57,3 +57,16 @@ def test_a_grouped_down_gemm_finds_the_routing_that_the_first_quantisation_write
     plan = pra.mlp_plan(2, 8192, 1 << 19)
     assert plan["down"]["kernel"] == plan["gate_up"]["kernel"] == "stream"
     assert pra.linear_plan(2, 1 << 20, 8192)["kernel"] == "dense_few"
+
+
+@pytest.mark.parametrize("m,hidden,inter,kernel,tile", [
+    # gate_up with wide tiles, us: 2048 rows of 1024 x 3968 26.6 (192 x 384 tiles 30.4), 6510 of 640 x 5632 72.0 (81.4)
+    (2048, 1024, 3968, "tile_wide", None),
+    (6510, 640, 5632, "tile_wide", None),
+    (4096, 4096, 1408, "tile_wide", None),  # 58.6 (256 x 192 tiles 58.5: even)
+    (5047, 2304, 960, "dense", (256, 192)),  # 40.2 (37.7)
+    (7411, 3840, 1088, "dense", (192, 384)),  # 95.7 (80.1)
+])
+def test_gate_up_is_charged_for_the_results_it_stores(pra, m, hidden, inter, kernel, tile):
+    plan = pra.mlp_plan(m, hidden, inter)["gate_up"]
+    assert (plan["kernel"], plan["tile"]) == (kernel, tile)
