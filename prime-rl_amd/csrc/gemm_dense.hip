@@ -373,12 +373,10 @@ const Config kConfigs[] = {
 // 768 36.2 / 39.2.
 const Config kWide = {256, 256, 1, 5.61f, 0.95f, 10.70f, 7.08f, 1e9f, nullptr, nullptr};
 
-// The largest tiles of kConfigs for results of more than kThroughBytes (no launch that the estimates would choose has so many in
-// smaller ones).
+// Those tiles of kConfigs that the estimates choose for results of more than kThroughBytes (of 800 000 random ones up to 4 GB: a large
+// result fills the chip with the larger tiles, and 128 x 128 with one workgroup per compute unit and 128 x 192 are for those that do not).
 const Config kLarge[] = {
-    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 4, 4, 2, 1, 0.77f, 3.27f, 4.54f, 3.74f, 1e9f),
     MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 2, 2, 2, 2, 0.22f, 4.29f, 7.73f, 5.34f, 1e9f),
-    MOE_I8_DENSE_STORES(false, 128, 192, 1, 4, 2, 3, 2, 1, 0.35f, 4.31f, 6.18f, 4.63f, 1e9f),
     MOE_I8_DENSE_STORES(false, 256, 192, 1, 4, 2, 2, 2, 1, 0.0f, 7.04f, 10.80f, 7.67f, 1e9f),
     MOE_I8_DENSE_STORES(false, 192, 320, 1, 4, 2, 2, 2, 1, 0.0f, 7.86f, 12.92f, 10.01f, 1e9f),
     MOE_I8_DENSE_STORES(false, 192, 384, 1, 2, 4, 2, 2, 1, 0.0f, 8.42f, 15.58f, 11.33f, 1e9f),

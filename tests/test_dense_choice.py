@@ -14,18 +14,26 @@ def _reached(pra, cases):
     linear, gate_up = set(), set()
     for m, n, k in cases:
         p = pra.linear_plan(m, n, k)
-        linear.add((p["kernel"], p["entry"]))
+        linear.add((p["kernel"], p["entry"], p["through"]))
         inter = n // 2 // 64 * 64
         if inter:
             p = pra.mlp_plan(m, k, inter)["gate_up"]
-            gate_up.add((p["kernel"], p["entry"]))
+            gate_up.add((p["kernel"], p["entry"], p["through"]))
     return linear, gate_up
 
 
 def test_every_tile_of_rows_that_their_workgroups_quantise_is_run(pra):
     linear, gate_up = _reached(pra, _cases(gpu.test_rows_quantised_by_their_tiles, gpu.test_rows_quantised_by_wide_tiles))
-    assert linear == {("dense_rows", i) for i in range(10)}
+    assert linear == {("dense_rows", i, True) for i in range(10)}
     assert gate_up >= linear
+
+
+def test_every_tile_of_the_dense_kernel_is_run(pra):
+    linear, gate_up = _reached(pra, _cases(gpu.test_linear_and_mlp, gpu.test_large_tiles, gpu.test_tiles_of_96,
+                                           gpu.test_tiles_of_few_and_of_short_problems, gpu.test_results_of_more_than_96_mb))
+    every = {("dense", i, True) for i in range(13)} | {("dense", i, False) for i in (8, 10, 11, 12)}
+    assert linear >= every and gate_up >= every
+    assert {p for p in linear | gate_up if p[0] == "dense"} == every
 
 
 def test_the_kernel_of_a_few_rows_is_run_with_every_number_of_rows_a_wavefront_can_have(pra):

@@ -123,3 +123,20 @@ def test_most_rows_in_one_launch(pra, oracle, M, N, K):
     assert pra.linear_plan(M, N, K)["kernel"] == "dense_few"
     assert pra.mlp_plan(M, K, N // 2 // 64 * 64)["gate_up"]["kernel"] == "dense_few"
     test_few_rows_in_one_launch(pra, oracle, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 160, 8384), (21, 208, 5056), (23, 9008, 2496), (4717, 688, 64), (1182, 3680, 64)])  # 16 x 16, 32 x 64, 128 x 128
+def test_tiles_of_few_and_of_short_problems(pra, oracle, M, N, K):
+    test_linear_and_mlp(pra, oracle, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1371, 75024, 192),   # 128 x 128, two workgroups to a compute unit
+    (967, 106960, 448),   # 256 x 192
+    (37219, 2832, 192),   # 192 x 320
+    (25597, 3984, 64),    # 192 x 384
+])
+def test_results_of_more_than_96_mb(pra, oracle, M, N, K):
+    """Results that are left in the L2s, gate_up's as well (M x N / 2), in every tile that is picked for so many."""
+    assert not pra.linear_plan(M, N, K)["through"] and not pra.mlp_plan(M, K, N // 2 // 64 * 64)["gate_up"]["through"]
+    test_large_tiles(pra, oracle, M, N, K)
