@@ -306,16 +306,18 @@ const Config kConfigs[] = {
 
 }  // namespace
 
-// A row more costs the kernel of a few rows a pass over its registers' weights, this one nothing up to 16: us there / here at 8 rows
-// 9168 x 1280 8.5 / 5.0, 11376 x 640 6.7 / 4.3, 2928 x 1408 4.5 / 4.5, 1776 x 3584 6.0 / 6.6; at 5 9264 x 1024 5.4 / 4.5, 3024 x 1024
-// 3.9 / 4.1.  Its time is about 3.48 + 0.0603 W + 0.0262 m W + 0.05 m us with W = n * k / 10^6 (rms error 9 %); it keeps what is within
-// 7 % of that (5 rows of 4096 x 1408, 4.83 by the estimates against 4.67: the gated MLP 10.0 / 10.75) and up to 4 rows everything,
-// where it is the faster one or even on all but the widest matrices.  A quantisation launch adds about 3.06 us + 0.69 per 5 MB that it moves to the
-// dense kernels' estimate.
+// A row more costs the kernel of a few rows a pass over its registers' weights, this one nothing up to 16.  Up to 4 rows that kernel is the
+// faster one or even on all but the widest matrices (4 x 8848 x 1536 6.3 / 5.1).  From 5 on it takes, on the device, about 2.1 + 0.1 W +
+// 0.0235 m W + 0.22 m us with W = n * k / 10^6 (rms error 12 %); the constants above, fitted to calls from a host that sends one every 3.7 us,
+// are 0.4 us high for the shorter reductions.  Over 405 problems of 5 to 16 rows, launches of a captured graph, the choice takes 0.6 % longer than the
+// faster of the two, 4 % by estimates fitted to such calls with 7 % in favour of the other kernel (which it had not in a graph); from the host
+// 0.7 and 2.1 % (578 problems).  us there / here: 6 x 6272 x 192 5.2 / 3.6, 7 x 4496 x 256 4.8 / 3.3, 16 x 640 x 1280 6.7 / 4.3, 5 x 1792 x 832 3.5 / 4.2,
+// 5 x 3760 x 2368 4.6 / 5.7; wrong by most 5 x 3200 x 704 3.6 / 4.2 and 6 x 16000 x 2304 10.9 / 13.5.  A quantisation launch adds about
+// 3.06 us + 0.69 per 5 MB that it moves to the dense kernels' estimate.
 int dense_rows_pick(int64_t m, int n, int k, bool few, float us) {
   if (m < kDenseRowsFrom || (int64_t)n * k >= (1ll << 32) || n % 16 != 0 || k % 64 != 0) return -1;
   const float w = (float)n * (float)k * 1e-6f;
-  float least = few ? 0.93f * (3.48f + 0.0603f * w + 0.0262f * (float)m * w + 0.05f * (float)m)
+  float least = few ? 2.1f + 0.1f * w + 0.0235f * (float)m * w + 0.22f * (float)m + (k <= 1024 ? 0.4f : 0.0f)
                     : us + 3.06f + 0.69f * (float)m * (float)k * (3.0f / 5e6f);
   int best = -1;
   const float kb = (float)k / 1024.0f, cus = (float)device_cu_count();

@@ -78,3 +78,15 @@ def test_a_grouped_down_gemm_finds_the_routing_that_the_first_quantisation_write
 def test_gate_up_is_charged_for_the_results_it_stores(pra, m, hidden, inter, kernel, tile):
     plan = pra.mlp_plan(m, hidden, inter)["gate_up"]
     assert (plan["kernel"], plan["tile"]) == (kernel, tile)
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    # us in the kernel of a few rows / in the one that quantises its tiles' rows: 5.2 / 3.6, 4.8 / 3.3, 4.5 / 3.2, 6.7 / 4.3
+    (6, 6272, 192, "dense_rows"), (7, 4496, 256, "dense_rows"), (11, 864, 256, "dense_rows"), (16, 640, 1280, "dense_rows"),
+    (4, 6272, 192, "dense_few"),  # up to 4 rows whatever the reduction
+    # 3.5 / 4.2, 4.6 / 5.7, 5.0 / 7.2
+    (5, 1792, 832, "dense_few"), (5, 3760, 2368, "dense_few"), (5, 640, 3904, "dense_few"),
+    (5, 4096, 1408, "dense_few"),  # the gated MLP of it 10.0 / 10.75
+])
+def test_line_between_the_kernels_that_quantise_their_rows(pra, m, n, k, kernel):
+    assert pra.linear_plan(m, n, k)["kernel"] == kernel
