@@ -39,12 +39,21 @@ constexpr int kStepK = 64;    // reduction bytes per MFMA
 // Two wavefronts halve the reduction of a tile pair: workgroups of half the length and twice as many.  With whole ones a launch takes
 // 5 to 25 % longer from 513 and from 769 workgroups on, two and three to a compute unit.  Layer us, whole / halved: 129 experts of 4096 x 1408 with
 // skewed routing at 5 / 7 / 8 / 10 / 14 tokens 75.5 / 76.1, 71.1 / 71.6, 94.1 / 83.7, 94.5 / 83.7, 94.4 / 87.1, 128 of them
-// evenly routed at 5 / 8 / 12 105 / 103, 162 / 159, 197 / 193; 256 of 7168 x 2048 at 6 / 8 314 / 312, 388 / 377; 64 of 2048 x 1408,
-// skewed, at 6 / 12 43.9 / 38.5, 47.9 / 46.4, even, at 6 / 8 56.4 / 58.7, 67.9 / 65.0; 16 of 4096 x 4096 at 6 / 10 96.7 / 86.3, 117 /
-// 104.  A gate_up launch with fewer bytes per expert stays whole: 128 of 2048 x 768 at 9 to 16 tokens 0.6 % slower on average
-// (55.9 / 57.1 .. 69.3 / 67.1).  Quarters, or workgroups of two wavefronts: less, and losses of up to 4 % where halves have none.
+// evenly routed at 5 / 8 / 12 105 / 103, 162 / 159, 197 / 193; 256 of 7168 x 2048 at 6 / 8 314 / 312, 388 / 377; 16 of 4096 x 4096 at 6 / 10
+// 96.7 / 86.3, 117 / 104.  Quarters, or workgroups of two wavefronts: less, and losses of up to 4 % where halves have none.  (The halved
+// instances keep 18 and 20 registers in scratch, the whole ones 6 and 8, of 168.)
+// gate_up: halved from 4 MB an expert and reductions of 1536 on.  By how many per cent a layer takes longer with it halved, evenly routed | Zipf
+// routing, mean over 5 to 16 tokens, by MB and reduction: 2.0 (512 channels x 2048) -1 | -4, 3.0 (768 x 2048) 0 | -6, 3.8 (1280 x 1536) 0 | -3,
+// 4.0 (512 x 4096) -3 | -5, 4.0 (1024 x 2048) -1 | -1, 5.0 (1024 x 2560) -2 | -7, 5.5 (1408 x 2048) -1 | -2, 6.0 (2048 x 1536) 0 | -1, 8.0 (1024 x
+// 4096) -2 | -5, 16 (1024 x 8192) -3 | -7; shorter reductions: 4.5 (3072 x 768) 5 | 3, 4.0 (2048 x 1024) 3 | 3, 5.5 (2816 x 1024, 64 experts) 3 | 2, 8.0
+// (4096 x 1024) 3 | 2, 5.0 (2048 x 1280) 2 | 2, 5.6 (2560 x 1152) 4 | 4, 8.0 (8192 x 512) 4 | 5.  Given away: the gains below 4 MB.
+// down (that reads quantised rows): always.  By output channels x reduction, as above: 1536 x 1280 0 | -4, 2048 x 1152 0 | 1, 2048 x 1408 0 | -5, 2048 x
+// 1536 0 | -4, 1024 x 2048 (32 experts) -4 | -7, (64) 2 | -6, 768 x 3072 -7 | -18, 2880 x 2880 -3 | -2, 4096 x 4096 -2 | -8, 4096 x 14336 -9 | -12.  Evenly
+// routed experts of 2 to 3 MB lose up to 4 % at single numbers of tokens, where the halves are a few more than fit the device at a time; a line by
+// size would give away more than that under Zipf routing.
 constexpr int kParts = 2;
 constexpr int64_t kSplitBytes = 4 << 20;
+constexpr int kSplitReduction = 1536;
 constexpr int kTiles = 2;     // 16-row weight tiles per wavefront
 constexpr int kWinBytes = 256;                              // bytes of every weight row per window
 constexpr int kWinSteps = kWinBytes / kStepK;               // MFMA steps per window
@@ -368,8 +377,8 @@ __device__ __forceinline__ int stream_pass(const StreamParams& p, int blk, int e
   return nvalid;
 }
 
-// grid.x * grid.y: one workgroup of kWaves wavefronts per kWaves tile pairs and per block of the
-// row list's capacity (grid.z: see below).  NS = sub-tiles per pass.
+// grid.x * grid.y: one workgroup of kWaves wavefronts per kWaves / KS tile pairs and per block of the
+// row list's capacity (grid.z: see below).  NS = sub-tiles per pass, KS = wavefronts that share a tile pair's reduction.
 template <int MODE, bool kFused, int NS, int KS>
 __global__ __launch_bounds__(kThreads, NS == 1 ? 3 : 2) void gemm_stream_kernel(StreamParams p) {
   __shared__ __align__(16) char lds[kWaves * kWaveLds];
@@ -470,7 +479,7 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   if (blocks > 65535 || blocks * ((waves + kWaves - 1) / kWaves) >= (1ll << 31)) return hipErrorInvalidValue;
   const bool two = !kFused && a.num_pairs > (int64_t)kPairRowsPerExpert * a.num_experts;
   const bool split = MODE != kAccI32 && !kFused && !two && a.k > kWinBytes &&
-                     (MODE == kDown || (int64_t)a.n * a.k >= kSplitBytes);
+                     (MODE == kDown || (a.k >= kSplitReduction && (int64_t)a.n * a.k >= kSplitBytes));
   // Passes per block that can be needed: no expert holds more rows than there are tokens (or pairs,
   // when the caller did not say).  One workgroup per pass once there can be more than one.
   const int ns = two ? 2 : 1;
