@@ -21,12 +21,10 @@
 // bytes (the quantiser writes them), which lets a reduction of any multiple of 64 run on the same path.
 #include <iterator>
 
-#include "lds_loads.hpp"
+#include "dense_body.hpp"
 
 namespace moe_i8 {
 namespace {
-
-constexpr int kXcds = 8;
 
 struct DenseParams {
   const int8_t* a_q;     // [M, lda], zero between K and lda
@@ -54,27 +52,17 @@ constexpr int64_t kThroughBytes = 96 << 20;
 // THROUGH: results are written through to memory.  (A template argument: decided at run time it cost the smallest launches 0.2 of 7 us.)
 template <int MODE, bool THROUGH, int TM, int TN, int KS, int WM, int WN, int S, int WPE>
 __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(DenseParams p) {
-  constexpr int G = WM * WN;                   // wavefronts of a group: they share the group's stages
-  constexpr int kThreads = 64 * KS * G;
-  constexpr int L = (TM + TN) / 8 / G;         // 1 KB loads per wavefront and step
-  static_assert((TM + TN) % (8 * G) == 0, "a group's loads divide evenly");
-  static_assert((S - 2) * L <= 63 && S >= 2, "counted waits");
-  constexpr int kGroupBytes = (TM + TN) * kStepBytes;
-  constexpr int kStage = KS * kGroupBytes;
-  constexpr int MT = TM / WM, NT = TN / WN;
-  constexpr int kPartRow = TN * 4 + 16;        // bytes of a token's row of partial sums
-  constexpr int kPart = TM * kPartRow;
+  using T = DenseTiling<TM, TN, KS, WM, WN, S, TM + TN>;
+  using F = typename T::F;
+  constexpr int G = T::G, L = T::L, kThreads = T::kThreads, MT = T::MT, NT = T::NT, MF = T::MF, MI = T::MI, NI = T::NI;
   // Sums that are not partial, of tiles whose int32 sums would not fit or that are pairs of half as many results: finished in registers,
   // they meet in LDS as bf16 (gate_up of 128 x 128: 1-1.4 % of an MLP; plain results of it, 1-3 % slower, stay below).
   // For gate_up 16 weight rows of 32 are then gate rows and 16 the matching up rows: a lane has both in its registers.
   constexpr bool kFinished = KS == 1 && (TM * TN > 128 * 128 || MODE == kGateUpSilu);
   constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;  // output channels of the tile
   constexpr int kOutRow = kOut * 2 + 16;
-  constexpr int MF = MT % 32 == 0 && NT % 32 == 0 ? 32 : 16;
-  constexpr int MI = MT / MF, NI = NT / MF;
-  using F = Mfma<MF>;
-  constexpr int kResults = kFinished ? TM * kOutRow : KS * kPart;
-  constexpr int kLds = S * kStage > kResults ? S * kStage : kResults;
+  constexpr int kResults = kFinished ? TM * kOutRow : KS * T::kPart;
+  constexpr int kLds = S * T::kStage > kResults ? S * T::kStage : kResults;
   static_assert(kLds + 4 * (TM + TN) <= 160 * 1024, "LDS");
   __shared__ __align__(16) char lds[kLds];
   __shared__ __align__(16) float scales[(TM + TN + 63) / 64 * 64];
@@ -84,32 +72,15 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
   const int g = wave / G, wg = wave % G;
   const int wm = wg / WN, wn = wg % WN;
 
-  // tile of this workgroup: the workgroups of one XCD (id % 8) take neighbouring tiles, token tiles fastest
-  const int total = p.mtiles * p.ntiles;
-  const int per_xcd = (total + kXcds - 1) / kXcds;
-  const int tile = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
-  if (tile >= total || (int)(blockIdx.x / kXcds) >= per_xcd) return;
+  int tile;
+  if (!dense_tile(p.mtiles * p.ntiles, tile)) return;
   constexpr int kBand = 8;  // token tiles that run together over all channel tiles
   const int band = tile / (kBand * p.ntiles);
   const int in_band = tile - band * kBand * p.ntiles;
   const int band_m = p.mtiles - band * kBand < kBand ? p.mtiles - band * kBand : kBand;
   const int m0 = (band * kBand + in_band % band_m) * TM;
   const int nt = in_band / band_m;
-  const int inter = p.N / 2;
-
-  auto weight_row = [&](int r) {  // LDS weight row r of the tile -> row of w
-    if constexpr (MODE == kGateUpSilu && kFinished) {
-      const int ch = nt * kOut + r / 32 * 16 + r % 16;
-      return (ch < inter ? ch : inter - 1) + (r % 32 < 16 ? 0 : inter);
-    } else if constexpr (MODE == kGateUpSilu) {
-      const int half = TN / 2;
-      const int ch = nt * half + (r < half ? r : r - half);
-      return (ch < inter ? ch : inter - 1) + (r < half ? 0 : inter);
-    } else {
-      const int n = nt * TN + r;
-      return n < p.N ? n : p.N - 1;
-    }
-  };
+  auto weight_row = [&](int r) { return dense_weight_row<MODE, TN, kFinished>(nt, r, p.N); };
 
   const uint32_t lds0 = lds_address(lds);
   // scales of the tile's channels and rows, the first things in flight
@@ -143,7 +114,7 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
   auto issue = [&](int s, int slot, int from, int to) {
     const int piece = s * KS + g;
     const int koff = piece * kStepBytes;
-    const uint32_t base = lds0 + slot * kStage + g * kGroupBytes;
+    const uint32_t base = lds0 + slot * T::kStage + g * T::kGroupBytes;
     // Last 64 bytes of a ragged reduction: the activation rows are zero there, so the weights may be anything
     // readable: the lower half again (the next row would lie past the end of the matrix for the last one).
     const uint32_t back = ragged && piece == nk - 1 ? 64u : 0u;
@@ -165,7 +136,7 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
 #pragma unroll
   for (int kk = 0; kk < F::kSub; ++kk) chunk[kk] = ((kk * (64 / MF) + lane / MF) ^ swizzle_of_row(lrow)) * 16;
 
-  typename F::Acc acc[NI][MI];
+  typename T::Acc acc;
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -189,7 +160,7 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
     const int fill = slot == 0 ? S - 1 : slot - 1;  // the slot of step s - 1: everybody is done reading it
     const bool more = s + S - 1 < mine;
     if (s < mine) {
-      const char* st = lds + slot * kStage + g * kGroupBytes;
+      const char* st = lds + slot * T::kStage + g * T::kGroupBytes;
       v4i a[2][NI], b[2][MI];
       auto read = [&](int kk) {
 #pragma unroll
@@ -215,9 +186,9 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
   wait_vmcnt<0>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-  constexpr int kPieces = kOut / 8;                        // 16-byte pieces of an output row
-  const int width = MODE == kGateUpSilu ? inter : p.N;
   if constexpr (kFinished) {
+    constexpr int kPieces = kOut / 8;  // 16-byte pieces of an output row
+    const int width = MODE == kGateUpSilu ? p.N / 2 : p.N;
     static_assert(MODE != kGateUpSilu || NT % 32 == 0, "gate and up rows in turns of 16");
     constexpr int kSets = MODE == kGateUpSilu ? NI * F::kRegs / 8 : NI * F::kRegs / 4;  // of 4 channels of a lane and token
 #pragma unroll
@@ -252,51 +223,8 @@ __global__ __launch_bounds__(64 * KS * WM * WN, WPE) void gemm_dense_kernel(Dens
       const int m = m0 + tok, n = nt * kOut + c;
       if (m < p.M && n < width) store16(p.out + (int64_t)m * width + n, *reinterpret_cast<const v4i*>(lds + tok * kOutRow + c * 2), THROUGH);
     }
-    return;
-  }
-
-  // ---- partial sums of the KS groups meet in LDS, [group][token][channel] ----
-  char* part = lds + g * kPart;
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < MI; ++j)
-#pragma unroll
-      for (int q = 0; q < F::kRegs / 4; ++q) {
-        const int tok = wm * MT + j * MF + lrow;
-        const int ch = wn * NT + i * MF + (MF == 32 ? 8 * q : 0) + 4 * (lane / MF);
-        *reinterpret_cast<v4i*>(part + tok * kPartRow + ch * 4) =
-            v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-      }
-  __syncthreads();
-
-  auto total4 = [&](int tok, int ch, int (&v)[4]) {
-    v4i s = *reinterpret_cast<const v4i*>(lds + tok * kPartRow + ch * 4);
-#pragma unroll
-    for (int k = 1; k < KS; ++k) s += *reinterpret_cast<const v4i*>(lds + k * kPart + tok * kPartRow + ch * 4);
-    v[0] = s[0], v[1] = s[1], v[2] = s[2], v[3] = s[3];
-  };
-  for (int u = threadIdx.x; u < TM * kPieces; u += kThreads) {
-    const int tok = u / kPieces, c = u % kPieces * 8;
-    const int m = m0 + tok, n = nt * kOut + c;
-    if (m >= p.M || n >= width) continue;
-    const float as = scales[TN + tok];
-    uint2 o[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int ch = c + 4 * h;
-      int v[4];
-      total4(tok, ch, v);
-      const float4 ws = *reinterpret_cast<const float4*>(scales + ch);
-      if constexpr (MODE == kGateUpSilu) {
-        int up[4];
-        total4(tok, ch + kOut, up);
-        o[h] = silu_mul_epilogue4(v, up, as, ws, *reinterpret_cast<const float4*>(scales + ch + kOut));
-      } else {
-        o[h] = down_epilogue4(v, as, ws, 1.0f);
-      }
-    }
-    store16(p.out + (int64_t)m * width + n, v4i{(int)o[0].x, (int)o[0].y, (int)o[1].x, (int)o[1].y}, THROUGH);
+  } else {
+    dense_results<T, MODE, THROUGH, TM, TN, KS>(acc, lds, g, wm * MT, wn * NT, scales, scales + TN, m0, nt, p.M, p.N, p.out);
   }
 }
 

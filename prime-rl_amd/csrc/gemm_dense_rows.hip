@@ -12,13 +12,12 @@
 // 17..1000 rows x 512..14336 channels x 192..4200, taken where the estimates say so, 22 % faster on average.
 #include <iterator>
 
-#include "lds_loads.hpp"
+#include "dense_body.hpp"
 #include "quant_body.hpp"
 
 namespace moe_i8 {
 namespace {
 
-constexpr int kXcds = 8;
 constexpr int kWaves = 8;
 
 struct DenseRowsParams {
@@ -37,24 +36,15 @@ struct DenseRowsParams {
 // bf16 row (K <= 512 * V).
 template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int V>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRowsParams p) {
-  constexpr int G = WM * WN;
-  static_assert(KS * G == kWaves && TM % kWaves == 0 && S >= 2);
-  constexpr int kThreads = 64 * kWaves;
-  constexpr int L = TN / 8 / G;                // 1 KB loads per wavefront and step
-  static_assert(TN % (8 * G) == 0 && (S - 2) * L <= 63);
+  using T = DenseTiling<TM, TN, KS, WM, WN, S, TN>;
+  constexpr int G = T::G, L = T::L, kThreads = T::kThreads, MT = T::MT, NT = T::NT, MF = T::MF, MI = T::MI, NI = T::NI;
+  using F = typename T::F;
+  static_assert(KS * G == kWaves && TM % kWaves == 0);
   constexpr int R = TM / kWaves;               // rows that a wavefront quantises
-  constexpr int kGroupBytes = TN * kStepBytes;
-  constexpr int kStage = KS * kGroupBytes;
   constexpr int kPiece = TM * kStepBytes;      // 128 reduction bytes of all rows
-  constexpr int kRowsAt = S * kStage;          // quantised rows, behind the stages: [piece][row][128]
-  constexpr int MT = TM / WM, NT = TN / WN;
-  constexpr int MF = MT % 32 == 0 && NT % 32 == 0 ? 32 : 16;
-  constexpr int MI = MT / MF, NI = NT / MF;
-  using F = Mfma<MF>;
-  constexpr int kPartRow = TN * 4 + 16;        // bytes of a token's row of partial sums
-  constexpr int kPart = TM * kPartRow;
+  constexpr int kRowsAt = S * T::kStage;          // quantised rows, behind the stages: [piece][row][128]
   constexpr int kUsed = kRowsAt + V * 4 * kPiece;
-  constexpr int kLds = kUsed > KS * kPart ? kUsed : KS * kPart;
+  constexpr int kLds = kUsed > KS * T::kPart ? kUsed : KS * T::kPart;
   static_assert(kLds + 4 * (TM + TN) <= 160 * 1024, "LDS");
   __shared__ __align__(16) char lds[kLds];
   __shared__ __align__(16) float scales[(TN + 63) / 64 * 64 + TM];
@@ -65,14 +55,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRo
   const int g = wave / G, wg = wave % G;
   const int wm = wg / WN, wn = wg % WN;
 
-  // tile of this workgroup: the workgroups of one XCD (id % 8) take neighbouring tiles, token tiles fastest
-  const int total = p.mtiles * p.ntiles;
-  const int per_xcd = (total + kXcds - 1) / kXcds;
-  const int tile = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
-  if (tile >= total || (int)(blockIdx.x / kXcds) >= per_xcd) return;
+  int tile;  // token tiles fastest
+  if (!dense_tile(p.mtiles * p.ntiles, tile)) return;
   const int m0 = tile % p.mtiles * TM;
   const int nt = tile / p.mtiles;
-  const int inter = p.N / 2;
   const int K = p.K;
 
   // ---- the tile's rows, the first things in flight (rows behind the last one: that one again) ----
@@ -87,16 +73,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRo
       if (i < vectors) v[r][i] = i * kWave + lane < K / kQuantVec ? x[i * kWave + lane] : make_uint4(0u, 0u, 0u, 0u);
   }
 
-  auto weight_row = [&](int r) {  // LDS weight row r of the tile -> row of w
-    if constexpr (MODE == kGateUpSilu) {
-      const int half = TN / 2;
-      const int ch = nt * half + (r < half ? r : r - half);
-      return (ch < inter ? ch : inter - 1) + (r < half ? 0 : inter);
-    } else {
-      const int n = nt * TN + r;
-      return n < p.N ? n : p.N - 1;
-    }
-  };
+  auto weight_row = [&](int r) { return dense_weight_row<MODE, TN>(nt, r, p.N); };
   const uint32_t lds0 = lds_address(lds);
   uint32_t off[L];
   bool hi[L];  // chunk in the upper 64 bytes of the step
@@ -113,7 +90,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRo
   const bool ragged = K % kStepBytes != 0;
   auto issue = [&](int s, int slot, int from, int to) {
     const int piece = s * KS + g;
-    const uint32_t base = lds0 + slot * kStage + g * kGroupBytes + wg * L * 1024;
+    const uint32_t base = lds0 + slot * T::kStage + g * T::kGroupBytes + wg * L * 1024;
     // Last 64 bytes of a ragged reduction: the rows are zero there, so the weights may be anything readable: the lower half
     // again (the next row would lie past the end of the matrix for the last one).
     const uint32_t back = ragged && piece == nk - 1 ? 64u : 0u;
@@ -159,7 +136,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRo
 #pragma unroll
   for (int kk = 0; kk < F::kSub; ++kk) chunk[kk] = ((kk * (64 / MF) + lane / MF) ^ swizzle_of_row(lrow)) * 16;
 
-  typename F::Acc acc[NI][MI];
+  typename T::Acc acc;
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -180,7 +157,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRo
     const int fill = slot == 0 ? S - 1 : slot - 1;  // the slot of step s - 1: everybody is done reading it
     const bool more = s + S - 1 < mine;
     if (s < mine) {
-      const char* st = lds + slot * kStage + g * kGroupBytes;
+      const char* st = lds + slot * T::kStage + g * T::kGroupBytes;
       const char* rows = lds + (s * KS + g) * kPiece;
       v4i a[2][NI], b[2][MI];
       auto read = [&](int kk) {
@@ -206,53 +183,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_dense_rows_kernel(DenseRo
   }
   wait_vmcnt<0>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-
-  // ---- partial sums of the KS groups meet in LDS, [group][token][channel] ----
-  char* part = lds + g * kPart;
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < MI; ++j)
-#pragma unroll
-      for (int q = 0; q < F::kRegs / 4; ++q) {
-        const int tok = wm * MT + j * MF + lrow;
-        const int ch = wn * NT + i * MF + (MF == 32 ? 8 * q : 0) + 4 * (lane / MF);
-        *reinterpret_cast<v4i*>(part + tok * kPartRow + ch * 4) =
-            v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-      }
-  __syncthreads();
-
-  constexpr int kOut = MODE == kGateUpSilu ? TN / 2 : TN;  // output channels of the tile
-  constexpr int kPieces = kOut / 8;                        // 16-byte pieces of an output row
-  const int width = MODE == kGateUpSilu ? inter : p.N;
-  auto total4 = [&](int tok, int ch, int (&v)[4]) {
-    v4i s = *reinterpret_cast<const v4i*>(lds + tok * kPartRow + ch * 4);
-#pragma unroll
-    for (int k = 1; k < KS; ++k) s += *reinterpret_cast<const v4i*>(lds + k * kPart + tok * kPartRow + ch * 4);
-    v[0] = s[0], v[1] = s[1], v[2] = s[2], v[3] = s[3];
-  };
-  for (int u = threadIdx.x; u < TM * kPieces; u += kThreads) {
-    const int tok = u / kPieces, c = u % kPieces * 8;
-    const int m = m0 + tok, n = nt * kOut + c;
-    if (m >= p.M || n >= width) continue;
-    const float as = scales[kRowScales + tok];
-    uint2 o[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int ch = c + 4 * h;
-      int v[4];
-      total4(tok, ch, v);
-      const float4 ws = *reinterpret_cast<const float4*>(scales + ch);
-      if constexpr (MODE == kGateUpSilu) {
-        int up[4];
-        total4(tok, ch + kOut, up);
-        o[h] = silu_mul_epilogue4(v, up, as, ws, *reinterpret_cast<const float4*>(scales + ch + kOut));
-      } else {
-        o[h] = down_epilogue4(v, as, ws, 1.0f);
-      }
-    }
-    store16(p.out + (int64_t)m * width + n, v4i{(int)o[0].x, (int)o[0].y, (int)o[1].x, (int)o[1].y}, true);
-  }
+  dense_results<T, MODE, true, TM, TN, KS>(acc, lds, g, wm * MT, wn * NT, scales, scales + kRowScales, m0, nt, p.M, p.N, p.out);
 }
 
 template <int MODE, int TM, int TN, int KS, int WM, int WN, int S, int V>
