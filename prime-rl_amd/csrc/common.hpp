@@ -370,6 +370,7 @@ struct DenseFewArgs {
 };
 constexpr int kDenseFewRows = 16;
 bool dense_few_takes(int64_t m, int n, int k);
+float dense_few_estimate(int64_t m, int n, int k);  // us, against the tiles of the kernel below
 hipError_t launch_dense_few(const DenseFewArgs& a, hipStream_t stream);
 // The dense kernel that quantises its own rows (ties to even): the entry of its table for this problem, -1 if it is not the one.
 // `few`: the kernel of a few rows would run it otherwise; if not, `us`: what the quantised product is expected to take.

@@ -136,14 +136,19 @@ hipError_t launch_rows(const DenseFewArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// As many weight rows per wavefront, up to 16 KB, as leave work for every compute unit.
+int rows_per_wave(int n, int pieces) {
+  const int most = n / (kWaves * 200);
+  return pieces <= 2 && most >= 8 ? 8 : pieces <= 4 && most >= 4 ? 4 : 2;
+}
+
 template <int MODE, int C>
 hipError_t launch_pieces(const DenseFewArgs& a, hipStream_t stream) {
-  // as many weight rows per wavefront, up to 16 KB, as leave work for every compute unit
-  const int most = a.n / (kWaves * 200);
+  const int rows = rows_per_wave(a.n, C);
   if constexpr (C <= 2)
-    if (most >= 8) return launch_rows<MODE, C, 8>(a, stream);
+    if (rows == 8) return launch_rows<MODE, C, 8>(a, stream);
   if constexpr (C <= 4)
-    if (most >= 4) return launch_rows<MODE, C, 4>(a, stream);
+    if (rows == 4) return launch_rows<MODE, C, 4>(a, stream);
   return launch_rows<MODE, C, 2>(a, stream);
 }
 
@@ -171,6 +176,15 @@ bool dense_few_takes(int64_t m, int n, int k) {
   const int64_t weights = (int64_t)n * k;
   const int64_t most = weights <= 1 << 20 ? kDenseFewRows : weights <= 12 << 20 ? 8 : weights <= 40 << 20 ? 6 : 4;
   return m <= most && n % 16 == 0 && k % 16 == 0 && k <= 8 * 1024;
+}
+
+// Least-squares fit to 1200 problems of 5 to 16 rows, the mean of the times with weights from memory and from the last-level cache (rms error
+// 3 % with a seventh term, 0.08 us per MB of weights, which the kernel that it is weighed against takes as well: both leave it out).
+float dense_few_estimate(int64_t m, int n, int k) {
+  const int pieces = (k + 1023) / 1024, rows = rows_per_wave(n, pieces), per_round = kWaves * rows * device_cu_count();
+  const float rounds = (float)((n + per_round - 1) / per_round), held = rounds * (float)(rows * pieces);
+  return 1.91f + 0.236f * (float)pieces + 0.271f * (float)((m + kWaves - 1) / kWaves - 1) + 0.022f * held +
+         (float)m * (0.131f * rounds + 0.0292f * held);
 }
 
 hipError_t launch_dense_few(const DenseFewArgs& a, hipStream_t stream) {

@@ -1,4 +1,5 @@
-// Dense int8 GEMM that quantises its own rows, for gfx950: linear layers and gated MLPs of about ten to some hundreds of rows.
+// Dense int8 GEMM that quantises its own rows, for gfx950: linear layers and gated MLPs of 5 rows and more, mostly tens to
+// hundreds (thousands where the channels are few: 6000 rows x 128 channels x 768).
 //
 // At this size a dense layer is two dependent launches, quantisation and product, and little else: 100 rows x 1000 channels x 1024
 // took 7.7 us for 0.1 us of bytes and 0.3 of operations.  Here a workgroup quantises the token rows of its tile itself, into
@@ -202,9 +203,10 @@ hipError_t launch_config(const DenseRowsParams& p0, hipStream_t stream) {
 // One way to cut the problem up and what it costs: a launch takes about
 //   start + rounds * (per_round + per_k * K / 1024) + waves * (per_wave + per_wave_k * K / 1024)
 // where a round is as many workgroups as the device holds at a time and a wave as many as it has compute units (the same, where a
-// unit holds one: then the second term is 0).  Least-squares fits to 540 problems of 2..1000 rows x 512..24576 channels x 192..4200
-// (rms error of a fit 4-7 %).  The choice between these and the launches they replace takes on average 0.6 % longer than the fastest
-// way, 1.9 % with up to 16 rows.
+// unit holds one: then the second term is 0).  Least-squares fits to 2600 problems of 5..8192 rows x 64..20000 channels x 64..4096, the mean of the
+// times with weights from memory and from the last-level cache (rms error of a fit 4-9 %).  Over 1300 problems of 5 rows and more the choice
+// between these and the launches that they replace takes on average 0.2 % longer than the fastest way with weights from memory and 0.1 % with cached
+// ones, 0.2 % in a captured graph (3000 problems).
 // The 256 and 512 channel tiles are one round where the 128 channel ones are two, and a workgroup's rows serve twice as many channels; no
 // split of the reduction is left, and none is missed: 16 x 256 is faster than 32 x 128, which was here, also where both are one round
 // (170 rows x 4112 channels x 256 4.7 / 4.2 us).  Without / with the three of them, 60 drawn linear layers that they are picked for:
@@ -223,33 +225,29 @@ struct Config {
   {TM, TN, 512 * V, PER_CU, START, ROUND, PER_K, WAVE, WAVE_K, launch_config<kGateUpSilu, TM, TN, KS, WM, WN, S, V>, \
    launch_config<kDown, TM, TN, KS, WM, WN, S, V>}
 const Config kConfigs[] = {
-    MOE_I8_ROWS(16, 32, 4, 1, 2, 3, 2, 2, 1.97f, 1.87f, -1.06f, -0.06f, 1.37f),
-    MOE_I8_ROWS(16, 64, 2, 1, 4, 3, 2, 2, 1.89f, 1.94f, -0.87f, -0.11f, 1.62f),
-    MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 2, 1, 1.23f, 2.27f, 1.54f, 0.0f, 0.0f),
-    MOE_I8_ROWS(16, 256, 1, 1, 8, 3, 2, 1, 0.98f, 2.44f, 2.91f, 0.0f, 0.0f),
-    MOE_I8_ROWS(32, 256, 1, 1, 8, 3, 2, 1, 0.75f, 3.59f, 3.33f, 0.0f, 0.0f),
-    MOE_I8_ROWS(32, 512, 1, 1, 8, 2, 1, 1, 0.53f, 4.37f, 4.63f, 0.0f, 0.0f),
-    MOE_I8_ROWS(16, 32, 8, 1, 1, 3, 4, 1, 1.12f, 2.41f, 0.83f, 0.0f, 0.0f),
-    MOE_I8_ROWS(16, 64, 4, 1, 2, 3, 4, 1, 1.02f, 2.57f, 1.18f, 0.0f, 0.0f),
-    MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 4, 1, 0.78f, 2.70f, 1.83f, 0.0f, 0.0f),
-    MOE_I8_ROWS(16, 32, 8, 1, 1, 2, 8, 1, 0.17f, 2.82f, 1.12f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 32, 4, 1, 2, 3, 2, 2, 1.63f, 0.80f, 0.23f, 0.73f, 0.63f),
+    MOE_I8_ROWS(16, 64, 2, 1, 4, 3, 2, 2, 1.48f, 0.98f, 0.51f, 0.66f, 0.85f),
+    MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 2, 1, 0.76f, 2.41f, 1.93f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 256, 1, 1, 8, 3, 2, 1, 0.57f, 2.65f, 3.26f, 0.0f, 0.0f),
+    MOE_I8_ROWS(32, 256, 1, 1, 8, 3, 2, 1, 0.15f, 4.07f, 3.42f, 0.0f, 0.0f),
+    MOE_I8_ROWS(32, 512, 1, 1, 8, 2, 1, 1, -0.52f, 4.94f, 5.82f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 32, 8, 1, 1, 3, 4, 1, 0.55f, 2.86f, 0.88f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 64, 4, 1, 2, 3, 4, 1, 0.23f, 3.31f, 1.20f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 128, 2, 1, 4, 3, 4, 1, -0.29f, 3.81f, 1.81f, 0.0f, 0.0f),
+    MOE_I8_ROWS(16, 32, 8, 1, 1, 2, 8, 1, -0.51f, 3.93f, 1.05f, 0.0f, 0.0f),
 };
 
 }  // namespace
 
 // A row more costs the kernel of a few rows a pass over its registers' weights, this one nothing up to 16.  Up to 4 rows that kernel is the
-// faster one or even on all but the widest matrices (4 x 8848 x 1536 6.3 / 5.1).  From 5 on it takes, on the device, about 2.1 + 0.1 W +
-// 0.0235 m W + 0.22 m us with W = n * k / 10^6 (rms error 12 %); the constants above, fitted to calls from a host that sends one every 3.7 us,
-// are 0.4 us high for the shorter reductions.  Over 405 problems of 5 to 16 rows, launches of a captured graph, the choice takes 0.6 % longer than the
-// faster of the two, 4 % by estimates fitted to such calls with 7 % in favour of the other kernel (which it had not in a graph); from the host
-// 0.7 and 2.1 % (578 problems).  us there / here: 6 x 6272 x 192 5.2 / 3.6, 7 x 4496 x 256 4.8 / 3.3, 16 x 640 x 1280 6.7 / 4.3, 5 x 1792 x 832 3.5 / 4.2,
-// 5 x 3760 x 2368 4.6 / 5.7; wrong by most 5 x 3200 x 704 3.6 / 4.2 and 6 x 16000 x 2304 10.9 / 13.5.  A quantisation launch adds about
-// 3.06 us + 0.69 per 5 MB that it moves to the dense kernels' estimate.
+// faster one or even on all but the widest matrices (4 x 8848 x 1536 6.3 / 5.1).  From 5 on both are estimated.  Over 1200 problems of 5 to 16 rows the choice
+// takes 0.1 % longer than the faster of the two, 0.2 % in a captured graph (3500 problems); by fits to calls that a host sends one every 3.7 us, which hide
+// how long a kernel of 3 us takes, 5 and 7 %.  us there / here in a graph: 6 x 6272 x 192 5.2 / 3.6, 7 x 4496 x 256 4.8 / 3.3, 16 x 640 x 1280 6.7 / 4.3, 5 x
+// 1792 x 832 3.5 / 4.2, 5 x 3760 x 2368 4.6 / 5.7, 6 x 4080 x 3072 6.3 / 8.2, 5 x 3680 x 576 3.8 / 4.4; wrong by most 6 x 4464 x 4032 9.4 / 10.3 and 8 x 1216 x
+// 1088 4.6 / 4.9.  A quantisation launch adds about 3.0 us and 0.66 per 10^6 elements to the dense kernels' estimate.
 int dense_rows_pick(int64_t m, int n, int k, bool few, float us) {
   if (m < kDenseRowsFrom || (int64_t)n * k >= (1ll << 32) || n % 16 != 0 || k % 64 != 0) return -1;
-  const float w = (float)n * (float)k * 1e-6f;
-  float least = few ? 2.1f + 0.1f * w + 0.0235f * (float)m * w + 0.22f * (float)m + (k <= 1024 ? 0.4f : 0.0f)
-                    : us + 3.06f + 0.69f * (float)m * (float)k * (3.0f / 5e6f);
+  float least = few ? dense_few_estimate(m, n, k) : us + 3.0f + 0.66e-6f * (float)m * (float)k;
   int best = -1;
   const float kb = (float)k / 1024.0f, cus = (float)device_cu_count();
   for (int i = 0; i < (int)std::size(kConfigs); ++i) {

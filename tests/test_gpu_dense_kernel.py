@@ -55,7 +55,7 @@ def test_few_rows_in_one_launch(pra, oracle, M, N, K):
     (16, 16, 64), (17, 560, 576), (33, 1040, 1024), (64, 864, 384), (5, 10880, 384), (100, 2064, 960), (500, 272, 1024),
     (13, 11568, 256), (31, 8208, 512), (43, 11616, 640), (65, 8464, 192), (245, 2752, 1024), (600, 1552, 448), (54, 1248, 1152),
     (16, 4112, 2048), (28, 8208, 1088), (30, 8176, 2048), (47, 5008, 1984), (9, 16912, 1344), (45, 624, 2880), (17, 1040, 4096),
-    (15, 528, 2112), (16, 2544, 3968),
+    (15, 528, 2112), (16, 2544, 3968), (16, 64, 4096), (69, 1280, 3904), (31, 8496, 576),
 ])
 def test_rows_quantised_by_their_tiles(pra, oracle, M, N, K):
     """Rows quantised by the workgroups whose tiles they are in: every tile and length of its registers, rows and channels
