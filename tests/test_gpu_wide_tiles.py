@@ -11,7 +11,7 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("B", [64, 128])
-@pytest.mark.parametrize("H,I", [(256, 384), (384, 256), (1408, 640), (4096, 256)])  # (even tiles from a reduction of 4096 on)
+@pytest.mark.parametrize("H,I", [(256, 384), (384, 256), (1408, 640), (4096, 256), (1920, 256), (2048, 256)])  # (even tiles from a reduction of 2048 on)
 def test_rows_around_the_edges_of_row_tiles(pra, H, I, B):
     counts = [1, 31, 32, 33, 63, 65, 127, 128, 129, 160, 161, 0, 224, 255, 256, 257, 300, 511, 513]
     M = sum(counts)
