@@ -304,7 +304,7 @@ int moe_i8_w8a8_mlp(const void* x, const int8_t* w13, const float* w13_scale, co
  * demands a family that does not handle the shape.
  */
 #define MOE_I8_DENSE_FEW 16   /* a few rows, quantised by every workgroup */
-#define MOE_I8_DENSE_ROWS 17  /* some tens to hundreds of rows, quantised by the workgroups whose tiles they are in */
+#define MOE_I8_DENSE_ROWS 17  /* mostly tens to hundreds of rows, quantised by the workgroups whose tiles they are in */
 #define MOE_I8_DENSE_TILES 18 /* rows quantised by a launch of their own */
 typedef struct moe_i8_dense_kernel {
   int kernel;                    /* MOE_I8_DENSE_*, or MOE_I8_GEMM_* where a grouped family runs it */

@@ -989,7 +989,7 @@ bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
 enum DenseWay {
   kGrouped,  // quantised by a launch of its own, then the 256-row tiles or a demanded family, which read that launch's routing
   kDense,    // quantised by a launch of its own, then the dense kernel, which needs no routing
-  kRows,     // the product's own launch quantises some tens to hundreds of rows
+  kRows,     // the product's own launch quantises the rows, mostly tens to hundreds of them
   kFew,      // ... a few rows
 };
 struct DenseChoice {

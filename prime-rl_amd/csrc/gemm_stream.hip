@@ -41,7 +41,7 @@ constexpr int kStepK = 64;    // reduction bytes per MFMA
 // skewed routing at 5 / 7 / 8 / 10 / 14 tokens 75.5 / 76.1, 71.1 / 71.6, 94.1 / 83.7, 94.5 / 83.7, 94.4 / 87.1, 128 of them
 // evenly routed at 5 / 8 / 12 105 / 103, 162 / 159, 197 / 193; 256 of 7168 x 2048 at 6 / 8 314 / 312, 388 / 377; 16 of 4096 x 4096 at 6 / 10
 // 96.7 / 86.3, 117 / 104.  Quarters, or workgroups of two wavefronts: less, and losses of up to 4 % where halves have none.  (The halved
-// instances keep 18 and 20 registers in scratch, the whole ones 6 and 8, of 168.)
+// instances keep 18 and 20 registers in scratch, the whole ones 6 and 8, the self-quantising one 17, of 168.)
 // gate_up: halved from 4 MB an expert and reductions of 1536 on.  By how many per cent a layer takes longer with it halved, evenly routed | Zipf
 // routing, mean over 5 to 16 tokens, by MB and reduction: 2.0 (512 channels x 2048) -1 | -4, 3.0 (768 x 2048) 0 | -6, 3.8 (1280 x 1536) 0 | -3,
 // 4.0 (512 x 4096) -3 | -5, 4.0 (1024 x 2048) -1 | -1, 5.0 (1024 x 2560) -2 | -7, 5.5 (1408 x 2048) -1 | -2, 6.0 (2048 x 1536) 0 | -1, 8.0 (1024 x
