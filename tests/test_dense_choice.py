@@ -94,3 +94,12 @@ def test_gate_up_is_charged_for_the_results_it_stores(pra, m, hidden, inter, ker
 ])
 def test_line_between_the_kernels_that_quantise_their_rows(pra, m, n, k, kernel):
     assert pra.linear_plan(m, n, k)["kernel"] == kernel
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    # us in the dense tile that the estimates come to next / with wide tiles: 43.9 / 35.2, 77.8 / 63.0, 82.4 / 69.5, 67.4 / 53.2
+    (14508, 3328, 256, "tile_wide"), (9405, 11520, 256, "tile_wide"), (8747, 8448, 640, "tile_wide"), (5836, 14784, 256, "tile_wide"),
+    (5780, 2672, 512, "dense"),  # 19.4 / 24.8
+])
+def test_linear_layers_of_short_reductions_are_charged_for_their_results(pra, m, n, k, kernel):
+    assert pra.linear_plan(m, n, k)["kernel"] == kernel

@@ -78,8 +78,9 @@ def test_rows_quantised_by_their_tiles(pra, oracle, M, N, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
-    (673, 5552, 576), (643, 5392, 192), (1421, 5584, 576), (1300, 5904, 64), (2051, 5616, 576), (1800, 6176, 192),  # 128 x 192,
-    (2315, 6176, 576), (4804, 2912, 64), (2309, 6192, 1088),                            # 256 x 192, 192 x 320, 192 x 384
+    (673, 5552, 576), (643, 5392, 192), (1421, 5584, 576), (1300, 5904, 64), (2051, 5616, 576), (1800, 6176, 192),
+    (2315, 6176, 576), (4804, 2912, 64), (2309, 6192, 1088),
+    (9935, 1168, 448), (779, 14608, 448), (1054, 14592, 64),                            # 192 x 320 and 192 x 384
     (11398, 4416, 576), (18529, 2720, 64), (21775, 2592, 576), (21327, 2368, 576),      # more than 96 MB of results
 ])
 def test_large_tiles(pra, oracle, M, N, K):
@@ -131,10 +132,10 @@ def test_tiles_of_few_and_of_short_problems(pra, oracle, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    (1371, 75024, 192),   # 128 x 128, two workgroups to a compute unit
-    (967, 106960, 448),   # 256 x 192
-    (37219, 2832, 192),   # 192 x 320
-    (25597, 3984, 64),    # 192 x 384
+    (1371, 75024, 192), (967, 106960, 448), (37219, 2832, 192), (25597, 3984, 64),  # 128 x 128, two workgroups to a compute unit
+    (1926, 55008, 1216),  # 256 x 192
+    (85854, 1280, 448),   # 192 x 320
+    (960, 114992, 448),   # 192 x 384
 ])
 def test_results_of_more_than_96_mb(pra, oracle, M, N, K):
     """Results that are left in the L2s, gate_up's as well (M x N / 2), in every tile that is picked for so many."""
