@@ -141,12 +141,15 @@ def test_layer_quantises_long_rows_as_the_row_quantiser_does(pra, H, M):
 
 
 @pytest.mark.parametrize("E,k,H,I,M,B", [
-    (66, 8, 4160, 576, 9, 64),    # 17 windows and 3, the last of 64 bytes
-    (40, 4, 4096, 1088, 16, 16),  # starting windows; 5 windows
-    (33, 2, 7168, 320, 40, 64),   # up to 40 rows of an expert: several passes; 2 windows
+    (66, 8, 4160, 576, 9, 64),    # 17 windows, the last of 64 bytes; down whole
+    (40, 4, 4096, 1088, 16, 16),  # starting windows; down whole, the longest of its kind
+    (33, 2, 7168, 320, 40, 64),   # up to 40 rows of an expert: several passes; down whole
     (70, 4, 1088, 2064, 5, 32),   # a reduction too short to be halved: whole
     (70, 4, 1600, 2064, 5, 32),   # an odd number of tile pairs (gate_up alone takes it), 7 windows, the last of 64 bytes
     (40, 4, 1536, 1408, 9, 64),   # the shortest that gate_up halves: 6 windows
+    (40, 4, 4096, 1152, 16, 16),  # the shortest that down halves: 5 windows, the last of 128 bytes
+    (33, 2, 2048, 1216, 40, 64),  # down in several passes: 5 windows, the last of 192 bytes
+    (17, 2, 1024, 4096, 9, 32),   # starting windows in down
 ])
 def test_reductions_halved_between_wavefronts(pra, oracle, E, k, H, I, M, B):
     """The streaming kernel with a tile pair's reduction in two wavefronts: windows that do not halve evenly, a last
