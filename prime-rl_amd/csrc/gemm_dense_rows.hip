@@ -206,7 +206,8 @@ hipError_t launch_config(const DenseRowsParams& p0, hipStream_t stream) {
 // unit holds one: then the second term is 0).  Least-squares fits to 2600 problems of 5..8192 rows x 64..20000 channels x 64..4096, the mean of the
 // times with weights from memory and from the last-level cache (rms error of a fit 4-9 %).  Over 1300 problems of 5 rows and more the choice
 // between these and the launches that they replace takes on average 0.2 % longer than the fastest way with weights from memory and 0.1 % with cached
-// ones, 0.2 % in a captured graph (3000 problems).
+// ones, 0.2 % in a captured graph (3000 problems).  Wrong by most where a nearly full round of 32 x 256 has a long reduction: 2009 rows x 832 x 832 9.3 us, quantised
+// by a launch of its own 8.8.
 // The 256 and 512 channel tiles are one round where the 128 channel ones are two, and a workgroup's rows serve twice as many channels; no
 // split of the reduction is left, and none is missed: 16 x 256 is faster than 32 x 128, which was here, also where both are one round
 // (170 rows x 4112 channels x 256 4.7 / 4.2 us).  Without / with the three of them, 60 drawn linear layers that they are picked for:
