@@ -47,12 +47,13 @@ constexpr int kStepK = 64;    // reduction bytes per MFMA
 // 4.0 (512 x 4096) -3 | -5, 4.0 (1024 x 2048) -1 | -1, 5.0 (1024 x 2560) -2 | -7, 5.5 (1408 x 2048) -1 | -2, 6.0 (2048 x 1536) 0 | -1, 8.0 (1024 x
 // 4096) -2 | -5, 16 (1024 x 8192) -3 | -7; shorter reductions: 4.5 (3072 x 768) 5 | 3, 4.0 (2048 x 1024) 3 | 3, 5.5 (2816 x 1024, 64 experts) 3 | 2, 8.0
 // (4096 x 1024) 3 | 2, 5.0 (2048 x 1280) 2 | 2, 5.6 (2560 x 1152) 4 | 4, 8.0 (8192 x 512) 4 | 5.  Given away: the gains below 4 MB.
-// down (that reads quantised rows): from reductions of 1152 on.  By output channels x reduction, as above: 1536 x 1280 0 | -4, 2048 x 1152 0 | 1, 2048 x 1408 0 |
+// down (that reads quantised rows): from reductions of 1152 on, and where whole ones give less than two workgroups to a compute unit.  By output channels x reduction, as above: 1536 x 1280 0 | -4, 2048 x 1152 0 | 1, 2048 x 1408 0 |
 // -5, 2048 x 1536 0 | -4, 1024 x 2048 (32 experts) -4 | -7, (64) 2 | -6, 768 x 3072 -7 | -18, 2880 x 2880 -3 | -2, 4096 x 4096 -2 | -8, 4096 x 14336 -9 | -12.
 // Evenly routed experts of 2 to 3 MB lose up to 4 % at single numbers of tokens, where the halves are a few more than fit the device at a time; a line by
 // size would give away more than that under Zipf routing.  Shorter reductions, layer us whole / halved: 159 experts of 4480 x 448 at 116 tokens 188 / 204, 92
 // of 3712 x 576 at 214 123 / 129, 133 of 6912 x 576 at 153 168 / 177, 50 of 1920 x 576 at 35 44.6 / 47.2, 22 of 6656 x 384 at 16 42.3 / 43.6, 46 of 3200 x 832
-// at 62 83.0 / 84.9; at best 33 of 2816 x 576 at 16 41.4 / 40.6 and 24 of 1280 x 704 at 23 31.0 / 30.4.
+// at 62 83.0 / 84.9, at best 33 of 2816 x 576 at 16 41.4 / 40.6; up to 512 workgroups 52 of 896 x 1088 at 15 26.5 / 23.4, 30 of 768 x 448 at 24
+// 23.6 / 22.2, 33 of 1536 x 576 at 25 28.5 / 27.1, 16 of 640 x 576 at 40 24.7 / 23.7, 23 of 2432 x 320 at 41 25.9 / 25.6, others even (43 of 50 within 0.6 %).
 constexpr int kParts = 2;
 constexpr int64_t kSplitBytes = 4 << 20;
 constexpr int kSplitReduction = 1536;
@@ -481,8 +482,11 @@ hipError_t launch_mode(const GemmArgs& a, hipStream_t stream) {
   if (blocks == 0 || waves == 0) return hipSuccess;
   if (blocks > 65535 || blocks * ((waves + kWaves - 1) / kWaves) >= (1ll << 31)) return hipErrorInvalidValue;
   const bool two = !kFused && a.num_pairs > (int64_t)kPairRowsPerExpert * a.num_experts;
+  // workgroups of a pass with whole reductions, every expert routed to
+  const int64_t whole = (int64_t)((waves + kWaves - 1) / kWaves) * (a.num_pairs < a.num_experts ? a.num_pairs : a.num_experts);
+  const bool few = a.k > kWinBytes && whole <= 2 * device_cu_count();
   const bool split = MODE != kAccI32 && !kFused && !two &&
-                     (MODE == kDown ? a.k >= kSplitDownReduction : a.k >= kSplitReduction && (int64_t)a.n * a.k >= kSplitBytes);
+                     (MODE == kDown ? a.k >= kSplitDownReduction || few : a.k >= kSplitReduction && (int64_t)a.n * a.k >= kSplitBytes);
   // Passes per block that can be needed: no expert holds more rows than there are tokens (or pairs,
   // when the caller did not say).  One workgroup per pass once there can be more than one.
   const int ns = two ? 2 : 1;

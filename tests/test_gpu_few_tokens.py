@@ -144,6 +144,8 @@ def test_layer_quantises_long_rows_as_the_row_quantiser_does(pra, H, M):
     (66, 8, 4160, 576, 9, 64),    # 17 windows, the last of 64 bytes; down whole
     (40, 4, 4096, 1088, 16, 16),  # starting windows; down whole, the longest of its kind
     (33, 2, 7168, 320, 40, 64),   # up to 40 rows of an expert: several passes; down whole
+    (17, 4, 1600, 320, 40, 64),   # down of so few workgroups that its 2 windows are halved, several passes
+    (32, 4, 2048, 576, 9, 32),    # the most workgroups of that kind: 3 windows, the last of 64 bytes
     (70, 4, 1088, 2064, 5, 32),   # a reduction too short to be halved: whole
     (70, 4, 1600, 2064, 5, 32),   # an odd number of tile pairs (gate_up alone takes it), 7 windows, the last of 64 bytes
     (40, 4, 1536, 1408, 9, 64),   # the shortest that gate_up halves: 6 windows
