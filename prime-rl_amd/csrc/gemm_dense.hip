@@ -242,7 +242,7 @@ hipError_t launch_config(const DenseParams& p0, hipStream_t stream) {
 }
 
 // One way to cut the problem up and what it costs.  A launch takes about
-//   start + rounds * per_round + max((full rounds * per_k + the last one's share) * K / 1024, padded operations / rate) + per_mb * MB of results,
+//   start + rounds * per_round + (full rounds * per_k + the last one's share) * K / 1024 + per_mb * MB of results,
 // where a round is as many workgroups as the device holds at a time, and a last round of a few tiles takes per_k_few and one of many up to per_k
 // (the chip's power is the limit: its clock falls as more matrix cores work).  Small tiles are bound by a round's
 // latency and by how fast a compute unit takes in its two operands, large ones by the matrix pipes at the
@@ -254,20 +254,18 @@ struct Config {
   float per_round;  // us
   float per_k;      // us per 1024 reduction bytes of a full round
   float per_k_few;  // ... of a nearly empty one
-  float rate;       // 1e15 operations per second
   float per_mb, per_mb_gate_up;  // us per MB of results, plain ones and gate_up's with its SiLU
   hipError_t (*gate_up)(const DenseParams&, hipStream_t);
   hipError_t (*down)(const DenseParams&, hipStream_t);
 };
-#define MOE_I8_DENSE_STORES(THROUGH, TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, PER_K_FEW, RATE, MB, MB_GU) \
-  {TM, TN, PER_CU, START, ROUND, PER_K, PER_K_FEW, RATE, MB, MB_GU, launch_config<kGateUpSilu, THROUGH, TM, TN, KS, WM, WN, S, WPE>, \
+#define MOE_I8_DENSE_STORES(THROUGH, TM, TN, KS, WM, WN, S, WPE, PER_CU, START, ROUND, PER_K, PER_K_FEW, MB, MB_GU) \
+  {TM, TN, PER_CU, START, ROUND, PER_K, PER_K_FEW, MB, MB_GU, launch_config<kGateUpSilu, THROUGH, TM, TN, KS, WM, WN, S, WPE>, \
    launch_config<kDown, THROUGH, TM, TN, KS, WM, WN, S, WPE>}
 #define MOE_I8_DENSE(...) MOE_I8_DENSE_STORES(true, __VA_ARGS__)
-// The constants are least-squares fits: those of the tiles up to 64 x 64 to 150 problems drawn over 1..8192 rows, 512..16384
-// channels and 512..8192 reduction bytes (rms error of a fit 6-14 %), those of 64 x 128 and 96 x 96 to 320 problems of 250..8192 rows, the others' and the
-// 256-row ones' to 1700 linear layers and 1200 gate_up GEMMs of 500..16384 rows, 768..16384 weight rows and 256..6144 (5-6 %).  Over 400 linear layers and 400
-// gate_up GEMMs that they were not fitted to the choice takes on average 0.39 and 0.33 % longer than the fastest tile; without a charge for the
-// results of the dense tiles, and with one of the wide ones' that did not go by the mode or the reduction, 1.3 and 0.4 %.
+// The constants are least-squares fits: those of the tiles up to 96 x 96 to 2000 linear layers and 1500 gate_up GEMMs of 5..2500 rows, 64..14000 weight rows
+// and 64..8192 (rms error of a fit 6-10 %), the others' and the 256-row ones' to 1700 and 1200 of 500..16384, 768..16384 and 256..6144 (5-6 %).  The choice takes on
+// average 0.2 % longer than the fastest tile over the former; over 400 linear layers and 400 gate_up GEMMs that nothing was fitted to, of the latter's range, 0.38 and
+// 0.33 %.  Without a charge for the results of the dense tiles, and with one of the wide ones' that did not go by the mode or the reduction, it was 0.4 and 1.3 %.
 // The four largest are for problems that fill the chip badly in 128 x 128 tiles (more rounds of less) and in 256 x 256 ones (half a
 // round): linear layers, us without / with them, 1818 rows x 4384 channels x 3008 54.0 / 39.1, 4868 x 3456 x 7680 164 / 138, 6508 x
 // 3984 x 6592 231 / 193, 5755 x 1488 x 1536 33.6 / 28.1.  192 x 192, 192 x 256, 256 x 256, 320 x 192, 128 x 256, 256 x 128, 64 x 192,
@@ -278,19 +276,19 @@ struct Config {
 // 96 x 32 or six of 96 x 32 (three stages as well) it is up to 12 % slower over several rounds; 96 x 64, 64 x 96, 48 x 64, 80 x 64,
 // 48 x 96 and 96 x 128 (two stages only) beside it gain 0.1 % or nothing.
 const Config kConfigs[] = {
-    MOE_I8_DENSE(16, 16, 8, 1, 1, 2, 4, 1, 2.45f, 0.53f, 0.38f, 0.38f, 1e9f, 0.0f, 0.0f),
-    MOE_I8_DENSE(16, 32, 8, 1, 1, 3, 2, 1, 1.49f, 1.46f, 0.58f, 0.58f, 1e9f, 0.0f, 0.0f),
-    MOE_I8_DENSE(32, 32, 8, 1, 1, 2, 2, 1, 1.35f, 1.64f, 0.70f, 0.70f, 1e9f, 0.0f, 0.0f),
-    MOE_I8_DENSE(32, 64, 4, 1, 2, 3, 2, 1, 1.27f, 2.03f, 1.06f, 1.06f, 0.98f, 0.0f, 0.0f),
-    MOE_I8_DENSE(64, 64, 2, 2, 2, 4, 2, 1, 1.56f, 2.08f, 1.38f, 1.38f, 1.12f, 0.0f, 0.0f),
-    MOE_I8_DENSE(64, 128, 2, 2, 2, 3, 2, 1, 1.10f, 2.42f, 2.65f, 2.41f, 1e9f, 0.0f, 0.0f),
-    MOE_I8_DENSE(96, 96, 2, 2, 2, 3, 2, 1, 0.80f, 2.68f, 3.42f, 2.98f, 1e9f, 0.0f, 0.0f),
-    MOE_I8_DENSE(128, 128, 1, 2, 4, 4, 2, 1, 1.57f, 2.24f, 4.52f, 3.76f, 1e9f, 0.05f, 0.19f),
-    MOE_I8_DENSE(128, 128, 1, 2, 2, 2, 2, 2, 2.15f, 1.43f, 7.62f, 5.74f, 1e9f, 0.12f, 0.27f),
-    MOE_I8_DENSE(128, 192, 1, 4, 2, 3, 2, 1, 1.56f, 2.83f, 6.10f, 4.81f, 1e9f, 0.05f, 0.21f),
-    MOE_I8_DENSE(256, 192, 1, 4, 2, 2, 2, 1, 1.45f, 4.51f, 10.25f, 8.34f, 1e9f, 0.07f, 0.22f),
-    MOE_I8_DENSE(192, 320, 1, 4, 2, 2, 2, 1, 1.60f, 5.54f, 11.72f, 10.92f, 1e9f, 0.08f, 0.18f),
-    MOE_I8_DENSE(192, 384, 1, 2, 4, 2, 2, 1, 0.80f, 6.54f, 14.22f, 11.98f, 1e9f, 0.07f, 0.21f),
+    MOE_I8_DENSE(16, 16, 8, 1, 1, 2, 4, 1, 2.72f, 0.49f, 0.35f, 0.54f, 0.51f, 4.37f),
+    MOE_I8_DENSE(16, 32, 8, 1, 1, 3, 2, 1, 1.94f, 1.36f, 0.62f, 0.60f, 0.0f, 2.52f),
+    MOE_I8_DENSE(32, 32, 8, 1, 1, 2, 2, 1, 1.81f, 1.55f, 0.84f, 0.73f, 0.0f, 0.73f),
+    MOE_I8_DENSE(32, 64, 4, 1, 2, 3, 2, 1, 1.64f, 1.75f, 1.37f, 1.15f, 0.03f, 0.23f),
+    MOE_I8_DENSE(64, 64, 2, 2, 2, 4, 2, 1, 1.68f, 1.73f, 1.98f, 1.61f, 0.10f, 0.19f),
+    MOE_I8_DENSE(64, 128, 2, 2, 2, 3, 2, 1, 1.64f, 1.98f, 2.82f, 2.46f, 0.07f, 0.29f),
+    MOE_I8_DENSE(96, 96, 2, 2, 2, 3, 2, 1, 1.68f, 2.12f, 3.17f, 3.11f, 0.14f, 0.47f),
+    MOE_I8_DENSE(128, 128, 1, 2, 4, 4, 2, 1, 1.57f, 2.24f, 4.52f, 3.76f, 0.05f, 0.19f),
+    MOE_I8_DENSE(128, 128, 1, 2, 2, 2, 2, 2, 2.15f, 1.43f, 7.62f, 5.74f, 0.12f, 0.27f),
+    MOE_I8_DENSE(128, 192, 1, 4, 2, 3, 2, 1, 1.56f, 2.83f, 6.10f, 4.81f, 0.05f, 0.21f),
+    MOE_I8_DENSE(256, 192, 1, 4, 2, 2, 2, 1, 1.45f, 4.51f, 10.25f, 8.34f, 0.07f, 0.22f),
+    MOE_I8_DENSE(192, 320, 1, 4, 2, 2, 2, 1, 1.60f, 5.54f, 11.72f, 10.92f, 0.08f, 0.18f),
+    MOE_I8_DENSE(192, 384, 1, 2, 4, 2, 2, 1, 0.80f, 6.54f, 14.22f, 11.98f, 0.07f, 0.21f),
 };
 // The 256-row tiles of the grouped family (one persistent workgroup per compute unit).  Their stores are not hidden behind another round's product: 0.18
 // us per MB, where rows of the result begin inside 64 bytes 0.20 more, up to 0.09 of which a longer reduction hides (5780 rows x 2672 channels x 512:
@@ -299,15 +297,15 @@ const Config kConfigs[] = {
 // 69.5, 4025 x 15536 x 768 89.1 / 76.2; gate_up 2048 x 7936 x 1024 30.4 / 26.6, 6510 x 11264 x 640 81.4 / 72.0, 4096 x 2816 x 4096 58.5 / 58.6; left to the dense
 // tiles: gate_up of 5047 x 1920 x 2304 37.7 / 40.2; wrong by most: 1605 x 13504 x 512 28.1 / 25.3 and, between two
 // dense tiles, 8018 x 7088 x 512 72.4 in 128 x 128 / 63.8 in 192 x 320.
-const Config kWide = {256, 256, 1, 5.99f, 0.13f, 10.29f, 7.13f, 1e9f, 0.18f, 0.41f, nullptr, nullptr};
+const Config kWide = {256, 256, 1, 5.99f, 0.13f, 10.29f, 7.13f, 0.18f, 0.41f, nullptr, nullptr};
 
 // Those tiles of kConfigs that the estimates choose for results of more than kThroughBytes (of 200 000 random ones up to 4 GB: a large
 // result fills the chip with the larger tiles, and 128 x 128 with one workgroup per compute unit and 128 x 192 are for those that do not).
 const Config kLarge[] = {
-    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 2, 2, 2, 2, 2.15f, 1.43f, 7.62f, 5.74f, 1e9f, 0.12f, 0.27f),
-    MOE_I8_DENSE_STORES(false, 256, 192, 1, 4, 2, 2, 2, 1, 1.45f, 4.51f, 10.25f, 8.34f, 1e9f, 0.07f, 0.22f),
-    MOE_I8_DENSE_STORES(false, 192, 320, 1, 4, 2, 2, 2, 1, 1.60f, 5.54f, 11.72f, 10.92f, 1e9f, 0.08f, 0.18f),
-    MOE_I8_DENSE_STORES(false, 192, 384, 1, 2, 4, 2, 2, 1, 0.80f, 6.54f, 14.22f, 11.98f, 1e9f, 0.07f, 0.21f),
+    MOE_I8_DENSE_STORES(false, 128, 128, 1, 2, 2, 2, 2, 2, 2.15f, 1.43f, 7.62f, 5.74f, 0.12f, 0.27f),
+    MOE_I8_DENSE_STORES(false, 256, 192, 1, 4, 2, 2, 2, 1, 1.45f, 4.51f, 10.25f, 8.34f, 0.07f, 0.22f),
+    MOE_I8_DENSE_STORES(false, 192, 320, 1, 4, 2, 2, 2, 1, 1.60f, 5.54f, 11.72f, 10.92f, 0.08f, 0.18f),
+    MOE_I8_DENSE_STORES(false, 192, 384, 1, 2, 4, 2, 2, 1, 0.80f, 6.54f, 14.22f, 11.98f, 0.07f, 0.21f),
 };
 
 float estimate(const Config& c, int mode, int64_t m, int64_t n, int64_t k) {
@@ -316,12 +314,10 @@ float estimate(const Config& c, int mode, int64_t m, int64_t n, int64_t k) {
   const float full = (float)(tiles / room), last = (float)(tiles % room) / (float)room;
   const float rounds = last > 0.0f ? full + 1.0f : full;
   const float turns = full * c.per_k + (last > 0.0f ? c.per_k_few + last * (c.per_k - c.per_k_few) : 0.0f);
-  const float latency = turns * (float)k / 1024.0f;
-  const float ops = (float)(tiles * c.tm * c.tn) * (float)k * 2.0f / (c.rate * 1e9f);
   float per_mb = mode == kGateUpSilu ? c.per_mb_gate_up : c.per_mb;  // (rows that begin inside 64 bytes cost more)
-  if (mode != kGateUpSilu && n % 32 && per_mb > 0.0f) per_mb += &c == &kWide ? 0.195f - 0.121f * (k < 768 ? (float)k / 1024.0f : 0.75f) : 0.022f;
+  if (mode != kGateUpSilu && n % 32) per_mb += &c == &kWide ? 0.195f - 0.121f * (k < 768 ? (float)k / 1024.0f : 0.75f) : 0.022f;
   const float mb = (float)(mode == kGateUpSilu ? m * (n / 2) : m * n) * 2e-6f;
-  return c.start + rounds * c.per_round + (latency > ops ? latency : ops) + per_mb * mb;
+  return c.start + rounds * c.per_round + turns * (float)k / 1024.0f + per_mb * mb;
 }
 
 }  // namespace

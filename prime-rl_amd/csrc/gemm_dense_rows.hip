@@ -245,10 +245,10 @@ const Config kConfigs[] = {
 // takes 0.1 % longer than the faster of the two, 0.2 % in a captured graph (3500 problems); by fits to calls that a host sends one every 3.7 us, which hide
 // how long a kernel of 3 us takes, 5 and 7 %.  us there / here in a graph: 6 x 6272 x 192 5.2 / 3.6, 7 x 4496 x 256 4.8 / 3.3, 16 x 640 x 1280 6.7 / 4.3, 5 x
 // 1792 x 832 3.5 / 4.2, 5 x 3760 x 2368 4.6 / 5.7, 6 x 4080 x 3072 6.3 / 8.2, 5 x 3680 x 576 3.8 / 4.4; wrong by most 6 x 4464 x 4032 9.4 / 10.3 and 8 x 1216 x
-// 1088 4.6 / 4.9.  A quantisation launch adds about 3.0 us and 0.66 per 10^6 elements to the dense kernels' estimate.
+// 1088 4.6 / 4.9.  A quantisation launch adds about 2.6 us and 0.66 per 10^6 elements to the dense kernels' estimate.
 int dense_rows_pick(int64_t m, int n, int k, bool few, float us) {
   if (m < kDenseRowsFrom || (int64_t)n * k >= (1ll << 32) || n % 16 != 0 || k % 64 != 0) return -1;
-  float least = few ? dense_few_estimate(m, n, k) : us + 3.0f + 0.66e-6f * (float)m * (float)k;
+  float least = few ? dense_few_estimate(m, n, k) : us + 2.6f + 0.66e-6f * (float)m * (float)k;
   int best = -1;
   const float kb = (float)k / 1024.0f, cus = (float)device_cu_count();
   for (int i = 0; i < (int)std::size(kConfigs); ++i) {

@@ -25,8 +25,7 @@ def _reached(pra, cases):
 def test_every_tile_of_rows_that_their_workgroups_quantise_is_run(pra):
     linear, gate_up = _reached(pra, _cases(gpu.test_rows_quantised_by_their_tiles, gpu.test_rows_quantised_by_wide_tiles))
     every = {("dense_rows", i, True) for i in range(10)}
-    assert linear >= every and gate_up >= every
-    assert linear - every == {("dense", 0, True)}  # 17 x 1040 x 4096 and 16 x 2544 x 3968; the longest row is held by 16 x 64 x 4096
+    assert linear == every and gate_up >= every
 
 
 def test_every_tile_of_the_dense_kernel_is_run(pra):
